@@ -341,15 +341,17 @@ static int ensure_big(topk_ctx *ctx, uint64_t n) {
     return TOPK_OK;
 }
 
-// One FTE query over objects [0, n) of the columns q points at, results to
-// device pointers (status in the context's result block).  The
-// sample-seeded pipeline runs first; if its guess left too few candidates
-// (STATUS_RETRY) or too many for the buffer (STATUS_OVERFLOW), the
-// exact-prefix pipeline runs, and after an overflow there an n-entry
-// candidate buffer.
-static int fte_run_range(topk_ctx *ctx, uint32_t k, const QCols &q, uint64_t n, uint64_t *d_ids, float *d_sc,
-                         float *d_thr) {
-    uint32_t *d_status = reinterpret_cast<uint32_t *>(ctx->d_res + ctx->res.status_off);
+// One FTE query over objects [0, n) of the columns q points at: ids, scores
+// and threshold to fo (the context's pinned result block, or a shard's list
+// on the device), status and candidate count straight to pinned memory, so
+// the host only waits for the stream.  The sample-seeded pipeline runs first;
+// if its guess left too few candidates (STATUS_RETRY) or too many for the
+// buffer (STATUS_OVERFLOW), the exact-prefix pipeline runs, and after an
+// overflow there an n-entry candidate buffer.
+static int fte_run_range(topk_ctx *ctx, uint32_t k, const QCols &q, uint64_t n, FinalOut fo) {
+    volatile uint32_t *h_status = reinterpret_cast<uint32_t *>(ctx->h_res + ctx->res.status_off);
+    fo.status = reinterpret_cast<uint32_t *>(ctx->h_res + ctx->res.status_off);
+    fo.cand = &ctx->h_state->cand_last;
     Lane &L = ctx->lane[0];
     int mode = ctx->tune.fte_force_exact ? FTE_EXACT : FTE_SAMPLE;
     for (int attempt = 0; attempt < 3; attempt++) {
@@ -357,14 +359,13 @@ static int fte_run_range(topk_ctx *ctx, uint32_t k, const QCols &q, uint64_t n, 
             int rc = ensure_big(ctx, n);
             if (rc) return rc;
         }
-        int rc = fte_enqueue(ctx, L, k, q, d_ids, d_sc, d_thr, d_status, mode, n);
+        ctx->h_state->cand_last = 0;
+        int rc = fte_enqueue(ctx, L, k, q, fo, mode, n);
         if (rc) return rc;
-        TK_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, ctx->res.bytes, hipMemcpyDeviceToHost, L.stream));
-        TK_HIP(hipMemcpyAsync(ctx->h_state, L.st, sizeof(FteState), hipMemcpyDeviceToHost, L.stream));
         TK_HIP(hipStreamSynchronize(L.stream));
-        const uint32_t status = *reinterpret_cast<const uint32_t *>(ctx->h_res + ctx->res.status_off);
+        const uint32_t status = *h_status;
         if (!status) {
-            ctx->stats.candidates += ctx->h_state->cand_last;
+            ctx->stats.candidates += *static_cast<volatile unsigned int *>(&ctx->h_state->cand_last);
             return TOPK_OK;
         }
         TK_HIP(hipMemsetAsync(&L.st->status, 0, sizeof(uint32_t), L.stream));
@@ -383,30 +384,29 @@ static QCols shard_cols(const QCols &q, uint32_t s) {
     return r;
 }
 
-// Runs one FTE query into the context's result block and copies it to the
-// pinned host mirror: one run over the store, or one per id shard and a
-// device merge of their top-k lists.
+// Runs one FTE query into the context's pinned result block: one run over the
+// store, or one per id shard and a device merge of their top-k lists.
 static int fte_run_sync(topk_ctx *ctx, uint32_t k, const QCols &q) {
-    uint64_t *d_ids = reinterpret_cast<uint64_t *>(ctx->d_res + ctx->res.ids_off);
-    float *d_sc = reinterpret_cast<float *>(ctx->d_res + ctx->res.scores_off);
-    float *d_thr = reinterpret_cast<float *>(ctx->d_res + ctx->res.thr_off);
-    uint32_t *d_status = reinterpret_cast<uint32_t *>(ctx->d_res + ctx->res.status_off);
+    const FinalOut fo{reinterpret_cast<uint64_t *>(ctx->h_res + ctx->res.ids_off),
+                      reinterpret_cast<float *>(ctx->h_res + ctx->res.scores_off),
+                      reinterpret_cast<float *>(ctx->h_res + ctx->res.thr_off),
+                      reinterpret_cast<uint32_t *>(ctx->h_res + ctx->res.status_off)};
     ctx->stats.fallback = 0;
     ctx->stats.retried = 0;
     ctx->stats.fte_fallback = 0;
     ctx->stats.candidates = 0;
     const uint32_t S = id_shards(ctx->n);
-    if (S == 1) return fte_run_range(ctx, k, q, ctx->n, d_ids, d_sc, d_thr);
+    if (S == 1) return fte_run_range(ctx, k, q, ctx->n, fo);
     Lane &L = ctx->lane[0];
     for (uint32_t s = 0; s < S; s++) {
         const uint64_t n0 = (uint64_t)s * ID_SHARD, ns = ctx->n - n0 < ID_SHARD ? ctx->n - n0 : ID_SHARD;
-        const int rc = fte_run_range(ctx, k, shard_cols(q, s), ns, L.sh_ids + (uint64_t)s * TOPK_MAX_K,
-                                     L.sh_scores + (uint64_t)s * TOPK_MAX_K, nullptr);
+        const int rc = fte_run_range(ctx, k, shard_cols(q, s), ns,
+                                     FinalOut{L.sh_ids + (uint64_t)s * TOPK_MAX_K,
+                                              L.sh_scores + (uint64_t)s * TOPK_MAX_K, nullptr, nullptr});
         if (rc) return rc;
     }
-    shard_merge_enqueue(L.stream, L.sh_ids, L.sh_scores, ctx->n, S, k, FinalOut{d_ids, d_sc, d_thr, d_status});
+    shard_merge_enqueue(L.stream, L.sh_ids, L.sh_scores, ctx->n, S, k, fo);
     TK_HIP(hipGetLastError());
-    TK_HIP(hipMemcpyAsync(ctx->h_res, ctx->d_res, ctx->res.bytes, hipMemcpyDeviceToHost, L.stream));
     TK_HIP(hipStreamSynchronize(L.stream));
     return TOPK_OK;
 }
@@ -443,14 +443,16 @@ int topk_fte_async(topk_ctx *ctx, uint32_t k, uint8_t qq, const float *weights, 
     const uint32_t lanes = ctx->timing_on ? 1u : (uint32_t)ctx->tune.lanes;
     Lane &L = ctx->lane[ctx->next_lane % lanes];
     ctx->next_lane = (ctx->next_lane + 1) % lanes;
-    const int mode = ctx->tune.fte_force_exact ? FTE_EXACT : FTE_SAMPLE;
+    const int mode = ctx->tune.fte_force_exact ? FTE_EXACT : FTE_QUEUED;
     const uint32_t S = id_shards(ctx->n);
-    if (S == 1) return fte_enqueue(ctx, L, k, q, d_ids, d_scores, nullptr, nullptr, mode);
+    if (S == 1) return fte_enqueue(ctx, L, k, q, FinalOut{d_ids, d_scores, nullptr, nullptr}, mode);
     // per id shard into the lane's shard lists, then the merge
     for (uint32_t s = 0; s < S; s++) {
         const uint64_t n0 = (uint64_t)s * ID_SHARD, ns = ctx->n - n0 < ID_SHARD ? ctx->n - n0 : ID_SHARD;
-        rc = fte_enqueue(ctx, L, k, shard_cols(q, s), L.sh_ids + (uint64_t)s * TOPK_MAX_K,
-                         L.sh_scores + (uint64_t)s * TOPK_MAX_K, nullptr, nullptr, mode, ns);
+        rc = fte_enqueue(ctx, L, k, shard_cols(q, s),
+                         FinalOut{L.sh_ids + (uint64_t)s * TOPK_MAX_K, L.sh_scores + (uint64_t)s * TOPK_MAX_K, nullptr,
+                                  nullptr},
+                         mode, ns);
         if (rc) return rc;
     }
     shard_merge_enqueue(L.stream, L.sh_ids, L.sh_scores, ctx->n, S, k, FinalOut{d_ids, d_scores, nullptr, nullptr});

@@ -14,24 +14,47 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 
+// Wave-wide scans and reductions by DPP: four row shifts inside the 16-lane
+// rows, then two row broadcasts across them (about 60 cycles; the same steps
+// as LDS permutes take about 130 cycles each).  All 64 lanes take part.
+// Lane l's value of the next step; zero where the pattern has no source.
+#define TK_DPP(v, ctrl, rows) ((uint32_t)__builtin_amdgcn_update_dpp(0, (int)(v), ctrl, rows, 0xF, false))
+#define TK_DPP_STEPS(STEP)                                                    \
+    STEP(0x111, 0xF) /* row_shr 1 */ STEP(0x112, 0xF) /* row_shr 2 */         \
+    STEP(0x114, 0xF) /* row_shr 4 */ STEP(0x118, 0xF) /* row_shr 8 */         \
+    STEP(0x142, 0xA) /* row_bcast 15 into rows 1, 3 */                        \
+    STEP(0x143, 0xC) /* row_bcast 31 into rows 2, 3 */
+
 // Inclusive prefix sum across the 64 lanes of a wave.
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
-    const uint32_t l = lane_id();
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        uint32_t t = __shfl_up(v, o, 64);
-        if (l >= (uint32_t)o) v += t;
-    }
+#define TK_STEP(ctrl, rows) v += TK_DPP(v, ctrl, rows);
+    TK_DPP_STEPS(TK_STEP)
+#undef TK_STEP
     return v;
 }
 
-__device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        uint64_t t = __shfl_xor(v, o, 64);
-        v = t < v ? t : v;
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+#define TK_STEP(ctrl, rows)                       \
+    {                                             \
+        const uint32_t t = TK_DPP(v, ctrl, rows); \
+        v = t > v ? t : v;                        \
     }
-    return v;
+    TK_DPP_STEPS(TK_STEP)
+#undef TK_STEP
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// The high halves' maximum, then the largest low half among its holders.
+__device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
+    const uint32_t hi = wave_max_u32((uint32_t)(v >> 32));
+    const uint32_t lo = wave_max_u32((uint32_t)(v >> 32) == hi ? (uint32_t)v : 0u);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+__device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) { return ~wave_max_u64(~v); }
+
+__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan(v), 63);
 }
 
 // The last index i in [lo, hi) with key(i) <= t (key non-decreasing, key(lo)
@@ -51,19 +74,29 @@ __device__ __forceinline__ uint32_t wave_last_le(Key key, uint32_t lo, uint32_t 
     return lo;
 }
 
-__device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
+// Removes the largest of the ranking keys the wave's lanes hold (NPL per
+// lane, score half in hi, id half in lo; hi = 0: none) and returns it on
+// every lane; 0 once none is left.  Keys are distinct.
+template <int NPL>
+__device__ __forceinline__ uint64_t wave_pop_max(uint32_t (&hi)[NPL], const uint32_t (&lo)[NPL]) {
+    uint32_t m = 0;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        uint64_t t = __shfl_xor(v, o, 64);
-        v = t > v ? t : v;
+    for (int j = 0; j < NPL; j++) m = hi[j] > m ? hi[j] : m;
+    const uint32_t M = wave_max_u32(m);
+    if (M == 0) return 0;
+    uint32_t l = 0;
+#pragma unroll
+    for (int j = 0; j < NPL; j++) l = hi[j] == M && lo[j] > l ? lo[j] : l;
+    uint64_t b = __ballot(m == M);
+    if (b & (b - 1)) {  // several lanes hold the score: the largest id half
+        const uint32_t L = wave_max_u32(m == M ? l : 0u);
+        b = __ballot(m == M && l == L);
     }
-    return v;
-}
-
-__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
+    const uint32_t leader = (uint32_t)__builtin_ctzll(b);
+    const uint32_t L = (uint32_t)__builtin_amdgcn_readlane((int)l, (int)leader);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    for (int j = 0; j < NPL; j++) hi[j] = hi[j] == M && lo[j] == L && lane_id() == leader ? 0u : hi[j];
+    return ((uint64_t)M << 32) | L;
 }
 
 // Streaming 128-bit load that bypasses cache residency (data read once).
@@ -71,12 +104,14 @@ __device__ __forceinline__ f4 ld_stream(const float *p) {
     return __builtin_nontemporal_load(reinterpret_cast<const f4 *>(p));
 }
 
-// LDS scratch of the workgroup selection (histogram for up to 11-bit digits).
-struct SelectScratch {
-    uint32_t hist[2048];
+// LDS scratch of the workgroup selection (a histogram of BINS digits).
+template <int BINS>
+struct SelectScratchT {
+    uint32_t hist[BINS];
     uint32_t digit, need, bcnt, counter;
     unsigned long long kmin, kmax;
 };
+using SelectScratch = SelectScratchT<2048>;  // up to 11-bit digits
 
 // How many of the n keys a[0..n) (LDS, every lane reading the same word)
 // are above x and above y: eight reads in flight per step, so the loop
@@ -132,8 +167,8 @@ struct MemKeys {
 };
 
 // Block-wide min / max of u64 (all threads call; result on every thread).
-template <int BS>
-__device__ __forceinline__ void block_minmax(uint64_t &lo, uint64_t &hi, SelectScratch &s) {
+template <int BS, class Scratch>
+__device__ __forceinline__ void block_minmax(uint64_t &lo, uint64_t &hi, Scratch &s) {
     lo = wave_min_u64(lo);
     hi = wave_max_u64(hi);
     if (BS == 64) return;
@@ -160,9 +195,10 @@ __device__ __forceinline__ void block_minmax(uint64_t &lo, uint64_t &hi, SelectS
 // a lane prefix scan.  Rounds stop when the candidate set is one value, when
 // the k-th is its maximum, or when the whole set is inside the top k (then
 // the k-th is its minimum).
-template <int BS, class Src, int DB = 8>
-__device__ uint64_t block_kth_largest(const Src &src, uint32_t setcnt, uint32_t k, SelectScratch &s) {
+template <int BS, class Src, int DB = 8, class Scratch = SelectScratch>
+__device__ uint64_t block_kth_largest(const Src &src, uint32_t setcnt, uint32_t k, Scratch &s) {
     static_assert(DB >= 6 && DB <= 11, "digit width");
+    static_assert(sizeof(s.hist) >= sizeof(uint32_t) << DB, "one bin per digit");
     constexpr uint32_t NB = 1u << DB, PER = NB / 64;
     const uint32_t tid = threadIdx.x;
     uint64_t prefix = 0, mask = 0;
@@ -225,8 +261,8 @@ __device__ uint64_t block_kth_largest(const Src &src, uint32_t setcnt, uint32_t 
 // Writes every non-zero key >= thr of the source to out[] (order
 // unspecified) with a wave-aggregated LDS counter; returns the count.  All
 // threads of the block must call.
-template <int BS, class Src, class Out>
-__device__ uint32_t block_gather_ge(const Src &src, uint64_t thr, Out out, SelectScratch &s) {
+template <int BS, class Src, class Out, class Scratch>
+__device__ uint32_t block_gather_ge(const Src &src, uint64_t thr, Out out, Scratch &s) {
     if (threadIdx.x == 0) s.counter = 0;
     __syncthreads();
     src.for_each([&](uint64_t key) {
@@ -299,23 +335,6 @@ __device__ uint32_t block_excl_scan(uint32_t v, uint32_t *wave_sums, uint32_t *t
     const uint32_t r = wave_sums[w] + incl - v;
     __syncthreads();
     return r;
-}
-
-// The kth (1 <= kth <= 8) largest of the keys the wave's lanes hold (NPL
-// per lane; distinct except zeros), by kth rounds of a wave max.  Every lane
-// gets the result; keys below it stay in v, the chosen ones are zeroed.
-template <int NPL>
-__device__ __forceinline__ uint64_t wave_kth_largest(uint64_t (&v)[NPL], uint32_t kth) {
-    uint64_t mx = 0;
-    for (uint32_t r = 0; r < kth; r++) {
-        uint64_t lm = 0;
-#pragma unroll
-        for (int j = 0; j < NPL; j++) lm = v[j] > lm ? v[j] : lm;
-        mx = wave_max_u64(lm);
-#pragma unroll
-        for (int j = 0; j < NPL; j++) v[j] = v[j] == mx ? 0ull : v[j];
-    }
-    return mx;
 }
 
 // Sorts the got distinct keys in[0..got) descending into out[] by rank

@@ -1,26 +1,28 @@
 // FTE (full-table evaluation) top-k on gfx950.
 //
 // Reference: cpu/TPAc.h:118-358 (scoring order, heap semantics) and the
-// empty GPU stub gpu/GFA.h:47-50.  A query is three launches on the
-// context's stream with no host round trip:
+// empty GPU stub gpu/GFA.h:47-50.  A query is one launch on the context's
+// stream (fte_stream_kernel; exact mode: a seed launch before it):
 //
-//  1. seed pass    (fte_seed_kernel): a few 4096-object chunks are scored;
-//     each block keeps its top ks keys (register-resident radix select) and
-//     the last block to finish selects the ks-th largest of the block
-//     winners: tau.
-//       - sample mode: 16 chunks spread over the id range, small ks; tau is
-//         a guess whose safety is checked at the end (>= k candidates).
-//       - exact mode:  contiguous chunks [0, P), ks = k; the prefix's k-th
-//         key is a proven lower bound of the global k-th key, and the
+//  1. threshold tau, a ranking key:
+//       - own sample (stores up to 2^19 objects, calls that re-run on a bad
+//         guess): every workgroup takes the same sample of 4096 objects and
+//         the same element of it.
+//       - shared sample: the first 32 workgroups score up to 128 chunks of
+//         1024 objects spread over the id range and publish their best; tau
+//         is the ks-th largest of the whole sample.  The other workgroups
+//         have their first tile in flight meanwhile.  A guess like the own
+//         sample, checked at the end (>= k candidates).
+//       - exact (fte_seed_kernel): contiguous chunks [0, P); the prefix's
+//         k-th key is a proven lower bound of the global k-th key, and the
 //         prefix's top k are written to the candidate list.
-//  2. stream pass  (fte_stream_kernel): each block streams whole tiles of
-//     contiguous column segments, scores stay in registers, and keys >= tau
-//     go to the block's own candidate slots (wave ballot + one LDS atomic
-//     per wave; no global atomic).  No barrier in the loop: a pure HBM
-//     stream.
-//  3. final select (fte_final_kernel): one workgroup scans the per-block
-//     counts, checks the candidate total, selects the exact top k and
-//     rank-sorts them.
+//  2. stream: each workgroup streams whole tiles of contiguous column
+//     segments, scores stay in registers, and keys >= tau go to the
+//     workgroup's own candidate slots (wave ballot + one LDS atomic per
+//     wave; no global atomic).  No barrier in the loop: a pure HBM stream.
+//  3. select: the last workgroup to finish scans the per-workgroup counts,
+//     checks the candidate total, selects the exact top k and writes them
+//     best first, to device memory or straight to pinned host memory.
 //
 // Exactness: with c >= k candidates of key >= tau, every other object has a
 // key < tau and is beaten by c >= k objects, so the top k are among the
@@ -29,6 +31,7 @@
 // the exact mode, with an n-entry buffer if needed.
 #include <string.h>
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -40,35 +43,76 @@ namespace topk {
 
 constexpr int SEED_BS = 256;
 constexpr uint32_t SEED_TILE = 4096;     // exact mode: objects per seed block (16 per thread)
-constexpr uint32_t SAMPLE_TILE = 1024;   // sample mode: objects per seed block (4 per thread)
-constexpr uint32_t SAMPLE_CHUNKS = 128;  // sample mode: 128 x 1024 objects spread over the ids
-constexpr int STREAM_BS = 256;
-constexpr int FINAL_BS = 512;            // regular final select
+constexpr uint32_t SAMPLE_TILE = 1024;   // shared sample: objects per chunk
+constexpr uint32_t SAMPLE_CHUNKS = 128;  // shared sample: chunks at most, spread over the ids
+constexpr uint32_t SAMPLE_WGS = 32;      // workgroups that take the shared sample
+constexpr uint32_t SAMPLE_MAX_W = SAMPLE_WIN / SAMPLE_WGS;  // winners each of them publishes at most
+constexpr int STREAM_BS = 1024;
+constexpr int STREAM_NW = STREAM_BS / 64;
+constexpr int SAMPLE_VEC = SAMPLE_CHUNKS * SAMPLE_TILE / (SAMPLE_WGS * STREAM_BS * 4);  // float4 per thread
+constexpr int OWN_VEC = 4096 / (STREAM_BS * 4);  // own sample: float4 vectors per thread
+constexpr uint32_t OWN_OBJS = STREAM_BS * 4 * OWN_VEC;
+constexpr uint32_t OWN_SPOTS = OWN_OBJS / 16;   // own sample: 256 runs of 16 objects, one 64-byte line per column each
+constexpr uint64_t OWN_MAX_N = 1ull << 19;      // stores up to this size take their own sample
+constexpr uint32_t FUSE_CAP_MIN = 1024, FUSE_CAP_MAX = 4096;  // candidates the last stream workgroup selects in LDS
+constexpr uint32_t STREAM_GRID = 256;    // stream workgroups at most (one per CU), unless tuned
+constexpr int FINAL_BS = 512;            // separate final select
 constexpr int FINAL_KPT = 16;            // candidate keys per final-select thread (8192 in registers)
-constexpr uint32_t SEED_WAVE_MAX = 512;  // seed winners a stream wave can reduce to tau itself
 constexpr int FLAT_BS = 1024;            // fallback final select over a large flat list
+
+// Runtime-width scores of VPT float4 vectors v, v + step, ...: G columns'
+// loads are issued before the first of them is used (a loop of one column
+// per step waited on memory once per term), terms in query order; real-data
+// scores divide after every term.
+template <bool NT>
+__device__ __forceinline__ f4 ld_col(const float *p) {
+    if constexpr (NT) return ld_stream(p);
+    else return *reinterpret_cast<const f4 *>(p);
+}
+template <int VPT, bool NT = true, int G = 8>
+__device__ __forceinline__ void score_wide(const QCols &q, uint64_t v, uint32_t step, f4 (&acc)[VPT]) {
+#pragma unroll
+    for (int u = 0; u < VPT; u++) acc[u] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t j0 = 0; j0 < q.m; j0 += G) {
+        f4 x[G][VPT];
+#pragma unroll
+        for (int t = 0; t < G; t++)
+            if (j0 + t < q.m) {
+#pragma unroll
+                for (int u = 0; u < VPT; u++) x[t][u] = ld_col<NT>(q.col[j0 + t] + (v + u * step) * 4);
+            }
+#pragma unroll
+        for (int t = 0; t < G; t++)
+            if (j0 + t < q.m) {
+#pragma unroll
+                for (int u = 0; u < VPT; u++) {
+                    f4 p = x[t][u] * q.w[j0 + t];
+                    acc[u] = acc[u] + p;
+                    if (q.div != 0.0f) acc[u] = acc[u] / q.div;
+                }
+            }
+    }
+}
 
 // Score of the 4 objects of float4 vector v: acc = fl(acc + fl(x*w)) in
 // attribute order, accumulator starting at +0 (cpu/TPAc.h:129-142).
-template <int M>
+// NT: nontemporal loads (data read once).
+template <int M, bool NT = true>
 __device__ __forceinline__ f4 score_vec(const QCols &q, uint64_t v) {
     f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
     if constexpr (M > 0) {
         f4 x[M];
 #pragma unroll
-        for (int j = 0; j < M; j++) x[j] = ld_stream(q.col[j] + v * 4);
+        for (int j = 0; j < M; j++) x[j] = ld_col<NT>(q.col[j] + v * 4);
 #pragma unroll
         for (int j = 0; j < M; j++) {
             f4 p = x[j] * q.w[j];
             acc = acc + p;
         }
     } else {
-        for (uint32_t j = 0; j < q.m; j++) {
-            f4 xv = ld_stream(q.col[j] + v * 4);
-            f4 p = xv * q.w[j];
-            acc = acc + p;
-            if (q.div != 0.0f) acc = acc / q.div;
-        }
+        f4 s1[1];
+        score_wide<1, NT, 16>(q, v, 0, s1);
+        acc = s1[0];
     }
     return acc;
 }
@@ -78,7 +122,7 @@ __device__ __forceinline__ f4 score_vec(const QCols &q, uint64_t v) {
 // ---------------------------------------------------------------------------
 // Block b scores objects [b*chunk_stride, +256*OPT) of the first n_eff objects.
 // total_valid = number of non-zero keys the blocks deposit in blk.
-template <int M, int OPT, bool MERGE>
+template <int M, int OPT>
 __global__ __launch_bounds__(SEED_BS) void fte_seed_kernel(QCols q, uint64_t n_eff, uint64_t chunk_stride,
                                                            uint32_t ks, uint32_t total_valid,
                                                            uint64_t *__restrict__ blk,
@@ -110,8 +154,6 @@ __global__ __launch_bounds__(SEED_BS) void fte_seed_kernel(QCols q, uint64_t n_e
     uint64_t *out = blk + (uint64_t)blockIdx.x * ks;
     const uint32_t got = block_gather_ge<SEED_BS>(rk, thr, out, ss);
     for (uint32_t i = got + tid; i < ks; i += SEED_BS) out[i] = 0;
-    if constexpr (!MERGE) return;  // sample mode: each stream wave derives tau from blk itself
-
     // the last block to arrive merges the block winners
     __threadfence();
     __syncthreads();
@@ -142,13 +184,13 @@ struct SlotView {
     uint32_t npre;
     const uint64_t *keys;
     uint32_t slot;
-    const uint32_t *off;   // nblk + 2 entries; region nblk is the spill region
-    uint32_t nblk;
+    const uint32_t *off;
+    uint32_t nblk, total;  // keys in slots; the spill region's follow
     const uint64_t *spill;
     __device__ __forceinline__ uint64_t get(uint32_t p) const {
         if (p < npre) return pre[p];
         const uint32_t q = p - npre;
-        if (q >= off[nblk]) return spill[q - off[nblk]];
+        if (q >= total) return spill[q - total];
         uint32_t lo = 0, hi = nblk;  // largest b with off[b] <= q
         while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) >> 1;
@@ -160,91 +202,539 @@ struct SlotView {
 };
 
 
-// The ks-th largest of the nseed (<= 512) seed winners, computed by one wave.
-__device__ __forceinline__ uint64_t wave_seed_tau(const uint64_t *__restrict__ seed, uint32_t nseed,
-                                                  uint32_t ks) {
-    uint64_t v[8];
+// The ks-th largest of the keys the wave's lanes hold (NPL per lane; 0: no
+// key) -- 0 with fewer than ks keys -- by bisection on ballot counts, score
+// half first, then the id half among the keys that share the score (only if
+// several do).  32 steps of NPL compares whatever ks is (rounds of wave
+// maxima cost ks x 0.4 us).
+template <int NPL>
+__device__ __forceinline__ uint64_t wave_kth_bisect(const uint64_t (&v)[NPL], uint32_t ks) {
+    uint32_t t = 0;
+    for (int b = 31; b >= 0; b--) {
+        const uint32_t c = t | (1u << b);
+        uint32_t cnt = 0;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const uint32_t i = j * 64 + lane_id();
-        v[j] = i < nseed ? seed[i] : 0ull;
+        for (int j = 0; j < NPL; j++) cnt += (uint32_t)__popcll(__ballot((uint32_t)(v[j] >> 32) >= c));
+        if (cnt >= ks) t = c;
     }
-    return wave_kth_largest<8>(v, ks);
-}
-
-// Sample mode seed with few winners per block (ks <= 4): block b scores the
-// 1024 objects at b*chunk_stride, every wave keeps its top ks by wave-max
-// rounds, and wave 0 reduces the 4*ks wave winners to the block's top ks.
-// No radix select, one barrier.
-template <int M>
-__global__ __launch_bounds__(SEED_BS) void fte_sample_kernel(QCols q, uint64_t n, uint64_t chunk_stride,
-                                                             uint32_t ks, uint64_t *__restrict__ blk) {
-    __shared__ uint64_t wtop[SEED_BS / 64][4];
-    const uint32_t tid = threadIdx.x, w = tid / 64;
-    const uint64_t v = (uint64_t)blockIdx.x * chunk_stride / 4 + tid;
-    const f4 s = score_vec<M>(q, v);
-    uint64_t keys[4];
+    if (t == 0) return 0;
+    uint32_t above = 0, equal = 0;
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const uint64_t id = v * 4 + e;
-        keys[e] = id < n ? rkey(s[e], (uint32_t)id) : 0ull;
+    for (int j = 0; j < NPL; j++) {
+        above += (uint32_t)__popcll(__ballot((uint32_t)(v[j] >> 32) > t));
+        equal += (uint32_t)__popcll(__ballot((uint32_t)(v[j] >> 32) == t));
     }
-    for (uint32_t r = 0; r < ks; r++) {
-        uint64_t lm = 0;
+    const uint32_t need = ks - above;  // >= 1
+    uint32_t lo = 0;
+    if (equal == need && equal == 1) {
+        // one key holds the score: its id half
+        uint32_t mine = 0;
 #pragma unroll
-        for (int e = 0; e < 4; e++) lm = keys[e] > lm ? keys[e] : lm;
-        const uint64_t mx = wave_max_u64(lm);
+        for (int j = 0; j < NPL; j++) mine |= (uint32_t)(v[j] >> 32) == t ? (uint32_t)v[j] : 0u;
 #pragma unroll
-        for (int e = 0; e < 4; e++) keys[e] = keys[e] == mx ? 0ull : keys[e];
-        if (lane_id() == 0) wtop[w][r] = mx;
-    }
-    __syncthreads();
-    if (w == 0) {
-        uint64_t c[1];
-        const uint32_t i = lane_id();
-        c[0] = i < (SEED_BS / 64) * ks ? wtop[i / ks][i % ks] : 0ull;
-        for (uint32_t r = 0; r < ks; r++) {
-            const uint64_t mx = wave_max_u64(c[0]);
-            c[0] = c[0] == mx ? 0ull : c[0];
-            if (i == 0) blk[(uint64_t)blockIdx.x * ks + r] = mx;
+        for (int o = 32; o > 0; o >>= 1) mine |= (uint32_t)__shfl_xor((int)mine, o, 64);
+        lo = mine;
+    } else {
+        for (int b = 31; b >= 0; b--) {
+            const uint32_t c = lo | (1u << b);
+            uint32_t cnt = 0;
+#pragma unroll
+            for (int j = 0; j < NPL; j++)
+                cnt += (uint32_t)__popcll(__ballot((uint32_t)(v[j] >> 32) == t && (uint32_t)v[j] >= c));
+            if (cnt >= need) lo = c;
         }
     }
+    return ((uint64_t)t << 32) | lo;
+}
+
+__device__ __forceinline__ void store_agent(uint64_t *p, uint64_t v) {
+    __hip_atomic_store(reinterpret_cast<unsigned long long *>(p), (unsigned long long)v, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The ks-th largest of the wave's keys (hi / lo as wave_pop_max's): rounds of
+// maxima for a shallow rank (about 0.1 us each), else bisection.
+template <int NPL>
+__device__ __forceinline__ uint64_t wave_kth(uint32_t (&hi)[NPL], const uint32_t (&lo)[NPL], uint32_t ks) {
+    uint64_t r = 0;
+    if (ks <= 16) {
+        for (uint32_t i = 0; i < ks; i++) r = wave_pop_max<NPL>(hi, lo);
+        return r;
+    }
+    uint64_t v[NPL];
+#pragma unroll
+    for (int j = 0; j < NPL; j++) v[j] = hi[j] ? ((uint64_t)hi[j] << 32) | lo[j] : 0ull;
+    return wave_kth_bisect<NPL>(v, ks);
+}
+
+// The wave's W (<= 64) largest keys, largest first, key i on lane i (0: fewer).
+template <int NPL>
+__device__ __forceinline__ uint64_t wave_top(uint32_t (&hi)[NPL], const uint32_t (&lo)[NPL], uint32_t W) {
+    uint64_t mine = 0;
+    for (uint32_t i = 0; i < W; i++) {
+        const uint64_t key = wave_pop_max<NPL>(hi, lo);
+        mine = lane_id() == i ? key : mine;
+    }
+    return mine;
+}
+
+// Shared sample, producer side: workgroup p < wgs scores chunks p, p +
+// SAMPLE_WGS, ... of the sample (1024 objects each, at multiples of
+// chunk_stride) and publishes its W largest keys at st->win[p * W ...].
+// Producers are the workgroups with the lowest indexes, which are
+// dispatched first, and wait for nobody before they have published.
+struct SampleScratch {
+    uint64_t keys[STREAM_NW * SAMPLE_MAX_W];
+};
+template <int M>
+__device__ __forceinline__ void sample_publish(const QCols &q, uint64_t n, uint32_t chunks, uint64_t chunk_stride,
+                                               uint32_t W, FteState *__restrict__ st, SampleScratch &sc) {
+    const uint32_t tid = threadIdx.x, wave = tid / 64, lane = lane_id();
+    constexpr uint32_t PER = STREAM_BS * 4 / SAMPLE_TILE;  // chunks per step of the workgroup
+    {
+        uint32_t hi[4 * SAMPLE_VEC], lo[4 * SAMPLE_VEC];
+#pragma unroll
+        for (int u = 0; u < SAMPLE_VEC; u++) {
+            const uint32_t c = blockIdx.x + (u * PER + tid / (SAMPLE_TILE / 4)) * SAMPLE_WGS;
+            const uint64_t v = (c < chunks ? c * chunk_stride : 0ull) / 4 + tid % (SAMPLE_TILE / 4);
+            const f4 s = score_vec<(M > 8 ? 0 : M)>(q, v);  // 16 columns at once would spill
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint64_t id = v * 4 + e;
+                hi[u * 4 + e] = c < chunks && id < n ? okey(s[e]) : 0u;
+                lo[u * 4 + e] = 0xFFFFFFFFu - (uint32_t)id;
+            }
+        }
+        const uint64_t mine = wave_top<4 * SAMPLE_VEC>(hi, lo, W);
+        if (lane < W) sc.keys[wave * W + lane] = mine;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        constexpr int NB = STREAM_NW * SAMPLE_MAX_W / 64;
+        uint32_t hi[NB], lo[NB];
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const uint32_t i = j * 64 + lane;
+            const uint64_t v = i < STREAM_NW * W ? sc.keys[i] : 0ull;
+            hi[j] = (uint32_t)(v >> 32);
+            lo[j] = (uint32_t)v;
+        }
+        const uint64_t mine = wave_top<NB>(hi, lo, W);
+        if (lane < W) store_agent(reinterpret_cast<uint64_t *>(&st->win[blockIdx.x * W + lane]), mine ? mine : 1ull);
+    }
+    __syncthreads();
+}
+
+// Consumer side, one wave: polls the winners until every one is there (a
+// winner is its own flag: a store and a load apart, where a counter would
+// add two more trips to memory) and returns the ks-th largest.  The wait is
+// bounded: should it run out, a threshold of 0 admits every object and the
+// candidate count settles what happens.
+constexpr uint32_t SAMPLE_SPINS = 1u << 20;
+__device__ __forceinline__ uint64_t sample_tau(FteState *__restrict__ st, uint32_t nwin, uint32_t ks) {
+    constexpr int NPL = SAMPLE_WIN / 64;
+    for (uint32_t s = 0; s < SAMPLE_SPINS; s++) {
+        uint32_t hi[NPL], lo[NPL];
+        bool all = true;
+#pragma unroll
+        for (int j = 0; j < NPL; j++) {
+            const uint32_t i = j * 64 + lane_id();
+            uint64_t v = 0;
+            if (i < nwin) {
+                v = __hip_atomic_load(&st->win[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                all = all && v != 0;
+            }
+            hi[j] = (uint32_t)(v >> 32);
+            lo[j] = (uint32_t)v;
+        }
+        if (!__ballot(!all)) return wave_kth<NPL>(hi, lo, ks);
+        __builtin_amdgcn_s_sleep(8);
+    }
+    return 0;
+}
+
+// Own sample: tau of a stream workgroup from the same OWN_OBJS objects in
+// every workgroup -- OWN_SPOTS runs of 16 objects at the starts of equal
+// strata of the store (each wave's runs alternate over the whole range) --
+// as the ks-th largest of their keys, from each wave's W largest.  The id
+// half is widened to the end of the stratum the key lies in: among tied
+// scores a run's ids are consecutive, and the key of one of them alone would
+// admit only that run's ids.
+constexpr uint32_t OWN_MAX_W = 32;
+struct OwnScratch {
+    uint64_t keys[STREAM_NW * OWN_MAX_W];
+    uint64_t tau;
+};
+template <int M>
+__device__ __forceinline__ uint64_t own_sample_tau(const QCols &q, uint64_t n, uint32_t ks, OwnScratch &os) {
+    const uint32_t wave = threadIdx.x / 64, lane = lane_id();
+    const uint32_t lines = (uint32_t)((n + 15) / 16);
+    const uint32_t W = ks < 8 + ks / 4 ? ks : (8 + ks / 4 < OWN_MAX_W ? 8 + ks / 4 : OWN_MAX_W);
+    {
+        uint32_t hi[4 * OWN_VEC], lo[4 * OWN_VEC];
+#pragma unroll
+        for (int u = 0; u < OWN_VEC; u++) {
+            const uint32_t spot = lane / 4 * (STREAM_NW * OWN_VEC) + wave * OWN_VEC + u;
+            const uint32_t v = (uint32_t)((uint64_t)spot * lines / OWN_SPOTS) * 4 + (lane & 3);
+            const f4 s = score_vec<(M > 8 ? 0 : M), false>(q, v);  // every workgroup reads them: cached
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t o = v * 4 + e;
+                hi[u * 4 + e] = o < n ? okey(s[e]) : 0u;
+                lo[u * 4 + e] = 0xFFFFFFFFu - o;
+            }
+        }
+        const uint64_t mine = wave_top<4 * OWN_VEC>(hi, lo, W);
+        if (lane < W) os.keys[wave * W + lane] = mine;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        constexpr int NPL = STREAM_NW * OWN_MAX_W / 64;
+        uint32_t hi[NPL], lo[NPL];
+#pragma unroll
+        for (int j = 0; j < NPL; j++) {
+            const uint32_t i = j * 64 + lane;
+            const uint64_t v = i < STREAM_NW * W ? os.keys[i] : 0ull;
+            hi[j] = (uint32_t)(v >> 32);
+            lo[j] = (uint32_t)v;
+        }
+        uint64_t tau = wave_kth<NPL>(hi, lo, ks);
+        if (tau) {
+            const uint32_t id = rkey_id(tau);
+            const uint64_t next = (uint64_t)(id / 16) * OWN_SPOTS / lines + 1;  // the next run
+            const uint64_t end = next * lines / OWN_SPOTS * 16;
+            if (end > id) tau = (tau & ~0xFFFFFFFFull) | (0xFFFFFFFFu - (uint32_t)end);
+        }
+        if (lane == 0) os.tau = tau;
+    }
+    __syncthreads();
+    return os.tau;
 }
 
 // ---------------------------------------------------------------------------
 // 2. stream pass
 // ---------------------------------------------------------------------------
-// Each block streams whole tiles of TILE = 1024*VPT objects: for every
+constexpr uint32_t FUSE_BINS = 1024;
+constexpr uint32_t FUSE_BIN_MAX = 128;  // keys of one bin ranked against each other
+struct FuseScratch {
+    uint32_t bins[FUSE_BINS];
+    SelectScratchT<256> rs;
+    uint64_t wlo[STREAM_NW], whi[STREAM_NW];
+    uint32_t crowded;     // an interval too full to rank by pairs
+    uint32_t cut, ncut;   // the interval holding the k-th key, and the keys up to its end
+};
+
+// Writes the first want keys, best first, and sentinels up to k.
+template <int BS>
+__device__ __forceinline__ void emit_sorted(const uint64_t *sorted, uint32_t want, uint32_t k, const FinalOut &fo) {
+    for (uint32_t i = threadIdx.x; i < k; i += BS) {
+        const uint64_t x = i < want ? sorted[i] : 0ull;
+        fo.ids[i] = i < want ? (uint64_t)rkey_id(x) : ~0ull;
+        fo.scores[i] = i < want ? rkey_score(x) : -INFINITY;
+    }
+    if (threadIdx.x == 0 && fo.thr) *fo.thr = rkey_score(sorted[want - 1]);
+}
+
+// Exact top k of the candidates the stream's workgroups published, by the
+// last of them to finish.  The counts' offsets are scanned, the candidates
+// gathered into LDS (lkeys, cap keys), counting-sorted by 1024 equal
+// intervals of their key range -- only as far as the interval that holds the
+// k-th -- and each key is ranked inside its interval; results go out best
+// first.  Ties crowding one interval, and more candidates than cap, take a
+// radix select.  lkeys and regb hold cap keys each (2 * kp2 at least).
+template <int BS>
+__device__ void fused_select(FteState *__restrict__ st, const CandSet &cs, uint32_t k, uint32_t kreq, uint32_t cap,
+                             uint32_t kp2, const FinalOut &fo, uint64_t *lkeys, uint64_t *regb, FuseScratch &fs) {
+    __shared__ uint32_t wsum[BS / 64];
+    __shared__ uint32_t total, s_spill, s_pre;
+    uint32_t *off = reinterpret_cast<uint32_t *>(regb);
+    const uint32_t tid = threadIdx.x, wave = tid / 64;
+    if (cs.nblk <= 256) {
+        // wave 0 scans four counts per lane, the other waves clear
+        if (wave == 0) {
+            uint32_t n_[4], sum = 0;
+#pragma unroll
+            for (int j = 0; j < 4; j++) n_[j] = 4 * tid + j < cs.nblk ? cs.counts[4 * tid + j] : 0u;
+            if (tid == 0) {
+                s_spill = st->spill;
+                s_pre = cs.pre ? st->pre_count : 0u;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) sum += n_[j];
+            uint32_t at = wave_incl_scan(sum) - sum;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (4 * tid + j < cs.nblk) off[4 * tid + j] = at;
+                at += n_[j];
+            }
+            if (tid == 63) total = at;
+        } else {
+            for (uint32_t b = tid - 64; b < FUSE_BINS; b += BS - 64) fs.bins[b] = 0;
+            if (tid == 64) fs.crowded = 0;
+        }
+    } else {
+        for (uint32_t b = tid; b < cs.nblk; b += BS) off[b] = cs.counts[b];
+        for (uint32_t b = tid; b < FUSE_BINS; b += BS) fs.bins[b] = 0;
+        if (tid == 0) {
+            fs.crowded = 0;
+            s_spill = st->spill;
+            s_pre = cs.pre ? st->pre_count : 0u;
+        }
+        __syncthreads();
+        const uint32_t per = (cs.nblk + BS - 1) / BS;
+        const uint32_t b0 = tid * per < cs.nblk ? tid * per : cs.nblk;
+        const uint32_t b1 = b0 + per < cs.nblk ? b0 + per : cs.nblk;
+        uint32_t mine = 0;
+        for (uint32_t b = b0; b < b1; b++) mine += off[b];
+        uint32_t run = block_excl_scan<BS>(mine, wsum, &total);
+        for (uint32_t b = b0; b < b1; b++) {
+            const uint32_t c = off[b];
+            off[b] = run;
+            run += c;
+        }
+    }
+    __syncthreads();
+    const uint32_t spilled = s_spill, npre = s_pre;
+    const uint32_t nspill = spilled < cs.spill_cap ? spilled : cs.spill_cap;
+    const uint32_t ntotal = total, c = npre + ntotal + nspill;
+    const uint32_t bad = spilled > cs.spill_cap ? STATUS_OVERFLOW : (c < kreq ? STATUS_RETRY : 0u);
+    if (tid == 0) {
+        // ready for the next query
+        st->spill = 0;
+        st->arrive = 0;
+        st->ticket = 0;
+        if (bad) st->status |= bad;
+        else st->cand_last = c;
+        if (!bad && fo.cand) *fo.cand = c;
+        if (fo.status) *fo.status = bad;
+    }
+    if (tid < ARRIVE_GROUPS) st->group[tid * ARRIVE_STRIDE] = 0;
+    if (tid < SAMPLE_WIN) st->win[tid] = 0;
+    if (bad) return;
+    const SlotView v{cs.pre, npre, cs.keys, cs.slot, off, cs.nblk, ntotal, cs.spill};
+    const uint32_t want = c < k ? c : k;  // results
+    uint64_t *sorted;
+    if (c <= BS / 4) {
+        // few: each key's rank counted by four threads, a quarter of the keys each
+        const uint32_t i = tid % (BS / 4), part = tid / (BS / 4), q4 = (c + 3) / 4;
+        uint64_t x = 0;
+        if (part == 0 && i < c) lkeys[i] = x = v.get(i);
+        if (part == 1) fs.bins[i] = 0;  // the ranks
+        __syncthreads();
+        if (i < c) {
+            x = lkeys[i];
+            const uint32_t j1 = (part + 1) * q4 < c ? (part + 1) * q4 : c;
+            uint32_t r = 0;
+            for (uint32_t j = part * q4; j < j1; j++) r += lkeys[j] > x ? 1u : 0u;
+            if (r) atomicAdd(&fs.bins[i], r);
+        }
+        __syncthreads();
+        if (tid < c) regb[fs.bins[tid]] = x;  // the offsets are used up
+        __syncthreads();
+        emit_sorted<BS>(regb, want, k, fo);
+        return;
+    }
+    if (c <= cap) {
+        uint64_t lo = ~0ull, hi = 0;
+        for (uint32_t i = tid; i < c; i += BS) {
+            const uint64_t x = v.get(i);
+            lkeys[i] = x;
+            lo = x < lo ? x : lo;
+            hi = x > hi ? x : hi;
+        }
+        lo = wave_min_u64(lo);
+        hi = wave_max_u64(hi);
+        if (lane_id() == 0) {
+            fs.wlo[wave] = lo;
+            fs.whi[wave] = hi;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < BS / 64; w++) {
+            lo = fs.wlo[w] < lo ? fs.wlo[w] : lo;
+            hi = fs.whi[w] > hi ? fs.whi[w] : hi;
+        }
+        const int width = 64 - (hi > lo ? __builtin_clzll(hi - lo) : 63);
+        const int shift = width > 10 ? width - 10 : 0;  // interval 0 holds the largest keys
+        for (uint32_t i = tid; i < c; i += BS) atomicAdd(&fs.bins[(uint32_t)((hi - lkeys[i]) >> shift)], 1u);
+        __syncthreads();
+        constexpr int BPT = FUSE_BINS / BS;
+        uint32_t n_[BPT], sum = 0;
+#pragma unroll
+        for (int j = 0; j < BPT; j++) {
+            n_[j] = fs.bins[tid * BPT + j];
+            sum += n_[j];
+        }
+        uint32_t at = block_excl_scan<BS>(sum, wsum, &total);
+#pragma unroll
+        for (int j = 0; j < BPT; j++) {
+            fs.bins[tid * BPT + j] = at;
+            if (at < want) {
+                if (n_[j] > FUSE_BIN_MAX) fs.crowded = 1;
+                if (at + n_[j] >= want) {  // holds the last result
+                    fs.cut = tid * BPT + j;
+                    fs.ncut = at + n_[j];
+                }
+            }
+            at += n_[j];
+        }
+        __syncthreads();
+        if (!fs.crowded) {
+            // the intervals up to the cut, in order; bins[] turns from an
+            // interval's start into its end (the offsets in regb are used up)
+            for (uint32_t i = tid; i < c; i += BS) {
+                const uint64_t x = lkeys[i];
+                const uint32_t b = (uint32_t)((hi - x) >> shift);
+                if (b <= fs.cut) regb[atomicAdd(&fs.bins[b], 1u)] = x;
+            }
+            __syncthreads();
+            sorted = lkeys;
+            for (uint32_t i = tid; i < fs.ncut; i += BS) {
+                const uint64_t x = regb[i];
+                const uint32_t b = (uint32_t)((hi - x) >> shift);
+                const uint32_t s0 = b ? fs.bins[b - 1] : 0u, s1 = fs.bins[b];
+                uint32_t r = s0;
+                for (uint32_t j = s0; j < s1; j++) r += regb[j] > x ? 1u : 0u;
+                if (r < want) sorted[r] = x;
+            }
+            __syncthreads();
+        }
+    }
+    if (c > cap || fs.crowded) {
+        uint32_t got;
+        if (c <= cap) {
+            const uint64_t thr =
+                c > k ? block_kth_largest<BS, MemKeys<BS>, 8>(MemKeys<BS>{lkeys, c}, c, k, fs.rs) : 1ull;
+            got = block_gather_ge<BS>(MemKeysUniform<BS>{lkeys, c}, thr, regb, fs.rs);
+            sorted = regb;
+        } else {
+            const uint64_t thr = block_kth_largest<BS, ViewKeys<BS, SlotView, false>, 8>(
+                ViewKeys<BS, SlotView, false>{v, c}, c, k, fs.rs);
+            got = block_gather_ge<BS>(ViewKeys<BS, SlotView, true>{v, c}, thr, lkeys, fs.rs);
+            sorted = lkeys;
+        }
+        if (got <= (uint32_t)BS) {  // a rank pass, else a bitonic sort (got^2 compares grow past it)
+            const uint64_t x = tid < got ? sorted[tid] : 0ull;
+            uint32_t r = 0, unused = 0;
+            rank2_lds(sorted, got, x, x, r, unused);
+            __syncthreads();
+            if (tid < got) sorted[r] = x;
+            __syncthreads();
+        } else {
+            for (uint32_t i = got + tid; i < kp2; i += BS) sorted[i] = 0;
+            __syncthreads();
+            bitonic_sort_desc<BS>(sorted, kp2);
+        }
+    }
+    emit_sorted<BS>(sorted, want, k, fo);
+}
+
+// Where a stream workgroup takes tau from.
+enum { TAU_ALL = 0, TAU_STATE = 1, TAU_SHARED = 2, TAU_OWN = 3 };
+
+// One stream pass.
+struct StreamArgs {
+    uint64_t n, obj_begin, ntiles;
+    uint64_t nstatic;      // tiles dealt out in turn; the rest as workgroups get free
+    FteState *st;
+    CandSet cs;
+    int tau;               // TAU_*: every object a candidate, st->tau, the shared sample, the own sample
+    uint32_t ks;           // rank of tau in the sample
+    uint32_t chunks, wgs, W;  // shared sample: chunks, producers, winners per producer
+    uint64_t chunk_stride; // objects between the chunks' first objects
+    int select;            // the last workgroup selects and emits (else a later launch does)
+    uint32_t cap, kp2, k, kreq;
+    FinalOut fo;
+    const uint32_t *gate;
+};
+
+// Each workgroup streams whole tiles of TILE = 4096*VPT objects: for every
 // queried column it reads one contiguous TILE*4-byte segment (VPT float4 per
 // lane).  Block-contiguous segments keep HBM near 88% of peak where a
 // thread-level grid stride over the columns stays near 72%.  The column
 // store is padded by one tile, so tile loads need no bounds check.
-// tau comes from st->tau (published by a merging seed pass) or, when nseed
-// > 0, from the ks-th largest of the nseed seed winners in seed[].
+//
+// One workgroup of 16 waves per CU holds 8 or more loads of 16 bytes per lane
+// in flight, which is all HBM needs (512 to 3072 workgroups of 256 threads
+// stream at the same 6.7 TB/s), leaves few arrivals at the end and 1024
+// threads to the select.  Of two workgroups on a CU the older one goes
+// first: two of 512 threads per CU ended between 203 and 334 us at N = 2^26.
+//
+// XCDs do not run at one speed either (at N = 2^26 four of the eight are 6%
+// behind), so the last tiles are handed out by a ticket, taken while the
+// tile before is processed (device atomics on one address serialise at
+// about 20 ns, so only the last ones).
+//
+// Bound by HBM above a few million objects (6.9 TB/s at N = 2^26, m = 8),
+// by the chain of launch, sample, arrival and select below.  A synchronous
+// call, before (seed, stream and select launches, two result copies) and
+// now: 16k objects 50 -> 35 us, 2^20 65 -> 39, 8M x 7 divided 114 -> 78, 4.2M
+// x 20 with k = 1000 245 -> 106, 2^26 x 8 373 -> 349; 32 queued queries of
+// 16M x 5 1945 -> 1807.  At 2^20 tau is known after 10 us, the last
+// workgroup arrives at 13 and has selected at 19.
+//
+// The select runs in the last workgroup to finish.  Its inputs cross XCDs
+// without an L2 write-back per workgroup: candidates, counts and spilled
+// keys are agent-scope (write-through) stores, each wave waits for its own
+// before the workgroup takes its arrival ticket, and the last workgroup
+// invalidates its caches once.  Arrivals are counted in ARRIVE_GROUPS
+// groups on cache lines of their own and then across groups: on one counter
+// they serialise at about 20 ns each.
 template <int M, int VPT>
-__global__ __launch_bounds__(STREAM_BS) void fte_stream_kernel(QCols q, uint64_t n, uint64_t obj_begin,
-                                                               uint64_t ntiles, FteState *__restrict__ st,
-                                                               CandSet cs, const uint64_t *__restrict__ seed,
-                                                               uint32_t nseed, uint32_t ks,
-                                                               const uint32_t *__restrict__ gate) {
+__global__ __launch_bounds__(STREAM_BS, 4) void fte_stream_kernel(QCols q, StreamArgs a) {
     constexpr uint32_t TILE = STREAM_BS * 4 * VPT;
-    __shared__ uint32_t lcount;
-    if (gate && *gate == 0) return;
-    if (threadIdx.x == 0) lcount = 0;
-    __syncthreads();
-    const uint64_t tau = nseed ? wave_seed_tau(seed, nseed, ks) : st->tau;
-    const uint32_t tau_hi = (uint32_t)(tau >> 32);
+    extern __shared__ uint64_t dyn[];  // cap keys | block offsets, later cap keys
+    __shared__ uint32_t lcount, is_last, s_next[2];
+    __shared__ uint64_t s_tau;
+    __shared__ union {
+        OwnScratch own;
+        SampleScratch sam;
+        FuseScratch sel;
+    } sh;
+    if (a.gate && *a.gate == 0) return;
     const uint32_t lane = lane_id();
-    uint64_t *my = cs.keys + (uint64_t)blockIdx.x * cs.slot;
-    for (uint64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-        const uint64_t v0 = (obj_begin + t * TILE) / 4 + threadIdx.x;
-        f4 s[VPT];
+    if (threadIdx.x == 0) lcount = 0;
+    if (a.tau == TAU_SHARED && blockIdx.x < a.wgs)
+        sample_publish<M>(q, a.n, a.chunks, a.chunk_stride, a.W, a.st, sh.sam);
+    // the first tile's loads are in flight while tau is found
+    constexpr int MX = M > 0 ? M : 1;
+    f4 x[MX][VPT];
+    uint64_t t = blockIdx.x;
+    auto load = [&](uint64_t v0) {
         if constexpr (M > 0) {
-            f4 x[M][VPT];
 #pragma unroll
             for (int j = 0; j < M; j++)
 #pragma unroll
                 for (int u = 0; u < VPT; u++) x[j][u] = ld_stream(q.col[j] + (v0 + u * STREAM_BS) * 4);
+        }
+    };
+    load((a.obj_begin + t * TILE) / 4 + threadIdx.x);  // the grid never exceeds the tiles
+    uint64_t tau = 0;
+    if (a.tau == TAU_OWN) {
+        tau = own_sample_tau<M>(q, a.n, a.ks, sh.own);
+    } else if (a.tau != TAU_ALL) {
+        if (threadIdx.x < 64) {
+            const uint64_t v = a.tau == TAU_SHARED ? sample_tau(a.st, a.wgs * a.W, a.ks) : a.st->tau;
+            if (lane == 0) s_tau = v;
+        }
+        __syncthreads();
+        tau = s_tau;
+    } else {
+        __syncthreads();
+    }
+    const uint32_t tau_hi = (uint32_t)(tau >> 32);
+    const CandSet &cs = a.cs;
+    uint64_t *my = cs.keys + (uint64_t)blockIdx.x * cs.slot;
+    for (bool first = true, par = false;; first = false) {
+        // past the dealt tiles, the next one's ticket travels while this one is processed
+        const bool draw = t + gridDim.x >= a.nstatic && a.nstatic < a.ntiles;  // uniform
+        uint32_t nx = 0;
+        if (draw && threadIdx.x == 0)
+            nx = __hip_atomic_fetch_add(&a.st->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t v0 = (a.obj_begin + t * TILE) / 4 + threadIdx.x;
+        f4 s[VPT];
+        if constexpr (M > 0) {
+            if (!first) load(v0);
 #pragma unroll
             for (int u = 0; u < VPT; u++) {
                 f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -256,8 +746,7 @@ __global__ __launch_bounds__(STREAM_BS) void fte_stream_kernel(QCols q, uint64_t
                 s[u] = acc;
             }
         } else {
-#pragma unroll
-            for (int u = 0; u < VPT; u++) s[u] = score_vec<0>(q, v0 + u * STREAM_BS);
+            score_wide<VPT>(q, v0, STREAM_BS, s);
         }
         // filter: key >= tau (score key first; the id only matters on ties)
         uint32_t npass = 0;
@@ -269,7 +758,7 @@ __global__ __launch_bounds__(STREAM_BS) void fte_stream_kernel(QCols q, uint64_t
                 const uint64_t id = (v0 + u * STREAM_BS) * 4 + e;
                 const uint32_t ok = okey(s[u][e]);
                 const uint64_t key = rkey_from_okey(ok, (uint32_t)id);
-                const bool p = ok >= tau_hi && key >= tau && id < n;
+                const bool p = ok >= tau_hi && key >= tau && id < a.n;
                 kk[u * 4 + e] = p ? key : 0ull;
                 npass += p ? 1u : 0u;
             }
@@ -285,7 +774,7 @@ __global__ __launch_bounds__(STREAM_BS) void fte_stream_kernel(QCols q, uint64_t
             const uint32_t nspill = base + wtotal > first_spill ? base + wtotal - first_spill : 0u;
             uint32_t sbase = 0;
             if (nspill) {
-                if (lane == 63) sbase = atomicAdd(&st->spill, nspill);
+                if (lane == 63) sbase = atomicAdd(&a.st->spill, nspill);
                 sbase = __shfl(sbase, 63, 64);
             }
             uint32_t pos = base + incl - npass;
@@ -293,28 +782,56 @@ __global__ __launch_bounds__(STREAM_BS) void fte_stream_kernel(QCols q, uint64_t
             for (int j = 0; j < VPT * 4; j++) {
                 if (kk[j]) {
                     if (pos < cs.slot) {
-                        my[pos] = kk[j];
+                        store_agent(my + pos, kk[j]);
                     } else {
                         const uint32_t sp = sbase + (pos - first_spill);
-                        if (sp < cs.spill_cap) cs.spill[sp] = kk[j];
+                        if (sp < cs.spill_cap) store_agent(cs.spill + sp, kk[j]);
                     }
                     pos++;
                 }
             }
         }
+        if (draw) {
+            if (threadIdx.x == 0) s_next[par] = nx;
+            __syncthreads();
+            t = a.nstatic + s_next[par];
+            par = !par;
+        } else {
+            t += gridDim.x;
+        }
+        if (t >= a.ntiles) break;
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's candidates have reached memory
     __syncthreads();
-    if (threadIdx.x == 0) cs.counts[blockIdx.x] = lcount < cs.slot ? lcount : cs.slot;
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(&cs.counts[blockIdx.x], lcount < cs.slot ? lcount : cs.slot, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+        if (a.select) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            // group g counts workgroups g, g + ARRIVE_GROUPS, ...
+            const uint32_t G = gridDim.x, g = blockIdx.x % ARRIVE_GROUPS;
+            const uint32_t members = (G - g + ARRIVE_GROUPS - 1) / ARRIVE_GROUPS;
+            bool last = __hip_atomic_fetch_add(&a.st->group[g * ARRIVE_STRIDE], 1u, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT) == members - 1;
+            if (last)
+                last = __hip_atomic_fetch_add(&a.st->arrive, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                       (G < ARRIVE_GROUPS ? G : ARRIVE_GROUPS) - 1;
+            is_last = last;
+        }
+    }
+    if (!a.select) return;
+    __syncthreads();
+    if (!is_last) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    fused_select<STREAM_BS>(a.st, cs, a.k, a.kreq, a.cap, a.kp2, a.fo, dyn, dyn + a.cap, sh.sel);
 }
 
-// 3. final select: one workgroup after the stream pass.  (A last-block merge
-// inside the stream pass would need an agent-scope release fence in every
-// one of its ~2000 blocks; each is an L2 write-back on gfx950 and together
-// they cost more than a launch.)
+// Final select as a launch of its own (one workgroup): partition queries,
+// and stores that fit the exact seed's prefix.
 __global__ __launch_bounds__(FINAL_BS) void fte_final_kernel(FteState *__restrict__ st, CandSet cs, uint32_t k,
                                                              uint32_t kreq, FinalOut fo,
                                                              const uint32_t *__restrict__ gate) {
-    __shared__ uint32_t off[MAX_STREAM_GRID + 2];
+    __shared__ uint32_t off[MAX_STREAM_GRID];
     if (gate && *gate == 0) return;
     __shared__ uint64_t top[TOPK_MAX_K];
     __shared__ uint64_t sorted[TOPK_MAX_K];
@@ -338,14 +855,10 @@ __global__ __launch_bounds__(FINAL_BS) void fte_final_kernel(FteState *__restric
     }
     const uint32_t spilled = st->spill;
     const uint32_t nspill = spilled < cs.spill_cap ? spilled : cs.spill_cap;
-    if (tid == 0) {
-        off[cs.nblk] = total;
-        off[cs.nblk + 1] = total + nspill;
-    }
     __syncthreads();
     if (tid == 0) st->spill = 0;  // ready for the next query
     const uint32_t npre = cs.pre ? st->pre_count : 0u;
-    const uint32_t c = npre + off[cs.nblk + 1];
+    const uint32_t c = npre + total + nspill;
     const uint32_t bad = spilled > cs.spill_cap ? STATUS_OVERFLOW : (c < kreq ? STATUS_RETRY : 0u);
     if (bad) {
         if (tid == 0) {
@@ -358,7 +871,7 @@ __global__ __launch_bounds__(FINAL_BS) void fte_final_kernel(FteState *__restric
         st->cand_last = c;
         if (fo.cand) *fo.cand = c;
     }
-    const SlotView v{cs.pre, npre, cs.keys, cs.slot, off, cs.nblk, cs.spill};
+    const SlotView v{cs.pre, npre, cs.keys, cs.slot, off, cs.nblk, total, cs.spill};
     select_and_emit<FINAL_BS, FINAL_KPT>(v, c, k, fo, top, sorted, ss);
 }
 
@@ -412,7 +925,10 @@ __global__ __launch_bounds__(FLAT_BS) void fte_final_flat_kernel(FteState *__res
         }
         return;
     }
-    if (threadIdx.x == 0) st->cand_last = c;
+    if (threadIdx.x == 0) {
+        st->cand_last = c;
+        if (fo.cand) *fo.cand = c;
+    }
     select_and_emit<FLAT_BS, 8>(FlatView{flat}, c, k, fo, top, sorted, ss);
 }
 
@@ -429,7 +945,7 @@ static uint32_t exact_prefix_blocks(uint64_t n, uint32_t k) {
 }
 
 static uint32_t stream_grid(uint32_t grid_cap, uint64_t ntiles) {
-    const uint64_t cap = grid_cap ? (uint64_t)grid_cap : 2048;
+    const uint64_t cap = grid_cap ? (uint64_t)grid_cap : STREAM_GRID;
     const uint64_t g = ntiles < cap ? ntiles : cap;
     return (uint32_t)(g < 1 ? 1 : g);
 }
@@ -438,36 +954,74 @@ static uint32_t stream_grid(uint32_t grid_cap, uint64_t ntiles) {
 // flight per lane (about 8-16) without exhausting registers.
 static int stream_vpt(uint32_t m) {
     if (m <= 1) return 8;
-    if (m <= 4) return 4;
-    if (m <= 8) return 2;
+    if (m <= 2) return 4;
+    if (m <= 4) return 2;
     return 1;
 }
 
-// Chooses the seed geometry for a query: sample mode when n is large enough
-// that a spread sample leaves many candidates, exact prefix mode otherwise.
-// Returns true for the sample geometry.
-static bool seed_plan(uint64_t n, uint32_t k, bool exact, uint32_t &blocks, uint64_t &stride, uint64_t &n_eff,
-                      uint32_t &ks, uint32_t &total_valid) {
-    const uint64_t s = (uint64_t)SAMPLE_CHUNKS * SAMPLE_TILE;
-    if (!exact && n > 4 * s) {
-        blocks = SAMPLE_CHUNKS;
-        stride = ((n / SAMPLE_CHUNKS) / SAMPLE_TILE) * SAMPLE_TILE;
-        n_eff = n;
-        // expected candidates ~ ks * n / s; aim for >= 8k
-        const uint64_t want = (8ull * k * s + n - 1) / n;
-        ks = (uint32_t)(want < 4 ? 4 : (want > k ? k : want));
-        total_valid = blocks * ks;
-        return true;
+// Samples above the ks-th largest of a random sample of s of the n objects
+// leave ks * n / s candidates on average, spread like a Gamma(ks) variable.
+// The smallest ks that leaves fewer than k with a chance of about 1e-4, from
+// q = k * s / n (the expected number of the top k in the sample): ks - 3.7
+// sqrt(ks) + 3.6 >= q, e.g. 17 k candidates at ks = 4, 5 k at 8, 2 k at 32.
+static uint32_t sample_rank(double q) {
+    uint32_t ks = 4;
+    while (ks < 4096 && ks - 3.7 * std::sqrt((double)ks) + 3.6 < q) ks++;
+    return ks;
+}
+
+// How a query gets its threshold.
+struct SeedPlan {
+    int tau;               // TAU_*
+    uint32_t blocks, ks;   // chunks of the sample or blocks of the exact seed; rank of tau (exact: winners per block)
+    uint32_t W;            // shared sample: winners per producer
+    uint64_t stride;       // objects between the chunks' first objects
+    uint64_t n_eff;        // exact: objects of the prefix
+    uint32_t total_valid;  // exact: keys the blocks deposit
+    double expect;         // candidates expected
+};
+
+// FTE_SAMPLE may guess on any store (the caller re-runs a bad guess): every
+// object of a store that fits the select, the own sample up to 2^19 objects,
+// the shared sample above.  FTE_QUEUED guesses only above 2^19 objects:
+// nothing re-runs it.
+static SeedPlan seed_plan(uint64_t n, uint32_t k, int mode) {
+    SeedPlan p{};
+    if (mode == FTE_SAMPLE && n <= FUSE_CAP_MAX) {
+        p.tau = TAU_ALL;
+        p.expect = (double)n;
+    } else if (mode == FTE_SAMPLE && n <= OWN_MAX_N) {
+        p.tau = TAU_OWN;
+        p.ks = sample_rank((double)k * OWN_OBJS / (double)n);
+        p.expect = (double)p.ks * n / OWN_OBJS;
+        if (p.expect >= n) p.tau = TAU_ALL;
+    } else if ((mode == FTE_SAMPLE || mode == FTE_QUEUED) && n > OWN_MAX_N) {
+        p.tau = TAU_SHARED;
+        // As many chunks as make tau the 8th largest of the sample (q =
+        // 1.13).  A long list on a small store would leave few of them, large
+        // jumps of the id range: below 32 chunks, all 128 and a deeper rank.
+        const uint64_t c8 = (uint64_t)(1.13 * (double)n / ((double)k * SAMPLE_TILE));
+        p.blocks = c8 >= SAMPLE_CHUNKS / 4 && c8 < SAMPLE_CHUNKS ? (uint32_t)c8 : SAMPLE_CHUNKS;
+        p.stride = ((n / p.blocks) / SAMPLE_TILE) * SAMPLE_TILE;
+        const double s = (double)p.blocks * SAMPLE_TILE;
+        p.ks = sample_rank(k * s / (double)n);
+        // each producer's share of the ks best: all of them up to 16 (the
+        // producers' chunks alternate over the id range, so more than 16 of
+        // a deep rank's best rarely meet in one; missing some lowers tau)
+        p.W = p.ks < SAMPLE_MAX_W ? p.ks : SAMPLE_MAX_W;
+        p.expect = (double)p.ks * n / s;
     } else {
-        blocks = exact_prefix_blocks(n, k);
-        stride = SEED_TILE;
-        const uint64_t p = (uint64_t)blocks * SEED_TILE;
-        n_eff = n < p ? n : p;
-        ks = k;
-        const uint64_t full = n_eff / SEED_TILE, rem = n_eff % SEED_TILE;
-        total_valid = (uint32_t)(full * (k < SEED_TILE ? k : SEED_TILE) + (rem < k ? rem : k));
-        return false;
+        p.tau = TAU_STATE;
+        p.blocks = exact_prefix_blocks(n, k);
+        p.stride = SEED_TILE;
+        const uint64_t pre = (uint64_t)p.blocks * SEED_TILE;
+        p.n_eff = n < pre ? n : pre;
+        p.ks = k;
+        const uint64_t full = p.n_eff / SEED_TILE, rem = p.n_eff % SEED_TILE;
+        p.total_valid = (uint32_t)(full * (k < SEED_TILE ? k : SEED_TILE) + (rem < k ? rem : k));
+        p.expect = 2.0 * k;
     }
+    return p;
 }
 
 // Everything one run of the FTE pipeline needs besides the query: the store
@@ -490,65 +1044,71 @@ struct FteRun {
     topk_ctx *timed;      // non-null: bracket the stream pass for topk_timing_*
 };
 
-// Enqueues seed -> stream -> final select for one query on r.s.  Returns the
-// candidate set the final select read (pta.hip re-uses the final stage).
+// Enqueues the threshold pass, if the plan has one, and the stream pass (with
+// the select, unless r.big leaves it to the caller) for one query on r.s.
+// Returns the candidate set the select reads.
 static CandSet fte_launch(const FteRun &r, uint32_t k, const QCols &q, const FinalOut &fo, int mode) {
     const uint64_t n = r.n;
-    const bool exact = mode != FTE_SAMPLE;
     hipStream_t s = r.s;
-
-    uint32_t blocks, ks, total_valid;
-    uint64_t stride, n_eff;
-    const bool sampled = seed_plan(n, k, exact, blocks, stride, n_eff, ks, total_valid);
+    const SeedPlan sp = seed_plan(n, k, mode);
+    const bool exact = sp.tau == TAU_STATE;
     uint64_t *pre = exact ? r.pre : nullptr;
-    // sample mode with few winners: no merge in the seed pass, every stream
-    // wave reduces the winners to tau itself
-    const bool wave_tau = sampled && ks <= 4 && blocks * ks <= SEED_WAVE_MAX;
     // kernels unrolled for the query width, or the runtime-width ones (the
     // only ones that divide real-data scores)
     const uint32_t msw = q.div != 0.0f ? 0u : q.m;
-#define TK_SEED(MM, OPT, MERGE)                                                                           \
-    hipLaunchKernelGGL((fte_seed_kernel<MM, OPT, MERGE>), dim3(blocks), dim3(SEED_BS), 0, s, q, n_eff, stride, \
-                       ks, total_valid, r.blk, pre, r.st, r.gate)
-#define TK_SEED_SAMPLE(MM) TK_SEED(MM, SAMPLE_TILE / SEED_BS, true)
-#define TK_SEED_EXACT(MM) TK_SEED(MM, SEED_TILE / SEED_BS, true)
-#define TK_SAMPLE(MM) \
-    hipLaunchKernelGGL(fte_sample_kernel<MM>, dim3(blocks), dim3(SEED_BS), 0, s, q, n_eff, stride, ks, r.blk)
-    if (wave_tau) {
-        TK_SWITCH_M(msw, TK_SAMPLE);
-    } else if (sampled) {
-        TK_SWITCH_M(msw, TK_SEED_SAMPLE);
-    } else {
-        TK_SWITCH_M(msw, TK_SEED_EXACT);
-    }
+#define TK_SEED(MM)                                                                                              \
+    hipLaunchKernelGGL((fte_seed_kernel<MM, SEED_TILE / SEED_BS>), dim3(sp.blocks), dim3(SEED_BS), 0, s, q, sp.n_eff, \
+                       sp.stride, sp.ks, sp.total_valid, r.blk, pre, r.st, r.gate)
+    if (exact) TK_SWITCH_M(msw, TK_SEED);
 #undef TK_SEED
-#undef TK_SAMPLE
-#undef TK_SEED_SAMPLE
-#undef TK_SEED_EXACT
-    const uint32_t nseed = wave_tau ? blocks * ks : 0u;
 
     // exact mode streams only the objects after the prefix
-    const uint64_t first = exact ? n_eff : 0;
-    const uint32_t kreq = (uint32_t)(n < k ? n : k);
-    const int vpt = r.vpt ? r.vpt : stream_vpt(q.m);
+    const uint64_t first = exact ? sp.n_eff : 0;
+    // smaller tiles where the wide ones would leave workgroups without one
+    int vpt = r.vpt ? r.vpt : stream_vpt(q.m);
+    while (!r.vpt && vpt > 1 && n - first < (uint64_t)STREAM_GRID * STREAM_BS * 4 * vpt) vpt /= 2;
     const uint64_t tile = (uint64_t)STREAM_BS * 4 * vpt;
-    const uint64_t ntiles = n > first ? (n - first + tile - 1) / tile : 0;
-    const uint32_t g = ntiles ? stream_grid(r.grid_cap, ntiles) : 0;
-    CandSet cs;
+    StreamArgs a{};
+    a.n = n;
+    a.obj_begin = first;
+    a.ntiles = n > first ? (n - first + tile - 1) / tile : 0;
+    a.st = r.st;
+    a.tau = sp.tau;
+    a.ks = sp.ks;
+    a.chunks = sp.blocks;
+    a.W = sp.W;
+    a.chunk_stride = sp.stride;
+    a.select = r.big ? 0 : 1;
+    a.k = k;
+    a.kreq = (uint32_t)(n < k ? n : k);
+    a.fo = fo;
+    a.gate = r.gate;
+    // room in LDS for twice the candidates expected, and for the sort of k
+    a.kp2 = next_pow2(k);
+    uint32_t cap = FUSE_CAP_MIN;
+    while (cap < FUSE_CAP_MAX && (cap < 2 * a.kp2 || cap < 2 * sp.expect)) cap += FUSE_CAP_MIN;
+    a.cap = cap;
+    const uint32_t g = a.ntiles ? stream_grid(r.grid_cap, a.ntiles) : 0;
+    // the last tiles by ticket; a run whose slots hold a block's every object
+    // deals all of them
+    a.nstatic = a.ntiles;
+    if (!r.big && a.ntiles > 2ull * g) a.nstatic = (a.ntiles - std::max<uint64_t>(a.ntiles / 12, 2ull * g) + g - 1) / g * g;
+    a.wgs = g < SAMPLE_WGS ? g : SAMPLE_WGS;
+    CandSet &cs = a.cs;
     cs.keys = r.cand;
     cs.counts = r.counts;
     cs.nblk = g;
     cs.pre = pre;
     cs.spill = r.spill;
     cs.spill_cap = r.spill_cap;
-    if (r.big) cs.slot = g ? (uint32_t)(((ntiles + g - 1) / g) * tile) : 0;  // a block's every object fits
+    if (r.big) cs.slot = g ? (uint32_t)(((a.ntiles + g - 1) / g) * tile) : 0;  // a block's every object fits
     else cs.slot = g ? (uint32_t)(r.cand_cap / g) : 0;
     if (g) {
+        const size_t lds = sizeof(uint64_t) * ((size_t)cap + std::max((g + 3) / 2, cap));
         hipEvent_t ev0 = nullptr;
         if (r.timed) timing_begin(r.timed, s, ev0);
-#define TK_STREAM(MM, VPT)                                                                                   \
-    hipLaunchKernelGGL((fte_stream_kernel<MM, VPT>), dim3(g), dim3(STREAM_BS), 0, s, q, n, first, ntiles, \
-                       r.st, cs, r.blk, nseed, ks, r.gate)
+#define TK_STREAM(MM, VPT) \
+    hipLaunchKernelGGL((fte_stream_kernel<MM, VPT>), dim3(g), dim3(STREAM_BS), lds, s, q, a)
 #define TK_STREAM1(MM) TK_STREAM(MM, 1)
 #define TK_STREAM2(MM) TK_STREAM(MM, 2)
 #define TK_STREAM4(MM) TK_STREAM(MM, 4)
@@ -565,13 +1125,13 @@ static CandSet fte_launch(const FteRun &r, uint32_t k, const QCols &q, const Fin
 #undef TK_STREAM4
 #undef TK_STREAM8
         if (r.timed) timing_end(r.timed, s, "fte_stream", ev0);
+    } else if (!r.big) {
+        hipLaunchKernelGGL(fte_final_kernel, dim3(1), dim3(FINAL_BS), 0, s, r.st, cs, k, a.kreq, fo, r.gate);
     }
-    if (!r.big) hipLaunchKernelGGL(fte_final_kernel, dim3(1), dim3(FINAL_BS), 0, s, r.st, cs, k, kreq, fo, r.gate);
     return cs;
 }
 
-int fte_enqueue(topk_ctx *ctx, Lane &L, uint32_t k, const QCols &q, uint64_t *d_ids, float *d_scores,
-                float *d_thr, uint32_t *d_status, int mode, uint64_t n) {
+int fte_enqueue(topk_ctx *ctx, Lane &L, uint32_t k, const QCols &q, const FinalOut &fo, int mode, uint64_t n) {
     if (!n) n = ctx->n;
     if (n >= ID_LIMIT) return TOPK_ERR_UNSUPPORTED;  // a run's ids are 32-bit: callers split larger stores
     FteRun r{};
@@ -590,7 +1150,6 @@ int fte_enqueue(topk_ctx *ctx, Lane &L, uint32_t k, const QCols &q, uint64_t *d_
     r.grid_cap = ctx->tune.stream_grid;
     r.timed = ctx;
     const uint32_t kreq = (uint32_t)(n < k ? n : k);
-    const FinalOut fo{d_ids, d_scores, d_thr, d_status};
     const CandSet cs = fte_launch(r, k, q, fo, mode);
     if (r.big) final_enqueue(ctx, L, cs, k, kreq, fo, true);
     TK_HIP(hipGetLastError());
@@ -684,7 +1243,7 @@ void final_enqueue(topk_ctx *ctx, Lane &L, const CandSet &cs, uint32_t k, uint32
 // failure.  Nothing waits on the host, so the call can be captured in a graph.
 constexpr uint64_t NA_CAND = 1ull << 20;   // candidate slots (8 MiB)
 constexpr uint32_t NA_SPILL = 1u << 18;    // spill region (2 MiB)
-constexpr uint64_t NA_BLK = (uint64_t)SAMPLE_CHUNKS * TOPK_MAX_K;  // seed winners, either mode (1 MiB)
+constexpr uint64_t NA_BLK = (uint64_t)SAMPLE_CHUNKS * TOPK_MAX_K;  // seed winners, any plan (1 MiB)
 struct NoAllocScratch {
     FteState st;
     uint32_t pass[2];  // final-select status of the first and the second run (0: settled)
@@ -724,11 +1283,10 @@ static int noalloc_scratch(NoAllocScratch **out) {
 
 // Clears what the pipeline expects at zero (a kernel, not a memset node).
 __global__ void noalloc_clear_kernel(NoAllocScratch *__restrict__ sc) {
-    if (threadIdx.x == 0) {
-        sc->st = FteState{};
-        sc->pass[0] = 0;
-        sc->pass[1] = 0;
-    }
+    static_assert(sizeof(FteState) % 8 == 0, "cleared by words");
+    uint64_t *w = reinterpret_cast<uint64_t *>(&sc->st);
+    for (uint32_t i = threadIdx.x; i < sizeof(FteState) / 8; i += blockDim.x) w[i] = 0;
+    if (threadIdx.x < 2) sc->pass[threadIdx.x] = 0;
 }
 
 // Caller-visible status: TOPK_OK when either run settled the query.
@@ -776,11 +1334,9 @@ extern "C" int topk_fte_noalloc(const float *d_cols, uint64_t n, uint32_t d, uin
     r.cand_cap = NA_CAND;
     r.spill = sc->spill;
     r.spill_cap = NA_SPILL;
-    hipLaunchKernelGGL(noalloc_clear_kernel, dim3(1), dim3(64), 0, r.s, sc);
-    uint32_t blocks, ks, total_valid;
-    uint64_t stride, n_eff;
-    const bool sampled = seed_plan(n, k, false, blocks, stride, n_eff, ks, total_valid);
-    fte_launch(r, k, q, FinalOut{d_ids, d_scores, d_threshold, &sc->pass[0]}, FTE_SAMPLE);
+    hipLaunchKernelGGL(noalloc_clear_kernel, dim3(1), dim3(256), 0, r.s, sc);
+    const bool sampled = seed_plan(n, k, FTE_QUEUED).tau != TAU_STATE;
+    fte_launch(r, k, q, FinalOut{d_ids, d_scores, d_threshold, &sc->pass[0]}, FTE_QUEUED);
     if (sampled) {
         // too few candidates (the sample guessed high) or a full buffer: the
         // exact-prefix run, skipped on the device when the first one settled

@@ -26,17 +26,22 @@ struct QCols {
     float div;
 };
 
-// Device-side state of one FTE / PTA query pipeline.
+// Device-side state of one FTE / PTA query pipeline.  Words that many
+// workgroups hit at once sit on cache lines of their own.
+constexpr uint32_t ARRIVE_GROUPS = 16, ARRIVE_STRIDE = 32;
+constexpr uint32_t SAMPLE_WIN = 512;
 struct FteState {
-    unsigned long long tau;   // threshold key published by the seed pass
+    unsigned long long tau;   // threshold key published by the exact seed pass
     unsigned int pre_count;   // exact mode: prefix keys the seed pass stored in pre[]
-    unsigned int arrive;      // arrival ticket of the seed pass (last block merges)
+    unsigned int arrive;      // arrival ticket of the seed or stream pass (the last block merges or selects)
     unsigned int status;      // sticky device error bits (STATUS_*)
     unsigned int scored;      // PTA: partitions scored
     unsigned int total;       // flat-gather mode: candidates gathered
     unsigned int cand_last;   // candidates seen by the last final select
     unsigned int spill;       // candidates that spilled past their block's slot region
-    unsigned int pad;
+    alignas(128) unsigned int ticket;  // next tile of the stream's shared part
+    alignas(128) unsigned int group[ARRIVE_GROUPS * ARRIVE_STRIDE];  // arrivals of the stream workgroups, by group
+    alignas(128) unsigned long long win[SAMPLE_WIN];  // the shared sample's winners (0: not published yet)
 };
 
 // Candidate keys of one query.  Stream block b owns keys[b*slot, (b+1)*slot)
@@ -58,9 +63,11 @@ struct CandSet {
 
 enum : unsigned int { STATUS_OVERFLOW = 1u, STATUS_RETRY = 2u };
 
-// FTE pipeline modes: sample-seeded (fast path), exact-prefix-seeded with
-// the regular candidate buffer, and exact with an n-entry buffer.
-enum { FTE_SAMPLE = 0, FTE_EXACT = 1, FTE_EXACT_BIG = 2 };
+// FTE pipeline modes: sample-seeded (the caller re-runs a bad guess),
+// exact-prefix-seeded with the regular candidate buffer, exact with an
+// n-entry buffer, and queued: sample-seeded above 2^19 objects, exact below
+// (nothing re-runs it).
+enum { FTE_SAMPLE = 0, FTE_EXACT = 1, FTE_EXACT_BIG = 2, FTE_QUEUED = 3 };
 
 constexpr uint32_t MAX_STREAM_GRID = 4096;
 
@@ -332,8 +339,7 @@ void final_enqueue(topk_ctx *ctx, Lane &L, const CandSet &cs, uint32_t k, uint32
                    bool flat_fallback);
 // One FTE pipeline run over objects [0, n) of the columns q points at (n = 0:
 // the whole store; ids are local to those columns).
-int fte_enqueue(topk_ctx *ctx, Lane &L, uint32_t k, const QCols &q, uint64_t *d_ids, float *d_scores,
-                float *d_thr, uint32_t *d_status, int mode, uint64_t n = 0);
+int fte_enqueue(topk_ctx *ctx, Lane &L, uint32_t k, const QCols &q, const FinalOut &fo, int mode, uint64_t n = 0);
 // Merges the top-k lists of `shards` id shards (shard s: sh_ids / sh_scores
 // + s * TOPK_MAX_K, min(k, objects of the shard) entries, best first) into
 // fo with global ids, on stream s (fte.hip).
