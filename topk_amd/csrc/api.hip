@@ -233,6 +233,7 @@ int topk_ctx_destroy(topk_ctx *ctx) {
     batch_free(ctx);
     aux_free(ctx);
     pta_release(ctx);
+    if (ctx->pta.h_report) hipHostFree(ctx->pta.h_report);
     if (ctx->stream) hipStreamDestroy(ctx->stream);
     delete ctx;
     return TOPK_OK;

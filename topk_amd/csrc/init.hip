@@ -19,6 +19,7 @@ namespace topk {
 
 int pta_build(topk_ctx *ctx);
 void pta_release(topk_ctx *ctx);
+void pta_stale(topk_ctx *ctx);
 int pta_query(topk_ctx *ctx, uint32_t k, uint8_t qq, const float *weights, const uint8_t *attr, const FinalOut &fo);
 
 // Per column max (starting at 0) and min (starting at FLT_MAX) as monotone
@@ -221,10 +222,16 @@ int topk_init(topk_ctx *ctx, uint32_t flags) {
     const double t0 = now_ms();
     int rc = TOPK_OK;
     if (flags & TOPK_INIT_NORMALIZE) {
-        pta_release(ctx);  // a layout built from the old values would be stale
+        // a layout built from the old values would be stale; one built next
+        // reuses its memory
+        if (flags & TOPK_INIT_PTA) pta_stale(ctx);
+        else pta_release(ctx);
         ctx->store_gen++;
         rc = normalize_store(ctx);
-        if (rc) return rc;
+        if (rc) {
+            pta_release(ctx);
+            return rc;
+        }
     }
     if (flags & TOPK_INIT_PTA) {
         rc = pta_build(ctx);

@@ -226,6 +226,10 @@ struct PtaLayout {
     uint64_t generation = 0;     // bumped whenever the layout is freed (rebuilt or released)
     uint64_t npos = 0;           // positions incl. padding (poff[nparts])
     uint64_t ld = 0;             // column stride of pcols
+    // pcols and the bitmaps are allocations of their own, the other device
+    // arrays pieces of the arena; a build's scratch is kept for the next one
+    unsigned char *arena = nullptr, *scratch = nullptr;
+    size_t arena_cap = 0, pcols_cap = 0, scratch_cap = 0;  // bytes
     float *pcols = nullptr;      // d columns in partition order, + one stream tile of padding
     uint32_t *pid = nullptr;     // global object id per position (0xFFFFFFFF: padding)
     uint32_t *cminid = nullptr;  // nchunks: smallest object id of each chunk (0xFFFFFFFF: none)
@@ -241,7 +245,8 @@ struct PtaLayout {
     uint32_t *wchunks = nullptr; // query scratch: chunks to score per cut workgroup
     uint2 *wstat = nullptr;      // query scratch: partitions and objects to score per cut workgroup
     int cus = 0;                 // compute units of the device (the scoring grid)
-    uint32_t *h_report = nullptr; // pinned, written by the query: candidates, partitions, objects (u64)
+    uint32_t *h_report = nullptr; // pinned, written by the query: candidates, partitions, objects (u64); kept
+                                  // over rebuilds (the build reports its sizes there), freed with the context
     // Bound tree: an implicit binary tree over partition ids padded to p2 (a
     // power of two); node v has children 2v, 2v+1 and leaf p is node p2 + p.
     // Leaves are numbered in k-d tree order, so a node is a contiguous,
@@ -277,6 +282,7 @@ struct PtaLayout {
     double tt_build_ms = 0;
 };
 constexpr uint32_t PTA_CHUNK = 256;
+constexpr uint32_t PTA_CUT_GROUPS = 4096;  // cut workgroups of a query at most (the scoring pass scans their totals in LDS)
 constexpr uint32_t PART_ALIGN = 256;
 static_assert(PART_ALIGN % PTA_CHUNK == 0, "partitions start on chunk boundaries");
 

@@ -6,15 +6,11 @@
 // idea -- group similar objects, bound each group, skip groups that cannot
 // reach the running k-th score -- with its own partitioning and bound:
 //
-//  * layout (topk_init with TOPK_INIT_PTA): a k-d tree whose split planes
-//    come from a deterministic sample (median splits on the axis of largest
-//    spread, built on the host); every object is routed to its leaf on the
-//    GPU, objects are counting-sorted by leaf, then ordered inside each
-//    partition by attribute sum (largest first, ties by id); the columns are
-//    gathered into partition order and each partition keeps per-attribute
-//    max/min, the max of its objects' attribute sums and the sum of its
-//    minima, and each 256-object chunk the same statistics over itself and
-//    every later chunk of its partition (suffix rows).
+//  * layout (pta_build.hip): the leaves of a k-d tree, objects ordered by
+//    attribute sum inside each; per partition max/min per attribute, the max
+//    of its objects' attribute sums and the sum of its minima, and each
+//    256-object chunk the same statistics over itself and every later chunk
+//    of its partition (suffix rows).
 //  * bound: the largest weighted sum any point of the partition's box can
 //    reach under the attribute-sum limit (a fractional-knapsack LP, solved
 //    greedily in FP64), plus a margin covering binary32 rounding of a score,
@@ -30,11 +26,6 @@
 #include <string.h>
 
 #include <algorithm>
-#include <chrono>
-#include <cmath>
-#include <numeric>
-#include <thread>
-#include <vector>
 
 #include "bound.hpp"
 #include "device.hpp"
@@ -43,593 +34,12 @@
 namespace topk {
 
 constexpr int PTA_BS = 256;
-constexpr uint32_t PTA_CUT_GROUPS = 4096;  // cut workgroups at most (the scoring pass scans their totals in LDS)
-constexpr uint32_t PTA_SORT_MAX = 8192;      // partitions up to this size are sorted in LDS (larger: scatter order)
 constexpr uint32_t PTA_SEED_OBJS = 1024;     // leading objects (largest attribute sums) of a seed partition
 constexpr uint32_t PTA_MIN_SEED = 16;        // seed partitions at least
 constexpr uint32_t PTA_SEED_RANK = 1024;     // block maxima ranked in LDS by the seed kernel
 constexpr uint32_t PTA_MAX_SEED = 64;
 constexpr int PTA_SEED_REG = 16;             // seed winners per thread the merge reads at once
 constexpr uint32_t PTA_SEED_LDS = PTA_SEED_REG * PTA_BS;  // seed winners the merge ranks in LDS
-
-struct KdNode {
-    float split;
-    uint32_t axis;
-    int32_t left;   // >= 0: internal node, < 0: leaf -(leaf + 1)
-    int32_t right;
-};
-
-// ---------------------------------------------------------------------------
-// layout build kernels
-// ---------------------------------------------------------------------------
-__global__ void pta_sample_kernel(const float *__restrict__ cols, uint64_t ld, uint32_t d, uint64_t n, uint64_t s,
-                                  float *__restrict__ rows) {
-    const uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= s) return;
-    const uint64_t i = j * n / s;
-    for (uint32_t m = 0; m < d; m++) rows[j * d + m] = cols[(uint64_t)m * ld + i];
-}
-
-__global__ void pta_assign_kernel(const float *__restrict__ cols, uint64_t ld, uint64_t n,
-                                  const KdNode *__restrict__ nodes, int32_t root, uint32_t *__restrict__ leaf,
-                                  uint32_t *__restrict__ cnt) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int32_t c = root;
-    while (c >= 0) {
-        const KdNode nd = nodes[c];
-        c = cols[(uint64_t)nd.axis * ld + i] < nd.split ? nd.left : nd.right;
-    }
-    const uint32_t l = (uint32_t)(-c - 1);
-    leaf[i] = l;
-    atomicAdd(&cnt[l], 1u);
-}
-
-__global__ void pta_scatter_kernel(uint64_t n, const uint32_t *__restrict__ leaf, const uint32_t *__restrict__ poff,
-                                   uint32_t *__restrict__ cursor, uint32_t *__restrict__ perm) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t l = leaf[i];
-    perm[poff[l] + atomicAdd(&cursor[l], 1u)] = (uint32_t)i;
-}
-
-// Sorts each partition's objects by attribute sum, largest first (ties by
-// lower id): consecutive positions then hold objects of similar sum, so a
-// chunk's statistics bound its objects more tightly than the partition's.
-// The sum only orders; any rounding is fine.
-__global__ __launch_bounds__(1024) void pta_sort_kernel(const float *__restrict__ cols, uint64_t ld, uint32_t d,
-                                                        const uint32_t *__restrict__ poff,
-                                                        const uint32_t *__restrict__ psz,
-                                                        uint32_t *__restrict__ perm) {
-    __shared__ uint64_t a[PTA_SORT_MAX];
-    const uint32_t p = blockIdx.x, s = psz[p];
-    if (s < 2 || s > PTA_SORT_MAX) return;
-    uint32_t *seg = perm + poff[p];
-    uint32_t n2 = 1;
-    while (n2 < s) n2 <<= 1;
-    for (uint32_t i = threadIdx.x; i < n2; i += 1024) {
-        uint64_t key = 0;
-        if (i < s) {
-            const uint32_t id = seg[i];
-            float sum = 0.0f;
-            for (uint32_t m = 0; m < d; m++) sum += cols[(uint64_t)m * ld + id];
-            key = rkey(sum, id);
-        }
-        a[i] = key;
-    }
-    __syncthreads();
-    for (uint32_t size = 2; size <= n2; size <<= 1)
-        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-            for (uint32_t t = threadIdx.x; t < n2 / 2; t += 1024) {
-                const uint32_t lo = 2 * stride * (t / stride) + (t & (stride - 1)), hi = lo + stride;
-                const bool desc = (lo & size) == 0;
-                const uint64_t x = a[lo], y = a[hi];
-                if ((x < y) == desc) {
-                    a[lo] = y;
-                    a[hi] = x;
-                }
-            }
-            __syncthreads();
-        }
-    for (uint32_t i = threadIdx.x; i < s; i += 1024) seg[i] = rkey_id(a[i]);
-}
-
-__global__ void pta_gather_kernel(const float *__restrict__ cols, uint64_t ld, uint32_t d, uint64_t npos,
-                                  const uint32_t *__restrict__ perm, float *__restrict__ pcols, uint64_t ldp,
-                                  uint32_t *__restrict__ pid) {
-    const uint64_t pos = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (pos >= npos) return;
-    const uint32_t id = perm[pos];
-    pid[pos] = id;
-    for (uint32_t m = 0; m < d; m++) pcols[(uint64_t)m * ldp + pos] = id != 0xFFFFFFFFu ? cols[(uint64_t)m * ld + id] : 0.0f;
-}
-
-// One block per partition: per-attribute max/min, the max attribute sum
-// (FP64, rounded up) and the sum of the minima (FP64, rounded down).
-__global__ __launch_bounds__(PTA_BS) void pta_bounds_kernel(const float *__restrict__ pcols, uint64_t ldp, uint32_t d,
-                                                            const uint32_t *__restrict__ poff,
-                                                            const uint32_t *__restrict__ psz,
-                                                            float *__restrict__ pmax, float *__restrict__ pmin,
-                                                            float *__restrict__ psum, float *__restrict__ pminsum) {
-    __shared__ float smax[PTA_BS / 64], smin[PTA_BS / 64];
-    __shared__ double ssum[PTA_BS / 64];
-    __shared__ float colmin[TOPK_MAX_DIMS];
-    const uint32_t p = blockIdx.x, start = poff[p], s = psz[p];
-    const uint32_t w = threadIdx.x / 64;
-    for (uint32_t m = 0; m < d; m++) {
-        float mx = -INFINITY, mn = INFINITY;
-        for (uint32_t i = threadIdx.x; i < s; i += PTA_BS) {
-            const float v = pcols[(uint64_t)m * ldp + start + i];
-            mx = v > mx ? v : mx;
-            mn = v < mn ? v : mn;
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-            mn = fminf(mn, __shfl_xor(mn, o, 64));
-        }
-        if (lane_id() == 0) { smax[w] = mx; smin[w] = mn; }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            for (int j = 1; j < PTA_BS / 64; j++) { mx = fmaxf(mx, smax[j]); mn = fminf(mn, smin[j]); }
-            pmax[(uint64_t)p * d + m] = s ? mx : 0.0f;
-            pmin[(uint64_t)p * d + m] = s ? mn : 0.0f;
-            colmin[m] = s ? mn : 0.0f;
-        }
-        __syncthreads();
-    }
-    double best = -INFINITY;
-    for (uint32_t i = threadIdx.x; i < s; i += PTA_BS) {
-        double t = 0;
-        for (uint32_t m = 0; m < d; m++) t += (double)pcols[(uint64_t)m * ldp + start + i];
-        best = t > best ? t : best;
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        const double t = __shfl_xor(best, o, 64);
-        best = t > best ? t : best;
-    }
-    if (lane_id() == 0) ssum[w] = best;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int j = 1; j < PTA_BS / 64; j++) best = ssum[j] > best ? ssum[j] : best;
-        double ms = 0;
-        for (uint32_t m = 0; m < d; m++) ms += (double)colmin[m];
-        psum[p] = s ? f32_round_up(best) : -INFINITY;
-        pminsum[p] = s ? f32_round_down(ms) : 0.0f;
-    }
-}
-
-// One wave per chunk of PTA_CHUNK positions: element e of chunk c (at
-// cstat[e * nchunks + c]) holds the chunk's per-attribute maxima (e in
-// [0, d)) and minima ([d, 2d)), the largest attribute sum of its objects
-// (FP64, rounded up) at 2d and the sum of its minima (FP64, rounded down)
-// at 2d + 1.  A chunk without objects has sum -inf.  cminid[c] gets the
-// chunk's smallest object id (0xFFFFFFFF: none).
-__global__ __launch_bounds__(256) void pta_chunk_kernel(const float *__restrict__ pcols, uint64_t ldp, uint32_t d,
-                                                        const uint32_t *__restrict__ pid, uint64_t nchunks,
-                                                        float *__restrict__ cstat, uint32_t *__restrict__ cminid) {
-    const uint64_t c = (uint64_t)blockIdx.x * 4 + threadIdx.x / 64;
-    if (c >= nchunks) return;
-    const uint32_t lane = lane_id();
-    constexpr uint32_t PER = PTA_CHUNK / 64;
-    const uint64_t pos0 = c * PTA_CHUNK + lane * PER;
-    bool ok[PER];
-    bool any = false;
-    uint32_t idmin = 0xFFFFFFFFu;  // padding positions hold id 0xFFFFFFFF
-#pragma unroll
-    for (uint32_t j = 0; j < PER; j++) {
-        const uint32_t id = pid[pos0 + j];
-        ok[j] = id != 0xFFFFFFFFu;
-        any |= ok[j];
-        idmin = id < idmin ? id : idmin;
-    }
-    const bool nonempty = __ballot(any) != 0;
-    for (int o = 32; o > 0; o >>= 1) {
-        const uint32_t t = (uint32_t)__shfl_xor((int)idmin, o, 64);
-        idmin = t < idmin ? t : idmin;
-    }
-    if (lane == 0) cminid[c] = idmin;
-    float *row = cstat + c;  // element e at row[e * nchunks]
-    double best = -INFINITY, minsum = 0.0;
-    double sums[PER];
-#pragma unroll
-    for (uint32_t j = 0; j < PER; j++) sums[j] = 0.0;
-    for (uint32_t m = 0; m < d; m++) {
-        float mx = -INFINITY, mn = INFINITY;
-#pragma unroll
-        for (uint32_t j = 0; j < PER; j++) {
-            const float v = pcols[(uint64_t)m * ldp + pos0 + j];
-            if (ok[j]) {
-                mx = v > mx ? v : mx;
-                mn = v < mn ? v : mn;
-                sums[j] += (double)v;
-            }
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-            mn = fminf(mn, __shfl_xor(mn, o, 64));
-        }
-        minsum += (double)mn;
-        if (lane == 0) {
-            row[m * nchunks] = nonempty ? mx : 0.0f;
-            row[(d + m) * nchunks] = nonempty ? mn : 0.0f;
-        }
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < PER; j++) best = ok[j] && sums[j] > best ? sums[j] : best;
-    for (int o = 32; o > 0; o >>= 1) {
-        const double t = __shfl_xor(best, o, 64);
-        best = t > best ? t : best;
-    }
-    if (lane == 0) {
-        row[2 * d * nchunks] = nonempty ? f32_round_up(best) : -INFINITY;
-        row[(2 * d + 1) * nchunks] = nonempty ? f32_round_down(minsum) : 0.0f;
-    }
-}
-
-// One thread per partition turns its chunk rows into suffix rows: row c
-// then bounds chunks c, c + 1, ... of the partition (per-attribute maxima and
-// minima, the largest attribute sum, and the sum of the union's minima in
-// FP64 rounded down), so a partition's row bounds never increase with c.
-__global__ __launch_bounds__(256) void pta_chunk_suffix_kernel(uint32_t L, uint32_t d,
-                                                               const uint32_t *__restrict__ poff,
-                                                               const uint32_t *__restrict__ psz, uint64_t nchunks,
-                                                               float *__restrict__ cstat) {
-    const uint32_t p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= L || psz[p] == 0) return;
-    const uint32_t c0 = poff[p] / PTA_CHUNK, n = (psz[p] + PTA_CHUNK - 1) / PTA_CHUNK;
-    const uint64_t S = nchunks;  // element stride
-    for (uint32_t i = n - 1; i > 0; i--) {
-        const float *nx = cstat + (c0 + i);
-        float *row = cstat + (c0 + i - 1);
-        double ms = 0.0;
-        for (uint32_t m = 0; m < d; m++) {
-            row[m * S] = fmaxf(row[m * S], nx[m * S]);
-            row[(d + m) * S] = fminf(row[(d + m) * S], nx[(d + m) * S]);
-            ms += (double)row[(d + m) * S];
-        }
-        row[2 * d * S] = fmaxf(row[2 * d * S], nx[2 * d * S]);
-        row[(2 * d + 1) * S] = f32_round_down(ms);
-    }
-}
-
-// ---------------------------------------------------------------------------
-// host: k-d tree on the sample
-// ---------------------------------------------------------------------------
-namespace {
-
-struct KdBuilder {
-    const float *rows;
-    uint32_t d;
-    std::vector<uint32_t> idx;
-    std::vector<KdNode> nodes;  // internal node for the split between leaves m-1 and m is nodes[m-1]
-
-    // Builds the subtree holding leaves [leaf_lo, leaf_lo + nl) from sample
-    // rows idx[lo, hi); returns its node code.
-    int32_t build(size_t lo, size_t hi, uint32_t leaf_lo, uint32_t nl, int depth) {
-        if (nl == 1) return -(int32_t)leaf_lo - 1;
-        const uint32_t nleft = nl / 2;
-        const size_t mid = lo + (hi - lo) * nleft / nl;
-        uint32_t axis = 0;
-        float split = INFINITY;
-        if (hi > lo) {
-            float best = -1.0f;
-            for (uint32_t m = 0; m < d; m++) {
-                float mn = INFINITY, mx = -INFINITY;
-                for (size_t j = lo; j < hi; j++) {
-                    const float v = rows[(size_t)idx[j] * d + m];
-                    mn = v < mn ? v : mn;
-                    mx = v > mx ? v : mx;
-                }
-                if (mx - mn > best) { best = mx - mn; axis = m; }
-            }
-            if (mid < hi) {
-                auto less = [&](uint32_t a, uint32_t b) {
-                    const float va = rows[(size_t)a * d + axis], vb = rows[(size_t)b * d + axis];
-                    return va < vb || (va == vb && a < b);
-                };
-                std::nth_element(idx.begin() + lo, idx.begin() + mid, idx.begin() + hi, less);
-                split = rows[(size_t)idx[mid] * d + axis];
-            }
-        }
-        const int32_t me = (int32_t)(leaf_lo + nleft - 1);
-        int32_t l, r;
-        if (depth < 4 && hi - lo > 65536) {
-            std::thread th([&] { l = build(lo, mid, leaf_lo, nleft, depth + 1); });
-            r = build(mid, hi, leaf_lo + nleft, nl - nleft, depth + 1);
-            th.join();
-        } else {
-            l = build(lo, mid, leaf_lo, nleft, depth + 1);
-            r = build(mid, hi, leaf_lo + nleft, nl - nleft, depth + 1);
-        }
-        nodes[me] = KdNode{split, axis, l, r};
-        return me;
-    }
-};
-
-}  // namespace
-
-static double now_ms() {
-    return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now().time_since_epoch()).count();
-}
-
-static float round_down_f32(double x) {
-    float f = (float)x;
-    if ((double)f > x) f = std::nextafter(f, -INFINITY);
-    return f;
-}
-
-// Aggregates the per-partition bounds bottom-up into the bound tree.
-static int build_bound_tree(PtaLayout &P, uint32_t d, hipStream_t s) {
-    const uint32_t L = P.nparts;
-    uint32_t p2 = 1;
-    while (p2 < L) p2 <<= 1;
-    const size_t nn = 2 * (size_t)p2;
-    std::vector<float> mx(nn * d, -INFINITY), mn(nn * d, INFINITY), sm(nn, -INFINITY), ms(nn, 0.0f);
-    std::vector<uint32_t> sz(L), off(L + 1), cmin(P.nchunks), idm(nn, 0xFFFFFFFFu);
-    TK_HIP(hipMemcpyAsync(mx.data() + (size_t)p2 * d, P.pmax, sizeof(float) * L * d, hipMemcpyDeviceToHost, s));
-    TK_HIP(hipMemcpyAsync(mn.data() + (size_t)p2 * d, P.pmin, sizeof(float) * L * d, hipMemcpyDeviceToHost, s));
-    TK_HIP(hipMemcpyAsync(sm.data() + p2, P.psum, sizeof(float) * L, hipMemcpyDeviceToHost, s));
-    TK_HIP(hipMemcpyAsync(ms.data() + p2, P.pminsum, sizeof(float) * L, hipMemcpyDeviceToHost, s));
-    TK_HIP(hipMemcpyAsync(sz.data(), P.psz, sizeof(uint32_t) * L, hipMemcpyDeviceToHost, s));
-    TK_HIP(hipMemcpyAsync(off.data(), P.poff, sizeof(uint32_t) * (L + 1), hipMemcpyDeviceToHost, s));
-    if (P.nchunks)
-        TK_HIP(hipMemcpyAsync(cmin.data(), P.cminid, sizeof(uint32_t) * P.nchunks, hipMemcpyDeviceToHost, s));
-    TK_HIP(hipStreamSynchronize(s));
-    // smallest id per partition (its chunks), then per node
-    for (uint32_t p = 0; p < L; p++) {
-        uint32_t m = 0xFFFFFFFFu;
-        if (sz[p])
-            for (uint64_t c = off[p] / PTA_CHUNK; c < ((uint64_t)off[p] + sz[p] + PTA_CHUNK - 1) / PTA_CHUNK; c++)
-                m = std::min(m, cmin[c]);
-        idm[p2 + p] = m;
-    }
-    for (size_t v = p2 - 1; v >= 1; v--) idm[v] = std::min(idm[2 * v], idm[2 * v + 1]);
-    for (uint32_t p = 0; p < L; p++)
-        if (!sz[p]) {  // empty partition: identity box
-            for (uint32_t m = 0; m < d; m++) {
-                mx[(size_t)(p2 + p) * d + m] = -INFINITY;
-                mn[(size_t)(p2 + p) * d + m] = INFINITY;
-            }
-            sm[p2 + p] = -INFINITY;
-        }
-    for (size_t v = p2 - 1; v >= 1; v--) {
-        const size_t a = 2 * v, b = 2 * v + 1;
-        bool any = false;
-        for (uint32_t m = 0; m < d; m++) {
-            mx[v * d + m] = std::max(mx[a * d + m], mx[b * d + m]);
-            mn[v * d + m] = std::min(mn[a * d + m], mn[b * d + m]);
-        }
-        sm[v] = std::max(sm[a], sm[b]);
-        any = sm[v] > -INFINITY;
-        double t = 0;
-        for (uint32_t m = 0; m < d; m++) t += any ? (double)mn[v * d + m] : 0.0;
-        ms[v] = any ? round_down_f32(t) : 0.0f;
-    }
-    P.p2 = p2;
-    // attribute-major copies for the device: attribute m of node v at [m * nn + v]
-    std::vector<float> mxt(nn * d), mnt(nn * d);
-    for (size_t v = 0; v < nn; v++)
-        for (uint32_t m = 0; m < d; m++) {
-            mxt[m * nn + v] = mx[v * d + m];
-            mnt[m * nn + v] = mn[v * d + m];
-        }
-    TK_HIP(hipMalloc(&P.tmax, sizeof(float) * nn * d));
-    TK_HIP(hipMalloc(&P.tmin, sizeof(float) * nn * d));
-    TK_HIP(hipMalloc(&P.tsum, sizeof(float) * nn));
-    TK_HIP(hipMalloc(&P.tminsum, sizeof(float) * nn));
-    TK_HIP(hipMalloc(&P.tminid, sizeof(uint32_t) * nn));
-    TK_HIP(hipMemcpyAsync(P.tminid, idm.data(), sizeof(uint32_t) * nn, hipMemcpyHostToDevice, s));
-    TK_HIP(hipMemcpyAsync(P.tmax, mxt.data(), sizeof(float) * nn * d, hipMemcpyHostToDevice, s));
-    TK_HIP(hipMemcpyAsync(P.tmin, mnt.data(), sizeof(float) * nn * d, hipMemcpyHostToDevice, s));
-    TK_HIP(hipMemcpyAsync(P.tsum, sm.data(), sizeof(float) * nn, hipMemcpyHostToDevice, s));
-    TK_HIP(hipMemcpyAsync(P.tminsum, ms.data(), sizeof(float) * nn, hipMemcpyHostToDevice, s));
-    TK_HIP(hipStreamSynchronize(s));
-    return TOPK_OK;
-}
-
-static void pta_free(PtaLayout &P) {
-    hipFree(P.pcols);
-    hipFree(P.pid);
-    hipFree(P.poff);
-    hipFree(P.psz);
-    hipFree(P.pmax);
-    hipFree(P.pmin);
-    hipFree(P.psum);
-    hipFree(P.pminsum);
-    hipFree(P.pbound);
-    hipFree(P.bmax);
-    hipFree(P.pcut);
-    hipFree(P.wchunks);
-    hipFree(P.wstat);
-    if (P.h_report) hipHostFree(P.h_report);
-    hipFree(P.tmax);
-    hipFree(P.tmin);
-    hipFree(P.tsum);
-    hipFree(P.tminsum);
-    hipFree(P.cstat);
-    hipFree(P.cminid);
-    hipFree(P.tminid);
-    hipFree(P.xbits);
-    const uint32_t psize = P.psize;
-    const uint64_t gen = P.generation;
-    P = PtaLayout();
-    P.psize = psize;
-    P.generation = gen + 1;
-}
-
-// One wave per (row, word): lane i reads object 64 w + i of the attribute
-// and the ballot of "equals the store's largest / smallest value" is the word.
-__global__ __launch_bounds__(256) void extreme_bits_kernel(const float *__restrict__ cols, uint64_t ld, uint64_t n,
-                                                           uint32_t d, const float *__restrict__ rmax,
-                                                           const float *__restrict__ rmin, uint64_t rstride,
-                                                           uint64_t nw, uint64_t *__restrict__ bits) {
-    const uint32_t lane = lane_id();
-    const uint64_t nwaves = (uint64_t)gridDim.x * 4;
-    for (uint64_t v = (uint64_t)blockIdx.x * 4 + threadIdx.x / 64; v < (uint64_t)d * nw; v += nwaves) {
-        const uint32_t a = (uint32_t)(v / nw);
-        const uint64_t w = v - (uint64_t)a * nw, id = 64 * w + lane;
-        const float x = id < n ? cols[(uint64_t)a * ld + id] : 0.0f;
-        const uint64_t hi = __ballot(id < n && x == rmax[a * rstride]);
-        const uint64_t lo = __ballot(id < n && x == rmin[a * rstride]);
-        if (lane == 0) {
-            bits[(uint64_t)a * nw + w] = hi;
-            bits[(uint64_t)(d + a) * nw + w] = lo;
-        }
-    }
-}
-
-int pta_extreme_bits(topk_ctx *ctx) {
-    PtaLayout &P = ctx->pta;
-    if (!P.built) return TOPK_ERR_STATE;
-    if (P.xbits) return TOPK_OK;
-    const uint64_t nw = ((ctx->n + 63) / 64 + 15) & ~15ull;  // padding words hold ids >= n: zero
-    TK_HIP(hipMalloc(&P.xbits, sizeof(uint64_t) * 2 * ctx->d * nw));
-    P.nw = nw;
-    const uint64_t waves = (uint64_t)ctx->d * nw;
-    const uint32_t grid = (uint32_t)std::min<uint64_t>((waves + 3) / 4, 65536);
-    hipLaunchKernelGGL(extreme_bits_kernel, dim3(grid), dim3(256), 0, ctx->stream, ctx->cols, ctx->ld, ctx->n, ctx->d,
-                       P.tmax + 1, P.tmin + 1, 2 * (uint64_t)P.p2, nw, P.xbits);
-    TK_HIP(hipGetLastError());
-    TK_HIP(hipStreamSynchronize(ctx->stream));
-    return TOPK_OK;
-}
-
-void pta_release(topk_ctx *ctx) {
-    batch_quiesce(ctx);  // batches in flight read the layout
-    pta_free(ctx->pta);
-}
-
-int pta_build(topk_ctx *ctx) {
-    const double t0 = now_ms();
-    PtaLayout &P = ctx->pta;
-    pta_release(ctx);
-    const uint64_t n = ctx->n;
-    const uint32_t d = ctx->d;
-    hipStream_t s = ctx->stream;
-    if (n >= ID_LIMIT) return TOPK_ERR_UNSUPPORTED;  // positions and partition ids are 32-bit
-    const uint64_t want = (n + P.psize - 1) / P.psize;
-    const uint32_t L = (uint32_t)(want < PTA_MAX_PARTS ? want : PTA_MAX_PARTS);
-
-    // 1. deterministic sample -> host k-d tree with L leaves
-    uint64_t ns = (uint64_t)L * 64;
-    if (ns < (1u << 20)) ns = 1u << 20;
-    if (ns > n) ns = n;
-    std::vector<float> rows((size_t)ns * d);
-    {
-        float *d_rows = nullptr;
-        TK_HIP(hipMalloc(&d_rows, sizeof(float) * ns * d));
-        hipLaunchKernelGGL(pta_sample_kernel, dim3((uint32_t)((ns + 255) / 256)), dim3(256), 0, s, ctx->cols,
-                           ctx->ld, d, n, ns, d_rows);
-        hipError_t e = hipMemcpyAsync(rows.data(), d_rows, sizeof(float) * ns * d, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        hipFree(d_rows);
-        TK_HIP(e);
-    }
-    KdBuilder kb{rows.data(), d, std::vector<uint32_t>(ns), std::vector<KdNode>(L > 1 ? L - 1 : 1)};
-    std::iota(kb.idx.begin(), kb.idx.end(), 0u);
-    const int32_t root = kb.build(0, ns, 0, L, 0);
-
-    // 2. route every object to its leaf and count
-    KdNode *d_nodes = nullptr;
-    uint32_t *leaf = nullptr, *cnt = nullptr, *cursor = nullptr, *perm = nullptr;
-    int rc = TOPK_OK;
-    auto cleanup = [&] {
-        hipFree(d_nodes);
-        hipFree(leaf);
-        hipFree(cnt);
-        hipFree(cursor);
-    };
-#define TK_TRY(call)                                              \
-    do {                                                          \
-        hipError_t e_ = (call);                                   \
-        if (e_ != hipSuccess) { rc = hip_status(e_); goto fail; } \
-    } while (0)
-    {
-        TK_TRY(hipMalloc(&d_nodes, sizeof(KdNode) * kb.nodes.size()));
-        TK_TRY(hipMemcpyAsync(d_nodes, kb.nodes.data(), sizeof(KdNode) * kb.nodes.size(), hipMemcpyHostToDevice, s));
-        TK_TRY(hipMalloc(&leaf, sizeof(uint32_t) * n));
-        TK_TRY(hipMalloc(&cnt, sizeof(uint32_t) * L));
-        TK_TRY(hipMalloc(&cursor, sizeof(uint32_t) * L));
-        TK_TRY(hipMemsetAsync(cnt, 0, sizeof(uint32_t) * L, s));
-        TK_TRY(hipMemsetAsync(cursor, 0, sizeof(uint32_t) * L, s));
-        hipLaunchKernelGGL(pta_assign_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, ctx->cols, ctx->ld, n,
-                           d_nodes, root, leaf, cnt);
-        std::vector<uint32_t> h_cnt(L), h_off(L + 1);
-        TK_TRY(hipMemcpyAsync(h_cnt.data(), cnt, sizeof(uint32_t) * L, hipMemcpyDeviceToHost, s));
-        TK_TRY(hipStreamSynchronize(s));
-        uint64_t acc = 0;
-        for (uint32_t p = 0; p < L; p++) {
-            P.nonempty += h_cnt[p] ? 1u : 0u;
-            P.maxsz = h_cnt[p] > P.maxsz ? h_cnt[p] : P.maxsz;
-            h_off[p] = (uint32_t)acc;
-            acc += ((uint64_t)h_cnt[p] + PART_ALIGN - 1) / PART_ALIGN * PART_ALIGN;
-        }
-        h_off[L] = (uint32_t)acc;
-        if (acc >= 0xFFFFFFFFull) { rc = TOPK_ERR_UNSUPPORTED; goto fail; }
-        P.nparts = L;
-        P.npos = acc;
-        P.ld = (acc + 8191) / 8192 * 8192;
-        TK_TRY(hipMalloc(&P.poff, sizeof(uint32_t) * (L + 1)));
-        TK_TRY(hipMalloc(&P.psz, sizeof(uint32_t) * L));
-        TK_TRY(hipMemcpyAsync(P.poff, h_off.data(), sizeof(uint32_t) * (L + 1), hipMemcpyHostToDevice, s));
-        TK_TRY(hipMemcpyAsync(P.psz, h_cnt.data(), sizeof(uint32_t) * L, hipMemcpyHostToDevice, s));
-        TK_TRY(hipStreamSynchronize(s));  // host vectors go out of scope
-
-        // 3. counting sort by leaf, then by attribute sum inside each partition
-        TK_TRY(hipMalloc(&perm, sizeof(uint32_t) * P.ld));
-        TK_TRY(hipMemsetAsync(perm, 0xFF, sizeof(uint32_t) * P.ld, s));
-        hipLaunchKernelGGL(pta_scatter_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, s, n, leaf, P.poff,
-                           cursor, perm);
-        hipLaunchKernelGGL(pta_sort_kernel, dim3(L), dim3(1024), 0, s, ctx->cols, ctx->ld, d, P.poff, P.psz, perm);
-
-        // 4. partition-order columns and bounds
-        const size_t pfl = P.ld * d + 8192;
-        TK_TRY(hipMalloc(&P.pcols, sizeof(float) * pfl));
-        TK_TRY(hipMemsetAsync(P.pcols, 0, sizeof(float) * pfl, s));
-        P.pid = perm;
-        perm = nullptr;
-        hipLaunchKernelGGL(pta_gather_kernel, dim3((uint32_t)((P.ld + 255) / 256)), dim3(256), 0, s, ctx->cols,
-                           ctx->ld, d, P.ld, P.pid, P.pcols, P.ld, P.pid);
-        TK_TRY(hipMalloc(&P.pmax, sizeof(float) * L * d));
-        TK_TRY(hipMalloc(&P.pmin, sizeof(float) * L * d));
-        TK_TRY(hipMalloc(&P.psum, sizeof(float) * L));
-        TK_TRY(hipMalloc(&P.pminsum, sizeof(float) * L));
-        hipLaunchKernelGGL(pta_bounds_kernel, dim3(L), dim3(PTA_BS), 0, s, P.pcols, P.ld, d, P.poff, P.psz, P.pmax,
-                           P.pmin, P.psum, P.pminsum);
-        P.nchunks = P.npos / PTA_CHUNK;
-        P.crow = 2 * d + 2;
-        TK_TRY(hipMalloc(&P.cstat, sizeof(float) * (P.nchunks ? P.nchunks : 1) * P.crow));
-        TK_TRY(hipMalloc(&P.cminid, sizeof(uint32_t) * (P.nchunks ? P.nchunks : 1)));
-        if (P.nchunks)
-            hipLaunchKernelGGL(pta_chunk_kernel, dim3((uint32_t)((P.nchunks + 3) / 4)), dim3(256), 0, s, P.pcols, P.ld,
-                               d, P.pid, (uint64_t)P.nchunks, P.cstat, P.cminid);
-        if (P.nchunks)
-            hipLaunchKernelGGL(pta_chunk_suffix_kernel, dim3((L + 255) / 256), dim3(256), 0, s, L, d, P.poff, P.psz,
-                               (uint64_t)P.nchunks, P.cstat);
-        TK_TRY(hipMalloc(&P.pbound, sizeof(uint64_t) * L));
-        TK_TRY(hipMalloc(&P.bmax, sizeof(uint64_t) * ((L + PTA_BS - 1) / PTA_BS)));
-        TK_TRY(hipMalloc(&P.pcut, sizeof(uint32_t) * L));
-        TK_TRY(hipMalloc(&P.wchunks, sizeof(uint32_t) * PTA_CUT_GROUPS));
-        TK_TRY(hipMalloc(&P.wstat, sizeof(uint2) * PTA_CUT_GROUPS));
-        TK_TRY(hipHostMalloc(&P.h_report, sizeof(uint32_t) * 4, hipHostMallocDefault));
-        TK_TRY(hipDeviceGetAttribute(&P.cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-        if (P.cus < 1) P.cus = 1;
-        TK_TRY(hipGetLastError());
-        TK_TRY(hipStreamSynchronize(s));
-        rc = build_bound_tree(P, d, s);
-        if (rc) goto fail;
-    }
-#undef TK_TRY
-    cleanup();
-    P.built = true;
-    P.tt_build_ms = now_ms() - t0;
-    return TOPK_OK;
-fail:
-    cleanup();
-    hipFree(perm);
-    pta_free(P);
-    return rc;
-}
 
 // ---------------------------------------------------------------------------
 // query kernels
