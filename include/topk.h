@@ -373,7 +373,8 @@ void *topk_stream(topk_ctx *ctx);
  *                     (1024 for d <= 8 with batch_vpt 4)
  *   "batch_qpi"       query budget of a batch work item (16..1024): a
  *                     partition is loaded once per item and scored for up
- *                     to this many of the queries that reach it
+ *                     to this many of the queries that reach it (0 = 4..64,
+ *                     by the entries of the batch's work lists)
  *   "batch_digit"     radix digit width of the per-query select: 8 or 11
  *   "batch_grid"      persistent batch scoring workgroups
  *   "batch_item"      objects of a partition per batch work item (a multiple
@@ -394,8 +395,9 @@ void *topk_stream(topk_ctx *ctx);
  *                     persistent scoring kernel); 2 = the query-major fused
  *                     pass: one workgroup per query bounds the groups,
  *                     partitions and chunks and scores the chunks that
- *                     reach the threshold, with no work list (0 = 1, or the
- *                     autotuner's choice)
+ *                     reach the threshold, with no work list (0 = the
+ *                     autotuner's choice, else 1 if a work-item shape
+ *                     above is set, else 2 for few queries x objects)
  *   "mlp_train"       predictor training: 0 = two launches per mini-batch
  *                     step (default), 1 = one cooperative launch for all
  *                     steps (same parameters)

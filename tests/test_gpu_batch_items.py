@@ -1,0 +1,50 @@
+"""Candidate staging, item order and the choice of pass of the batched path
+against the oracle (cpu/TPAc.h:209-254 findTopKsimdMQ), bit for bit."""
+import numpy as np
+import pytest
+
+import topk_amd
+from test_gpu_batch import make_queries, oracle_batch
+
+pytestmark = pytest.mark.gpu
+
+
+def check(eng, x, qs):
+    ref = oracle_batch(x, x.shape[1], qs)
+    for i, ((gi, gs, _), (ri, rs)) in enumerate(zip(eng.batch(qs), ref)):
+        assert np.array_equal(gi, ri) and np.array_equal(gs.view(np.uint32), rs.view(np.uint32)), i
+
+
+SHAPES = [(8, 4, 256), (8, 8, 512), (8, 16, 256), (8, 16, 512), (8, 4, 1024), (16, 2, 256), (16, 4, 512), (16, 8, 256),
+          (20, 2, 512), (20, 4, 256)]
+
+
+@pytest.mark.parametrize("d,vpt,bs", SHAPES)
+def test_stage_fills(gpu, d, vpt, bs):
+    """Few distinct values: every tile of a query is full of candidates and of
+    ties, the stage overflows inside an item; 70 queries cross a lane block."""
+    rng = np.random.default_rng(d * vpt + bs)
+    n = 30_001
+    x = (np.rint(rng.random((d, n)) * 3) / 3).astype(np.float32)
+    for order in ("sorted", "shuffled"):
+        qs = make_queries(rng, 70, d, [1, 64, 1024], order=order, mmax=4)
+        with topk_amd.Engine(x) as eng:
+            for name, v in (("batch_fused", 1), ("batch_vpt", vpt), ("batch_bs", bs)):
+                eng.set_tuning(name, v)
+            for qpi in (0, 16, 128):
+                eng.set_tuning("batch_qpi", qpi)
+                check(eng, x, qs)
+
+
+@pytest.mark.parametrize("nq", [1, 3, 64, 65, 1024])
+@pytest.mark.parametrize("d,n", [(6, 1), (8, 4097), (8, 262_144), (8, 262_145), (12, 16_384), (12, 16_385), (17, 5000)])
+def test_choice_of_pass(gpu, d, n, nq):
+    """Both sides of the limits between the two passes, and the smallest and
+    largest query budgets the entries give."""
+    rng = np.random.default_rng(n + nq)
+    x = topk_amd.generate(n, d, topk_amd.ANTICORRELATED, n)
+    qs = make_queries(rng, nq, d, [1, 16, 100])
+    with topk_amd.Engine(x) as eng:
+        check(eng, x, qs)
+        eng.set_tuning("batch_fused", 1)
+        check(eng, x, qs)

@@ -22,12 +22,13 @@
 //     reaches tau_q, then their partitions; q is appended to the query list
 //     of every partition whose bound reaches tau_q.
 //  3. compaction (one thread per partition): each query list becomes work
-//     items of at most qpi queries over object chunks; items with many
-//     (object, query) pairs go to the front of the list.
+//     items of at most qpi queries (by default as the entries allow) over
+//     object chunks; items with many (object, query) pairs go to the front
+//     of the list.
 //  4. scoring (persistent workgroups taking items from a global ticket):
 //     a workgroup loads the chunk's objects into registers once and scores
-//     them for every query of the item; survivors are appended to the
-//     query's candidate list (wave-aggregated atomic).  Scores use the
+//     them for every query of the item; survivors are staged in LDS and
+//     appended to the queries' candidate lists.  Scores use the
 //     query's own term order: a fixed ascending register walk when the terms
 //     are ascending, else a wave-uniform switch on the attribute id.
 //  5. final select per query (one workgroup each): radix select over the
@@ -530,13 +531,17 @@ __global__ __launch_bounds__(BMASK_BS) void batch_mask_query_kernel(const BatchQ
                                                                     uint32_t G, uint32_t H, uint32_t L, uint32_t nq,
                                                                     unsigned int *__restrict__ pcnt,
                                                                     uint16_t *__restrict__ plist,
+                                                                    unsigned int *__restrict__ ctr,
                                                                     const uint32_t *__restrict__ qflag) {
     constexpr int U = 32 / NB;
     __shared__ uint32_t list[BMASK_PAIRS];
-    __shared__ uint32_t nlist;
+    __shared__ uint32_t nlist, nent;
     const uint32_t q = blockIdx.x, y = blockIdx.y, S = gridDim.y, tid = threadIdx.x;
     if (qflag && qflag[q] == QF_DONE) return;  // second pass: settled queries take no part
-    if (tid == 0) nlist = 0;
+    if (tid == 0) {
+        nlist = 0;
+        nent = 0;
+    }
     __syncthreads();
     const BoundArgs &b = qb[q];
     const float tau = qs[q].tau;
@@ -548,6 +553,7 @@ __global__ __launch_bounds__(BMASK_BS) void batch_mask_query_kernel(const BatchQ
     }
     __syncthreads();
     const uint32_t nl = nlist, per = 1u << H, total = nl * per;
+    uint32_t mine = 0;
     for (uint32_t i0 = tid; i0 < total; i0 += U * BMASK_BS) {
         uint32_t p[U];
         bool in[U];
@@ -563,8 +569,15 @@ __global__ __launch_bounds__(BMASK_BS) void batch_mask_query_kernel(const BatchQ
         for (int u = 0; u < U; u++) pos[u] = in[u] ? atomicAdd(&pcnt[p[u]], 1u) : 0u;
 #pragma unroll
         for (int u = 0; u < U; u++)
-            if (in[u]) plist[(uint64_t)p[u] * nq + pos[u]] = (uint16_t)q;
+            if (in[u]) {
+                plist[(uint64_t)p[u] * nq + pos[u]] = (uint16_t)q;
+                mine++;
+            }
     }
+    mine = wave_sum_u32(mine);
+    if (lane_id() == 0 && mine) atomicAdd(&nent, mine);
+    __syncthreads();
+    if (tid == 0 && nent) atomicAdd(reinterpret_cast<unsigned long long *>(ctr + 2), (unsigned long long)nent);
 }
 
 // Group-major mask: workgroup (g, y) takes group g of 2^H partitions (tree node G + g) and
@@ -581,6 +594,7 @@ __global__ __launch_bounds__(BMASK_BS) void batch_mask_kernel(const BatchQuery *
                                                               uint32_t G, uint32_t H, uint32_t L, uint32_t nq,
                                                               uint32_t QS, unsigned int *__restrict__ pcnt,
                                                               uint16_t *__restrict__ plist,
+                                                              unsigned int *__restrict__ ctr,
                                                               const uint32_t *__restrict__ qflag) {
     constexpr int U = 32 / NB;  // bounds in flight per thread (registers: ~4 NB per bound)
     __shared__ uint16_t lq[BMASK_PAIRS];   // listed queries
@@ -621,9 +635,12 @@ __global__ __launch_bounds__(BMASK_BS) void batch_mask_kernel(const BatchQuery *
         }
     }
     __syncthreads();
-    if (tid < per) {
-        const uint32_t c = lcnt[tid];
+    static_assert(BMASK_MAX_PER == 64, "wave 0 holds a group's partitions");
+    if (tid < 64) {
+        const uint32_t c = tid < per ? lcnt[tid] : 0u;
         lbase[tid] = c ? atomicAdd(&pcnt[p0 + tid], c) : 0u;
+        const uint32_t all = wave_sum_u32(c);
+        if (tid == 0 && all) atomicAdd(reinterpret_cast<unsigned long long *>(ctr + 2), (unsigned long long)all);
     }
     __syncthreads();
     for (uint32_t i = tid; i < total; i += BMASK_BS) {
@@ -636,22 +653,44 @@ __global__ __launch_bounds__(BMASK_BS) void batch_mask_kernel(const BatchQuery *
 }
 
 // One thread per partition: its query list is cut into ranges of at most
-// qmax queries and every range into object chunks of ochunk.  Ranges holding
+// qmax queries (qfix, or by the number of (query, partition) entries the mask
+// counted) and every range into object chunks of ochunk.  Ranges holding
 // at least qmax / 2 queries are "heavy" and fill the item list from the
 // front, the others from the back (index cap - 1 - i), so the persistent
 // scoring kernel starts the long items first; only a list's last range can
-// be light.  One global atomic per workgroup reserves its items, two more
-// add its pair counts.  The items of a partition are written by the whole
-// wave (a partition many queries reach has a hundred or more).
+// be light.  One global atomic per workgroup reserves its items, one more
+// adds its pair count.
+//
+// Order: a wave takes 64 partitions spread over the whole store and writes
+// their first ranges, then their second ones, and so on.  The candidates a
+// full list keeps (the first BATCH_CAP) then come from everywhere, and the
+// second pass's threshold, their k-th key, is close to the k-th of all;
+// partition after partition, neighbours filled the lists (anticorrelated, N
+// = 2^24, d = 8, k <= 256: 512 queries 4.0 -> 2.5 ms, 1024 queries 4.7 ->
+// 3.9 ms, and fewer queries that overflow twice).
+//
+// qmax: a wave walks an item's queries one after another (about 1 us each
+// alone on its SIMD), so few entries are cut into short items until `target`
+// of them exist, while long lists keep enough queries an item to pay for the
+// load of its objects.  Correlated, d = 8, 128 queries, N = 2^18: 128
+// queries an item 451 us, 16 206 us, 4 169 us; anticorrelated, d = 16, 1024
+// queries, N = 2^24: 128 and 64 27.4 ms, 32 29.4 ms, 16 33.3 ms.
+constexpr uint32_t QPI_MIN = 4, QPI_MAX = 64, QPI_ITEMS = 4096;
 __global__ __launch_bounds__(BAUX_BS) void batch_compact_kernel(const unsigned int *__restrict__ pcnt, uint32_t L,
-                                                                uint32_t qmax, uint32_t ochunk, uint64_t cap,
+                                                                uint32_t qfix, uint32_t target, uint32_t ochunk, uint64_t cap,
                                                                 const uint32_t *__restrict__ psz,
                                                                 BatchItem *__restrict__ items,
                                                                 unsigned int *__restrict__ ctr) {
     __shared__ uint32_t wsum[BAUX_BS / 64];
-    __shared__ unsigned long long wstat[BAUX_BS / 64][2];
+    __shared__ unsigned long long wstat[BAUX_BS / 64];
     __shared__ uint32_t tot_h, tot_l, base_h, base_l;
-    const uint32_t p = blockIdx.x * BAUX_BS + threadIdx.x, lane = lane_id();
+    const uint32_t lane = lane_id();
+    const uint32_t p = (lane * (BAUX_BS / 64) + threadIdx.x / 64) * gridDim.x + blockIdx.x;
+    uint32_t qmax = qfix;
+    if (!qfix) {
+        const unsigned long long e = *reinterpret_cast<const unsigned long long *>(ctr + 2) / target;
+        qmax = e < QPI_MIN ? QPI_MIN : (e > QPI_MAX ? QPI_MAX : (uint32_t)e);
+    }
     const uint32_t cnt = p < L ? pcnt[p] : 0u;
     const uint32_t sz = cnt ? psz[p] : 0u;
     const uint32_t nch = (sz + ochunk - 1) / ochunk;
@@ -662,15 +701,9 @@ __global__ __launch_bounds__(BAUX_BS) void batch_compact_kernel(const unsigned i
     const uint32_t nh = nhr * nch, nl = (nr - nhr) * nch;
     const uint32_t offh = block_excl_scan<BAUX_BS>(nh, wsum, &tot_h);
     const uint32_t offl = block_excl_scan<BAUX_BS>(nl, wsum, &tot_l);
-    unsigned long long pairs = cnt, objs = (unsigned long long)cnt * sz;
-    for (int o = 32; o > 0; o >>= 1) {
-        pairs += __shfl_xor(pairs, o, 64);
-        objs += __shfl_xor(objs, o, 64);
-    }
-    if (lane == 0) {
-        wstat[threadIdx.x / 64][0] = pairs;
-        wstat[threadIdx.x / 64][1] = objs;
-    }
+    unsigned long long objs = (unsigned long long)cnt * sz;
+    for (int o = 32; o > 0; o >>= 1) objs += __shfl_xor(objs, o, 64);
+    if (lane == 0) wstat[threadIdx.x / 64] = objs;
     __syncthreads();
     if (threadIdx.x == 0) {
         // heavy items count in ctr[0], light in ctr[1]: one 64-bit atomic
@@ -681,31 +714,26 @@ __global__ __launch_bounds__(BAUX_BS) void batch_compact_kernel(const unsigned i
                           : 0ull;
         base_h = (uint32_t)r;
         base_l = (uint32_t)(r >> 32);
-        unsigned long long sp = 0, so = 0;
-        for (int w = 0; w < BAUX_BS / 64; w++) {
-            sp += wstat[w][0];
-            so += wstat[w][1];
-        }
-        if (sp) {
-            atomicAdd(reinterpret_cast<unsigned long long *>(ctr + 2), sp);
-            atomicAdd(reinterpret_cast<unsigned long long *>(ctr + 4), so);
-        }
+        unsigned long long so = 0;
+        for (int w = 0; w < BAUX_BS / 64; w++) so += wstat[w];
+        if (so) atomicAdd(reinterpret_cast<unsigned long long *>(ctr + 4), so);
     }
     __syncthreads();
-    const uint32_t kh0 = base_h + offh, kl0 = base_l + offl;
-    for (uint64_t m = __ballot(nr != 0); m; m &= m - 1) {
-        const int src = __ffsll((long long)m) - 1;
-        const uint32_t sp_ = __shfl(p, src, 64), scnt = __shfl(cnt, src, 64), snch = __shfl(nch, src, 64);
-        const uint32_t snr = __shfl(nr, src, 64), snhr = __shfl(nhr, src, 64);
-        const uint32_t skh = __shfl(kh0, src, 64), skl = __shfl(kl0, src, 64);
-        for (uint32_t i = lane; i < snr * snch; i += 64) {
-            const uint32_t r = i / snch, c = i - r * snch;
-            const uint32_t q0 = r * qmax, qn = scnt - q0 < qmax ? scnt - q0 : qmax;
-            const BatchItem it{sp_, q0, qn, c};
-            if (r < snhr) items[skh + i] = it;           // heavy ranges come first
-            else items[cap - 1 - (skl + c)] = it;        // the light last range
+    uint32_t kh = base_h + (uint32_t)__builtin_amdgcn_readfirstlane((int)offh);
+    uint32_t kl = base_l + (uint32_t)__builtin_amdgcn_readfirstlane((int)offl);
+    const uint32_t maxc = wave_max_u32(nch), maxr = wave_max_u32(nr);
+    const uint64_t below = (1ull << lane) - 1ull;
+    for (uint32_t r = 0; r < maxr; r++)
+        for (uint32_t c = 0; c < maxc; c++) {
+            const bool on = r < nr && c < nch, heavy = on && r < nhr;
+            const uint64_t mh = __ballot(heavy), ml = __ballot(on && !heavy);
+            const uint32_t q0 = r * qmax;
+            const BatchItem it{p, q0, cnt - q0 < qmax ? cnt - q0 : qmax, c};
+            if (heavy) items[kh + (uint32_t)__popcll(mh & below)] = it;
+            else if (on) items[cap - 1 - (kl + (uint32_t)__popcll(ml & below))] = it;
+            kh += (uint32_t)__popcll(mh);
+            kl += (uint32_t)__popcll(ml);
         }
-    }
 }
 
 struct ScoreArgs {
@@ -775,11 +803,29 @@ __device__ __forceinline__ void load_objs(const float *__restrict__ p, float (&x
 // queries whose bound reaches their threshold, loads its objects only if one
 // does, and a query that fails stays out of the wave's later tiles, which
 // ends the wave's walk through the item once every query has failed.
+//
+// Candidates: scores that reach their query's threshold are staged per wave
+// (score, position, query) and appended once per 64 queries of an item, or
+// before a query the stage may not have room for.  An id load and an atomic
+// per (tile, query) with a candidate put 2 us of latency each into the query
+// loop: 1024 queries, k <= 256, d = 16, 128 queries an item took 31.3 ms and
+// take 27.4 ms (anticorrelated, N = 2^24), 5.8 and 5.1 ms (N = 2^22, 512
+// queries), 1.16 and 0.86 ms (correlated, N = 2^20).
+template <int VPT>
+struct ScoreStage {
+    float score[64 * VPT];
+    uint32_t pos[64 * VPT];
+    uint32_t count[64];
+    uint8_t query[64 * VPT];
+};
 template <int D, int VPT, int BS>
 __global__ __launch_bounds__(BS) void batch_score_kernel(ScoreArgs a) {
     constexpr bool LANE_W = D <= 16;
+    constexpr int R = VPT < 4 ? VPT : 4;  // staged scores a lane appends at once
     __shared__ uint32_t s_it[2];
+    __shared__ ScoreStage<VPT> stage[BS / 64];
     const uint32_t tid = threadIdx.x, lane = lane_id();
+    ScoreStage<VPT> &st = stage[__builtin_amdgcn_readfirstlane(tid / 64)];
     const uint32_t nheavy = __builtin_amdgcn_readfirstlane(a.ctr[0]);
     const uint32_t nlight = __builtin_amdgcn_readfirstlane(a.ctr[1]);
     const uint32_t nitems = nheavy + nlight;
@@ -822,6 +868,45 @@ __global__ __launch_bounds__(BS) void batch_score_kernel(ScoreArgs a) {
                 nxt = atomicAdd(&a.ctr[6], 1u);
                 ticket = false;
             }
+            uint32_t nst = 0;
+            // Appends the staged scores, 256 at a time: ids read at once, ties
+            // past tau_id dropped, the rest ranked per query in LDS; lane j
+            // takes the room of query j, all queries in one atomic.
+            auto flush = [&]() {
+                wave_lds_sync();
+#pragma unroll 1
+                for (uint32_t r = 0; r < nst; r += 64 * R) {
+                    uint32_t of[R], id[R], rank[R];
+                    st.count[lane] = 0;
+#pragma unroll
+                    for (int v = 0; v < R; v++) {
+                        const uint32_t i = r + 64 * v + lane;
+                        of[v] = i < nst ? st.query[i] : 0u;
+                        id[v] = i < nst ? a.pid[st.pos[i]] : 0u;
+                    }
+                    wave_lds_sync();
+#pragma unroll
+                    for (int v = 0; v < R; v++) {
+                        const uint32_t i = r + 64 * v + lane;
+                        const float tau = __shfl(lt[0], (int)of[v], 64);
+                        const uint32_t tau_id = (uint32_t)__shfl(__float_as_int(lt[1]), (int)of[v], 64);
+                        const bool in = i < nst && (st.score[i] != tau || id[v] <= tau_id);
+                        rank[v] = in ? atomicAdd(&st.count[of[v]], 1u) : BATCH_CAP;
+                    }
+                    wave_lds_sync();
+                    const uint32_t c = st.count[lane];
+                    const uint32_t base = c ? atomicAdd(&a.ccount[lq], c) : 0u;
+#pragma unroll
+                    for (int v = 0; v < R; v++) {
+                        const uint32_t i = r + 64 * v + lane;
+                        const uint32_t at = (uint32_t)__shfl((int)base, (int)of[v], 64) + rank[v];
+                        const uint32_t q = (uint32_t)__shfl((int)lq, (int)of[v], 64);
+                        if (at < BATCH_CAP) a.cand[(uint64_t)q * BATCH_CAP + at] = rkey(st.score[i], id[v]);
+                    }
+                    wave_lds_sync();
+                }
+                nst = 0;
+            };
             // lanes whose query may still reach its threshold on the wave's
             // remaining objects (suffix bounds: once below, below for good)
             bool alive = lane < nqb;
@@ -940,35 +1025,30 @@ __global__ __launch_bounds__(BS) void batch_score_kernel(ScoreArgs a) {
                                 }
                             }
                         }
-                        // admitted: key (s, id) >= (tau, tau_id); the id is read only on a tie
+                        // scores that reach tau are staged; ids and ties wait for the flush
                         const float tau = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lt[0]), (int)qi));
-                        const uint32_t tau_id = (uint32_t)__builtin_amdgcn_readlane(__float_as_int(lt[1]), (int)qi);
                         uint32_t adm = 0;
 #pragma unroll
-                        for (int e = 0; e < VPT; e++) {
-                            bool in = (uint32_t)e < nvalid && s[e] >= tau;
-                            if (in && s[e] == tau && tau_id != 0xFFFFFFFFu) in = a.pid[start + i0 + e] <= tau_id;
-                            adm |= in ? 1u << e : 0u;
-                        }
-                        const uint32_t np = (uint32_t)__popc(adm);
-                        if (__ballot(np != 0)) {
-                            const uint32_t incl = wave_incl_scan(np);
-                            const uint32_t tot = __shfl(incl, 63, 64);
-                            uint32_t base = 0;
-                            if (lane == 63) base = atomicAdd(&a.ccount[q], tot);
-                            base = __shfl(base, 63, 64);
-                            uint32_t pos = base + incl - np;
-                            uint64_t *out = a.cand + (uint64_t)q * BATCH_CAP;
+                        for (int e = 0; e < VPT; e++) adm |= (uint32_t)e < nvalid && s[e] >= tau ? 1u << e : 0u;
+                        if (__ballot(adm != 0)) {
+                            const uint32_t c = (uint32_t)__popc(adm);
+                            const uint32_t inc = wave_incl_scan(c);
+                            const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+                            if (nst + all > 64u * VPT) flush();
+                            uint32_t at = nst + inc - c;
 #pragma unroll
-                            for (int e = 0; e < VPT; e++) {
+                            for (int e = 0; e < VPT; e++)
                                 if ((adm >> e) & 1u) {
-                                    if (pos < BATCH_CAP) out[pos] = rkey(s[e], a.pid[start + i0 + e]);
-                                    pos++;
+                                    st.score[at] = s[e];
+                                    st.pos[at] = start + i0 + e;
+                                    st.query[at] = (uint8_t)qi;
+                                    at++;
                                 }
-                            }
+                            nst += all;
                         }
                     }
                 }
+            flush();  // the lanes' queries change
             }
         if (ticket) nxt = atomicAdd(&a.ctr[6], 1u);  // no wave of tid 0 reached the queries
         if (tid == 0) s_it[slot] = nxt;
@@ -1601,7 +1681,7 @@ static uint64_t bq_task_entries(uint32_t nq, uint32_t p2, uint32_t H) {
 }
 
 struct BatchVariant {
-    int vpt, bs, qpi, digit, grid;
+    int vpt, bs, qpi, digit, grid;  // qpi 0: chosen on the device by the batch's entries
     int item;   // objects per work item (a multiple of PTA_CHUNK)
     int fused;  // 1: the query-major fused pass replaces mask, compaction and item scoring
 };
@@ -1790,8 +1870,10 @@ static int ensure(topk_ctx *ctx, BatchState &B, uint32_t nq, uint32_t ks, int si
     HostSlot &H = B.slot[si];
     const uint32_t L = P.nparts, nw = (nq + 63) / 64;
     const size_t in_need = InLayout::make(nq).bytes, out_need = OutLayout::make(nq, ks).bytes;
+    // a budget of 16 queries or more: 4 nw + 1 ranges a partition at most; a
+    // smaller one: at most 1.25 QPI_ITEMS ranges and one a partition
     const uint64_t items_need =
-        (uint64_t)L * (4 * nw + 1) * ((P.maxsz + ITEM_MIN_OBJECTS - 1) / ITEM_MIN_OBJECTS + 1);
+        ((uint64_t)L * (4 * nw + 1) + 5ull * QPI_ITEMS / 4) * ((P.maxsz + ITEM_MIN_OBJECTS - 1) / ITEM_MIN_OBJECTS + 1);
     const uint64_t te = bq_task_entries(nq, P.p2, group_height(P.p2));
     const bool grow = B.gen != P.generation || nq > H.nq_cap || in_need > H.din_cap || out_need > H.dout_cap ||
                       in_need > H.in_cap || out_need > H.out_cap || (uint64_t)L * nq > H.plist_cap ||
@@ -1859,7 +1941,7 @@ static int ensure(topk_ctx *ctx, BatchState &B, uint32_t nq, uint32_t ks, int si
     H.stream = ctx->lane[si].stream;
     rc = grow_dev(H.d_plist, H.plist_cap, (uint64_t)L * nq, changed);
     if (!rc) rc = grow_dev(H.d_pcnt, H.pcnt_cap, (uint64_t)L, changed);
-    // budget >= 16 queries, chunks >= ITEM_MIN_OBJECTS objects
+    // chunks >= ITEM_MIN_OBJECTS objects
     if (!rc) rc = grow_dev(H.d_items, H.item_cap, items_need, changed);
     if (rc) return rc;
     {
@@ -1916,16 +1998,33 @@ static uint32_t item_objects(const BatchVariant &v) {
     return o > ITEM_MIN_OBJECTS ? o : ITEM_MIN_OBJECTS;
 }
 
-static BatchVariant pick_variant(const topk_ctx *ctx, const BatchState &B) {
+static BatchVariant pick_variant(const topk_ctx *ctx, const BatchState &B, uint32_t nq) {
     const int D = dims_class(ctx->d);
     BatchVariant v;
     v.vpt = ctx->tune.batch_vpt ? ctx->tune.batch_vpt : (D == 8 ? 8 : (D == 16 ? 4 : 2));
     v.bs = ctx->tune.batch_bs ? ctx->tune.batch_bs : 256;
-    v.qpi = ctx->tune.batch_qpi ? ctx->tune.batch_qpi : 128;
+    v.qpi = ctx->tune.batch_qpi;
     v.digit = ctx->tune.batch_digit ? ctx->tune.batch_digit : 11;
     v.grid = ctx->tune.batch_grid ? ctx->tune.batch_grid : B.cus * (v.bs == 256 ? 4 : 2);
     v.item = ctx->tune.batch_item ? ctx->tune.batch_item : 4096;
-    v.fused = ctx->tune.batch_fused == 2 ? 1 : 0;
+    // The query-major pass when neither it nor a work-item shape was asked
+    // for: no work list to build and no
+    // reuse of loaded objects, so it is ahead while queries x objects are
+    // few.  Measured limits, worst distribution (anticorrelated or
+    // independent) and best (correlated), work items against query-major in
+    // us, k <= 256:
+    //   d <= 8:  2^28 pairs in at most 2^22 objects; 2^20 x 128: 518 / 479
+    //            and 181 / 148, 2^18 x 1024: 643 / 702 and 369 / 351;
+    //            2^22 x 512: 1250 / 1520 and 337 / 296;
+    //            8 queries over 2^24 (one workgroup bounds a whole tree):
+    //            209 / 247
+    //   d <= 16: 2^24 pairs in at most 2^18 objects; 2^18 x 32: 321 / 315
+    //            and 160 / 126; 2^20 x 8: 297 / 337; 2^20 x 32: 491 / 586
+    //            and 187 / 154
+    const bool shaped = ctx->tune.batch_vpt || ctx->tune.batch_bs || ctx->tune.batch_qpi || ctx->tune.batch_grid ||
+                        ctx->tune.batch_item || ctx->tune.batch_mask;
+    const uint64_t most = D == 8 ? 1ull << 28 : (D == 16 ? 1ull << 24 : 0), most_n = D == 8 ? 1ull << 22 : 1ull << 18;
+    v.fused = ctx->tune.batch_fused ? ctx->tune.batch_fused == 2 : !shaped && ctx->n <= most_n && ctx->n * nq <= most;
     return v;
 }
 
@@ -2060,21 +2159,25 @@ static int enqueue_pass(topk_ctx *ctx, BatchState &B, hipStream_t s, uint32_t nq
         auto mask = NB == 8 ? batch_mask_query_kernel<8>
                             : (NB == 16 ? batch_mask_query_kernel<16> : batch_mask_query_kernel<32>);
         hipLaunchKernelGGL(mask, dim3(nq, S), dim3(BMASK_BS), 0, s, dq, db, ta, G, H, L, nq, B.slot[B.cur].d_pcnt, B.slot[B.cur].d_plist,
-                           pass_flags);
+                           B.slot[B.cur].d_ctr, pass_flags);
     } else {
         const uint32_t QS = BMASK_PAIRS >> H, Y = (nq + QS - 1) / QS;
         auto mask = NB == 8 ? batch_mask_kernel<8> : (NB == 16 ? batch_mask_kernel<16> : batch_mask_kernel<32>);
         hipLaunchKernelGGL(mask, dim3(G, Y), dim3(BMASK_BS), 0, s, dq, db, ta, G, H, L, nq, QS, B.slot[B.cur].d_pcnt,
-                           B.slot[B.cur].d_plist, pass_flags);
+                           B.slot[B.cur].d_plist, B.slot[B.cur].d_ctr, pass_flags);
     }
     const uint32_t ochunk = item_objects(v);
+    BatchVariant vs = v;
+    if (second) vs.grid = v.grid / 8 > 32 ? v.grid / 8 : 32;  // the second pass has few items
+    // Items a workgroup: 4 of the short ones at d <= 8, 2 of the longer ones
+    // above (4 against 2, 1024 queries, k <= 256: 736 against 798 us at d = 8,
+    // N = 2^24; 648 against 604 us at d = 16, N = 2^22; both correlated).
+    const uint32_t target = std::min((ctx->d <= 8 ? 4u : 2u) * (uint32_t)vs.grid, QPI_ITEMS);
     hipLaunchKernelGGL(batch_compact_kernel, dim3((L + BAUX_BS - 1) / BAUX_BS), dim3(BAUX_BS), 0, s, B.slot[B.cur].d_pcnt, L,
-                       (uint32_t)v.qpi, ochunk, B.slot[B.cur].item_cap, P.psz, B.slot[B.cur].d_items, B.slot[B.cur].d_ctr);
+                       (uint32_t)v.qpi, target, ochunk, B.slot[B.cur].item_cap, P.psz, B.slot[B.cur].d_items, B.slot[B.cur].d_ctr);
     ScoreArgs sa{P.pcols, P.ld, ctx->d,    P.poff,     P.psz,  P.pid,  B.slot[B.cur].d_items, B.slot[B.cur].item_cap,
                  ochunk,  B.slot[B.cur].d_plist, nq, B.slot[B.cur].d_ctr, dq, B.slot[B.cur].d_cand, B.slot[B.cur].d_ccount, P.cstat,  P.crow, (uint64_t)P.nchunks,
                  B.slot[B.cur].d_scored, P.cminid};
-    BatchVariant vs = v;
-    if (second) vs.grid = v.grid / 8 > 32 ? v.grid / 8 : 32;  // the second pass has few items
     hipEvent_t ev0 = nullptr;
     timing_begin(ctx, s, ev0);
     launch_score(dims_class(ctx->d), vs, s, sa);
@@ -2358,8 +2461,8 @@ static int batch_submit(topk_ctx *ctx, uint32_t nq, const topk_query *qs, uint32
     int rc = batch_complete(ctx, B, si);
     if (!rc) rc = ensure(ctx, B, nq, ks, si);
     if (rc) return rc;
-    const BatchVariant v = force ? *force : pick_variant(ctx, B);  // after ensure: the CU count is known
-    if (!variant_ok(dims_class(ctx->d), v.vpt, v.bs) || v.qpi < 16 || v.qpi > 1024 ||
+    const BatchVariant v = force ? *force : pick_variant(ctx, B, nq);  // after ensure: the CU count is known
+    if (!variant_ok(dims_class(ctx->d), v.vpt, v.bs) || (v.qpi && v.qpi < 16) || v.qpi > 1024 ||
         (v.digit != 8 && v.digit != 11) || v.grid < 1 || v.grid > (int)BATCH_MAX_GRID || v.item < (int)PTA_CHUNK ||
         v.item % PTA_CHUNK)
         return TOPK_ERR_INVALID;
@@ -2460,7 +2563,7 @@ int topk_batch_autotune(topk_ctx *ctx, uint32_t nq, const topk_query *qs, uint32
         memcpy(B.slot[0].h_in + InLayout::make(nq).od_off, &od, sizeof(od));
     }
     const int D = dims_class(ctx->d);
-    const BatchVariant def = pick_variant(ctx, B);
+    const BatchVariant def = pick_variant(ctx, B, nq);
     std::vector<BatchVariant> cand;
     static const int vpts[] = {2, 4, 8, 16}, qpis[] = {16, 32, 64, 128}, per_cu[] = {2, 4, 8};
     for (int vpt : vpts)
@@ -2517,6 +2620,17 @@ int topk_batch_autotune(topk_ctx *ctx, uint32_t nq, const topk_query *qs, uint32
             best = v;
         }
     }
+    if (!rc && best.qpi && !best.fused) {  // the budget by the batch's entries, with the best shape
+        BatchVariant v = best;
+        v.qpi = 0;
+        double ms;
+        rc = time_one(v, ms);
+        extra++;
+        if (!rc && ms < best_ms) {
+            best_ms = ms;
+            best = v;
+        }
+    }
     for (int it : {2048, 4096, 8192, 16384}) {  // objects per work item, with the best shape
         if (rc || it == best.item || best.fused) continue;
         BatchVariant v = best;
@@ -2542,7 +2656,7 @@ int topk_batch_autotune(topk_ctx *ctx, uint32_t nq, const topk_query *qs, uint32
     if (out) {
         out->vpt = (uint32_t)best.vpt;
         out->bs = (uint32_t)best.bs;
-        out->qpi = (uint32_t)best.qpi;
+        out->qpi = best.qpi ? (uint32_t)best.qpi : QPI_MAX;
         out->digit = (uint32_t)best.digit;
         out->grid = (uint32_t)best.grid;
         out->item = (uint32_t)best.item;

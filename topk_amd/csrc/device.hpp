@@ -25,6 +25,14 @@ __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
     STEP(0x142, 0xA) /* row_bcast 15 into rows 1, 3 */                        \
     STEP(0x143, 0xC) /* row_bcast 31 into rows 2, 3 */
 
+// Orders a wave's own LDS accesses: what its lanes wrote before is what any of
+// them reads after (no instruction beyond the waits the compiler inserts).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Inclusive prefix sum across the 64 lanes of a wave.
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
 #define TK_STEP(ctrl, rows) v += TK_DPP(v, ctrl, rows);
