@@ -39,6 +39,8 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
+#include <new>
 #include <string>
 #include <thread>
 #include <vector>
@@ -52,8 +54,8 @@ constexpr uint32_t CSV_BS = 256;
 constexpr uint32_t CSV_TILE = 65536;             // text bytes per workgroup in the newline passes
 constexpr uint32_t CSV_LDS_WORDS = 8192;        // text staged in LDS per parse workgroup (32 KiB)
 constexpr uint32_t CSV_SCAN_BS = 1024;
-constexpr uint64_t STAGE_BYTES = 64ull << 20;    // pinned staging buffer (two alternate)
 constexpr uint32_t IO_THREADS = 16;
+constexpr uint64_t COUNT_CHUNK = 256ull << 10;   // file bytes the host counts lines in at once
 
 // Status of a runtime call; with TOPK_DEBUG set in the environment a
 // failure also names the call on stderr.
@@ -422,66 +424,110 @@ struct MappedFile {
     }
 };
 
-// Reads [off, off+bytes) of fd with IO_THREADS preads.
-static bool pread_all(int fd, char *dst, uint64_t off, uint64_t bytes) {
-    std::atomic<bool> ok{true};
-    const uint64_t per = (bytes + IO_THREADS - 1) / IO_THREADS;
-    auto work = [&](uint64_t b, uint64_t e) {
-        while (b < e) {
-            const ssize_t r = ::pread(fd, dst + b, e - b, (off_t)(off + b));
-            if (r <= 0) {
-                if (r < 0 && errno == EINTR) continue;
-                ok = false;
-                return;
-            }
-            b += (uint64_t)r;
+static bool pread_full(int fd, char *dst, uint64_t off, uint64_t bytes) {
+    while (bytes) {
+        const ssize_t r = ::pread(fd, dst, bytes, (off_t)off);
+        if (r <= 0) {
+            if (r < 0 && errno == EINTR) continue;
+            return false;
         }
-    };
-    if (bytes < (4ull << 20)) {
-        work(0, bytes);
-        return ok;
+        dst += r;
+        off += (uint64_t)r;
+        bytes -= (uint64_t)r;
     }
-    std::vector<std::thread> th;
-    for (uint32_t t = 0; t < IO_THREADS; t++) {
-        const uint64_t b = t * per, e = std::min(bytes, b + per);
-        if (b < e) th.emplace_back(work, b, e);
-    }
-    for (auto &t : th) t.join();
-    return ok;
+    return true;
 }
 
-// Streams file bytes to device memory through two pinned buffers: the
-// read of one chunk overlaps the copy of the previous one.
-struct Uploader {
-    char *stage[2] = {nullptr, nullptr};
-    hipEvent_t done[2] = {nullptr, nullptr};
+// Runs f(worker, chunk) for every chunk on nw workers, the caller one of
+// them; a chunk goes to the next free worker, and an f that returns a status
+// ends the run with it.  A thread that cannot be started leaves its share to
+// the others.
+template <class F>
+static int for_chunks(uint32_t nw, uint64_t chunks, F f) {
+    std::atomic<uint64_t> next{0};
+    std::atomic<int> rc{TOPK_OK};
+    auto work = [&](uint32_t w) {
+        for (uint64_t c; rc == TOPK_OK && (c = next++) < chunks;) {
+            const int r = f(w, c);
+            if (r) rc = r;
+        }
+    };
+    std::vector<std::thread> th;
+    try {
+        th.reserve(nw);
+        for (uint32_t w = 1; w < nw && w < chunks; w++) th.emplace_back(work, w);
+    } catch (...) {
+    }
+    work(0);
+    for (auto &t : th) t.join();
+    return rc;
+}
+
+// Copies between a file or pageable memory and the device through one small
+// pinned slot per worker: while one slot is on the bus the other workers
+// read the file, or write the caller's pages (whose first touch costs more
+// than the copy: 4.1 ms for 16 MiB from the runtime's own staging, 0.9 ms
+// here).  Pinned pages cost 0.4 ms a MiB when the host first writes them,
+// so the slots are reused and grow with the bytes to move; a copy costs its
+// call, so each worker has two to make below 64 MiB.  The read of 37.7 MB of
+// text into 16.8 MB (both directions, 8 workers) took 2.5 ms; with four
+// copies a worker 2.7, with eight 3.4, with one 6.1; two 64 MiB buffers and
+// the runtime's copy back 5 ms.
+struct Stager {
+    char *buf = nullptr;
+    hipEvent_t done[IO_THREADS] = {};
     hipStream_t st = nullptr;
-    int init(hipStream_t s) {
+    uint64_t slot = 0;
+    uint32_t nw = 0;
+    int dev = 0;
+    int init(hipStream_t s, uint64_t total) {
         st = s;
-        for (int i = 0; i < 2; i++) {
-            IK_HIP(hipHostMalloc(&stage[i], STAGE_BYTES, hipHostMallocDefault));
-            IK_HIP(hipEventCreateWithFlags(&done[i], hipEventDisableTiming));
-        }
+        nw = total < (2ull << 20) ? 1u : (total < (256ull << 20) ? IO_THREADS / 2 : IO_THREADS);
+        slot = std::min<uint64_t>(std::max<uint64_t>(total / (2 * nw), 256ull << 10), 4ull << 20) & ~0xFFFFull;
+        IK_HIP(hipGetDevice(&dev));
+        IK_HIP(hipHostMalloc(&buf, slot * nw, hipHostMallocDefault));
+        for (uint32_t i = 0; i < nw; i++) IK_HIP(hipEventCreateWithFlags(&done[i], hipEventDisableTiming));
         return TOPK_OK;
     }
-    // Appends [off, off+bytes) of fd to dst (device).
-    int copy(int fd, uint64_t off, uint64_t bytes, char *dst, int &slot) {
-        for (uint64_t b = 0; b < bytes; b += STAGE_BYTES) {
-            const uint64_t c = std::min<uint64_t>(STAGE_BYTES, bytes - b);
-            IK_HIP(hipEventSynchronize(done[slot]));
-            if (!pread_all(fd, stage[slot], off + b, c)) return TOPK_ERR_IO;
-            IK_HIP(hipMemcpyAsync(dst + b, stage[slot], c, hipMemcpyHostToDevice, st));
-            IK_HIP(hipEventRecord(done[slot], st));
-            slot ^= 1;
-        }
+    // [off, off+bytes) of fd to dst (device); complete in stream order.
+    int upload(int fd, uint64_t off, uint64_t bytes, char *dst) {
+        return for_chunks(nw, (bytes + slot - 1) / slot, [&](uint32_t w, uint64_t c) -> int {
+            const uint64_t b = c * slot, n = std::min(slot, bytes - b);
+            char *stage = buf + w * slot;
+            IK_HIP(hipSetDevice(dev));  // per thread
+            IK_HIP(hipEventSynchronize(done[w]));
+            if (!pread_full(fd, stage, off + b, n)) return TOPK_ERR_IO;
+            IK_HIP(hipMemcpyAsync(dst + b, stage, n, hipMemcpyHostToDevice, st));
+            IK_HIP(hipEventRecord(done[w], st));
+            return TOPK_OK;
+        });
+    }
+    // bytes of src (device) to out (host); complete on return.
+    int download(const char *src, uint64_t bytes, char *out) {
+        return for_chunks(nw, (bytes + slot - 1) / slot, [&](uint32_t w, uint64_t c) -> int {
+            const uint64_t b = c * slot, n = std::min(slot, bytes - b);
+            char *stage = buf + w * slot;
+            IK_HIP(hipSetDevice(dev));
+            IK_HIP(hipMemcpyAsync(stage, src + b, n, hipMemcpyDeviceToHost, st));
+            IK_HIP(hipEventRecord(done[w], st));
+            IK_HIP(hipEventSynchronize(done[w]));
+            memcpy(out + b, stage, n);
+            return TOPK_OK;
+        });
+    }
+    // One 64-bit word of device memory, through the first slot (idle: the
+    // caller has synchronised since the last upload).
+    int word(const void *src, uint64_t &v) {
+        IK_HIP(hipMemcpyAsync(buf, src, sizeof(v), hipMemcpyDeviceToHost, st));
+        IK_HIP(hipStreamSynchronize(st));
+        memcpy(&v, buf, sizeof(v));
         return TOPK_OK;
     }
-    ~Uploader() {
+    ~Stager() {
         if (st) hipStreamSynchronize(st);
-        for (int i = 0; i < 2; i++) {
-            if (stage[i]) hipHostFree(stage[i]);
-            if (done[i]) hipEventDestroy(done[i]);
-        }
+        if (buf) hipHostFree(buf);
+        for (auto e : done)
+            if (e) hipEventDestroy(e);
     }
 };
 
@@ -512,18 +558,21 @@ static uint32_t first_line_fields(const char *t, uint64_t size) {
 struct CsvText {
     MappedFile f;
     hipStream_t st = nullptr;
+    Stager io;
     char *text = nullptr;       // size rounded up to whole tiles, zero padded
     uint64_t *ends = nullptr;   // newline offsets
     uint64_t *row_base = nullptr;  // exclusive prefix of non-blank lines per group
+    CsvSlow *slow = nullptr;    // lines left to the host
+    unsigned long long *nslow = nullptr;
+    char *mem[2] = {nullptr, nullptr};  // the text with its tile counts; everything sized by the lines
     uint64_t ntiles = 0, nl = 0, groups = 0, rows = 0;
     uint32_t fields = 0;
     double ms_read = 0, ms_index = 0;
 
     ~CsvText() {
         if (st) hipStreamSynchronize(st);
-        hipFree(text);
-        hipFree(ends);
-        hipFree(row_base);
+        hipFree(mem[0]);
+        hipFree(mem[1]);
     }
 
     int load(const char *path, hipStream_t s) {
@@ -536,49 +585,41 @@ struct CsvText {
         auto t0 = std::chrono::steady_clock::now();
         ntiles = (f.size + CSV_TILE - 1) / CSV_TILE;
         const uint64_t cap = ntiles * CSV_TILE;
-        IK_HIP(hipMalloc(&text, cap));
+        // text | tile_base (ntiles + 1) | tile_nl (ntiles)
+        IK_HIP(hipMalloc(&mem[0], cap + 8 * (ntiles + 1) + 4 * ntiles));
+        text = mem[0];
+        uint64_t *tile_base = reinterpret_cast<uint64_t *>(text + cap);
+        uint32_t *tile_nl = reinterpret_cast<uint32_t *>(tile_base + ntiles + 1);
         IK_HIP(hipMemsetAsync(text + f.size, 0, cap - f.size, st));
-        {
-            Uploader up;
-            rc = up.init(st);
-            int slot = 0;
-            if (!rc) rc = up.copy(f.fd, 0, f.size, text, slot);
-            if (rc) return rc;
-        }  // drains the stream
-        ms_read = ms_since(t0);
-        t0 = std::chrono::steady_clock::now();
-        uint32_t *tile_nl = nullptr;
-        uint64_t *tile_base = nullptr;
-        IK_HIP(hipMalloc(&tile_nl, sizeof(uint32_t) * ntiles));
-        IK_HIP(hipMalloc(&tile_base, sizeof(uint64_t) * (ntiles + 1)));
+        rc = io.init(st, f.size);
+        if (!rc) rc = io.upload(f.fd, 0, f.size, text);
+        if (rc) return rc;
         hipLaunchKernelGGL(csv_count_kernel, dim3((uint32_t)ntiles), dim3(CSV_BS), 0, st, (const uint4 *)text,
                            tile_nl);
         hipLaunchKernelGGL(csv_scan_kernel, dim3(1), dim3(CSV_SCAN_BS), 0, st, tile_nl, ntiles, tile_base);
-        rc = IK_ST(hipGetLastError());
-        if (!rc) rc = IK_ST(hipMemcpyAsync(&nl, tile_base + ntiles, sizeof(nl), hipMemcpyDeviceToHost, st));
-        if (!rc) rc = IK_ST(hipStreamSynchronize(st));
-        if (!rc && hipMalloc(&ends, sizeof(uint64_t) * (nl + 1)) != hipSuccess) rc = TOPK_ERR_NOMEM;
-        if (!rc) {
-            hipLaunchKernelGGL(csv_index_kernel, dim3((uint32_t)ntiles), dim3(CSV_BS), 0, st, (const uint4 *)text,
-                               tile_base, ends);
-            rc = IK_ST(hipGetLastError());
-        }
-        if (!rc) rc = IK_ST(hipStreamSynchronize(st));
-        hipFree(tile_nl);
-        hipFree(tile_base);
+        IK_HIP(hipGetLastError());
+        IK_HIP(hipStreamSynchronize(st));
+        ms_read = ms_since(t0);
+        t0 = std::chrono::steady_clock::now();
+        rc = io.word(tile_base + ntiles, nl);
         if (rc) return rc;
         // lines: nl terminated ones plus the text after the last newline
         groups = (nl + 1 + CSV_BS - 1) / CSV_BS;
-        uint32_t *grp = nullptr;
-        IK_HIP(hipMalloc(&grp, sizeof(uint32_t) * groups));
-        IK_HIP(hipMalloc(&row_base, sizeof(uint64_t) * (groups + 1)));
+        // slow (nl + 1) | ends (nl + 1) | row_base (groups + 1) | nslow | grp (groups)
+        if (hipMalloc(&mem[1], 24 * (nl + 1) + 8 * (groups + 2) + 4 * groups) != hipSuccess) return TOPK_ERR_NOMEM;
+        static_assert(sizeof(CsvSlow) == 16, "slow lines lead the block");
+        slow = reinterpret_cast<CsvSlow *>(mem[1]);
+        ends = reinterpret_cast<uint64_t *>(slow + nl + 1);
+        row_base = ends + nl + 1;
+        nslow = reinterpret_cast<unsigned long long *>(row_base + groups + 1);
+        uint32_t *grp = reinterpret_cast<uint32_t *>(nslow + 1);
+        hipLaunchKernelGGL(csv_index_kernel, dim3((uint32_t)ntiles), dim3(CSV_BS), 0, st, (const uint4 *)text,
+                           tile_base, ends);
         hipLaunchKernelGGL(csv_rows_kernel, dim3((uint32_t)groups), dim3(CSV_BS), 0, st, (const uint32_t *)text,
                            ends, nl, f.size, grp);
         hipLaunchKernelGGL(csv_scan_kernel, dim3(1), dim3(CSV_SCAN_BS), 0, st, grp, groups, row_base);
-        rc = IK_ST(hipGetLastError());
-        if (!rc) rc = IK_ST(hipMemcpyAsync(&rows, row_base + groups, sizeof(rows), hipMemcpyDeviceToHost, st));
-        if (!rc) rc = IK_ST(hipStreamSynchronize(st));
-        hipFree(grp);
+        IK_HIP(hipGetLastError());
+        rc = io.word(row_base + groups, rows);
         ms_index = ms_since(t0);
         return rc;
     }
@@ -586,24 +627,12 @@ struct CsvText {
     // Parses the first n rows (d fields each) into out[m*cs + i*rs] (device).
     int parse(uint64_t n, uint32_t d, float *out, uint64_t cs, uint64_t rs, uint64_t &slow_lines, double &ms) {
         auto t0 = std::chrono::steady_clock::now();
-        unsigned long long *cnt = nullptr;
-        CsvSlow *slow = nullptr;
-        const uint64_t cap = std::min<uint64_t>(n, nl + 1);
-        IK_HIP(hipMalloc(&cnt, sizeof(unsigned long long)));
-        int rc = IK_ST(hipMalloc(&slow, sizeof(CsvSlow) * cap));
-        if (!rc) rc = IK_ST(hipMemsetAsync(cnt, 0, sizeof(unsigned long long), st));
-        if (!rc) {
-            hipLaunchKernelGGL(csv_parse_kernel, dim3((uint32_t)groups), dim3(CSV_BS), 0, st,
-                               (const uint32_t *)text, ends, nl, f.size, row_base, n, d, out, cs, rs, cnt, slow);
-            rc = IK_ST(hipGetLastError());
-        }
-        unsigned long long hs = 0;
-        if (!rc) rc = IK_ST(hipMemcpyAsync(&hs, cnt, sizeof(hs), hipMemcpyDeviceToHost, st));
-        if (!rc) rc = IK_ST(hipStreamSynchronize(st));
-        slow_lines = hs;
-        if (!rc && hs) rc = patch(slow, hs, d, out, cs, rs);
-        hipFree(cnt);
-        hipFree(slow);
+        IK_HIP(hipMemsetAsync(nslow, 0, sizeof(unsigned long long), st));
+        hipLaunchKernelGGL(csv_parse_kernel, dim3((uint32_t)groups), dim3(CSV_BS), 0, st, (const uint32_t *)text,
+                           ends, nl, f.size, row_base, n, d, out, cs, rs, nslow, slow);
+        IK_HIP(hipGetLastError());
+        int rc = io.word(nslow, slow_lines);
+        if (!rc && slow_lines) rc = patch(slow, slow_lines, d, out, cs, rs);
         ms = ms_since(t0);
         return rc;
     }
@@ -740,12 +769,11 @@ static int load_colfile(topk_ctx *ctx, const char *path, uint64_t n, uint32_t d,
     ctx->d = d;
     rc = ctx_alloc(ctx);
     if (!rc) {
-        Uploader up;
-        rc = up.init(ctx->stream);
-        int slot = 0;
+        Stager io;
+        rc = io.init(ctx->stream, n * 4);
         for (uint32_t m = 0; m < d && !rc; m++)
-            rc = up.copy(f.fd, h.data_offset + (uint64_t)m * h.n * 4, n * 4,
-                         reinterpret_cast<char *>(ctx->cols + (uint64_t)m * ctx->ld), slot);
+            rc = io.upload(f.fd, h.data_offset + (uint64_t)m * h.n * 4, n * 4,
+                           reinterpret_cast<char *>(ctx->cols + (uint64_t)m * ctx->ld));
     }  // drains the copies
     const double ms_read = ms_since(t0);
     if (!rc) rc = check_finite(ctx);
@@ -789,18 +817,53 @@ int topk_csv_count(const char *path, uint64_t *rows, uint32_t *fields) {
     int rc = f.open(path);
     if (rc) return rc;
     const uint32_t fl = f.size ? first_line_fields(f.map, f.size) : 0;
-    uint64_t r = 0;
-    uint64_t p = 0;
-    while (p < f.size) {
-        const char *nlp = static_cast<const char *>(memchr(f.map + p, '\n', f.size - p));
-        const uint64_t e = nlp ? (uint64_t)(nlp - f.map) : f.size;
-        for (uint64_t i = p; i < e; i++)
-            if (!csv_ws((unsigned char)f.map[i])) {
-                r++;
+    // Per chunk: the non-blank lines that begin and end in it, and whether
+    // its text before the first and after the last newline (all of it, with
+    // none) is non-blank.  37.7 MB, 524309 lines: 0.5 ms (one thread over
+    // the mapping: 4 ms).
+    struct Seg {
+        uint32_t mid = 0;
+        bool nl = false, head = false, tail = false;
+    };
+    const uint64_t chunks = (f.size + COUNT_CHUNK - 1) / COUNT_CHUNK;
+    std::unique_ptr<Seg[]> seg(new (std::nothrow) Seg[chunks]);
+    const uint32_t nw = (uint32_t)std::min<uint64_t>(IO_THREADS / 2, std::max<uint64_t>(chunks / 4, 1));
+    std::unique_ptr<char[]> bufs(new (std::nothrow) char[nw * COUNT_CHUNK]);
+    if (!seg || !bufs) return TOPK_ERR_NOMEM;
+    rc = for_chunks(nw, chunks, [&](uint32_t w, uint64_t c) -> int {
+        char *t = bufs.get() + w * COUNT_CHUNK;
+        const uint64_t n = std::min<uint64_t>(COUNT_CHUNK, f.size - c * COUNT_CHUNK);
+        const char *end = t + n;
+        if (!pread_full(f.fd, t, c * COUNT_CHUNK, n)) return TOPK_ERR_IO;
+        Seg g;
+        for (const char *p = t;;) {
+            const char *e = static_cast<const char *>(memchr(p, '\n', (size_t)(end - p)));
+            const char *le = e ? e : end;
+            while (p < le && csv_ws((unsigned char)*p)) p++;
+            const bool text = p < le;
+            if (!g.nl) g.head = text;
+            else if (e) g.mid += text ? 1u : 0u;
+            if (!e) {
+                g.tail = text;
                 break;
             }
-        p = e + 1;
+            g.nl = true;
+            p = e + 1;
+        }
+        seg[c] = g;
+        return TOPK_OK;
+    });
+    if (rc) return rc;
+    uint64_t r = 0;
+    bool open = false;  // the line at the end of the chunks so far has text
+    for (uint64_t c = 0; c < chunks; c++) {
+        const Seg &g = seg[c];
+        open = open || g.head;
+        if (!g.nl) continue;
+        r += (open ? 1u : 0u) + g.mid;
+        open = g.tail;
     }
+    r += open ? 1u : 0u;
     *rows = r;
     *fields = fl;
     return TOPK_OK;
@@ -824,8 +887,7 @@ int topk_csv_read(const char *path, uint64_t n, uint32_t d, uint32_t flags, floa
         const bool rowmajor = flags & TOPK_ROWMAJOR;
         rc = t->parse(n, d, dout, rowmajor ? 1 : n, rowmajor ? d : 1, slow, ms_parse);
     }
-    if (!rc) rc = IK_ST(hipMemcpyAsync(out, dout, sizeof(float) * n * d, hipMemcpyDeviceToHost, st));
-    if (!rc) rc = IK_ST(hipStreamSynchronize(st));
+    if (!rc) rc = t->io.download(reinterpret_cast<const char *>(dout), sizeof(float) * n * d, reinterpret_cast<char *>(out));
     if (!rc)
         fill_report(rep, 0, t->f.size, t->nl + (t->f.size && t->f.map[t->f.size - 1] != '\n' ? 1 : 0), n, d, slow,
                     t->ms_read, t->ms_index + ms_parse, ms_since(t0));
