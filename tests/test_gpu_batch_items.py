@@ -48,3 +48,23 @@ def test_choice_of_pass(gpu, d, n, nq):
         check(eng, x, qs)
         eng.set_tuning("batch_fused", 1)
         check(eng, x, qs)
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 129, 4096, 16_385, 300_007])
+@pytest.mark.parametrize("levels", [2, 1000, 0])
+def test_select_ends(gpu, n, levels):
+    """Lists of 63 to 65 keys and more, k at both ends, few distinct values
+    and many; single queries and batches over the same store."""
+    rng = np.random.default_rng(n + levels)
+    d = 5
+    x = rng.random((d, n)).astype(np.float32)
+    if levels:
+        x = np.rint(x * levels).astype(np.float32) / np.float32(levels)
+    ks = [k for k in (1, 2, 63, 64, 65, 66, 1024) if k <= n]
+    qs = make_queries(rng, 3 * len(ks), d, ks)
+    with topk_amd.Engine(x) as eng:
+        check(eng, x, qs)
+        ref = oracle_batch(x, n, qs)
+        for (k, w, a), (ri, rs) in zip(qs, ref):
+            for got in (eng.fte(k, w, a), eng.pta(k, w, a)):
+                assert np.array_equal(got[0], ri) and np.array_equal(got[1].view(np.uint32), rs.view(np.uint32))

@@ -234,12 +234,20 @@ __device__ __forceinline__ float batch_score_one(const BatchQuery &Q, const floa
     return s;
 }
 
-// Seed pass, one workgroup per query.  Wave 0 walks the bound tree from the
-// root keeping the 4 children with the largest bounds at every level (a
-// beam search); the first objects of the 4 partitions it reaches (16384 in
-// all) are scored, and the exact k-th largest key among them is a lower
-// bound of the query's k-th key: its score is tau.  Fewer than k objects:
-// tau = -inf (every object is a candidate).
+// Seed pass, one workgroup per query.  Wave 0 descends the bound tree to the
+// query's partitions with large bounds, a node per lane: the 64 nodes six
+// levels down, then the 16 descendants four levels down of each of the best
+// 4 (a level at a time was 13 rounds of loads, bound and ranking at 8192
+// partitions, now 3).  The first objects of the 4 partitions it reaches
+// (16384 in all) are scored, and the exact k-th largest key among them is a
+// lower bound of the query's k-th key: its score is tau.  Fewer than k
+// objects: tau = -inf (every object is a candidate).
+//
+// Bound by its chain of dependent loads: the objects of a thread come as
+// four 16-byte loads a term and BSEED_U terms are in flight together.
+// 1024 queries, d = 16, N = 2^25: 103 -> 52 us; 32 queries, d = 8, N =
+// 2^20: 38 -> 28 us.
+constexpr int BSEED_U = 4;
 template <int NB>
 __global__ __launch_bounds__(BSEED_BS) void batch_seed_kernel(BatchQuery *__restrict__ qs,
                                                               const BoundArgs *__restrict__ qb, TreeArgs t,
@@ -260,27 +268,28 @@ __global__ __launch_bounds__(BSEED_BS) void batch_seed_kernel(BatchQuery *__rest
         const uint32_t lane = tid;
         uint32_t beam[BSEED_T] = {1u, 0u, 0u, 0u};
         uint32_t nb = 1;
-        while (beam[0] < t.p2) {  // all beam nodes sit on one level
+        const uint32_t leaf = 31u - (uint32_t)__builtin_clz(t.p2);  // level of the partitions
+        for (uint32_t level = 0; nb && level < leaf;) {  // all beam nodes sit on one level
+            const uint32_t most = nb == 1 ? 6u : 4u, down = leaf - level < most ? leaf - level : most;
             uint64_t key = 0;
-            if (lane < 2 * nb) {
-                uint32_t parent = beam[0];
+            if (lane < nb << down) {
+                uint32_t from = beam[0];
 #pragma unroll
-                for (uint32_t i = 1; i < BSEED_T; i++) parent = lane / 2 == i ? beam[i] : parent;
-                const uint32_t c = 2 * parent + (lane & 1);
+                for (uint32_t i = 1; i < BSEED_T; i++) from = lane >> down == i ? beam[i] : from;
+                const uint32_t c = (from << down) + (lane & ((1u << down) - 1u));
                 const float ub = node_bound<NB>(b, t, c);
                 if (ub > -INFINITY) key = ((uint64_t)okey(ub) << 32) | c;
             }
-            uint32_t got = 0;
+            level += down;
+            nb = 0;
 #pragma unroll
             for (uint32_t r = 0; r < BSEED_T; r++) {
                 const uint64_t m = wave_max_u64(key);
                 if (m == 0) break;
                 beam[r] = (uint32_t)(m & 0xFFFFFFFFu);
                 key = key == m ? 0ull : key;
-                got++;
+                nb++;
             }
-            nb = got;
-            if (!nb) break;
         }
         if (lane == 0) {
             uint32_t c = 0;
@@ -293,7 +302,7 @@ __global__ __launch_bounds__(BSEED_BS) void batch_seed_kernel(BatchQuery *__rest
     }
     __syncthreads();
     const uint32_t T = nbest;
-    const uint32_t per = T ? BSEED_OBJS / T : 0u;
+    const uint32_t per = T ? BSEED_OBJS / T & ~3u : 0u;
     uint32_t start[BSEED_T], lim[BSEED_T], total = 0;
 #pragma unroll
     for (uint32_t i = 0; i < BSEED_T; i++) {
@@ -302,14 +311,14 @@ __global__ __launch_bounds__(BSEED_BS) void batch_seed_kernel(BatchQuery *__rest
         lim[i] = i < T ? (psz[p] < per ? psz[p] : per) : 0u;
         total += lim[i];
     }
-    // object slot j of this thread: position pos[j] (valid when ok[j]); the
-    // terms run outside the objects so each term's loads are in flight together
-    uint32_t pos[BSEED_KPT];
-    bool ok[BSEED_KPT];
-    float sc[BSEED_KPT];
+    // group j of this thread: four objects from position pos[j], nv[j] of
+    // them valid (loads past the last one stay in the partition's padding)
+    constexpr int GRP = BSEED_KPT / 4;
+    uint32_t pos[GRP], nv[GRP];
+    f4 sc[GRP];
 #pragma unroll
-    for (int j = 0; j < BSEED_KPT; j++) {
-        const uint32_t g = j * BSEED_BS + tid;
+    for (int j = 0; j < GRP; j++) {
+        const uint32_t g = 4 * (j * BSEED_BS + tid);
         const uint32_t i = per ? g / per : BSEED_T, o = per ? g - i * per : 0u;
         uint32_t st = 0, lm = 0;
 #pragma unroll
@@ -317,26 +326,42 @@ __global__ __launch_bounds__(BSEED_BS) void batch_seed_kernel(BatchQuery *__rest
             st = i == u ? start[u] : st;
             lm = i == u ? lim[u] : lm;
         }
-        ok[j] = i < T && o < lm;
-        pos[j] = ok[j] ? st + o : 0u;
-        sc[j] = 0.0f;
+        nv[j] = i < T && o < lm ? (lm - o < 4u ? lm - o : 4u) : 0u;
+        pos[j] = nv[j] ? st + o : 0u;
+        sc[j] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    for (uint32_t t = 0; t < Q.m; t++) {
-        const float *col = pcols + (uint64_t)Q.attr[t] * ld;
-        const float w = Q.w[t];
+    const uint32_t m = Q.m;
+    for (uint32_t t0 = 0; t0 < m; t0 += BSEED_U) {
+        f4 x[BSEED_U][GRP];
 #pragma unroll
-        for (int j = 0; j < BSEED_KPT; j++) {
-            const float pr = col[pos[j]] * w;
-            sc[j] = sc[j] + pr;
+        for (int u = 0; u < BSEED_U; u++) {
+            const float *col = pcols + (uint64_t)Q.attr[t0 + u < m ? t0 + u : t0] * ld;
+#pragma unroll
+            for (int j = 0; j < GRP; j++) x[u][j] = *reinterpret_cast<const f4 *>(col + pos[j]);
         }
+#pragma unroll
+        for (int u = 0; u < BSEED_U; u++)
+            if (t0 + u < m) {
+                const float w = Q.w[t0 + u];
+#pragma unroll
+                for (int j = 0; j < GRP; j++) {
+                    const f4 pr = x[u][j] * w;
+                    sc[j] = sc[j] + pr;
+                }
+            }
     }
     RegKeys<BSEED_KPT> rk;
 #pragma unroll
-    for (int j = 0; j < BSEED_KPT; j++) rk.k[j] = ok[j] ? rkey(sc[j], pid[pos[j]]) : 0ull;
+    for (int j = 0; j < GRP; j++) {
+        const uint4 id = *reinterpret_cast<const uint4 *>(pid + pos[j]);
+        const uint32_t ids[4] = {id.x, id.y, id.z, id.w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) rk.k[4 * j + e] = (uint32_t)e < nv[j] ? rkey(sc[j][e], ids[e]) : 0ull;
+    }
     float tau = -INFINITY;
     uint32_t tau_id = 0xFFFFFFFFu;
     if (total >= Q.k) {
-        const uint64_t kth = block_kth_largest<BSEED_BS>(rk, total, Q.k, ss);
+        const uint64_t kth = block_kth_largest<BSEED_BS, RegKeys<BSEED_KPT>, 11>(rk, total, Q.k, ss);
         tau = rkey_score(kth);
         tau_id = rkey_id(kth);
     }
@@ -362,7 +387,7 @@ __global__ __launch_bounds__(BSEED_BS) void batch_seed_kernel(BatchQuery *__rest
 // project more than `budget` ids to reach k; such queries then take all
 // ties as candidates or their learned score threshold, by the projected
 // number of ties (end of the kernel).  No query leaves it marked.
-constexpr uint64_t BXB_BUDGET = 1ull << 20;  // ids a scan may cover
+constexpr uint64_t BXB_BUDGET = 1ull << 19;  // ids a scan may cover
 constexpr int BXB_BS = 256;                  // threads per scan workgroup
 constexpr int BXB_R0 = 4;                    // rows ANDed for every word
 // W words of one row from 16-byte loads (rows are 128-byte aligned and w
@@ -381,7 +406,14 @@ __device__ __forceinline__ void load_words(const uint64_t *__restrict__ p, uint6
 // step a thread ANDs the first BXB_R0 rows of its W words, then reads the
 // other rows only if that partial AND is nonzero -- past a few attributes
 // most words hold no common tie, and their remaining rows are never
-// fetched.  The rows of each phase are loaded all at once.
+// fetched.  The rows of each phase are loaded all at once, the first ones
+// of the next step before this step's others.
+//
+// Bound by the queries that scan the whole budget, 1 MB of rows through one
+// CU: 1024 queries (d = 16, N = 2^24, mixed, k <= 256) take 5, 10, 16 and 25
+// us at budgets of 2^16, 2^18, 2^19 and 2^20 ids, and the whole batch 1104
+// (2^17), 1039, 1023 and 1045 us: past 2^19 ids the scan costs more than the
+// pairs it saves.  512 or 1024 threads a query took no less.
 template <int MAXR, int W>
 __global__ __launch_bounds__(BXB_BS) void batch_tiebits_kernel(BatchQuery *__restrict__ qs,
                                                             const uint64_t *__restrict__ xbits, uint32_t d,
@@ -389,6 +421,8 @@ __global__ __launch_bounds__(BXB_BS) void batch_tiebits_kernel(BatchQuery *__res
     __shared__ uint32_t wsum[BXB_BS / 64], wtot[2][BXB_BS / 64];
     __shared__ uint32_t total, nrows;
     __shared__ uint32_t rrow[MAXR];
+    constexpr int R = MAXR <= 16 ? MAXR - BXB_R0 : (MAXR - BXB_R0) / 2;  // rows at a time after the first
+    static_assert((MAXR - BXB_R0) % R == 0, "whole groups of rows");
     const uint32_t tid = threadIdx.x, q = blockIdx.x;
     if (!qs[q].seed) return;  // uniform over the workgroup
     const BatchQuery &Q = qs[q];
@@ -414,48 +448,53 @@ __global__ __launch_bounds__(BXB_BS) void batch_tiebits_kernel(BatchQuery *__res
     const uint64_t lim = n < budget ? n : budget, wlim = (lim + 63) / 64;
     uint32_t found = 0, step = 0;
     uint64_t scanned = lim;  // ids read when the scan stops
+    uint64_t x0[BXB_R0][W];  // the first rows' words of the step
+    auto load_first = [&](uint64_t w) {
+#pragma unroll
+        for (int r = 0; r < BXB_R0; r++) {
+            if ((uint32_t)r < nr) {
+                load_words<W>(rowp[r] + w, x0[r]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < W; i++) x0[r][i] = ~0ull;
+            }
+        }
+    };
+    // a thread past wlim reads words 0.. (in bounds) and masks them out;
+    // words in [wlim, wb + W) lie inside the padded row
+    load_first((uint64_t)tid * W < wlim ? (uint64_t)tid * W : 0);
     for (uint64_t w0 = 0; w0 < wlim; w0 += BXB_BS * W) {
         const uint64_t wb = w0 + (uint64_t)tid * W;
-        // a thread past wlim reads words 0.. (in bounds) and masks them out;
-        // words in [wlim, wb + W) lie inside the padded row
-        const uint64_t wr = wb < wlim ? wb : 0;
+        const uint64_t wr = wb < wlim ? wb : 0, wn = wb + BXB_BS * W;
         uint64_t acc[W];
 #pragma unroll
         for (int i = 0; i < W; i++) acc[i] = wb + i < wlim ? ~0ull : 0ull;
-        {
-            uint64_t x[BXB_R0][W];
 #pragma unroll
-            for (int r = 0; r < BXB_R0; r++) {
-                if ((uint32_t)r < nr) {
-                    load_words<W>(rowp[r] + wr, x[r]);
-                } else {
+        for (int r = 0; r < BXB_R0; r++)
 #pragma unroll
-                    for (int i = 0; i < W; i++) x[r][i] = ~0ull;
+            for (int i = 0; i < W; i++) acc[i] &= x0[r][i];
+        if (w0 + BXB_BS * W < wlim) load_first(wn < wlim ? wn : 0);
+#pragma unroll
+        for (int r0 = BXB_R0; r0 < MAXR; r0 += R) {
+            uint64_t any = 0;
+#pragma unroll
+            for (int i = 0; i < W; i++) any |= acc[i];
+            if ((uint32_t)r0 < nr && any) {
+                uint64_t x[R][W];
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    if ((uint32_t)(r0 + r) < nr) {
+                        load_words<W>(rowp[r0 + r] + wr, x[r]);
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < W; i++) x[r][i] = ~0ull;
+                    }
                 }
+#pragma unroll
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int i = 0; i < W; i++) acc[i] &= x[r][i];
             }
-#pragma unroll
-            for (int r = 0; r < BXB_R0; r++)
-#pragma unroll
-                for (int i = 0; i < W; i++) acc[i] &= x[r][i];
-        }
-        uint64_t any = 0;
-#pragma unroll
-        for (int i = 0; i < W; i++) any |= acc[i];
-        if (nr > (uint32_t)BXB_R0 && any) {
-            uint64_t x[MAXR - BXB_R0][W];
-#pragma unroll
-            for (int r = BXB_R0; r < MAXR; r++) {
-                if ((uint32_t)r < nr) {
-                    load_words<W>(rowp[r] + wr, x[r - BXB_R0]);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < W; i++) x[r - BXB_R0][i] = ~0ull;
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < MAXR - BXB_R0; r++)
-#pragma unroll
-                for (int i = 0; i < W; i++) acc[i] &= x[r][i];
         }
         uint32_t c = 0;
 #pragma unroll

@@ -562,11 +562,69 @@ __global__ __launch_bounds__(MLP_BS) void mlp_train_kernel(MlpTrainArgs a) {
     }
 }
 
+// The features of query base + q, as mlp_features sums them, into X[q] by
+// the 16 lanes 16 q .. 16 q + 15 of the workgroup: lane a the weight and
+// sketch of attribute a, then a sum per lane over the attributes in order.
+// One thread per query spent 5 of the tau kernel's 13 us here (a chain of 32
+// x 16 selects); the kernel now takes 7.
+__device__ void tile_features(const BatchQuery *qs, uint32_t nr, const Sketch &S, float (*X)[MLP_XP], float *fsc,
+                              float *fmx) {
+    static_assert(MLP_BS == 16 * MLP_TR && LRN_MAX_D == 16 && MLP_IN == 96, "one lane per attribute");
+    const uint32_t q = threadIdx.x / 16, a = threadIdx.x % 16, first = lane_id() & ~15u;
+    const bool valid = q < nr;
+    const BatchQuery &Q = qs[valid ? q : 0];
+    const uint32_t m = valid ? Q.m : 0u;
+    const float wlo = Q.w[a], whi = Q.w[16 + a];
+    const uint32_t alo = Q.attr[a], ahi = Q.attr[16 + a];
+    const float lk = log2f((float)Q.k);
+    float wa = 0.0f;
+#pragma unroll
+    for (int j = 0; j < TOPK_MAX_DIMS; j++) {
+        const uint32_t at = (uint32_t)__shfl((int)(j < 16 ? alo : ahi), (int)(first + j % 16), 64);
+        const float w = __shfl(j < 16 ? wlo : whi, (int)(first + j % 16), 64);
+        wa = (uint32_t)j < m && at == a ? wa + w : wa;
+    }
+    float sabs = 0.0f;
+#pragma unroll
+    for (int i = 0; i < LRN_MAX_D; i++) sabs += fabsf(__shfl(wa, (int)(first + i), 64));
+    const float inv = sabs > 0.0f ? 1.0f / sabs : 0.0f;
+    const float wn = wa * inv;
+    // lane 0: sum, 1: of squares, 2: maximum, 3: with the maxima, 4..7: with
+    // the quantiles
+    float s = a == 2 ? -1.0f : 0.0f;
+#pragma unroll
+    for (int i = 0; i < LRN_MAX_D; i++) {
+        const float v = __shfl(wn, (int)(first + i), 64);
+        float f = a == 0 ? 1.0f : v;
+        f = a == 3 ? S.cmax[i] : f;
+#pragma unroll
+        for (int t = 0; t < 4; t++) f = a == 4u + t ? S.q[i][t] : f;
+        const float p = v * f;
+        s = a == 2 ? (v > s ? v : s) : s + p;
+    }
+    float *f = X[q];
+    const float z = valid ? 1.0f : 0.0f;  // rows past nr: zero, as mlp_tile pads them
+    f[a] = valid ? wn : 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; t++) f[17 + 4 * a + t] = z * S.q[a][t];
+    float e = 0.0f;
+    e = a == 8 ? lk * 0.1f : e;
+    e = a == 9 ? (float)m * 0.0625f : e;
+    e = a == 10 ? S.log2n * 0.03125f : e;
+    e = a == 11 ? (lk - S.log2n) * 0.03125f : e;
+    const uint32_t at = a < 3 ? 82u + a : (a == 3 ? 91u : (a < 8 ? 83u + a : (a == 8 ? 16u : (a == 9 ? 81u : (a < 12 ? 75u + a : 80u + a)))));
+    f[at] = valid ? (a < 8 ? s : e) : 0.0f;
+    if (a == 3) {
+        fsc[q] = valid ? sabs : 0.0f;
+        fmx[q] = valid ? s : 0.0f;
+    }
+}
+
 // Threshold per batch query: tau = (prediction - margin) * sum |W| (or
 // -inf when the weights are all zero).  pred (optional) gets the unlowered
-// prediction in score units.  One workgroup per 16 queries: lanes 0..15 of
-// the first wave build the queries' feature rows in the LDS tile while
-// every wave loads its B operands, then the forward pass runs on FP32
+// prediction in score units.  One workgroup per 16 queries: 16
+// lanes a query build its feature row in the LDS tile behind the loads of
+// every wave's B operands, then the forward pass runs on FP32
 // matrix cores with exactly the operation sequence of mlp_tile's forward
 // part -- the predictions equal those the calibration computed (mlp_pass
 // over the same features), bit for bit, and the weights are read once per
@@ -592,19 +650,7 @@ __global__ __launch_bounds__(MLP_BS) void mlp_tau_kernel(const float *__restrict
         for (int t = 0; t < 4; t++) w2[t] = p2[t];
     }
     const float b1 = P[OFF_B1 + unit], b2 = P[OFF_B2 + unit], w3 = P[OFF_W3 + unit], b3 = P[OFF_B3];
-    if (tid < MLP_TR) {
-        float f[MLP_IN], sc = 0.0f;
-        if (tid < nr) {
-            mlp_features(qs[base + tid], S, f, &sc);
-        } else {
-#pragma unroll
-            for (int i = 0; i < MLP_IN; i++) f[i] = 0.0f;  // rows past nr: zero, as mlp_tile pads them
-        }
-#pragma unroll
-        for (int i = 0; i < MLP_IN; i += 4) *reinterpret_cast<f4 *>(&T.X[tid][i]) = f4{f[i], f[i + 1], f[i + 2], f[i + 3]};
-        fsc[tid] = sc;
-        fmx[tid] = f[91];
-    }
+    tile_features(qs + base, nr, S, T.X, fsc, fmx);
     __syncthreads();
     // layer 1 (K = 96), as in mlp_tile
     f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
