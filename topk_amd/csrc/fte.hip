@@ -38,6 +38,7 @@
 #include "device.hpp"
 #include "emit.hpp"
 #include "internal.hpp"
+#include "select.hpp"
 
 namespace topk {
 
@@ -47,14 +48,11 @@ constexpr uint32_t SAMPLE_TILE = 1024;   // shared sample: objects per chunk
 constexpr uint32_t SAMPLE_CHUNKS = 128;  // shared sample: chunks at most, spread over the ids
 constexpr uint32_t SAMPLE_WGS = 32;      // workgroups that take the shared sample
 constexpr uint32_t SAMPLE_MAX_W = SAMPLE_WIN / SAMPLE_WGS;  // winners each of them publishes at most
-constexpr int STREAM_BS = 1024;
-constexpr int STREAM_NW = STREAM_BS / 64;
 constexpr int SAMPLE_VEC = SAMPLE_CHUNKS * SAMPLE_TILE / (SAMPLE_WGS * STREAM_BS * 4);  // float4 per thread
 constexpr int OWN_VEC = 4096 / (STREAM_BS * 4);  // own sample: float4 vectors per thread
 constexpr uint32_t OWN_OBJS = STREAM_BS * 4 * OWN_VEC;
 constexpr uint32_t OWN_SPOTS = OWN_OBJS / 16;   // own sample: 256 runs of 16 objects, one 64-byte line per column each
 constexpr uint64_t OWN_MAX_N = 1ull << 19;      // stores up to this size take their own sample
-constexpr uint32_t FUSE_CAP_MIN = 1024, FUSE_CAP_MAX = 4096;  // candidates the last stream workgroup selects in LDS
 constexpr uint32_t STREAM_GRID = 256;    // stream workgroups at most (one per CU), unless tuned
 constexpr int FINAL_BS = 512;            // separate final select
 constexpr int FINAL_KPT = 16;            // candidate keys per final-select thread (8192 in registers)
@@ -177,30 +175,6 @@ __global__ __launch_bounds__(SEED_BS) void fte_seed_kernel(QCols q, uint64_t n_e
 // ---------------------------------------------------------------------------
 // final select + sort
 // ---------------------------------------------------------------------------
-// Flat index -> key over pre[0..npre) followed by the blocks' slot regions;
-// off[] (LDS) holds the exclusive prefix of the per-block counts.
-struct SlotView {
-    const uint64_t *pre;
-    uint32_t npre;
-    const uint64_t *keys;
-    uint32_t slot;
-    const uint32_t *off;
-    uint32_t nblk, total;  // keys in slots; the spill region's follow
-    const uint64_t *spill;
-    __device__ __forceinline__ uint64_t get(uint32_t p) const {
-        if (p < npre) return pre[p];
-        const uint32_t q = p - npre;
-        if (q >= total) return spill[q - total];
-        uint32_t lo = 0, hi = nblk;  // largest b with off[b] <= q
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (off[mid] <= q) lo = mid;
-            else hi = mid;
-        }
-        return keys[(uint64_t)lo * slot + (q - off[lo])];
-    }
-};
-
 
 // The ks-th largest of the keys the wave's lanes hold (NPL per lane; 0: no
 // key) -- 0 with fewer than ks keys -- by bisection on ballot counts, score
@@ -245,11 +219,6 @@ __device__ __forceinline__ uint64_t wave_kth_bisect(const uint64_t (&v)[NPL], ui
         }
     }
     return ((uint64_t)t << 32) | lo;
-}
-
-__device__ __forceinline__ void store_agent(uint64_t *p, uint64_t v) {
-    __hip_atomic_store(reinterpret_cast<unsigned long long *>(p), (unsigned long long)v, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The ks-th largest of the wave's keys (hi / lo as wave_pop_max's): rounds of
@@ -414,221 +383,6 @@ __device__ __forceinline__ uint64_t own_sample_tau(const QCols &q, uint64_t n, u
 // ---------------------------------------------------------------------------
 // 2. stream pass
 // ---------------------------------------------------------------------------
-constexpr uint32_t FUSE_BINS = 1024;
-constexpr uint32_t FUSE_BIN_MAX = 128;  // keys of one bin ranked against each other
-struct FuseScratch {
-    uint32_t bins[FUSE_BINS];
-    SelectScratchT<256> rs;
-    uint64_t wlo[STREAM_NW], whi[STREAM_NW];
-    uint32_t crowded;     // an interval too full to rank by pairs
-    uint32_t cut, ncut;   // the interval holding the k-th key, and the keys up to its end
-};
-
-// Writes the first want keys, best first, and sentinels up to k.
-template <int BS>
-__device__ __forceinline__ void emit_sorted(const uint64_t *sorted, uint32_t want, uint32_t k, const FinalOut &fo) {
-    for (uint32_t i = threadIdx.x; i < k; i += BS) {
-        const uint64_t x = i < want ? sorted[i] : 0ull;
-        fo.ids[i] = i < want ? (uint64_t)rkey_id(x) : ~0ull;
-        fo.scores[i] = i < want ? rkey_score(x) : -INFINITY;
-    }
-    if (threadIdx.x == 0 && fo.thr) *fo.thr = rkey_score(sorted[want - 1]);
-}
-
-// Exact top k of the candidates the stream's workgroups published, by the
-// last of them to finish.  The counts' offsets are scanned, the candidates
-// gathered into LDS (lkeys, cap keys), counting-sorted by 1024 equal
-// intervals of their key range -- only as far as the interval that holds the
-// k-th -- and each key is ranked inside its interval; results go out best
-// first.  Ties crowding one interval, and more candidates than cap, take a
-// radix select.  lkeys and regb hold cap keys each (2 * kp2 at least).
-template <int BS>
-__device__ void fused_select(FteState *__restrict__ st, const CandSet &cs, uint32_t k, uint32_t kreq, uint32_t cap,
-                             uint32_t kp2, const FinalOut &fo, uint64_t *lkeys, uint64_t *regb, FuseScratch &fs) {
-    __shared__ uint32_t wsum[BS / 64];
-    __shared__ uint32_t total, s_spill, s_pre;
-    uint32_t *off = reinterpret_cast<uint32_t *>(regb);
-    const uint32_t tid = threadIdx.x, wave = tid / 64;
-    if (cs.nblk <= 256) {
-        // wave 0 scans four counts per lane, the other waves clear
-        if (wave == 0) {
-            uint32_t n_[4], sum = 0;
-#pragma unroll
-            for (int j = 0; j < 4; j++) n_[j] = 4 * tid + j < cs.nblk ? cs.counts[4 * tid + j] : 0u;
-            if (tid == 0) {
-                s_spill = st->spill;
-                s_pre = cs.pre ? st->pre_count : 0u;
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++) sum += n_[j];
-            uint32_t at = wave_incl_scan(sum) - sum;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if (4 * tid + j < cs.nblk) off[4 * tid + j] = at;
-                at += n_[j];
-            }
-            if (tid == 63) total = at;
-        } else {
-            for (uint32_t b = tid - 64; b < FUSE_BINS; b += BS - 64) fs.bins[b] = 0;
-            if (tid == 64) fs.crowded = 0;
-        }
-    } else {
-        for (uint32_t b = tid; b < cs.nblk; b += BS) off[b] = cs.counts[b];
-        for (uint32_t b = tid; b < FUSE_BINS; b += BS) fs.bins[b] = 0;
-        if (tid == 0) {
-            fs.crowded = 0;
-            s_spill = st->spill;
-            s_pre = cs.pre ? st->pre_count : 0u;
-        }
-        __syncthreads();
-        const uint32_t per = (cs.nblk + BS - 1) / BS;
-        const uint32_t b0 = tid * per < cs.nblk ? tid * per : cs.nblk;
-        const uint32_t b1 = b0 + per < cs.nblk ? b0 + per : cs.nblk;
-        uint32_t mine = 0;
-        for (uint32_t b = b0; b < b1; b++) mine += off[b];
-        uint32_t run = block_excl_scan<BS>(mine, wsum, &total);
-        for (uint32_t b = b0; b < b1; b++) {
-            const uint32_t c = off[b];
-            off[b] = run;
-            run += c;
-        }
-    }
-    __syncthreads();
-    const uint32_t spilled = s_spill, npre = s_pre;
-    const uint32_t nspill = spilled < cs.spill_cap ? spilled : cs.spill_cap;
-    const uint32_t ntotal = total, c = npre + ntotal + nspill;
-    const uint32_t bad = spilled > cs.spill_cap ? STATUS_OVERFLOW : (c < kreq ? STATUS_RETRY : 0u);
-    if (tid == 0) {
-        // ready for the next query
-        st->spill = 0;
-        st->arrive = 0;
-        st->ticket = 0;
-        if (bad) st->status |= bad;
-        else st->cand_last = c;
-        if (!bad && fo.cand) *fo.cand = c;
-        if (fo.status) *fo.status = bad;
-    }
-    if (tid < ARRIVE_GROUPS) st->group[tid * ARRIVE_STRIDE] = 0;
-    if (tid < SAMPLE_WIN) st->win[tid] = 0;
-    if (bad) return;
-    const SlotView v{cs.pre, npre, cs.keys, cs.slot, off, cs.nblk, ntotal, cs.spill};
-    const uint32_t want = c < k ? c : k;  // results
-    uint64_t *sorted;
-    if (c <= BS / 4) {
-        // few: each key's rank counted by four threads, a quarter of the keys each
-        const uint32_t i = tid % (BS / 4), part = tid / (BS / 4), q4 = (c + 3) / 4;
-        uint64_t x = 0;
-        if (part == 0 && i < c) lkeys[i] = x = v.get(i);
-        if (part == 1) fs.bins[i] = 0;  // the ranks
-        __syncthreads();
-        if (i < c) {
-            x = lkeys[i];
-            const uint32_t j1 = (part + 1) * q4 < c ? (part + 1) * q4 : c;
-            uint32_t r = 0;
-            for (uint32_t j = part * q4; j < j1; j++) r += lkeys[j] > x ? 1u : 0u;
-            if (r) atomicAdd(&fs.bins[i], r);
-        }
-        __syncthreads();
-        if (tid < c) regb[fs.bins[tid]] = x;  // the offsets are used up
-        __syncthreads();
-        emit_sorted<BS>(regb, want, k, fo);
-        return;
-    }
-    if (c <= cap) {
-        uint64_t lo = ~0ull, hi = 0;
-        for (uint32_t i = tid; i < c; i += BS) {
-            const uint64_t x = v.get(i);
-            lkeys[i] = x;
-            lo = x < lo ? x : lo;
-            hi = x > hi ? x : hi;
-        }
-        lo = wave_min_u64(lo);
-        hi = wave_max_u64(hi);
-        if (lane_id() == 0) {
-            fs.wlo[wave] = lo;
-            fs.whi[wave] = hi;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int w = 0; w < BS / 64; w++) {
-            lo = fs.wlo[w] < lo ? fs.wlo[w] : lo;
-            hi = fs.whi[w] > hi ? fs.whi[w] : hi;
-        }
-        const int width = 64 - (hi > lo ? __builtin_clzll(hi - lo) : 63);
-        const int shift = width > 10 ? width - 10 : 0;  // interval 0 holds the largest keys
-        for (uint32_t i = tid; i < c; i += BS) atomicAdd(&fs.bins[(uint32_t)((hi - lkeys[i]) >> shift)], 1u);
-        __syncthreads();
-        constexpr int BPT = FUSE_BINS / BS;
-        uint32_t n_[BPT], sum = 0;
-#pragma unroll
-        for (int j = 0; j < BPT; j++) {
-            n_[j] = fs.bins[tid * BPT + j];
-            sum += n_[j];
-        }
-        uint32_t at = block_excl_scan<BS>(sum, wsum, &total);
-#pragma unroll
-        for (int j = 0; j < BPT; j++) {
-            fs.bins[tid * BPT + j] = at;
-            if (at < want) {
-                if (n_[j] > FUSE_BIN_MAX) fs.crowded = 1;
-                if (at + n_[j] >= want) {  // holds the last result
-                    fs.cut = tid * BPT + j;
-                    fs.ncut = at + n_[j];
-                }
-            }
-            at += n_[j];
-        }
-        __syncthreads();
-        if (!fs.crowded) {
-            // the intervals up to the cut, in order; bins[] turns from an
-            // interval's start into its end (the offsets in regb are used up)
-            for (uint32_t i = tid; i < c; i += BS) {
-                const uint64_t x = lkeys[i];
-                const uint32_t b = (uint32_t)((hi - x) >> shift);
-                if (b <= fs.cut) regb[atomicAdd(&fs.bins[b], 1u)] = x;
-            }
-            __syncthreads();
-            sorted = lkeys;
-            for (uint32_t i = tid; i < fs.ncut; i += BS) {
-                const uint64_t x = regb[i];
-                const uint32_t b = (uint32_t)((hi - x) >> shift);
-                const uint32_t s0 = b ? fs.bins[b - 1] : 0u, s1 = fs.bins[b];
-                uint32_t r = s0;
-                for (uint32_t j = s0; j < s1; j++) r += regb[j] > x ? 1u : 0u;
-                if (r < want) sorted[r] = x;
-            }
-            __syncthreads();
-        }
-    }
-    if (c > cap || fs.crowded) {
-        uint32_t got;
-        if (c <= cap) {
-            const uint64_t thr =
-                c > k ? block_kth_largest<BS, MemKeys<BS>, 8>(MemKeys<BS>{lkeys, c}, c, k, fs.rs) : 1ull;
-            got = block_gather_ge<BS>(MemKeysUniform<BS>{lkeys, c}, thr, regb, fs.rs);
-            sorted = regb;
-        } else {
-            const uint64_t thr = block_kth_largest<BS, ViewKeys<BS, SlotView, false>, 8>(
-                ViewKeys<BS, SlotView, false>{v, c}, c, k, fs.rs);
-            got = block_gather_ge<BS>(ViewKeys<BS, SlotView, true>{v, c}, thr, lkeys, fs.rs);
-            sorted = lkeys;
-        }
-        if (got <= (uint32_t)BS) {  // a rank pass, else a bitonic sort (got^2 compares grow past it)
-            const uint64_t x = tid < got ? sorted[tid] : 0ull;
-            uint32_t r = 0, unused = 0;
-            rank2_lds(sorted, got, x, x, r, unused);
-            __syncthreads();
-            if (tid < got) sorted[r] = x;
-            __syncthreads();
-        } else {
-            for (uint32_t i = got + tid; i < kp2; i += BS) sorted[i] = 0;
-            __syncthreads();
-            bitonic_sort_desc<BS>(sorted, kp2);
-        }
-    }
-    emit_sorted<BS>(sorted, want, k, fo);
-}
-
 // Where a stream workgroup takes tau from.
 enum { TAU_ALL = 0, TAU_STATE = 1, TAU_SHARED = 2, TAU_OWN = 3 };
 
@@ -808,15 +562,7 @@ __global__ __launch_bounds__(STREAM_BS, 4) void fte_stream_kernel(QCols q, Strea
                            __HIP_MEMORY_SCOPE_AGENT);
         if (a.select) {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            // group g counts workgroups g, g + ARRIVE_GROUPS, ...
-            const uint32_t G = gridDim.x, g = blockIdx.x % ARRIVE_GROUPS;
-            const uint32_t members = (G - g + ARRIVE_GROUPS - 1) / ARRIVE_GROUPS;
-            bool last = __hip_atomic_fetch_add(&a.st->group[g * ARRIVE_STRIDE], 1u, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_AGENT) == members - 1;
-            if (last)
-                last = __hip_atomic_fetch_add(&a.st->arrive, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                       (G < ARRIVE_GROUPS ? G : ARRIVE_GROUPS) - 1;
-            is_last = last;
+            is_last = last_to_arrive(a.st);
         }
     }
     if (!a.select) return;
@@ -826,8 +572,8 @@ __global__ __launch_bounds__(STREAM_BS, 4) void fte_stream_kernel(QCols q, Strea
     fused_select<STREAM_BS>(a.st, cs, a.k, a.kreq, a.cap, a.kp2, a.fo, dyn, dyn + a.cap, sh.sel);
 }
 
-// Final select as a launch of its own (one workgroup): partition queries,
-// and stores that fit the exact seed's prefix.
+// Final select as a launch of its own (one workgroup): stores that fit the
+// exact seed's prefix.
 __global__ __launch_bounds__(FINAL_BS) void fte_final_kernel(FteState *__restrict__ st, CandSet cs, uint32_t k,
                                                              uint32_t kreq, FinalOut fo,
                                                              const uint32_t *__restrict__ gate) {
@@ -1131,6 +877,15 @@ static CandSet fte_launch(const FteRun &r, uint32_t k, const QCols &q, const Fin
     return cs;
 }
 
+// The select of a run with an n-entry candidate buffer (FteRun::big).
+static void final_enqueue(topk_ctx *ctx, Lane &L, const CandSet &cs, uint32_t k, uint32_t kreq, const FinalOut &fo) {
+    hipStream_t s = L.stream;
+    hipLaunchKernelGGL(cand_offsets_kernel, dim3(1), dim3(FLAT_BS), 0, s, L.st, cs, ctx->offsets, ctx->flat);
+    if (cs.nblk)
+        hipLaunchKernelGGL(cand_compact_kernel, dim3(cs.nblk), dim3(256), 0, s, cs, ctx->offsets, ctx->flat);
+    hipLaunchKernelGGL(fte_final_flat_kernel, dim3(1), dim3(FLAT_BS), 0, s, L.st, ctx->flat, k, kreq, fo);
+}
+
 int fte_enqueue(topk_ctx *ctx, Lane &L, uint32_t k, const QCols &q, const FinalOut &fo, int mode, uint64_t n) {
     if (!n) n = ctx->n;
     if (n >= ID_LIMIT) return TOPK_ERR_UNSUPPORTED;  // a run's ids are 32-bit: callers split larger stores
@@ -1151,7 +906,7 @@ int fte_enqueue(topk_ctx *ctx, Lane &L, uint32_t k, const QCols &q, const FinalO
     r.timed = ctx;
     const uint32_t kreq = (uint32_t)(n < k ? n : k);
     const CandSet cs = fte_launch(r, k, q, fo, mode);
-    if (r.big) final_enqueue(ctx, L, cs, k, kreq, fo, true);
+    if (r.big) final_enqueue(ctx, L, cs, k, kreq, fo);
     TK_HIP(hipGetLastError());
     return TOPK_OK;
 }
@@ -1216,19 +971,6 @@ void shard_merge_enqueue(hipStream_t s, const uint64_t *sh_ids, const float *sh_
     }
     const uint32_t kreq = (uint32_t)(n < k ? n : k);
     hipLaunchKernelGGL(shard_merge_kernel, dim3(1), dim3(MERGE_BS), 0, s, sh_ids, sh_scores, c, k, kreq, fo);
-}
-
-void final_enqueue(topk_ctx *ctx, Lane &L, const CandSet &cs, uint32_t k, uint32_t kreq, const FinalOut &fo,
-                   bool flat_fallback) {
-    hipStream_t s = L.stream;
-    if (flat_fallback) {
-        hipLaunchKernelGGL(cand_offsets_kernel, dim3(1), dim3(FLAT_BS), 0, s, L.st, cs, ctx->offsets, ctx->flat);
-        if (cs.nblk)
-            hipLaunchKernelGGL(cand_compact_kernel, dim3(cs.nblk), dim3(256), 0, s, cs, ctx->offsets, ctx->flat);
-        hipLaunchKernelGGL(fte_final_flat_kernel, dim3(1), dim3(FLAT_BS), 0, s, L.st, ctx->flat, k, kreq, fo);
-    } else {
-        hipLaunchKernelGGL(fte_final_kernel, dim3(1), dim3(FINAL_BS), 0, s, L.st, cs, k, kreq, fo, nullptr);
-    }
 }
 
 // ---------------------------------------------------------------------------

@@ -241,9 +241,9 @@ struct PtaLayout {
     float *pminsum = nullptr;    // nparts: sum of the d minima (rounded down)
     uint64_t *pbound = nullptr;  // query scratch: bound key per partition
     uint64_t *bmax = nullptr;    // query scratch: max bound key per 256 partitions
-    uint32_t *pcut = nullptr;    // query scratch: chunks to score per partition (0: ruled out)
-    uint32_t *wchunks = nullptr; // query scratch: chunks to score per cut workgroup
-    uint2 *wstat = nullptr;      // query scratch: partitions and objects to score per cut workgroup
+    uint32_t *pcut = nullptr;    // query scratch: objects to score per partition, by cut group (0: ruled out)
+    uint32_t *wchunks = nullptr; // query scratch: chunks to score per cut group
+    uint2 *wstat = nullptr;      // query scratch: partitions and objects to score per cut group
     int cus = 0;                 // compute units of the device (the scoring grid)
     uint32_t *h_report = nullptr; // pinned, written by the query: candidates, partitions, objects (u64); kept
                                   // over rebuilds (the build reports its sizes there), freed with the context
@@ -282,7 +282,7 @@ struct PtaLayout {
     double tt_build_ms = 0;
 };
 constexpr uint32_t PTA_CHUNK = 256;
-constexpr uint32_t PTA_CUT_GROUPS = 4096;  // cut workgroups of a query at most (the scoring pass scans their totals in LDS)
+constexpr uint32_t PTA_CUT_GROUPS = 4096;  // cut groups of a query at most (the scoring pass scans their totals in LDS)
 constexpr uint32_t PART_ALIGN = 256;
 static_assert(PART_ALIGN % PTA_CHUNK == 0, "partitions start on chunk boundaries");
 
@@ -340,9 +340,6 @@ struct FinalOut {
 };
 
 // Launch helpers implemented in the .hip translation units.
-// Enqueues the final select over a candidate set on lane L (fte.hip).
-void final_enqueue(topk_ctx *ctx, Lane &L, const CandSet &cs, uint32_t k, uint32_t kreq, const FinalOut &fo,
-                   bool flat_fallback);
 // One FTE pipeline run over objects [0, n) of the columns q points at (n = 0:
 // the whole store; ids are local to those columns).
 int fte_enqueue(topk_ctx *ctx, Lane &L, uint32_t k, const QCols &q, const FinalOut &fo, int mode, uint64_t n = 0);

@@ -21,8 +21,8 @@
 //    score (skip iff bound < tau strictly), each up to its first suffix row
 //    whose bound falls below tau, as chunk ranges; the scoring pass spreads
 //    those chunks evenly over every wave of the GPU and keeps keys >= tau;
-//    the FTE final select writes the exact top k straight into pinned host
-//    memory.  Results equal topk_fte's.
+//    its last workgroup selects the exact top k, as the plain stream's does,
+//    straight into pinned host memory.  Results equal topk_fte's.
 #include <string.h>
 
 #include <algorithm>
@@ -30,6 +30,7 @@
 #include "bound.hpp"
 #include "device.hpp"
 #include "internal.hpp"
+#include "select.hpp"
 
 namespace topk {
 
@@ -44,6 +45,7 @@ constexpr uint32_t PTA_SEED_LDS = PTA_SEED_REG * PTA_BS;  // seed winners the me
 // ---------------------------------------------------------------------------
 // query kernels
 // ---------------------------------------------------------------------------
+template <int NB>
 __global__ __launch_bounds__(PTA_BS) void pta_bound_kernel(BoundArgs b, uint32_t L,
                                                            const uint32_t *__restrict__ psz,
                                                            const float *__restrict__ pmax,
@@ -55,7 +57,7 @@ __global__ __launch_bounds__(PTA_BS) void pta_bound_kernel(BoundArgs b, uint32_t
     const uint32_t p = blockIdx.x * PTA_BS + threadIdx.x;
     uint64_t key = 0;
     if (p < L && psz[p]) {
-        const float ub = lp_bound(b, pmax + (uint64_t)p * b.d, pmin + (uint64_t)p * b.d, psum[p], pminsum[p]);
+        const float ub = lp_bound<NB>(b, pmax + (uint64_t)p * b.d, pmin + (uint64_t)p * b.d, psum[p], pminsum[p]);
         key = rkey(ub, p);
     }
     if (p < L) pbound[p] = key;
@@ -86,6 +88,16 @@ struct SeedKeys {
 #pragma unroll
         for (int j = 0; j < KPT; j++) f(v[j]);
     }
+};
+
+// Key array written with agent-scope (write-through) stores.
+struct AgentOut {
+    uint64_t *p;
+    struct Ref {
+        uint64_t *p;
+        __device__ __forceinline__ void operator=(uint64_t v) const { store_agent(p, v); }
+    };
+    __device__ __forceinline__ Ref operator[](uint32_t i) const { return Ref{p + i}; }
 };
 
 // Block t scores the leading PTA_SEED_OBJS objects (largest attribute sums)
@@ -162,18 +174,20 @@ __global__ __launch_bounds__(PTA_BS) void pta_seed_kernel(QCols q, const uint64_
     }
     uint64_t thr = 1;
     if (size > k) thr = block_kth_largest<PTA_BS, RegKeys<PTA_SEED_OBJS / PTA_BS>, 11>(rk, size, k, ss);
-    uint64_t *out = blk + (uint64_t)blockIdx.x * k;
+    // written through to where the last block reads them: no cache write-back
+    const AgentOut out{blk + (uint64_t)blockIdx.x * k};
     const uint32_t got = block_gather_ge<PTA_BS>(rk, thr, out, ss);
     for (uint32_t i = got + tid; i < k; i += PTA_BS) out[i] = 0;
     // this block's k-th key (k keys at or above it), or 0 with fewer than k
-    if (tid == 0) bthr[blockIdx.x] = got >= k ? thr : 0ull;
+    if (tid == 0) store_agent(bthr + blockIdx.x, got >= k ? thr : 0ull);
 
-    __threadfence();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's keys have reached memory
     __syncthreads();
-    if (tid == 0) is_last = (atomicAdd(&st->arrive, 1u) == gridDim.x - 1);
+    if (tid == 0)
+        is_last = __hip_atomic_fetch_add(&st->arrive, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
     __syncthreads();
     if (!is_last) return;
-    __threadfence();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     const uint32_t nk = gridDim.x * k;
     if (tid == 0) nvalid = 0;
     __syncthreads();
@@ -183,8 +197,8 @@ __global__ __launch_bounds__(PTA_BS) void pta_seed_kernel(QCols q, const uint64_
         // block alone has k keys at or above it): only keys at or above it
         // compete.  They are gathered into LDS and the one with exactly k-1
         // larger keys is the k-th (keys are distinct).
-        uint64_t floor_key = 0;
-        for (uint32_t b = 0; b < gridDim.x; b++) floor_key = bthr[b] > floor_key ? bthr[b] : floor_key;
+        static_assert(PTA_MAX_SEED <= 64, "a lane per seed block");
+        const uint64_t floor_key = wave_max_u64(lane_id() < gridDim.x ? bthr[lane_id()] : 0ull);
         const SeedKeys<PTA_SEED_REG> wk{blk, nk};
         const uint32_t nc = block_gather_ge<PTA_BS>(wk, floor_key ? floor_key : 1ull, cands, ss);
         if (nc > k && nc <= 2 * PTA_BS) {
@@ -218,34 +232,49 @@ __global__ __launch_bounds__(PTA_BS) void pta_seed_kernel(QCols q, const uint64_
 // Cut per partition, as the number of its leading objects to score: 0 when
 // its bound is below tau's score (skip iff bound < tau strictly), else the
 // objects before its first chunk whose suffix-row bound falls below tau
-// (every later object of the partition scores below tau too).  Workgroup
-// g owns partitions [g * R, (g + 1) * R) (R a multiple of 16), four per
-// wave per round, 16 lanes each, one chunk row per lane (a 4096-object
-// partition in one round), and publishes its chunk total (wchunks[g]) and
-// its partitions and objects to score (wstat[g]).  No atomics: the
-// scoring pass scans the workgroup totals.
+// (every later object of the partition scores below tau too).
+//
+// A wave takes group g: the R <= 64 partitions g, g + G, g + 2 G, ... (the
+// ones that survive are neighbours, so they spread over the waves), a lane
+// each for the bounds.  The survivors are then cut four at a time, 16 lanes
+// each, one chunk row per lane (a 4096-object partition in one round).  The
+// group's cuts, chunk total and report go out without atomics; the scoring
+// pass scans the totals.  Bound by the chain of one wave's loads; one
+// workgroup per 16 partitions, most of which did not survive, took 11.5 us at
+// 65536 partitions, this 7.4.
 template <int NB>
-__global__ __launch_bounds__(PTA_BS) void pta_cut_kernel(BoundArgs b, uint32_t L, uint32_t R,
+__global__ __launch_bounds__(PTA_BS) void pta_cut_kernel(BoundArgs b, uint32_t L, uint32_t R, uint32_t G,
                                                          const uint64_t *__restrict__ pbound,
                                                          const uint32_t *__restrict__ poff,
                                                          const uint32_t *__restrict__ psz,
                                                          const float *__restrict__ cstat, uint64_t nchunks,
                                                          const FteState *__restrict__ st, uint32_t *__restrict__ cut,
                                                          uint32_t *__restrict__ wchunks, uint2 *__restrict__ wstat) {
-    __shared__ uint32_t wsum[PTA_BS / 64][3];
-    const uint32_t lane = lane_id(), wave = threadIdx.x / 64, g = lane / 16, gl = lane % 16;
+    const uint32_t lane = lane_id(), part = lane / 16, gl = lane % 16;
+    const uint32_t g = blockIdx.x * (PTA_BS / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    if (g >= G) return;
     const uint32_t tau_hi = (uint32_t)(st->tau >> 32);
     const uint32_t d = b.d;
+    const uint32_t p = lane < R ? lane * G + g : L;
+    const uint64_t pb = p < L ? pbound[p] : 0ull;  // key 0: an empty partition
+    const bool alive = pb != 0 && (uint32_t)(pb >> 32) >= tau_hi;
+    const uint32_t psz_ = alive ? psz[p] : 0u, poff_ = alive ? poff[p] : 0u;
+    if (lane < R && !alive) cut[g * R + lane] = 0;
+    const uint64_t mask = __ballot(alive);
+    const uint32_t na = (uint32_t)__popcll(mask);
+    // lane i: the owner of the i-th survivor (the other lanes push past them)
+    const uint32_t below = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+    const uint32_t owner = (uint32_t)__builtin_amdgcn_ds_permute((int)(4u * (alive ? below : na + lane - below)), (int)lane);
     uint32_t ch = 0, parts = 0, objs = 0;  // this lane's partitions (lanes gl == 0)
-    for (uint32_t r = 0; r < R; r += 16) {
-        const uint32_t p = blockIdx.x * R + r + wave * 4 + g;
-        const uint64_t pb = p < L ? pbound[p] : 0ull;  // key 0: an empty partition
-        const bool alive = pb != 0 && (uint32_t)(pb >> 32) >= tau_hi;
-        const uint32_t sz = alive ? psz[p] : 0u;
-        const uint32_t c0 = alive ? poff[p] / PTA_CHUNK : 0u;
+    for (uint32_t i0 = 0; i0 < na; i0 += 4) {
+        const bool on = i0 + part < na;
+        const uint32_t src = (uint32_t)__shfl((int)owner, (int)((i0 + part) & 63u), 64);
+        const uint32_t szs = (uint32_t)__shfl((int)psz_, (int)src, 64), offs = (uint32_t)__shfl((int)poff_, (int)src, 64);
+        const uint32_t sz = on ? szs : 0u;
+        const uint32_t c0 = offs / PTA_CHUNK;
         const uint32_t nc = (sz + PTA_CHUNK - 1) / PTA_CHUNK;
-        uint32_t first = nc;  // this group's answer, settled once `done`
-        bool done = !alive;
+        uint32_t first = nc;  // this partition's answer, settled once `done`
+        bool done = !on;
         for (uint32_t cb = 0; __ballot(!done); cb += 16) {
             const uint32_t c = cb + gl;
             bool fail = false;
@@ -254,7 +283,7 @@ __global__ __launch_bounds__(PTA_BS) void pta_cut_kernel(BoundArgs b, uint32_t L
                 fail = okey(lp_bound<NB>(b, row, row + d * nchunks, row[2 * d * nchunks],
                                          row[(2 * d + 1) * nchunks], nchunks)) < tau_hi;
             }
-            const uint32_t m = (uint32_t)(__ballot(fail) >> (16 * g)) & 0xFFFFu;
+            const uint32_t m = (uint32_t)(__ballot(fail) >> (16 * part)) & 0xFFFFu;
             if (!done) {
                 if (m) {
                     first = cb + (uint32_t)__builtin_ctz(m);
@@ -265,85 +294,82 @@ __global__ __launch_bounds__(PTA_BS) void pta_cut_kernel(BoundArgs b, uint32_t L
             }
         }
         // objects to score: the chunks before the cut, the last one partial
-        const uint32_t o = alive ? min(sz, first * PTA_CHUNK) : 0u;
-        if (gl == 0 && p < L) {
-            cut[p] = o;
+        const uint32_t o = min(sz, first * PTA_CHUNK);
+        if (gl == 0 && on) {
+            cut[g * R + src] = o;
             ch += (o + PTA_CHUNK - 1) / PTA_CHUNK;
             parts += o ? 1u : 0u;
             objs += o;
         }
     }
-    for (int x = 32; x > 0; x >>= 1) {
-        ch += __shfl_xor(ch, x, 64);
-        parts += __shfl_xor(parts, x, 64);
-        objs += __shfl_xor(objs, x, 64);
-    }
+    ch = wave_sum_u32(ch);
+    parts = wave_sum_u32(parts);
+    objs = wave_sum_u32(objs);
     if (lane == 0) {
-        wsum[wave][0] = ch;
-        wsum[wave][1] = parts;
-        wsum[wave][2] = objs;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t a = 0, bp = 0, bo = 0;
-        for (int w = 0; w < PTA_BS / 64; w++) {
-            a += wsum[w][0];
-            bp += wsum[w][1];
-            bo += wsum[w][2];
-        }
-        wchunks[blockIdx.x] = a;
-        wstat[blockIdx.x] = make_uint2(bp, bo);
+        wchunks[g] = ch;
+        wstat[g] = make_uint2(parts, objs);
     }
 }
 
 // Scores the chunks of the partitions the cut pass kept.  Every workgroup
-// first scans the G cut-workgroup chunk totals into LDS (E[g]: chunks
-// before group g).  The waves split the chunks into equal contiguous
-// ranges; a wave finds its group by a binary search of E, holds the
-// group's cuts (lane j: partition g * R + j) and their chunk prefix in
-// registers, and walks on, one chunk per step: 4 objects per lane, the
-// queried columns loaded together.  Keys >= tau go to the workgroup's own
-// slot region of the candidate buffer (an LDS counter; past the slot, the
-// shared spill region), its count to cs.counts[workgroup].  Workgroup 0
-// also reports the partitions and objects scored.
+// first scans the G groups' chunk totals into LDS (E[g]: chunks before group
+// g).  The waves split the chunks into equal contiguous ranges; a wave finds
+// its group by a binary search of E, holds the group's cuts (lane j:
+// partition g + j * G) and their chunk prefix in registers, and walks on,
+// one chunk per step: 4 objects per lane, the queried columns loaded
+// together.  Keys >= tau go to the workgroup's own slot region of the
+// candidate buffer (an LDS counter; past the slot, the shared spill region),
+// its count to cs.counts[workgroup]; the last workgroup selects, as the
+// plain stream's does.  One workgroup of 16 waves per CU keeps the arrivals
+// few and gives the select its threads; with four of 4 waves and a select
+// launch, scoring and select took 12 + 7 us at N = 2^28, now 14.2 together.
+// Workgroup 0 also reports the partitions and objects scored.
+struct ScoreSelect {
+    uint32_t cap, kp2, k, kreq;
+    FinalOut fo;
+};
 template <int M>
-__global__ __launch_bounds__(PTA_BS) void pta_score_kernel(QCols q, uint32_t L, uint32_t R, uint32_t G,
-                                                           const uint32_t *__restrict__ cut,
-                                                           const uint32_t *__restrict__ wchunks,
-                                                           const uint2 *__restrict__ wstat,
-                                                           const uint32_t *__restrict__ poff,
-                                                           const uint32_t *__restrict__ pid,
-                                                           FteState *__restrict__ st, CandSet cs,
-                                                           uint32_t *__restrict__ report) {
-    __shared__ uint32_t E[PTA_CUT_GROUPS + 1];
-    __shared__ uint32_t wtot[PTA_BS / 64];
-    __shared__ uint32_t wrep[PTA_BS / 64][2];
-    __shared__ uint32_t lcount;
+__global__ __launch_bounds__(STREAM_BS) void pta_score_kernel(QCols q, uint32_t L, uint32_t R, uint32_t G,
+                                                              const uint32_t *__restrict__ cut,
+                                                              const uint32_t *__restrict__ wchunks,
+                                                              const uint2 *__restrict__ wstat,
+                                                              const uint32_t *__restrict__ poff,
+                                                              const uint32_t *__restrict__ pid,
+                                                              FteState *__restrict__ st, CandSet cs,
+                                                              uint32_t *__restrict__ report, ScoreSelect a) {
+    extern __shared__ uint64_t dyn[];  // cap keys | workgroup offsets, later cap keys
+    constexpr uint32_t GPT = PTA_CUT_GROUPS / STREAM_BS;
+    __shared__ union {
+        uint32_t E[PTA_CUT_GROUPS + 1];
+        FuseScratch sel;
+    } sh;
+    uint32_t *E = sh.E;
+    __shared__ uint32_t wtot[STREAM_NW];
+    __shared__ uint32_t wrep[STREAM_NW][2];
+    __shared__ uint32_t lcount, is_last;
     // the wave index made visibly uniform: the chunk cursor and its loads
     // (group offsets, cuts, partition offsets) are then scalar
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(tid / 64);
-    // exclusive scan of the group totals: thread t owns groups [16t, 16t + 16)
+    // exclusive scan of the group totals, GPT consecutive groups a thread
     {
-        uint32_t v[16], sum = 0, pp = 0, oo = 0;
+        uint32_t v[GPT], sum = 0, pp = 0, oo = 0;
 #pragma unroll
-        for (int j = 0; j < 16; j++) {
-            const uint32_t gi = tid * 16 + j;
+        for (uint32_t j = 0; j < GPT; j++) {
+            const uint32_t gi = tid * GPT + j;
             v[j] = gi < G ? wchunks[gi] : 0u;
             sum += v[j];
         }
         if (blockIdx.x == 0) {
             // partitions and objects scored, for the report (fit 32 bits: positions do)
 #pragma unroll
-            for (int j = 0; j < 16; j++) {
-                const uint32_t gi = tid * 16 + j;
+            for (uint32_t j = 0; j < GPT; j++) {
+                const uint32_t gi = tid * GPT + j;
                 const uint2 w = gi < G ? wstat[gi] : make_uint2(0u, 0u);
                 pp += w.x;
                 oo += w.y;
             }
-            for (int x = 32; x > 0; x >>= 1) {
-                pp += __shfl_xor(pp, x, 64);
-                oo += __shfl_xor(oo, x, 64);
-            }
+            pp = wave_sum_u32(pp);
+            oo = wave_sum_u32(oo);
             if (lane == 0) {
                 wrep[wave][0] = pp;
                 wrep[wave][1] = oo;
@@ -354,31 +380,32 @@ __global__ __launch_bounds__(PTA_BS) void pta_score_kernel(QCols q, uint32_t L, 
         if (tid == 0) lcount = 0;
         __syncthreads();
         uint32_t run = incl - sum, all = 0;
-        for (uint32_t w = 0; w < PTA_BS / 64; w++) {
+#pragma unroll
+        for (uint32_t w = 0; w < STREAM_NW; w++) {
             run += w < wave ? wtot[w] : 0u;
             all += wtot[w];
         }
 #pragma unroll
-        for (int j = 0; j < 16; j++) {
-            const uint32_t gi = tid * 16 + j;
+        for (uint32_t j = 0; j < GPT; j++) {
+            const uint32_t gi = tid * GPT + j;
             if (gi < G) E[gi] = run;
             run += v[j];
         }
         if (tid == 0) E[G] = all;  // the total
         if (blockIdx.x == 0 && tid == 0) {
-            uint32_t a = 0, o = 0;
-            for (int w = 0; w < PTA_BS / 64; w++) {
-                a += wrep[w][0];
+            uint32_t parts = 0, o = 0;
+            for (uint32_t w = 0; w < STREAM_NW; w++) {
+                parts += wrep[w][0];
                 o += wrep[w][1];
             }
-            report[1] = a;
+            report[1] = parts;
             report[2] = o;
             report[3] = 0;
         }
         __syncthreads();
     }
     const uint32_t total = E[G];
-    const uint32_t nw = gridDim.x * (PTA_BS / 64), gw = blockIdx.x * (PTA_BS / 64) + wave;
+    const uint32_t nw = gridDim.x * STREAM_NW, gw = blockIdx.x * STREAM_NW + wave;
     const uint64_t tau = st->tau;
     const uint32_t tau_hi = (uint32_t)(tau >> 32);
     const uint32_t per = (total + nw - 1) / nw;
@@ -394,11 +421,13 @@ __global__ __launch_bounds__(PTA_BS) void pta_score_kernel(QCols q, uint32_t L, 
             else hi = mid;
         }
         uint32_t grp = lo;
-        uint32_t gbase = 0, lch = 0, lincl = 0;  // lane j: chunks of partition grp * R + j, inclusive prefix
+        uint32_t gbase = 0, lch = 0, lincl = 0;  // lane j: chunks of partition grp + j * G, inclusive prefix
+        uint32_t lobj = 0, loff = 0;             // its objects to score and first position
         auto load_group = [&]() {
             gbase = E[grp];
-            const uint32_t p = grp * R + lane;
-            const uint32_t o = lane < R && p < L ? cut[p] : 0u;
+            lobj = lane < R ? cut[grp * R + lane] : 0u;
+            loff = lobj ? poff[lane * G + grp] : 0u;
+            const uint32_t o = lobj;
             lch = (o + PTA_CHUNK - 1) / PTA_CHUNK;
             lincl = wave_incl_scan(lch);
         };
@@ -412,10 +441,10 @@ __global__ __launch_bounds__(PTA_BS) void pta_score_kernel(QCols q, uint32_t L, 
             const uint64_t pm = __ballot(gbase + lincl > c);
             const uint32_t j = (uint32_t)__builtin_ctzll(pm);
             const uint32_t pincl = (uint32_t)__shfl(lincl, (int)j, 64), pch = (uint32_t)__shfl(lch, (int)j, 64);
-            const uint32_t p = grp * R + j, lc = c - (gbase + pincl - pch);
-            const uint32_t objs_p = cut[p];  // objects to score (uniform load)
+            const uint32_t lc = c - (gbase + pincl - pch);
+            const uint32_t objs_p = (uint32_t)__shfl((int)lobj, (int)j, 64);
             const uint32_t first = lc * PTA_CHUNK + 4 * lane;
-            const uint64_t pos = (uint64_t)poff[p] + first;
+            const uint64_t pos = (uint64_t)(uint32_t)__shfl((int)loff, (int)j, 64) + first;
             f4 sc = {0.0f, 0.0f, 0.0f, 0.0f};
             if constexpr (M > 0) {
                 f4 x[M];
@@ -464,18 +493,28 @@ __global__ __launch_bounds__(PTA_BS) void pta_score_kernel(QCols q, uint32_t L, 
                 for (int e = 0; e < 4; e++)
                     if (kk[e]) {
                         if (pos_k < cs.slot) {
-                            my[pos_k] = kk[e];
+                            store_agent(my + pos_k, kk[e]);
                         } else {
                             const uint32_t sp = sbase + (pos_k - first_spill);
-                            if (sp < cs.spill_cap) cs.spill[sp] = kk[e];
+                            if (sp < cs.spill_cap) store_agent(cs.spill + sp, kk[e]);
                         }
                         pos_k++;
                     }
             }
         }
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's candidates have reached memory
     __syncthreads();
-    if (tid == 0) cs.counts[blockIdx.x] = lcount < cs.slot ? lcount : cs.slot;
+    if (tid == 0) {
+        __hip_atomic_store(&cs.counts[blockIdx.x], lcount < cs.slot ? lcount : cs.slot, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        is_last = last_to_arrive(st);
+    }
+    __syncthreads();
+    if (!is_last) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    fused_select<STREAM_BS>(st, cs, a.k, a.kreq, a.cap, a.kp2, a.fo, dyn, dyn + a.cap, sh.sel);
 }
 
 // ---------------------------------------------------------------------------
@@ -496,8 +535,10 @@ int pta_query(topk_ctx *ctx, uint32_t k, uint8_t qq, const float *weights, const
     hipStream_t s = Ln.stream;
     const uint32_t L = P.nparts;
     const uint32_t nb = (L + PTA_BS - 1) / PTA_BS;
-    hipLaunchKernelGGL(pta_bound_kernel, dim3(nb), dim3(PTA_BS), 0, s, b, L, P.psz, P.pmax, P.pmin, P.psum,
-                       P.pminsum, P.pbound, P.bmax);
+    const int NB = ctx->d <= 8 ? 8 : (ctx->d <= 16 ? 16 : TOPK_MAX_DIMS);
+    auto bound = NB == 8 ? pta_bound_kernel<8> : (NB == 16 ? pta_bound_kernel<16> : pta_bound_kernel<TOPK_MAX_DIMS>);
+    hipLaunchKernelGGL(bound, dim3(nb), dim3(PTA_BS), 0, s, b, L, P.psz, P.pmax, P.pmin, P.psum, P.pminsum, P.pbound,
+                       P.bmax);
     // seed partitions are ranked by their own bounds when there are few of
     // them (so a small layout still seeds from several partitions), else by
     // the block maxima
@@ -515,23 +556,16 @@ int pta_query(topk_ctx *ctx, uint32_t k, uint8_t qq, const float *weights, const
 #undef TK_SEED
     hipEvent_t ev0 = nullptr;
     timing_begin(ctx, s, ev0);
-    // cut pass: R partitions per workgroup (four per wave per round), at
-    // most PTA_CUT_GROUPS workgroups
-    uint32_t R = 16;
-    while ((L + R - 1) / R > PTA_CUT_GROUPS) R += 16;
-    if (R > 64) return TOPK_ERR_UNSUPPORTED;  // a scoring wave holds one group's cuts
+    // cut pass: R partitions a wave, four (one round) on small layouts, at
+    // most 64 (a lane each) and PTA_CUT_GROUPS waves
+    const uint32_t R = std::min(64u, std::max(4u, (L + 1023) / 1024));
     const uint32_t G = (L + R - 1) / R;
-    if (ctx->d <= 8)
-        hipLaunchKernelGGL(pta_cut_kernel<8>, dim3(G), dim3(PTA_BS), 0, s, b, L, R, P.pbound, P.poff, P.psz, P.cstat,
-                           (uint64_t)P.nchunks, Ln.st, P.pcut, P.wchunks, P.wstat);
-    else if (ctx->d <= 16)
-        hipLaunchKernelGGL(pta_cut_kernel<16>, dim3(G), dim3(PTA_BS), 0, s, b, L, R, P.pbound, P.poff, P.psz,
-                           P.cstat, (uint64_t)P.nchunks, Ln.st, P.pcut, P.wchunks, P.wstat);
-    else
-        hipLaunchKernelGGL(pta_cut_kernel<TOPK_MAX_DIMS>, dim3(G), dim3(PTA_BS), 0, s, b, L, R, P.pbound, P.poff,
-                           P.psz, P.cstat, (uint64_t)P.nchunks, Ln.st, P.pcut, P.wchunks, P.wstat);
-    // scoring: four resident 4-wave workgroups per CU, one slot region each
-    const uint32_t sg = std::min((uint32_t)P.cus * 4, MAX_STREAM_GRID);
+    if (G > PTA_CUT_GROUPS) return TOPK_ERR_UNSUPPORTED;
+    auto cutk = NB == 8 ? pta_cut_kernel<8> : (NB == 16 ? pta_cut_kernel<16> : pta_cut_kernel<TOPK_MAX_DIMS>);
+    hipLaunchKernelGGL(cutk, dim3((G + PTA_BS / 64 - 1) / (PTA_BS / 64)), dim3(PTA_BS), 0, s, b, L, R, G, P.pbound,
+                       P.poff, P.psz, P.cstat, (uint64_t)P.nchunks, Ln.st, P.pcut, P.wchunks, P.wstat);
+    // scoring and select: one 16-wave workgroup per CU, one slot region each
+    const uint32_t sg = std::min((uint32_t)P.cus, MAX_STREAM_GRID);
     CandSet cs;
     cs.keys = Ln.cand;
     cs.counts = Ln.counts;
@@ -540,16 +574,20 @@ int pta_query(topk_ctx *ctx, uint32_t k, uint8_t qq, const float *weights, const
     cs.pre = nullptr;
     cs.spill = Ln.spill;
     cs.spill_cap = ctx->spill_cap;
-#define TK_SCORE(MM)                                                                                          \
-    hipLaunchKernelGGL(pta_score_kernel<MM>, dim3(sg), dim3(PTA_BS), 0, s, q, L, R, G, P.pcut, P.wchunks, P.wstat, \
-                       P.poff, P.pid, Ln.st, cs, P.h_report)
+    ScoreSelect sel{};
+    sel.k = k;
+    sel.kreq = (uint32_t)(ctx->n < k ? ctx->n : k);
+    sel.kp2 = next_pow2(k);
+    sel.cap = std::min(FUSE_CAP_MAX, std::max(FUSE_CAP_MIN, 4 * sel.kp2));
+    sel.fo = fo;
+    sel.fo.cand = P.h_report;  // report[0]
+    const size_t lds = sizeof(uint64_t) * ((size_t)sel.cap + std::max((sg + 3) / 2, sel.cap));
+#define TK_SCORE(MM)                                                                                                \
+    hipLaunchKernelGGL(pta_score_kernel<MM>, dim3(sg), dim3(STREAM_BS), lds, s, q, L, R, G, P.pcut, P.wchunks, P.wstat, \
+                       P.poff, P.pid, Ln.st, cs, P.h_report, sel)
     TK_SWITCH_M(q.m, TK_SCORE);
 #undef TK_SCORE
     timing_end(ctx, s, "pta_stream", ev0);
-    const uint32_t kreq = (uint32_t)(ctx->n < k ? ctx->n : k);
-    FinalOut f = fo;
-    f.cand = P.h_report;  // report[0]
-    final_enqueue(ctx, Ln, cs, k, kreq, f, false);
     TK_HIP(hipGetLastError());
     return TOPK_OK;
 }

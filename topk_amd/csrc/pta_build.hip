@@ -1349,7 +1349,7 @@ int pta_build(topk_ctx *ctx) {
         c.take(P.pminsum, L);
         c.take(P.pbound, L);
         c.take(P.bmax, (L + 255) / 256);
-        c.take(P.pcut, L);
+        c.take(P.pcut, L + 64);  // by group: R L/R rounded up
         c.take(P.wchunks, PTA_CUT_GROUPS);
         c.take(P.wstat, PTA_CUT_GROUPS);
         c.take(P.tmax, nn * d);
