@@ -716,6 +716,15 @@ static uint32_t sample_rank(double q) {
     return ks;
 }
 
+// The same for a query nothing re-runs: fewer than k means that ks of the
+// top k fell into the sample, for about Poisson(q) of them less often than
+// exp(-q) (e q / ks)^ks (Chernoff), here at most 1e-8.
+static uint32_t queued_rank(double q) {
+    uint32_t ks = 4;
+    while (ks < 4096 && (ks <= q || ks * (std::log(ks / q) - 1.0) + q < 18.4)) ks++;
+    return ks;
+}
+
 // How a query gets its threshold.
 struct SeedPlan {
     int tau;               // TAU_*
@@ -750,7 +759,7 @@ static SeedPlan seed_plan(uint64_t n, uint32_t k, int mode) {
         p.blocks = c8 >= SAMPLE_CHUNKS / 4 && c8 < SAMPLE_CHUNKS ? (uint32_t)c8 : SAMPLE_CHUNKS;
         p.stride = ((n / p.blocks) / SAMPLE_TILE) * SAMPLE_TILE;
         const double s = (double)p.blocks * SAMPLE_TILE;
-        p.ks = sample_rank(k * s / (double)n);
+        p.ks = mode == FTE_QUEUED ? queued_rank(k * s / (double)n) : sample_rank(k * s / (double)n);
         // each producer's share of the ks best: all of them up to 16 (the
         // producers' chunks alternate over the id range, so more than 16 of
         // a deep rank's best rarely meet in one; missing some lowers tau)
