@@ -1152,14 +1152,17 @@ struct OutDesc {
 // Publishes a finished batch to pinned host memory, as the last step of
 // the batch on its slot's stream: direct, the ids, scores and thresholds
 // into the caller's arrays and the status words into the staging block;
-// otherwise the whole output block into the staging block.  Its time is
-// the host link's, and the other slot's batch runs meanwhile.
+// otherwise every query's own results and what follows the rows into the
+// staging block.  Its time is the host link's, and the other slot's batch
+// runs meanwhile (1024 queries of 16..256 results at a stride of 256: 73 us
+// with the padding, 37 without).
 constexpr uint32_t BPUB_GRID = 64;
 struct PublishArgs {
     const unsigned char *d_out;
     size_t ids_off, sc_off, thr_off, st_off, bytes;
     uint64_t nres;
-    uint32_t nq;
+    uint32_t nq, ks;
+    const BatchQuery *q;
     const OutDesc *od;
     unsigned char *h_out;
 };
@@ -1182,7 +1185,21 @@ __global__ __launch_bounds__(256) void batch_publish_kernel(PublishArgs a) {
         for (uint64_t i = t; i < a.nq; i += stride) thr[i] = dt[i];
         for (uint64_t i = a.st_off / 4 + t; i < a.bytes / 4; i += stride) hw[i] = dw[i];
     } else {
-        for (uint64_t i = t; i < a.bytes / 4; i += stride) hw[i] = dw[i];
+        // each query's own results, a wave per query; then what follows the rows
+        const uint32_t lane = lane_id();
+        for (uint64_t q = t / 64; q < a.nq; q += stride / 64) {
+            const uint32_t k = a.q[q].k;
+            const uint64_t o = q * a.ks;
+            const uint64_t *di = reinterpret_cast<const uint64_t *>(a.d_out + a.ids_off) + o;
+            const float *ds = reinterpret_cast<const float *>(a.d_out + a.sc_off) + o;
+            uint64_t *hi = reinterpret_cast<uint64_t *>(a.h_out + a.ids_off) + o;
+            float *hs = reinterpret_cast<float *>(a.h_out + a.sc_off) + o;
+            for (uint32_t i = lane; i < k; i += 64) {
+                hi[i] = di[i];
+                hs[i] = ds[i];
+            }
+        }
+        for (uint64_t i = a.thr_off / 4 + t; i < a.bytes / 4; i += stride) hw[i] = dw[i];
     }
 }
 
@@ -2255,7 +2272,7 @@ static int batch_enqueue(topk_ctx *ctx, BatchState &B, hipStream_t s, uint32_t n
     if (!rc) rc = enqueue_pass(ctx, B, s, nq, ks, mode, v, true);
     if (rc) return rc;
     const PublishArgs pa{H.d_out,  ol.ids_off, ol.sc_off, ol.thr_off, ol.st_off,
-                         ol.bytes, (uint64_t)nq * ks, nq, reinterpret_cast<const OutDesc *>(d_in + il.od_off), H.h_out};
+                         ol.bytes, (uint64_t)nq * ks, nq, ks, dq, reinterpret_cast<const OutDesc *>(d_in + il.od_off), H.h_out};
     hipLaunchKernelGGL(batch_publish_kernel, dim3(BPUB_GRID), dim3(256), 0, s, pa);
     TK_HIP(hipGetLastError());
     return TOPK_OK;
