@@ -68,3 +68,20 @@ def test_select_ends(gpu, n, levels):
         for (k, w, a), (ri, rs) in zip(qs, ref):
             for got in (eng.fte(k, w, a), eng.pta(k, w, a)):
                 assert np.array_equal(got[0], ri) and np.array_equal(got[1].view(np.uint32), rs.view(np.uint32))
+
+
+@pytest.mark.parametrize("nq", [17, 300, 1024, 1025])
+@pytest.mark.parametrize("mode", [1, 2])
+def test_many_second_passes(gpu, nq, mode):
+    """Long lists over anticorrelated objects and weights of both signs: a
+    third of the queries overflow their candidate list and rerun, few enough
+    and too many for 64 slices each, in batches on both sides of 1024."""
+    n, d = 1_000_003, 8
+    qs = make_queries(np.random.default_rng(nq), nq, d, [512, 1024], mmin=5, wlo=-1.0)
+    with topk_amd.Engine.generated(n, d, topk_amd.ANTICORRELATED, 5) as eng:
+        eng.set_tuning("batch_fused", mode)
+        got = eng.batch(qs)
+        assert eng.stats()["retried"] > 2
+        for i, (q, (gi, gs, gt)) in enumerate(zip(qs, got)):
+            ri, rs, rt = eng.fte(*q)
+            assert np.array_equal(gi, ri) and np.array_equal(gs.view(np.uint32), rs.view(np.uint32)) and gt == rt, i

@@ -1299,7 +1299,7 @@ __global__ __launch_bounds__(BFIN_BS) void batch_final_kernel(FinalArgs a) {
 // ---------------------------------------------------------------------------
 // query-major pass
 // ---------------------------------------------------------------------------
-// Three launches replace the mask, the compaction and the item scoring when
+// Two or three launches replace the mask, the compaction and the item scoring when
 // thresholds are tight (a trained predictor): each query then reaches a few
 // dozen partitions and a few chunks in each, and the time of the item path
 // goes to list building, contended partition counters and dependent loads.
@@ -1314,8 +1314,9 @@ __global__ __launch_bounds__(BFIN_BS) void batch_final_kernel(FinalArgs a) {
 //     u = q * S + s lists (partition, first chunk index) pairs in
 //     tasks[u * ucap ...], chunk indices as an exclusive prefix over the
 //     list, and ucnt[u] = (entries, chunks).
-//  2. batch_unit_scan_kernel (one workgroup): exclusive prefix of the units'
-//     chunk counts, uoff[0..U].
+//  2. with more than BC_UNITS units, batch_unit_scan_kernel (one workgroup):
+//     exclusive prefix of the units' chunk counts, uoff[0..U]; fewer are
+//     scanned by the next pass's workgroups.
 //  3. batch_chunk_kernel: the uoff[U] chunks of all units are split into
 //     equal contiguous ranges, one per wave; a wave walks its range (its
 //     first unit and list entry found by a 64-way search per level), scores
@@ -1345,13 +1346,28 @@ struct CutArgs {
     const float *cstat;  // element e of chunk c at [e * nchunks + c]
     uint64_t nchunks;
     uint2 *tasks;        // unit u: tasks[u * ucap ...] = (partition, first chunk index within the unit)
-    uint64_t ucap;
     uint2 *ucnt;         // unit u: (entries, chunks)
     unsigned int *ctr;
     const uint32_t *qflag;  // second pass: settled queries are skipped
     uint32_t S;             // slices per query (gridDim.y)
     const uint32_t *flist;  // second pass: the flagged queries ([0] count); workgroup x takes entries x, x + gridDim.x, ...
+    uint32_t most;          // second pass: units at most (0: any number)
 };
+
+// Units a scoring workgroup scans by itself.
+constexpr uint32_t BC_UNITS = 1024;
+
+// Slices per query of a pass: S, halved in a second pass (S a power of two)
+// until its units fit `most`, and the task entries of a unit (G is a power of
+// two: queries x slices x entries never grows).
+__device__ __forceinline__ uint32_t bq_pass_slices(const uint32_t *flist, uint32_t S, uint32_t most) {
+    if (flist && most)
+        while (S > 1 && S * flist[0] > most) S /= 2;
+    return S;
+}
+__device__ __forceinline__ uint64_t bq_unit_cap(uint32_t G, uint32_t H, uint32_t S) {
+    return (uint64_t)((G + S - 1) / S) << H;
+}
 
 // Index i < n of the last entry with off[i] <= t (off non-decreasing, off[0] = 0).
 __device__ __forceinline__ uint32_t last_le(const uint32_t *off, uint32_t n, uint32_t t) {
@@ -1435,10 +1451,13 @@ __global__ __launch_bounds__(BQ_BS, bq_waves_per_simd(NB)) void batch_cut_kernel
     __shared__ uint32_t wsum[BQ_BS / 64];
     __shared__ uint32_t ng, np, tot;
     const uint32_t sl = blockIdx.y, tid = threadIdx.x;
+    const uint32_t S = bq_pass_slices(a.flist, a.S, a.most);
+    if (sl >= S) return;
+    const uint64_t ucap = bq_unit_cap(a.G, a.H, S);
     const uint32_t nent_list = a.flist ? a.flist[0] : gridDim.x;
     for (uint32_t f = blockIdx.x; f < nent_list; f += gridDim.x) {
     const uint32_t q = a.flist ? a.flist[1 + f] : f;
-    const uint64_t u = (uint64_t)f * a.S + sl;
+    const uint64_t u = (uint64_t)f * S + sl;
     if (a.qflag && a.qflag[q] == QF_DONE) {
         if (tid == 0) a.ucnt[u] = make_uint2(0u, 0u);
         continue;
@@ -1453,7 +1472,7 @@ __global__ __launch_bounds__(BQ_BS, bq_waves_per_simd(NB)) void batch_cut_kernel
     }
     __syncthreads();
     // groups of this slice
-    for (uint32_t g = sl + a.S * tid; g < a.G; g += a.S * BQ_BS) {
+    for (uint32_t g = sl + S * tid; g < a.G; g += S * BQ_BS) {
         const float ub = node_bound<NB>(b, a.t, a.G + g);
         if (ub > -INFINITY && ub >= tau && !(sat && a.t.tminid[a.G + g] > tau_id))
             glist[atomicAdd(&ng, 1u)] = (uint16_t)g;
@@ -1461,7 +1480,7 @@ __global__ __launch_bounds__(BQ_BS, bq_waves_per_simd(NB)) void batch_cut_kernel
     __syncthreads();
     const uint32_t H = a.H, per = 1u << H, total = ng << H;
     constexpr uint32_t STEP = BQ_BS * U;  // partition bounds per step
-    uint2 *out = a.tasks + u * a.ucap;
+    uint2 *out = a.tasks + u * ucap;
     uint32_t parts = 0, nent = 0, nchk = 0;
     auto flush = [&]() {
         const uint32_t n = np;
@@ -1541,20 +1560,26 @@ struct ChunkArgs {
     uint64_t ld;
     const uint32_t *poff, *psz, *pid;
     const uint2 *tasks;
-    uint64_t ucap;
+    uint32_t G, H;
     const uint2 *ucnt;
-    const uint32_t *uoff;
+    const uint32_t *uoff;      // null: scanned here, by every workgroup
     uint32_t nu, S;            // units (nu_host) and slices per query
     const uint32_t *flist;     // second pass: unit u belongs to query flist[1 + u / S] ([0] count)
     uint64_t *cand;
     unsigned int *ccount;
     unsigned long long *scored;  // per workgroup
     const uint32_t *cminid;      // smallest object id per chunk
+    uint32_t most;               // as CutArgs
 };
 
 constexpr uint32_t BC_STAGE = 256;  // candidate keys a wave stages in LDS before one append
 
+// SCAN: at most BC_UNITS units, whose chunk counts every workgroup scans into
+// LDS, 1 to 2 us instead of a launch of 4.5 us a pass (32 queries over 2^20
+// objects: 104 -> 99 us; four learned batches at N = 2^26: 410 -> 399 us).
+template <bool SCAN>
 __global__ __launch_bounds__(BC_BS) void batch_chunk_kernel(ChunkArgs a) {
+    __shared__ uint32_t loff[SCAN ? BC_UNITS + 1 : 1], wsum[BC_BS / 64], ltot;
     __shared__ unsigned long long wpairs[BC_BS / 64][2];
     __shared__ uint64_t stage[BC_BS / 64][BC_STAGE];
     // the wave index made visibly uniform: the whole chunk cursor (unit,
@@ -1562,8 +1587,31 @@ __global__ __launch_bounds__(BC_BS) void batch_chunk_kernel(ChunkArgs a) {
     // are scalar (62 vector registers instead of 76: eight waves per SIMD)
     const uint32_t lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const uint32_t nwaves = gridDim.x * (BC_BS / 64), gw = blockIdx.x * (BC_BS / 64) + wave;
-    const uint32_t nu = a.flist ? a.flist[0] * a.S : a.nu;
-    const uint32_t total = a.uoff[nu];
+    const uint32_t S = bq_pass_slices(a.flist, a.S, a.most);
+    const uint64_t ucap = bq_unit_cap(a.G, a.H, S);
+    const uint32_t nu = a.flist ? a.flist[0] * S : a.nu;
+    if constexpr (SCAN) {
+        constexpr uint32_t PER = BC_UNITS / BC_BS;
+        uint32_t c[PER], mine = 0;
+#pragma unroll
+        for (uint32_t e = 0; e < PER; e++) {
+            const uint32_t i = threadIdx.x * PER + e;
+            c[e] = i < nu ? a.ucnt[i].y : 0u;
+            mine += c[e];
+        }
+        uint32_t run = block_excl_scan<BC_BS>(mine, wsum, &ltot);
+#pragma unroll
+        for (uint32_t e = 0; e < PER; e++) {
+            const uint32_t i = threadIdx.x * PER + e;
+            if (i < nu) loff[i] = run;
+            run += c[e];
+        }
+        if (threadIdx.x == 0) loff[nu] = ltot;
+        __syncthreads();
+    }
+    const uint32_t *uoff = SCAN ? loff : a.uoff;
+    auto first_chunk = [&](uint32_t i) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)uoff[i]); };
+    const uint32_t total = first_chunk(nu);
     const uint32_t per = (total + nwaves - 1) / nwaves;
     uint32_t t = gw * per;
     const uint32_t t_end = t + per < total ? t + per : total;
@@ -1571,13 +1619,12 @@ __global__ __launch_bounds__(BC_BS) void batch_chunk_kernel(ChunkArgs a) {
     unsigned long long terms = 0;
     uint64_t *wst = stage[wave];
     if (t < t_end) {
-        const uint32_t *uoff = a.uoff;
         uint32_t u = wave_last_le([&](uint32_t i) { return uoff[i]; }, 0u, nu, t);
-        uint32_t ub = uoff[u], ue = uoff[u + 1];
-        const uint2 *tl = a.tasks + (uint64_t)u * a.ucap;
+        uint32_t ub = first_chunk(u), ue = first_chunk(u + 1);
+        const uint2 *tl = a.tasks + (uint64_t)u * ucap;
         uint32_t ne = a.ucnt[u].x;
         uint32_t j = wave_last_le([&](uint32_t i) { return tl[i].y; }, 0u, ne, t - ub);
-        auto query_of = [&](uint32_t uu) { return a.flist ? a.flist[1 + uu / a.S] : uu / a.S; };
+        auto query_of = [&](uint32_t uu) { return a.flist ? a.flist[1 + uu / S] : uu / S; };
         uint32_t q = query_of(u);
         // the query's terms, lane j holding term j
         float lw = 0.0f, tau = 0.0f;
@@ -1615,9 +1662,9 @@ __global__ __launch_bounds__(BC_BS) void batch_chunk_kernel(ChunkArgs a) {
             while (t >= ue) {  // next unit with chunks
                 u++;
                 ub = ue;
-                ue = uoff[u + 1];
+                ue = first_chunk(u + 1);
                 if (t < ue) {
-                    tl = a.tasks + (uint64_t)u * a.ucap;
+                    tl = a.tasks + (uint64_t)u * ucap;
                     ne = a.ucnt[u].x;
                     j = 0;
                     jb = 0;
@@ -2037,7 +2084,7 @@ static int ensure(topk_ctx *ctx, BatchState &B, uint32_t nq, uint32_t ks, int si
         // allow, at most six, so two wave slots per SIMD stay free for the
         // other batch in flight (six measured 3% above eight)
         int nb = 0;
-        TK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_chunk_kernel, BC_BS, 0));
+        TK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, batch_chunk_kernel<true>, BC_BS, 0));
         B.chunk_wgs = nb < 1 ? 1 : (nb > 6 ? 6 : nb);
     }
     if (changed) drop_graphs(B);
@@ -2178,22 +2225,26 @@ static int enqueue_pass(topk_ctx *ctx, BatchState &B, hipStream_t s, uint32_t nq
     if (v.fused && B.slot[B.cur].d_tasks) {
         // a second pass re-runs few queries: each is spread over S slices
         const uint32_t S = bq_slices(nq, second, ctx->tune.batch_slices);
-        const uint64_t ucap = (uint64_t)((G + S - 1) / S) << H;
+        // few units: every scoring workgroup scans their chunk counts itself
+        // (a second pass thins its slices to fit)
+        const bool scan = (second ? nq : nq * S) <= BC_UNITS;
+        const uint32_t most = scan ? BC_UNITS : 0;
         // the second pass works through the list of flagged queries the
         // first final select wrote: a few workgroups per slice, not one per query
         const uint32_t *fl = second ? B.slot[B.cur].d_flist : nullptr;
         const uint32_t gx = second ? std::min(nq, 16u) : nq;
         const CutArgs ca{dq,       db,    ta,     G,       H,       L,         ctx->d,  P.poff, P.psz,
-                         P.cstat,  (uint64_t)P.nchunks, B.slot[B.cur].d_tasks, ucap, B.slot[B.cur].d_ucnt, B.slot[B.cur].d_ctr, pass_flags, S, fl};
+                         P.cstat,  (uint64_t)P.nchunks, B.slot[B.cur].d_tasks, B.slot[B.cur].d_ucnt, B.slot[B.cur].d_ctr, pass_flags, S, fl, most};
         auto ck = NB == 8 ? batch_cut_kernel<8> : (NB == 16 ? batch_cut_kernel<16> : batch_cut_kernel<32>);
         hipLaunchKernelGGL(ck, dim3(gx, S), dim3(BQ_BS), 0, s, ca);
-        hipLaunchKernelGGL(batch_unit_scan_kernel, dim3(1), dim3(1024), 0, s, B.slot[B.cur].d_ucnt, nq * S, fl, S, B.slot[B.cur].d_uoff);
+        if (!scan)
+            hipLaunchKernelGGL(batch_unit_scan_kernel, dim3(1), dim3(1024), 0, s, B.slot[B.cur].d_ucnt, nq * S, fl, S, B.slot[B.cur].d_uoff);
         const uint32_t g2 = (uint32_t)B.cus * (second ? 2 : (uint32_t)B.chunk_wgs);  // all resident at once
-        const ChunkArgs xa{dq, P.pcols, P.ld, P.poff, P.psz, P.pid, B.slot[B.cur].d_tasks, ucap, B.slot[B.cur].d_ucnt, B.slot[B.cur].d_uoff, nq * S, S,
-                           fl, B.slot[B.cur].d_cand, B.slot[B.cur].d_ccount, B.slot[B.cur].d_scored, P.cminid};
+        const ChunkArgs xa{dq, P.pcols, P.ld, P.poff, P.psz, P.pid, B.slot[B.cur].d_tasks, G, H, B.slot[B.cur].d_ucnt, scan ? nullptr : B.slot[B.cur].d_uoff, nq * S, S,
+                           fl, B.slot[B.cur].d_cand, B.slot[B.cur].d_ccount, B.slot[B.cur].d_scored, P.cminid, most};
         hipEvent_t ev0 = nullptr;
         timing_begin(ctx, s, ev0);
-        hipLaunchKernelGGL(batch_chunk_kernel, dim3(g2), dim3(BC_BS), 0, s, xa);
+        hipLaunchKernelGGL(scan ? batch_chunk_kernel<true> : batch_chunk_kernel<false>, dim3(g2), dim3(BC_BS), 0, s, xa);
         timing_end(ctx, s, second ? "batch_score_second" : "batch_score", ev0);
         fa.nscored = g2;
         if (v.digit == 8)
