@@ -387,7 +387,12 @@ __global__ __launch_bounds__(BSEED_BS) void batch_seed_kernel(BatchQuery *__rest
 // project more than `budget` ids to reach k; such queries then take all
 // ties as candidates or their learned score threshold, by the projected
 // number of ties (end of the kernel).  No query leaves it marked.
-constexpr uint64_t BXB_BUDGET = 1ull << 19;  // ids a scan may cover
+// Ids a scan may cover.  1024 queries, d = 16, mixed, k <= 256: at N = 2^24
+// the scan takes 5, 10, 16 and 25 us for 2^16, 2^18, 2^19 and 2^20 ids and
+// the whole batch 1104 (2^17), 1039, 1023 and 1045 us; the pairs a longer
+// scan saves grow with N: at 2^26 four batches take 4.00 ms with 2^19 and
+// 3.85 ms with 2^20.
+static uint64_t bxb_budget(uint64_t n) { return n <= 1ull << 25 ? 1ull << 19 : 1ull << 20; }
 constexpr int BXB_BS = 256;                  // threads per scan workgroup
 constexpr int BXB_R0 = 4;                    // rows ANDed for every word
 // W words of one row from 16-byte loads (rows are 128-byte aligned and w
@@ -409,11 +414,8 @@ __device__ __forceinline__ void load_words(const uint64_t *__restrict__ p, uint6
 // fetched.  The rows of each phase are loaded all at once, the first ones
 // of the next step before this step's others.
 //
-// Bound by the queries that scan the whole budget, 1 MB of rows through one
-// CU: 1024 queries (d = 16, N = 2^24, mixed, k <= 256) take 5, 10, 16 and 25
-// us at budgets of 2^16, 2^18, 2^19 and 2^20 ids, and the whole batch 1104
-// (2^17), 1039, 1023 and 1045 us: past 2^19 ids the scan costs more than the
-// pairs it saves.  512 or 1024 threads a query took no less.
+// Bound by the queries that scan the whole budget, 1 or 2 MB of rows through
+// one CU: 512 or 1024 threads a query took no less.
 template <int MAXR, int W>
 __global__ __launch_bounds__(BXB_BS) void batch_tiebits_kernel(BatchQuery *__restrict__ qs,
                                                             const uint64_t *__restrict__ xbits, uint32_t d,
@@ -2187,7 +2189,7 @@ static int enqueue_pass(topk_ctx *ctx, BatchState &B, hipStream_t s, uint32_t nq
             // extreme-value bitmaps, else a seed (key) threshold
             if (P.xbits) {
                 auto tk = ctx->d <= 16 ? batch_tiebits_kernel<16, 4> : batch_tiebits_kernel<32, 2>;
-                hipLaunchKernelGGL(tk, dim3(nq), dim3(BXB_BS), 0, s, dq, P.xbits, ctx->d, P.nw, ctx->n, BXB_BUDGET);
+                hipLaunchKernelGGL(tk, dim3(nq), dim3(BXB_BS), 0, s, dq, P.xbits, ctx->d, P.nw, ctx->n, bxb_budget(ctx->n));
             } else {  // no bitmaps (the layout was rebuilt after training): seeds
                 const int NB = dims_class(ctx->d);
                 auto seed = NB == 8 ? batch_seed_kernel<8> : (NB == 16 ? batch_seed_kernel<16> : batch_seed_kernel<32>);
