@@ -9,7 +9,7 @@ import topk_amd
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 3000, 1024 * 1030, 1024 * 4096 + 5, 1024 * 5000 + 1, 66_100_003])
+@pytest.mark.parametrize("n", [1, 3000, 1024 * 257, 1024 * 700, 1024 * 1030, 1024 * 4096 + 5, 1024 * 5000 + 1, 66_100_003])
 @pytest.mark.parametrize("d,distr", [(2, topk_amd.ANTICORRELATED), (9, topk_amd.CORRELATED), (17, topk_amd.INDEPENDENT)])
 def test_group_edges(gpu, n, d, distr):
     if n > 10**7 and d > 2:

@@ -37,7 +37,8 @@ namespace topk {
 constexpr int PTA_BS = 256;
 constexpr uint32_t PTA_SEED_OBJS = 1024;     // leading objects (largest attribute sums) of a seed partition
 constexpr uint32_t PTA_MIN_SEED = 16;        // seed partitions at least
-constexpr uint32_t PTA_SEED_RANK = 1024;     // block maxima ranked in LDS by the seed kernel
+constexpr uint32_t PTA_SEED_RANK = 1024;     // keys the seed kernel ranks at most
+static_assert(PTA_MAX_PARTS <= PTA_SEED_RANK * PTA_BS, "block maxima of any layout fit the ranking");
 constexpr uint32_t PTA_MAX_SEED = 64;
 constexpr int PTA_SEED_REG = 16;             // seed winners per thread the merge reads at once
 constexpr uint32_t PTA_SEED_LDS = PTA_SEED_REG * PTA_BS;  // seed winners the merge ranks in LDS
@@ -115,34 +116,42 @@ __global__ __launch_bounds__(PTA_BS) void pta_seed_kernel(QCols q, const uint64_
     __shared__ SelectScratch ss;
     __shared__ uint64_t pick;
     __shared__ uint32_t is_last, nvalid;
-    __shared__ uint64_t bm[PTA_SEED_RANK];
+    __shared__ uint64_t bm[PTA_BS];
     __shared__ uint64_t cands[PTA_SEED_LDS];
     __shared__ uint64_t kth;
     const uint32_t tid = threadIdx.x;
     if (tid == 0) pick = 0;
-    if (nb <= PTA_SEED_RANK) {
-        // the (t+1)-th largest block maximum: the nonzero key with exactly t
-        // larger ones (keys carry partition ids, so nonzero keys are distinct)
-        for (uint32_t i = tid; i < nb; i += PTA_BS) bm[i] = bmax[i];
+    // the (t+1)-th largest of the keys (they carry partition ids, so nonzero
+    // keys are distinct): up to one a thread, the key with exactly t larger
+    // ones; above, where that took 45 us at 1024 keys, a radix select
+    if (nb <= PTA_BS) {
+        const uint64_t v = tid < nb ? bmax[tid] : 0ull;
+        bm[tid] = v;
         __syncthreads();
-        for (uint32_t i = tid; i < nb; i += PTA_BS) {
-            const uint64_t v = bm[i];
-            uint32_t r = 0, unused = 0;
-            rank2_lds(bm, nb, v, v, r, unused);
-            if (v && r == blockIdx.x) pick = v;
+        uint32_t r = 0, unused = 0;
+        rank2_lds(bm, nb, v, v, r, unused);
+        if (v && r == blockIdx.x) pick = v;
+    } else {
+        RegKeys<PTA_SEED_RANK / PTA_BS> bk;
+        uint32_t mine = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < PTA_SEED_RANK / PTA_BS; j++) {
+            const uint32_t i = j * PTA_BS + tid;
+            bk.k[j] = i < nb ? bmax[i] : 0ull;
+            mine += bk.k[j] ? 1u : 0u;
         }
-    } else if (tid < 64) {
-        // (t+1)-th largest block maximum by wave-max rounds
-        uint64_t best = 0;
-        for (uint32_t r = 0; r <= blockIdx.x; r++) {
-            uint64_t lm = 0;
-            for (uint32_t i = lane_id(); i < nb; i += 64) {
-                const uint64_t v = bmax[i];
-                if (v > lm && (r == 0 || v < best)) lm = v;
-            }
-            best = wave_max_u64(lm);
+        if (tid == 0) nvalid = 0;
+        __syncthreads();
+        mine = wave_sum_u32(mine);
+        if (lane_id() == 0) atomicAdd(&nvalid, mine);
+        __syncthreads();
+        const uint32_t valid = nvalid;
+        __syncthreads();
+        if (blockIdx.x < valid) {  // uniform
+            const uint64_t v =
+                block_kth_largest<PTA_BS, RegKeys<PTA_SEED_RANK / PTA_BS>, 11>(bk, valid, blockIdx.x + 1, ss);
+            if (tid == 0) pick = v;
         }
-        if (tid == 0) pick = best;
     }
     __syncthreads();
     const uint64_t pk = pick;
