@@ -299,7 +299,7 @@ __device__ __forceinline__ void sample_publish(const QCols &q, uint64_t n, uint3
 // add two more trips to memory) and returns the ks-th largest.  The wait is
 // bounded: should it run out, a threshold of 0 admits every object and the
 // candidate count settles what happens.
-constexpr uint32_t SAMPLE_SPINS = 1u << 20;
+constexpr uint32_t SAMPLE_SPINS = 1u << 23;  // more than 10 s: past any stall of the producers
 __device__ __forceinline__ uint64_t sample_tau(FteState *__restrict__ st, uint32_t nwin, uint32_t ks) {
     constexpr int NPL = SAMPLE_WIN / 64;
     for (uint32_t s = 0; s < SAMPLE_SPINS; s++) {
@@ -847,10 +847,17 @@ static CandSet fte_launch(const FteRun &r, uint32_t k, const QCols &q, const Fin
     while (cap < FUSE_CAP_MAX && (cap < 2 * a.kp2 || cap < 2 * sp.expect)) cap += FUSE_CAP_MIN;
     a.cap = cap;
     const uint32_t g = a.ntiles ? stream_grid(r.grid_cap, a.ntiles) : 0;
-    // the last tiles by ticket; a run whose slots hold a block's every object
-    // deals all of them
+    // The last sixth of the tiles by ticket, at least two a workgroup, four
+    // where a tile lasts longer (above 8 columns): with a twelfth and two, a
+    // workgroup that the query before delays at its start (its last one
+    // selects) ended late.  Queued queries, 2^25 objects: 12 columns 251 ->
+    // 242 us, 8 columns 171 -> 164 (alone 202 -> 194); 2^24 x 12: 130 with
+    // two, 125 with four, 2^24 x 5: 58.3 and 59.7.  Up to four tiles a
+    // workgroup are all dealt (2^22 x 8: 37 -> 34 us), and so are those of a
+    // run whose slots hold a block's every object.
     a.nstatic = a.ntiles;
-    if (!r.big && a.ntiles > 2ull * g) a.nstatic = (a.ntiles - std::max<uint64_t>(a.ntiles / 12, 2ull * g) + g - 1) / g * g;
+    if (!r.big && a.ntiles > 4ull * g)
+        a.nstatic = (a.ntiles - std::max<uint64_t>(a.ntiles / 6, (q.m > 8 ? 4ull : 2ull) * g) + g - 1) / g * g;
     a.wgs = g < SAMPLE_WGS ? g : SAMPLE_WGS;
     CandSet &cs = a.cs;
     cs.keys = r.cand;
