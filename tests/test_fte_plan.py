@@ -1,0 +1,85 @@
+"""The plain query's launch plans (topk_amd/csrc/fte_plan.hpp) on the CPU:
+how far the stream's tiles and the exact seed read a column, and what the
+slots of an n-entry run take, over store sizes, widths, modes and the tuned
+tile and grid -- the sizes around every tile, pad and plan limit."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+HEADER = r"""
+#include <cstdint>
+#include <cstdio>
+#include <initializer_list>
+#include <vector>
+#include "fte_plan.hpp"
+using namespace topk;
+static int fails = 0;
+#define CHECK(c, ...) do { if (!(c)) { if (fails++ < 10) { std::printf("%s: ", #c); std::printf(__VA_ARGS__); std::printf("\n"); } } } while (0)
+"""
+
+REACH = HEADER + r"""
+int main() {
+    std::vector<uint64_t> sizes;
+    for (uint64_t c : {1ull, 4096ull, 8192ull, 32768ull, 1ull << 19, 1ull << 20, 1ull << 21, 3000001ull, 1ull << 23,
+                       8388609ull, 10000000ull, 150000000ull, 1ull << 28, (1ull << 32) - 8192})
+        for (int64_t o : {-8191, -4097, -4095, -1, 0, 1, 4, 4095, 4097, 8191})
+            if ((int64_t)c + o >= 1 && c + o < 0xFFFFFFFFull) sizes.push_back(c + o);
+    for (uint64_t n : sizes)
+        for (uint32_t m : {1u, 2u, 3u, 5u, 9u, 20u})
+            for (uint32_t k : {1u, 200u, 1024u})
+                for (int mode : {FTE_SAMPLE, FTE_EXACT, FTE_EXACT_BIG, FTE_QUEUED})
+                    for (int vpt : {0, 1, 2, 4, 8})
+                        for (uint32_t grid : {0u, 1u, 257u, MAX_STREAM_GRID}) {
+                            const SeedPlan s = seed_plan(n, k, mode);
+                            const uint64_t first = s.tau == TAU_STATE ? s.n_eff : 0, pad = (n + 3) / 4 * 4;
+                            const bool big = mode == FTE_EXACT_BIG;
+                            const StreamPlan p = stream_plan(n, first, m, big, vpt, grid, 1ull << 21);
+                            // the stream: every object of [first, n), nothing past the column's last vector
+                            CHECK(first + p.ntiles * p.tile >= n && (!p.ntiles || first % 4 == 0), "n %llu", (unsigned long long)n);
+                            const uint32_t last = (uint32_t)((n - 1) / 4);
+                            uint64_t most = 0;
+                            for (uint64_t t = p.ntiles > 2 ? p.ntiles - 2 : 0; t < p.ntiles; t++)
+                                for (uint64_t v = 0; v < p.tile / 4; v += v + 1 < p.tile / 4 && v ? p.tile / 4 - 1 - v : 1)
+                                    most = std::max<uint64_t>(most, 4ull * tile_vec((uint32_t)((first + t * p.tile) / 4 + v), last) + 4);
+                            CHECK(most <= pad, "n %llu m %u k %u mode %d vpt %d: reads %llu", (unsigned long long)n, m, k,
+                                  mode, vpt, (unsigned long long)most);
+                            // samples and the exact seed
+                            if (s.tau == TAU_STATE)
+                                CHECK(((s.n_eff + SEED_TILE - 1) / SEED_TILE) * SEED_TILE <= n + PAD_REACH, "n %llu",
+                                      (unsigned long long)n);
+                            if (s.tau == TAU_SHARED)
+                                CHECK((s.blocks - 1) * s.stride + SAMPLE_TILE <= n + SAMPLE_TILE - 1, "n %llu",
+                                      (unsigned long long)n);
+                            // slots: an n-entry run's hold every object of a workgroup's tiles, inside the buffer
+                            if (big && p.grid) {
+                                CHECK((uint64_t)p.slot >= (p.ntiles + p.grid - 1) / p.grid * p.tile, "n %llu",
+                                      (unsigned long long)n);
+                                CHECK((uint64_t)p.slot * p.grid <= big_slots(n), "n %llu m %u vpt %d grid %u",
+                                      (unsigned long long)n, m, vpt, grid);
+                            }
+                            CHECK(p.grid <= MAX_STREAM_GRID && p.grid <= std::max<uint64_t>(p.ntiles, 1), "grid %u", p.grid);
+                            CHECK(p.nstatic <= p.ntiles && (p.nstatic == p.ntiles || p.nstatic >= p.grid), "n %llu",
+                                  (unsigned long long)n);
+                        }
+    return fails ? 1 : 0;
+}
+"""
+
+
+def _run(program, tmp_path):
+    if not shutil.which("g++"):
+        pytest.skip("no g++")
+    src, exe = tmp_path / "plan.cpp", tmp_path / "plan"
+    src.write_text(program)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-I", os.path.join(ROOT, "topk_amd", "csrc"), str(src), "-o", str(exe)],
+                   check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout
+
+
+def test_reads_and_slots_stay_inside_their_buffers(tmp_path):
+    _run(REACH, tmp_path)

@@ -329,7 +329,7 @@ static void emit_result(topk_ctx *ctx, uint32_t k, uint64_t *out_ids, float *out
 // Fallback buffers: slots large enough that no stream block can overflow
 // (every block's objects fit in its slot) and a flat gather buffer.
 static int ensure_big(topk_ctx *ctx, uint64_t n) {
-    const uint64_t need = n + (uint64_t)MAX_STREAM_GRID * 8192 + TOPK_MAX_K;
+    const uint64_t need = big_slots(n);
     if (ctx->cand_big && ctx->cand_big_cap >= need) return TOPK_OK;
     hipFree(ctx->cand_big);
     hipFree(ctx->flat);

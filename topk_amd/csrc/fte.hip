@@ -37,28 +37,18 @@
 
 #include "device.hpp"
 #include "emit.hpp"
+#include "fte_plan.hpp"
 #include "internal.hpp"
 #include "select.hpp"
 
 namespace topk {
 
 constexpr int SEED_BS = 256;
-constexpr uint32_t SEED_TILE = 4096;     // exact mode: objects per seed block (16 per thread)
-constexpr uint32_t SAMPLE_TILE = 1024;   // shared sample: objects per chunk
-constexpr uint32_t SAMPLE_CHUNKS = 128;  // shared sample: chunks at most, spread over the ids
-constexpr uint32_t SAMPLE_WGS = 32;      // workgroups that take the shared sample
-constexpr uint32_t SAMPLE_MAX_W = SAMPLE_WIN / SAMPLE_WGS;  // winners each of them publishes at most
-constexpr int SAMPLE_VEC = SAMPLE_CHUNKS * SAMPLE_TILE / (SAMPLE_WGS * STREAM_BS * 4);  // float4 per thread
-constexpr int OWN_VEC = 4096 / (STREAM_BS * 4);  // own sample: float4 vectors per thread
-constexpr uint32_t OWN_OBJS = STREAM_BS * 4 * OWN_VEC;
-constexpr uint32_t OWN_SPOTS = OWN_OBJS / 16;   // own sample: 256 runs of 16 objects, one 64-byte line per column each
-constexpr uint64_t OWN_MAX_N = 1ull << 19;      // stores up to this size take their own sample
-constexpr uint32_t STREAM_GRID = 256;    // stream workgroups at most (one per CU), unless tuned
 constexpr int FINAL_BS = 512;            // separate final select
 constexpr int FINAL_KPT = 16;            // candidate keys per final-select thread (8192 in registers)
 constexpr int FLAT_BS = 1024;            // fallback final select over a large flat list
 
-// Runtime-width scores of VPT float4 vectors v, v + step, ...: G columns'
+// Runtime-width scores of VPT float4 vectors v, v + step, ... (at most last): G columns'
 // loads are issued before the first of them is used (a loop of one column
 // per step waited on memory once per term), terms in query order; real-data
 // scores divide after every term.
@@ -68,7 +58,7 @@ __device__ __forceinline__ f4 ld_col(const float *p) {
     else return *reinterpret_cast<const f4 *>(p);
 }
 template <int VPT, bool NT = true, int G = 8>
-__device__ __forceinline__ void score_wide(const QCols &q, uint64_t v, uint32_t step, f4 (&acc)[VPT]) {
+__device__ __forceinline__ void score_wide(const QCols &q, uint32_t v, uint32_t step, uint32_t last, f4 (&acc)[VPT]) {
 #pragma unroll
     for (int u = 0; u < VPT; u++) acc[u] = f4{0.0f, 0.0f, 0.0f, 0.0f};
     for (uint32_t j0 = 0; j0 < q.m; j0 += G) {
@@ -77,7 +67,7 @@ __device__ __forceinline__ void score_wide(const QCols &q, uint64_t v, uint32_t 
         for (int t = 0; t < G; t++)
             if (j0 + t < q.m) {
 #pragma unroll
-                for (int u = 0; u < VPT; u++) x[t][u] = ld_col<NT>(q.col[j0 + t] + (v + u * step) * 4);
+                for (int u = 0; u < VPT; u++) x[t][u] = ld_col<NT>(q.col[j0 + t] + (uint64_t)tile_vec(v + u * step, last) * 4);
             }
 #pragma unroll
         for (int t = 0; t < G; t++)
@@ -109,7 +99,7 @@ __device__ __forceinline__ f4 score_vec(const QCols &q, uint64_t v) {
         }
     } else {
         f4 s1[1];
-        score_wide<1, NT, 16>(q, v, 0, s1);
+        score_wide<1, NT, 16>(q, (uint32_t)v, 0, 0xFFFFFFFFu, s1);
         acc = s1[0];
     }
     return acc;
@@ -383,9 +373,6 @@ __device__ __forceinline__ uint64_t own_sample_tau(const QCols &q, uint64_t n, u
 // ---------------------------------------------------------------------------
 // 2. stream pass
 // ---------------------------------------------------------------------------
-// Where a stream workgroup takes tau from.
-enum { TAU_ALL = 0, TAU_STATE = 1, TAU_SHARED = 2, TAU_OWN = 3 };
-
 // One stream pass.
 struct StreamArgs {
     uint64_t n, obj_begin, ntiles;
@@ -405,8 +392,8 @@ struct StreamArgs {
 // Each workgroup streams whole tiles of TILE = 4096*VPT objects: for every
 // queried column it reads one contiguous TILE*4-byte segment (VPT float4 per
 // lane).  Block-contiguous segments keep HBM near 88% of peak where a
-// thread-level grid stride over the columns stays near 72%.  The column
-// store is padded by one tile, so tile loads need no bounds check.
+// thread-level grid stride over the columns stays near 72%.  A tile may end
+// past the store: its lanes there read the last vector (tile_vec).
 //
 // One workgroup of 16 waves per CU holds 8 or more loads of 16 bytes per lane
 // in flight, which is all HBM needs (512 to 3072 workgroups of 256 threads
@@ -454,15 +441,17 @@ __global__ __launch_bounds__(STREAM_BS, 4) void fte_stream_kernel(QCols q, Strea
     constexpr int MX = M > 0 ? M : 1;
     f4 x[MX][VPT];
     uint64_t t = blockIdx.x;
-    auto load = [&](uint64_t v0) {
+    const uint32_t last = (uint32_t)((a.n - 1) / 4);
+    auto load = [&](uint32_t v0) {
         if constexpr (M > 0) {
 #pragma unroll
             for (int j = 0; j < M; j++)
 #pragma unroll
-                for (int u = 0; u < VPT; u++) x[j][u] = ld_stream(q.col[j] + (v0 + u * STREAM_BS) * 4);
+                for (int u = 0; u < VPT; u++)
+                    x[j][u] = ld_stream(q.col[j] + (uint64_t)tile_vec(v0 + u * STREAM_BS, last) * 4);
         }
     };
-    load((a.obj_begin + t * TILE) / 4 + threadIdx.x);  // the grid never exceeds the tiles
+    load((uint32_t)((a.obj_begin + t * TILE) / 4) + threadIdx.x);  // the grid never exceeds the tiles
     uint64_t tau = 0;
     if (a.tau == TAU_OWN) {
         tau = own_sample_tau<M>(q, a.n, a.ks, sh.own);
@@ -485,7 +474,7 @@ __global__ __launch_bounds__(STREAM_BS, 4) void fte_stream_kernel(QCols q, Strea
         uint32_t nx = 0;
         if (draw && threadIdx.x == 0)
             nx = __hip_atomic_fetch_add(&a.st->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint64_t v0 = (a.obj_begin + t * TILE) / 4 + threadIdx.x;
+        const uint32_t v0 = (uint32_t)((a.obj_begin + t * TILE) / 4) + threadIdx.x;
         f4 s[VPT];
         if constexpr (M > 0) {
             if (!first) load(v0);
@@ -500,7 +489,7 @@ __global__ __launch_bounds__(STREAM_BS, 4) void fte_stream_kernel(QCols q, Strea
                 s[u] = acc;
             }
         } else {
-            score_wide<VPT>(q, v0, STREAM_BS, s);
+            score_wide<VPT>(q, v0, STREAM_BS, last, s);
         }
         // filter: key >= tau (score key first; the id only matters on ties)
         uint32_t npass = 0;
@@ -509,7 +498,7 @@ __global__ __launch_bounds__(STREAM_BS, 4) void fte_stream_kernel(QCols q, Strea
         for (int u = 0; u < VPT; u++) {
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const uint64_t id = (v0 + u * STREAM_BS) * 4 + e;
+                const uint64_t id = (uint64_t)(v0 + u * STREAM_BS) * 4 + e;
                 const uint32_t ok = okey(s[u][e]);
                 const uint64_t key = rkey_from_okey(ok, (uint32_t)id);
                 const bool p = ok >= tau_hi && key >= tau && id < a.n;
@@ -682,106 +671,6 @@ __global__ __launch_bounds__(FLAT_BS) void fte_final_flat_kernel(FteState *__res
 // host side
 // ---------------------------------------------------------------------------
 
-static uint32_t exact_prefix_blocks(uint64_t n, uint32_t k) {
-    const uint64_t need = (n + SEED_TILE - 1) / SEED_TILE;
-    uint32_t g = 32768u / (k ? k : 1);
-    if (g > 256) g = 256;
-    if (g < 8) g = 8;
-    return (uint32_t)(need < g ? need : g);
-}
-
-static uint32_t stream_grid(uint32_t grid_cap, uint64_t ntiles) {
-    const uint64_t cap = grid_cap ? (uint64_t)grid_cap : STREAM_GRID;
-    const uint64_t g = ntiles < cap ? ntiles : cap;
-    return (uint32_t)(g < 1 ? 1 : g);
-}
-
-// float4 vectors per lane per column of one stream tile: enough loads in
-// flight per lane (about 8-16) without exhausting registers.
-static int stream_vpt(uint32_t m) {
-    if (m <= 1) return 8;
-    if (m <= 2) return 4;
-    if (m <= 4) return 2;
-    return 1;
-}
-
-// Samples above the ks-th largest of a random sample of s of the n objects
-// leave ks * n / s candidates on average, spread like a Gamma(ks) variable.
-// The smallest ks that leaves fewer than k with a chance of about 1e-4, from
-// q = k * s / n (the expected number of the top k in the sample): ks - 3.7
-// sqrt(ks) + 3.6 >= q, e.g. 17 k candidates at ks = 4, 5 k at 8, 2 k at 32.
-static uint32_t sample_rank(double q) {
-    uint32_t ks = 4;
-    while (ks < 4096 && ks - 3.7 * std::sqrt((double)ks) + 3.6 < q) ks++;
-    return ks;
-}
-
-// The same for a query nothing re-runs: fewer than k means that ks of the
-// top k fell into the sample, for about Poisson(q) of them less often than
-// exp(-q) (e q / ks)^ks (Chernoff, ten times the truth): here 1e-8, and 1e-5
-// below q = 1, where every rank adds candidates the most (32 queries of 16M x
-// 5, k = 32, q = 0.25: rank 4, 1e-4, 1797 us; rank 6 1820; rank 8 1872).
-static uint32_t queued_rank(double q) {
-    const double rare = q < 1.0 ? 11.5 : 18.4;
-    uint32_t ks = 4;
-    while (ks < 4096 && (ks <= q || ks * (std::log(ks / q) - 1.0) + q < rare)) ks++;
-    return ks;
-}
-
-// How a query gets its threshold.
-struct SeedPlan {
-    int tau;               // TAU_*
-    uint32_t blocks, ks;   // chunks of the sample or blocks of the exact seed; rank of tau (exact: winners per block)
-    uint32_t W;            // shared sample: winners per producer
-    uint64_t stride;       // objects between the chunks' first objects
-    uint64_t n_eff;        // exact: objects of the prefix
-    uint32_t total_valid;  // exact: keys the blocks deposit
-    double expect;         // candidates expected
-};
-
-// FTE_SAMPLE may guess on any store (the caller re-runs a bad guess): every
-// object of a store that fits the select, the own sample up to 2^19 objects,
-// the shared sample above.  FTE_QUEUED guesses only above 2^19 objects:
-// nothing re-runs it.
-static SeedPlan seed_plan(uint64_t n, uint32_t k, int mode) {
-    SeedPlan p{};
-    if (mode == FTE_SAMPLE && n <= FUSE_CAP_MAX) {
-        p.tau = TAU_ALL;
-        p.expect = (double)n;
-    } else if (mode == FTE_SAMPLE && n <= OWN_MAX_N) {
-        p.tau = TAU_OWN;
-        p.ks = sample_rank((double)k * OWN_OBJS / (double)n);
-        p.expect = (double)p.ks * n / OWN_OBJS;
-        if (p.expect >= n) p.tau = TAU_ALL;
-    } else if ((mode == FTE_SAMPLE || mode == FTE_QUEUED) && n > OWN_MAX_N) {
-        p.tau = TAU_SHARED;
-        // As many chunks as make tau the 8th largest of the sample (q =
-        // 1.13).  A long list on a small store would leave few of them, large
-        // jumps of the id range: below 32 chunks, all 128 and a deeper rank.
-        const uint64_t c8 = (uint64_t)(1.13 * (double)n / ((double)k * SAMPLE_TILE));
-        p.blocks = c8 >= SAMPLE_CHUNKS / 4 && c8 < SAMPLE_CHUNKS ? (uint32_t)c8 : SAMPLE_CHUNKS;
-        p.stride = ((n / p.blocks) / SAMPLE_TILE) * SAMPLE_TILE;
-        const double s = (double)p.blocks * SAMPLE_TILE;
-        p.ks = mode == FTE_QUEUED ? queued_rank(k * s / (double)n) : sample_rank(k * s / (double)n);
-        // each producer's share of the ks best: all of them up to 16 (the
-        // producers' chunks alternate over the id range, so more than 16 of
-        // a deep rank's best rarely meet in one; missing some lowers tau)
-        p.W = p.ks < SAMPLE_MAX_W ? p.ks : SAMPLE_MAX_W;
-        p.expect = (double)p.ks * n / s;
-    } else {
-        p.tau = TAU_STATE;
-        p.blocks = exact_prefix_blocks(n, k);
-        p.stride = SEED_TILE;
-        const uint64_t pre = (uint64_t)p.blocks * SEED_TILE;
-        p.n_eff = n < pre ? n : pre;
-        p.ks = k;
-        const uint64_t full = p.n_eff / SEED_TILE, rem = p.n_eff % SEED_TILE;
-        p.total_valid = (uint32_t)(full * (k < SEED_TILE ? k : SEED_TILE) + (rem < k ? rem : k));
-        p.expect = 2.0 * k;
-    }
-    return p;
-}
-
 // Everything one run of the FTE pipeline needs besides the query: the store
 // size, the stream, the scratch its kernels use and the launch shape.
 struct FteRun {
@@ -822,14 +711,13 @@ static CandSet fte_launch(const FteRun &r, uint32_t k, const QCols &q, const Fin
 
     // exact mode streams only the objects after the prefix
     const uint64_t first = exact ? sp.n_eff : 0;
-    // smaller tiles where the wide ones would leave workgroups without one
-    int vpt = r.vpt ? r.vpt : stream_vpt(q.m);
-    while (!r.vpt && vpt > 1 && n - first < (uint64_t)STREAM_GRID * STREAM_BS * 4 * vpt) vpt /= 2;
-    const uint64_t tile = (uint64_t)STREAM_BS * 4 * vpt;
+    const StreamPlan pl = stream_plan(n, first, q.m, r.big, r.vpt, r.grid_cap, r.cand_cap);
+    const uint32_t g = pl.grid;
     StreamArgs a{};
     a.n = n;
     a.obj_begin = first;
-    a.ntiles = n > first ? (n - first + tile - 1) / tile : 0;
+    a.ntiles = pl.ntiles;
+    a.nstatic = pl.nstatic;
     a.st = r.st;
     a.tau = sp.tau;
     a.ks = sp.ks;
@@ -846,18 +734,6 @@ static CandSet fte_launch(const FteRun &r, uint32_t k, const QCols &q, const Fin
     uint32_t cap = FUSE_CAP_MIN;
     while (cap < FUSE_CAP_MAX && (cap < 2 * a.kp2 || cap < 2 * sp.expect)) cap += FUSE_CAP_MIN;
     a.cap = cap;
-    const uint32_t g = a.ntiles ? stream_grid(r.grid_cap, a.ntiles) : 0;
-    // The last sixth of the tiles by ticket, at least two a workgroup, four
-    // where a tile lasts longer (above 8 columns): with a twelfth and two, a
-    // workgroup that the query before delays at its start (its last one
-    // selects) ended late.  Queued queries, 2^25 objects: 12 columns 251 ->
-    // 242 us, 8 columns 171 -> 164 (alone 202 -> 194); 2^24 x 12: 130 with
-    // two, 125 with four, 2^24 x 5: 58.3 and 59.7.  Up to four tiles a
-    // workgroup are all dealt (2^22 x 8: 37 -> 34 us), and so are those of a
-    // run whose slots hold a block's every object.
-    a.nstatic = a.ntiles;
-    if (!r.big && a.ntiles > 4ull * g)
-        a.nstatic = (a.ntiles - std::max<uint64_t>(a.ntiles / 6, (q.m > 8 ? 4ull : 2ull) * g) + g - 1) / g * g;
     a.wgs = g < SAMPLE_WGS ? g : SAMPLE_WGS;
     CandSet &cs = a.cs;
     cs.keys = r.cand;
@@ -866,8 +742,7 @@ static CandSet fte_launch(const FteRun &r, uint32_t k, const QCols &q, const Fin
     cs.pre = pre;
     cs.spill = r.spill;
     cs.spill_cap = r.spill_cap;
-    if (r.big) cs.slot = g ? (uint32_t)(((a.ntiles + g - 1) / g) * tile) : 0;  // a block's every object fits
-    else cs.slot = g ? (uint32_t)(r.cand_cap / g) : 0;
+    cs.slot = pl.slot;
     if (g) {
         const size_t lds = sizeof(uint64_t) * ((size_t)cap + std::max((g + 3) / 2, cap));
         hipEvent_t ev0 = nullptr;
@@ -878,7 +753,7 @@ static CandSet fte_launch(const FteRun &r, uint32_t k, const QCols &q, const Fin
 #define TK_STREAM2(MM) TK_STREAM(MM, 2)
 #define TK_STREAM4(MM) TK_STREAM(MM, 4)
 #define TK_STREAM8(MM) TK_STREAM(MM, 8)
-        switch (vpt) {
+        switch (pl.vpt) {
             case 1: TK_SWITCH_M(msw, TK_STREAM1); break;
             case 2: TK_SWITCH_M(msw, TK_STREAM2); break;
             case 4: TK_SWITCH_M(msw, TK_STREAM4); break;

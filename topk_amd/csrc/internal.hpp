@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../../include/topk.h"
+#include "fte_plan.hpp"
 
 namespace topk {
 
@@ -29,7 +30,6 @@ struct QCols {
 // Device-side state of one FTE / PTA query pipeline.  Words that many
 // workgroups hit at once sit on cache lines of their own.
 constexpr uint32_t ARRIVE_GROUPS = 16, ARRIVE_STRIDE = 32;
-constexpr uint32_t SAMPLE_WIN = 512;
 struct FteState {
     unsigned long long tau;   // threshold key published by the exact seed pass
     unsigned int pre_count;   // exact mode: prefix keys the seed pass stored in pre[]
@@ -62,14 +62,6 @@ struct CandSet {
 };
 
 enum : unsigned int { STATUS_OVERFLOW = 1u, STATUS_RETRY = 2u };
-
-// FTE pipeline modes: sample-seeded (the caller re-runs a bad guess),
-// exact-prefix-seeded with the regular candidate buffer, exact with an
-// n-entry buffer, and queued: sample-seeded above 2^19 objects, exact below
-// (nothing re-runs it).
-enum { FTE_SAMPLE = 0, FTE_EXACT = 1, FTE_EXACT_BIG = 2, FTE_QUEUED = 3 };
-
-constexpr uint32_t MAX_STREAM_GRID = 4096;
 
 // Object ids.  Ranking keys carry a 32-bit id (0xFFFFFFFF is reserved), so a
 // store of 2^32 - 1 objects or more runs the FTE path per id shard of
@@ -294,7 +286,7 @@ struct topk_ctx {
     uint64_t n = 0;
     uint32_t d = 0;
     uint64_t ld = 0;            // padded column stride (multiple of 8192 objects)
-    float *cols = nullptr;      // d * ld + 8192 floats, zero padded (a stream tile never needs a bounds check)
+    float *cols = nullptr;      // d * ld + 8192 floats, zero padded
     // FTE pipeline lanes: queries alternate between them so one query's seed
     // and final passes overlap its neighbours' stream passes
     topk::Lane lane[topk::NUM_LANES > 2 ? topk::NUM_LANES : 2];

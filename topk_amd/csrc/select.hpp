@@ -7,9 +7,7 @@
 
 namespace topk {
 
-constexpr int STREAM_BS = 1024;
 constexpr int STREAM_NW = STREAM_BS / 64;
-constexpr uint32_t FUSE_CAP_MIN = 1024, FUSE_CAP_MAX = 4096;  // candidates the last stream workgroup selects in LDS
 
 __device__ __forceinline__ void store_agent(uint64_t *p, uint64_t v) {
     __hip_atomic_store(reinterpret_cast<unsigned long long *>(p), (unsigned long long)v, __ATOMIC_RELAXED,
