@@ -363,6 +363,9 @@ void *topk_stream(topk_ctx *ctx);
  *   "stream_grid"     blocks of the FTE stream pass (0 = default)
  *   "stream_vpt"      float4 vectors per lane per column of a stream tile:
  *                     1, 2, 4 or 8 (0 = chosen from the query width)
+ *   "sample_polls"    tries (about 1.5 us each) of an FTE stream workgroup to
+ *                     get the shared threshold sample before it scores the
+ *                     missing part of it itself (0 = default)
  *   "fte_force_exact" 1 = seed FTE queries with the exact prefix pass
  *   "lanes"           1 or 2: pipelines that consecutive topk_fte_async
  *                     calls alternate between (2 overlaps one query's seed

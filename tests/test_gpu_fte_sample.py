@@ -1,0 +1,70 @@
+"""The shared threshold sample when its pieces are late (forced from the host:
+one try, then every workgroup scores what is missing itself), bit for bit
+against the CPU oracle: synchronous queries, queries queued on both lanes,
+and two engines queueing at once."""
+import threading
+
+import numpy as np
+import pytest
+
+import oracle
+import topk_amd
+
+pytestmark = pytest.mark.gpu
+
+# (n, d, m, k): fewer workgroups than pieces' takers, ragged pieces, deep ranks, runtime-width scores
+CASES = [((1 << 19) + 1, 3, 2, 16), (1_300_003, 8, 8, 64), (2_100_001, 20, 20, 1000), (4_194_301, 5, 1, 1)]
+
+
+def _store(n, d):
+    return topk_amd.generate(n, d, topk_amd.INDEPENDENT, 3)
+
+
+@pytest.mark.parametrize("polls", [1, 2, 0])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c)))
+def test_late_sample(gpu, case, polls):
+    n, d, m, k = case
+    x = _store(n, d)
+    rng = np.random.default_rng(n)
+    w, attr = rng.uniform(-0.2, 1.0, d).astype(np.float32), rng.permutation(d)[:m]
+    rid, rsc, rthr = oracle.fte_topk(x, n, k, w, attr)
+    with topk_amd.Engine(x) as eng:
+        eng.set_tuning("sample_polls", polls)
+        for grid in (0, 5):
+            eng.set_tuning("stream_grid", grid)
+            for _ in range(2):
+                ids, sc, thr = eng.fte(k, w, attr)
+                assert np.array_equal(ids, rid) and np.array_equal(sc.view(np.uint32), rsc.view(np.uint32))
+                assert thr == rthr
+
+
+def _queue(eng, queries, k):
+    import torch
+    ids = [torch.empty(k, dtype=torch.int64, device="cuda") for _ in queries]
+    sc = [torch.empty(k, dtype=torch.float32, device="cuda") for _ in queries]
+    for i, (w, attr) in enumerate(queries):
+        eng.fte_async(k, w, attr, ids[i].data_ptr(), sc[i].data_ptr())
+    eng.sync()
+    return [t.cpu().numpy().view(np.uint64) for t in ids], [t.cpu().numpy() for t in sc]
+
+
+@pytest.mark.parametrize("polls", [1, 0])
+def test_late_sample_with_queries_queued_on_both_lanes(gpu, polls):
+    n, d, k = 1_300_003, 8, 32
+    x = _store(n, d)
+    rng = np.random.default_rng(1)
+    queries = [(rng.uniform(0.1, 1.0, d).astype(np.float32), rng.permutation(d)[:3 + i % 6]) for i in range(16)]
+    want = [oracle.fte_topk(x, n, k, w, a) for w, a in queries]
+    with topk_amd.Engine(x) as a, topk_amd.Engine(x) as b:
+        got = {}
+        for e in (a, b):
+            e.set_tuning("sample_polls", polls)
+        threads = [threading.Thread(target=lambda e=e, i=i: got.setdefault(i, _queue(e, queries, k)))
+                   for i, e in enumerate((a, b))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    for i in range(2):
+        for j, (rid, rsc, _) in enumerate(want):
+            assert np.array_equal(got[i][0][j], rid) and np.array_equal(got[i][1][j], rsc), (i, j)

@@ -483,6 +483,9 @@ int topk_set_tuning(topk_ctx *ctx, const char *name, int64_t value) {
     if (key == "stream_grid") {
         if (value < 0 || value > (int64_t)MAX_STREAM_GRID) return TOPK_ERR_INVALID;
         ctx->tune.stream_grid = (uint32_t)value;
+    } else if (key == "sample_polls") {
+        if (value < 0 || value > 1 << 20) return TOPK_ERR_INVALID;
+        ctx->tune.sample_polls = (uint32_t)value;
     } else if (key == "stream_vpt") {
         if (value != 0 && value != 1 && value != 2 && value != 4 && value != 8) return TOPK_ERR_INVALID;
         ctx->tune.stream_vpt = (int)value;

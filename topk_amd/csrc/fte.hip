@@ -11,8 +11,9 @@
 //       - shared sample: the first 32 workgroups score up to 128 chunks of
 //         1024 objects spread over the id range and publish their best; tau
 //         is the ks-th largest of the whole sample.  The other workgroups
-//         have their first tile in flight meanwhile.  A guess like the own
-//         sample, checked at the end (>= k candidates).
+//         have their first tile in flight meanwhile; what is late they score
+//         themselves.  A guess like the own sample, checked at the end (>= k
+//         candidates).
 //       - exact (fte_seed_kernel): contiguous chunks [0, P); the prefix's
 //         k-th key is a proven lower bound of the global k-th key, and the
 //         prefix's top k are written to the candidate list.
@@ -237,24 +238,33 @@ __device__ __forceinline__ uint64_t wave_top(uint32_t (&hi)[NPL], const uint32_t
     return mine;
 }
 
-// Shared sample, producer side: workgroup p < wgs scores chunks p, p +
-// SAMPLE_WGS, ... of the sample (1024 objects each, at multiples of
-// chunk_stride) and publishes its W largest keys at st->win[p * W ...].
-// Producers are the workgroups with the lowest indexes, which are
-// dispatched first, and wait for nobody before they have published.
+// Shared sample: its chunks (1024 objects each, at multiples of chunk_stride)
+// are dealt into wgs pieces, chunk c to piece c % SAMPLE_WGS, and the W
+// largest keys of piece p are published at st->win[p * W ...].  The workgroup
+// with index p takes piece p.
+//
+// No workgroup waits on another's progress: one that has polled for a while
+// in vain takes a missing piece itself and polls again.  A piece's winners
+// depend on the query alone, so it does not matter who publishes them or how
+// often, every workgroup gets the same tau, and after at most wgs pieces of
+// its own work all of them are there.  (The first workgroups of one launch
+// start first, but two launches in flight may hold each other's compute
+// units, each XCD starting another of them first.)
 struct SampleScratch {
     uint64_t keys[STREAM_NW * SAMPLE_MAX_W];
 };
+constexpr uint32_t NO_PIECE = 0xFFFFFFFFu;
 template <int M>
 __device__ __forceinline__ void sample_publish(const QCols &q, uint64_t n, uint32_t chunks, uint64_t chunk_stride,
-                                               uint32_t W, FteState *__restrict__ st, SampleScratch &sc) {
+                                               uint32_t W, uint32_t piece, FteState *__restrict__ st,
+                                               SampleScratch &sc) {
     const uint32_t tid = threadIdx.x, wave = tid / 64, lane = lane_id();
     constexpr uint32_t PER = STREAM_BS * 4 / SAMPLE_TILE;  // chunks per step of the workgroup
     {
         uint32_t hi[4 * SAMPLE_VEC], lo[4 * SAMPLE_VEC];
 #pragma unroll
         for (int u = 0; u < SAMPLE_VEC; u++) {
-            const uint32_t c = blockIdx.x + (u * PER + tid / (SAMPLE_TILE / 4)) * SAMPLE_WGS;
+            const uint32_t c = piece + (u * PER + tid / (SAMPLE_TILE / 4)) * SAMPLE_WGS;
             const uint64_t v = (c < chunks ? c * chunk_stride : 0ull) / 4 + tid % (SAMPLE_TILE / 4);
             const f4 s = score_vec<(M > 8 ? 0 : M)>(q, v);  // 16 columns at once would spill
 #pragma unroll
@@ -279,20 +289,21 @@ __device__ __forceinline__ void sample_publish(const QCols &q, uint64_t n, uint3
             lo[j] = (uint32_t)v;
         }
         const uint64_t mine = wave_top<NB>(hi, lo, W);
-        if (lane < W) store_agent(reinterpret_cast<uint64_t *>(&st->win[blockIdx.x * W + lane]), mine ? mine : 1ull);
+        if (lane < W) store_agent(reinterpret_cast<uint64_t *>(&st->win[piece * W + lane]), mine ? mine : 1ull);
     }
     __syncthreads();
 }
 
-// Consumer side, one wave: polls the winners until every one is there (a
-// winner is its own flag: a store and a load apart, where a counter would
-// add two more trips to memory) and returns the ks-th largest.  The wait is
-// bounded: should it run out, a threshold of 0 admits every object and the
-// candidate count settles what happens.
-constexpr uint32_t SAMPLE_SPINS = 1u << 23;  // more than 10 s: past any stall of the producers
-__device__ __forceinline__ uint64_t sample_tau(FteState *__restrict__ st, uint32_t nwin, uint32_t ks) {
+// Consumer side, one wave: polls the winners (a winner is its own flag: a
+// store and a load apart, where a counter would add two more trips to
+// memory).  With all of them there, tau is the ks-th largest and the result
+// NO_PIECE; after `polls` tries it is a missing piece, the first one from this
+// workgroup's own number on, so that many workgroups take different ones.
+__device__ __forceinline__ uint32_t sample_tau(FteState *__restrict__ st, uint32_t wgs, uint32_t W, uint32_t ks,
+                                               uint32_t polls, uint64_t &tau) {
     constexpr int NPL = SAMPLE_WIN / 64;
-    for (uint32_t s = 0; s < SAMPLE_SPINS; s++) {
+    const uint32_t nwin = wgs * W;
+    for (uint32_t s = 1;; s++) {
         uint32_t hi[NPL], lo[NPL];
         bool all = true;
 #pragma unroll
@@ -306,10 +317,24 @@ __device__ __forceinline__ uint64_t sample_tau(FteState *__restrict__ st, uint32
             hi[j] = (uint32_t)(v >> 32);
             lo[j] = (uint32_t)v;
         }
-        if (!__ballot(!all)) return wave_kth<NPL>(hi, lo, ks);
+        if (!__ballot(!all)) {
+            tau = wave_kth<NPL>(hi, lo, ks);
+            return NO_PIECE;
+        }
+        if (s >= polls) {
+            const uint32_t from = blockIdx.x % wgs;
+            uint32_t near = 0;  // wgs less the steps from there to the nearest missing piece
+#pragma unroll
+            for (int j = 0; j < NPL; j++) {
+                const uint32_t i = j * 64 + lane_id(), p = i / W;
+                const uint32_t left = p >= from ? wgs - (p - from) : from - p;
+                near = i < nwin && (hi[j] | lo[j]) == 0 && left > near ? left : near;
+            }
+            const uint32_t p = from + wgs - wave_max_u32(near);
+            return p < wgs ? p : p - wgs;
+        }
         __builtin_amdgcn_s_sleep(8);
     }
-    return 0;
 }
 
 // Own sample: tau of a stream workgroup from the same OWN_OBJS objects in
@@ -381,8 +406,9 @@ struct StreamArgs {
     CandSet cs;
     int tau;               // TAU_*: every object a candidate, st->tau, the shared sample, the own sample
     uint32_t ks;           // rank of tau in the sample
-    uint32_t chunks, wgs, W;  // shared sample: chunks, producers, winners per producer
+    uint32_t chunks, wgs, W;  // shared sample: chunks, pieces, winners per piece
     uint64_t chunk_stride; // objects between the chunks' first objects
+    uint32_t polls;        // tries before a workgroup takes a missing piece of the sample
     int select;            // the last workgroup selects and emits (else a later launch does)
     uint32_t cap, kp2, k, kreq;
     FinalOut fo;
@@ -425,7 +451,7 @@ template <int M, int VPT>
 __global__ __launch_bounds__(STREAM_BS, 4) void fte_stream_kernel(QCols q, StreamArgs a) {
     constexpr uint32_t TILE = STREAM_BS * 4 * VPT;
     extern __shared__ uint64_t dyn[];  // cap keys | block offsets, later cap keys
-    __shared__ uint32_t lcount, is_last, s_next[2];
+    __shared__ uint32_t lcount, is_last, s_next[2], s_piece;
     __shared__ uint64_t s_tau;
     __shared__ union {
         OwnScratch own;
@@ -435,8 +461,6 @@ __global__ __launch_bounds__(STREAM_BS, 4) void fte_stream_kernel(QCols q, Strea
     if (a.gate && *a.gate == 0) return;
     const uint32_t lane = lane_id();
     if (threadIdx.x == 0) lcount = 0;
-    if (a.tau == TAU_SHARED && blockIdx.x < a.wgs)
-        sample_publish<M>(q, a.n, a.chunks, a.chunk_stride, a.W, a.st, sh.sam);
     // the first tile's loads are in flight while tau is found
     constexpr int MX = M > 0 ? M : 1;
     f4 x[MX][VPT];
@@ -451,19 +475,41 @@ __global__ __launch_bounds__(STREAM_BS, 4) void fte_stream_kernel(QCols q, Strea
                     x[j][u] = ld_stream(q.col[j] + (uint64_t)tile_vec(v0 + u * STREAM_BS, last) * 4);
         }
     };
-    load((uint32_t)((a.obj_begin + t * TILE) / 4) + threadIdx.x);  // the grid never exceeds the tiles
+    const uint32_t first_v = (uint32_t)((a.obj_begin + t * TILE) / 4) + threadIdx.x;  // the grid never exceeds the tiles
     uint64_t tau = 0;
-    if (a.tau == TAU_OWN) {
-        tau = own_sample_tau<M>(q, a.n, a.ks, sh.own);
-    } else if (a.tau != TAU_ALL) {
-        if (threadIdx.x < 64) {
-            const uint64_t v = a.tau == TAU_SHARED ? sample_tau(a.st, a.wgs * a.W, a.ks) : a.st->tau;
-            if (lane == 0) s_tau = v;
+    if (a.tau == TAU_SHARED) {
+        auto publish = [&](uint32_t piece) {
+            sample_publish<M>(q, a.n, a.chunks, a.chunk_stride, a.W, piece, a.st, sh.sam);
+        };
+        auto missing = [&]() -> uint32_t {
+            if (threadIdx.x < 64) {
+                uint64_t v = 0;
+                const uint32_t p = sample_tau(a.st, a.wgs, a.W, a.ks, a.polls, v);
+                if (lane == 0) {
+                    s_tau = v;
+                    s_piece = p;
+                }
+            }
+            __syncthreads();
+            return __builtin_amdgcn_readfirstlane(s_piece);
+        };
+        if (blockIdx.x < a.wgs) publish(blockIdx.x);
+        load(first_v);
+        for (uint32_t piece = missing(); piece != NO_PIECE; piece = missing()) {
+            publish(piece);
+            uint32_t v0 = first_v;
+            asm volatile("" : "+v"(v0));  // the addresses are made anew, not kept over the sample
+            load(v0);
         }
-        __syncthreads();
         tau = s_tau;
     } else {
-        __syncthreads();
+        load(first_v);
+        if (a.tau == TAU_OWN) {
+            tau = own_sample_tau<M>(q, a.n, a.ks, sh.own);
+        } else {
+            if (a.tau == TAU_STATE) tau = a.st->tau;
+            __syncthreads();
+        }
     }
     const uint32_t tau_hi = (uint32_t)(tau >> 32);
     const CandSet &cs = a.cs;
@@ -687,6 +733,7 @@ struct FteRun {
     uint32_t spill_cap;
     int vpt;              // 0: chosen from the query width
     uint32_t grid_cap;    // 0: default
+    uint32_t polls;       // of the shared sample (0: default)
     const uint32_t *gate; // non-null: every kernel exits at once unless *gate != 0
     topk_ctx *timed;      // non-null: bracket the stream pass for topk_timing_*
 };
@@ -735,6 +782,7 @@ static CandSet fte_launch(const FteRun &r, uint32_t k, const QCols &q, const Fin
     while (cap < FUSE_CAP_MAX && (cap < 2 * a.kp2 || cap < 2 * sp.expect)) cap += FUSE_CAP_MIN;
     a.cap = cap;
     a.wgs = g < SAMPLE_WGS ? g : SAMPLE_WGS;
+    a.polls = r.polls ? r.polls : SAMPLE_POLLS;
     CandSet &cs = a.cs;
     cs.keys = r.cand;
     cs.counts = r.counts;
@@ -797,6 +845,7 @@ int fte_enqueue(topk_ctx *ctx, Lane &L, uint32_t k, const QCols &q, const FinalO
     r.spill_cap = ctx->spill_cap;
     r.vpt = ctx->tune.stream_vpt;
     r.grid_cap = ctx->tune.stream_grid;
+    r.polls = ctx->tune.sample_polls;
     r.timed = ctx;
     const uint32_t kreq = (uint32_t)(n < k ? n : k);
     const CandSet cs = fte_launch(r, k, q, fo, mode);

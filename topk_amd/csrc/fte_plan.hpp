@@ -28,6 +28,7 @@ constexpr uint32_t SAMPLE_CHUNKS = 128;  // shared sample: chunks at most, sprea
 constexpr uint32_t SAMPLE_WGS = 32;      // workgroups that take the shared sample
 constexpr uint32_t SAMPLE_WIN = 512;     // shared sample: winners of all workgroups at most
 constexpr uint32_t SAMPLE_MAX_W = SAMPLE_WIN / SAMPLE_WGS;  // winners each of them publishes at most
+constexpr uint32_t SAMPLE_POLLS = 32;    // tries before a workgroup takes a missing piece of the sample
 constexpr int SAMPLE_VEC = SAMPLE_CHUNKS * SAMPLE_TILE / (SAMPLE_WGS * STREAM_BS * 4);  // float4 per thread
 constexpr int OWN_VEC = 4096 / (STREAM_BS * 4);  // own sample: float4 vectors per thread
 constexpr uint32_t OWN_OBJS = STREAM_BS * 4 * OWN_VEC;
@@ -104,7 +105,7 @@ enum { TAU_ALL = 0, TAU_STATE = 1, TAU_SHARED = 2, TAU_OWN = 3 };
 struct SeedPlan {
     int tau;               // TAU_*
     uint32_t blocks, ks;   // chunks of the sample or blocks of the exact seed; rank of tau (exact: winners per block)
-    uint32_t W;            // shared sample: winners per producer
+    uint32_t W;            // shared sample: winners per piece
     uint64_t stride;       // objects between the chunks' first objects
     uint64_t n_eff;        // exact: objects of the prefix
     uint32_t total_valid;  // exact: keys the blocks deposit
@@ -135,8 +136,8 @@ static inline SeedPlan seed_plan(uint64_t n, uint32_t k, int mode) {
         p.stride = ((n / p.blocks) / SAMPLE_TILE) * SAMPLE_TILE;
         const double s = (double)p.blocks * SAMPLE_TILE;
         p.ks = mode == FTE_QUEUED ? queued_rank(k * s / (double)n) : sample_rank(k * s / (double)n);
-        // each producer's share of the ks best: all of them up to 16 (the
-        // producers' chunks alternate over the id range, so more than 16 of
+        // each piece's share of the ks best: all of them up to 16 (the
+        // pieces' chunks alternate over the id range, so more than 16 of
         // a deep rank's best rarely meet in one; missing some lowers tau)
         p.W = p.ks < SAMPLE_MAX_W ? p.ks : SAMPLE_MAX_W;
         p.expect = (double)p.ks * n / s;

@@ -76,6 +76,7 @@ inline uint32_t id_shards(uint64_t n) { return n >= ID_LIMIT ? (uint32_t)((n + I
 // Launch-shape knobs (set by topk_set_tuning / the autotuner).
 struct Tuning {
     uint32_t stream_grid = 0;   // 0: default grid cap
+    uint32_t sample_polls = 0;  // 0: default tries for the shared sample
     int stream_vpt = 0;         // float4 vectors per lane per column in a stream tile (0: by width)
     int fte_force_exact = 0;    // 1: skip the sample seed (testing / comparison)
     int lanes = 2;              // pipeline lanes used by asynchronous queries
