@@ -37,6 +37,23 @@ def test_last_tile_past_the_store(gpu, case):
     assert np.array_equal(sc.view(np.uint32), rsc.view(np.uint32)) and thr == rthr
 
 
+@pytest.mark.parametrize("m,vpt", [(12, 1), (13, 1), (6, 2), (7, 2), (3, 4), (4, 4), (1, 8), (2, 8)])
+@pytest.mark.parametrize("divide", [0, 1])
+def test_unrolled_and_runtime_widths(gpu, m, vpt, divide):
+    # the two sides of the unrolling limit, at a ragged size with a second tile per workgroup
+    n, k = 1_100_003 * vpt, 33
+    x = topk_amd.generate(n, m, topk_amd.INDEPENDENT, 5)
+    rng = np.random.default_rng(m)
+    w, attr = rng.uniform(-0.3, 1.0, m).astype(np.float32), rng.permutation(m)
+    rid, rsc, rthr = oracle.fte_topk(x, n, k, w, attr, divide=bool(divide))
+    with topk_amd.Engine(x) as eng:
+        eng.set_tuning("stream_vpt", vpt)
+        eng.set_tuning("score_divide", divide)
+        ids, sc, thr = eng.fte(k, w, attr)
+    assert np.array_equal(ids, rid)
+    assert np.array_equal(sc.view(np.uint32), rsc.view(np.uint32)) and thr == rthr
+
+
 def test_every_object_a_candidate(gpu):
     # best objects last: the prefix admits the whole store, past the regular
     # buffer, so the run with an n-entry one answers

@@ -49,16 +49,16 @@ constexpr int FINAL_BS = 512;            // separate final select
 constexpr int FINAL_KPT = 16;            // candidate keys per final-select thread (8192 in registers)
 constexpr int FLAT_BS = 1024;            // fallback final select over a large flat list
 
-// Runtime-width scores of VPT float4 vectors v, v + step, ... (at most last): G columns'
-// loads are issued before the first of them is used (a loop of one column
-// per step waited on memory once per term), terms in query order; real-data
-// scores divide after every term.
+// Runtime-width scores of VPT float4 vectors v, v + step, ... (at most last): the
+// loads of G columns, eight a lane, are issued before the first of them is used
+// (a loop of one column per step waited on memory once per term), terms in
+// query order; real-data scores divide after every term.
 template <bool NT>
 __device__ __forceinline__ f4 ld_col(const float *p) {
     if constexpr (NT) return ld_stream(p);
     else return *reinterpret_cast<const f4 *>(p);
 }
-template <int VPT, bool NT = true, int G = 8>
+template <int VPT, bool NT = true, int G = VPT < 8 ? 8 / VPT : 1>
 __device__ __forceinline__ void score_wide(const QCols &q, uint32_t v, uint32_t step, uint32_t last, f4 (&acc)[VPT]) {
 #pragma unroll
     for (int u = 0; u < VPT; u++) acc[u] = f4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -796,7 +796,7 @@ static CandSet fte_launch(const FteRun &r, uint32_t k, const QCols &q, const Fin
         hipEvent_t ev0 = nullptr;
         if (r.timed) timing_begin(r.timed, s, ev0);
 #define TK_STREAM(MM, VPT) \
-    hipLaunchKernelGGL((fte_stream_kernel<MM, VPT>), dim3(g), dim3(STREAM_BS), lds, s, q, a)
+    hipLaunchKernelGGL((fte_stream_kernel<stream_unroll(MM, VPT), VPT>), dim3(g), dim3(STREAM_BS), lds, s, q, a)
 #define TK_STREAM1(MM) TK_STREAM(MM, 1)
 #define TK_STREAM2(MM) TK_STREAM(MM, 2)
 #define TK_STREAM4(MM) TK_STREAM(MM, 4)

@@ -74,6 +74,16 @@ static inline int stream_vpt(uint32_t m) {
     return 1;
 }
 
+// Columns the stream kernel is unrolled for, its first tile's loads all in
+// flight while tau is found; 0: the runtime width, eight loads a lane at a
+// time.  16 waves a workgroup leave a lane 128 registers, and past 12 loads
+// of 16 bytes they spill.  2^25 objects, k = 64, unrolled and runtime width,
+// alone / queued: 9 columns 220 / 186 and 216 / 183 us, 12: 271 / 243 and 271
+// / 244, 13: 308 / 270 and 295 / 267, 16: 380 / 342 and 355 / 327; 2^22: 9:
+// 61 / 39 and 64 / 42, 12: 69 / 47 and 71 / 50, 13: 78 / 54 and 74 / 53, 16:
+// 91 / 65 and 83 / 62.
+constexpr int stream_unroll(int m, int vpt) { return m * vpt <= 12 ? m : 0; }
+
 // Samples above the ks-th largest of a random sample of s of the n objects
 // leave ks * n / s candidates on average, spread like a Gamma(ks) variable.
 // The smallest ks that leaves fewer than k with a chance of about 1e-4, from
