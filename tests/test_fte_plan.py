@@ -69,6 +69,24 @@ int main() {
 }
 """
 
+RANKS = HEADER + r"""
+int main() {
+    // a query nothing re-runs: no threshold above the one that k-th, or 8 k candidates', rank of 128 x 1024
+    // sampled objects gives
+    for (uint64_t n : {(1ull << 19) + 1, 524289ull, 700001ull, 1ull << 20, (1ull << 20) + 1, 1500000ull, 1ull << 21, 3000001ull,
+                       1ull << 23, 16777213ull, 1ull << 26, 1ull << 31})
+        for (uint32_t k = 1; k <= 1024; k++) {
+            const SeedPlan p = seed_plan(n, k, FTE_QUEUED);
+            const uint64_t s = 128 * 1024, want = (8ull * k * s + n - 1) / n;
+            const uint32_t floor_ = (uint32_t)(want < 4 ? 4 : (want > k ? k : want));
+            CHECK(p.tau == TAU_SHARED && p.blocks == 128 && p.ks >= floor_ && p.ks <= SAMPLE_WGS * p.W && p.W <= SAMPLE_MAX_W,
+                  "n %llu k %u: rank %u of %u, %u expected", (unsigned long long)n, k, p.ks, p.blocks, floor_);
+            if (n <= 1ull << 20) CHECK(p.ks >= k, "n %llu k %u", (unsigned long long)n, k);
+        }
+    return fails ? 1 : 0;
+}
+"""
+
 
 def _run(program, tmp_path):
     if not shutil.which("g++"):
@@ -83,3 +101,7 @@ def _run(program, tmp_path):
 
 def test_reads_and_slots_stay_inside_their_buffers(tmp_path):
     _run(REACH, tmp_path)
+
+
+def test_queued_ranks_are_as_deep_as_a_proven_bound(tmp_path):
+    _run(RANKS, tmp_path)

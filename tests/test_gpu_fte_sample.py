@@ -48,6 +48,34 @@ def _queue(eng, queries, k):
     return [t.cpu().numpy().view(np.uint64) for t in ids], [t.cpu().numpy() for t in sc]
 
 
+def _ordered(n, kind):
+    """One column whose score order follows the ids."""
+    i = np.arange(n, dtype=np.float32) / np.float32(n)
+    if kind == "best-first":
+        return i[::-1].copy().reshape(1, n)
+    if kind == "best-last":
+        return i.reshape(1, n)
+    x = topk_amd.generate(n, 1, topk_amd.INDEPENDENT, 2) * np.float32(0.5)
+    at = (n // 128 // 1024) * 1024 * 40  # the first object of a sampled chunk
+    x[0, at:at + 2000] += np.linspace(1, 0.5, 2000, dtype=np.float32)
+    return x
+
+
+@pytest.mark.parametrize("kind", ["best-first", "best-last", "clustered"])
+@pytest.mark.parametrize("n,ks", [(524_289, (14, 18, 300)), (700_001, (14, 24, 1024)), (1 << 20, (14, 16, 36, 64, 1000)),
+                                  (1_048_577, (16, 1000)), (2_097_153, (256, 1000))])
+def test_queued_queries_on_stores_in_score_order(gpu, kind, n, ks):
+    # nothing re-runs a queued query: its threshold holds for ordered stores too
+    x = _ordered(n, kind)
+    w = np.ones(1, np.float32)
+    with topk_amd.Engine(x) as eng:
+        for k in ks:
+            ids, sc = _queue(eng, [(w, [0])] * 2, k)
+            rid, rsc, _ = oracle.fte_topk(x, n, k, w, [0])
+            for j in range(2):
+                assert np.array_equal(ids[j], rid) and np.array_equal(sc[j], rsc), k
+
+
 @pytest.mark.parametrize("polls", [1, 0])
 def test_late_sample_with_queries_queued_on_both_lanes(gpu, polls):
     n, d, k = 1_300_003, 8, 32

@@ -238,15 +238,29 @@ __device__ __forceinline__ uint64_t wave_top(uint32_t (&hi)[NPL], const uint32_t
     return mine;
 }
 
+// The same of the cnt <= 64 * NPL keys at p (LDS).
+template <int NPL>
+__device__ __forceinline__ uint64_t top_of_list(const uint64_t *p, uint32_t cnt, uint32_t W) {
+    uint32_t hi[NPL], lo[NPL];
+#pragma unroll
+    for (int j = 0; j < NPL; j++) {
+        const uint32_t i = j * 64 + lane_id();
+        const uint64_t v = i < cnt ? p[i] : 0ull;
+        hi[j] = (uint32_t)(v >> 32);
+        lo[j] = (uint32_t)v;
+    }
+    return wave_top<NPL>(hi, lo, W);
+}
+
 // Shared sample: its chunks (1024 objects each, at multiples of chunk_stride)
-// are dealt into wgs pieces, chunk c to piece c % SAMPLE_WGS, and the W
+// are dealt into SAMPLE_WGS pieces, chunk c to piece c % SAMPLE_WGS, and the W
 // largest keys of piece p are published at st->win[p * W ...].  The workgroup
-// with index p takes piece p.
+// with index p takes piece p; of fewer workgroups, any takes the pieces left.
 //
 // No workgroup waits on another's progress: one that has polled for a while
 // in vain takes a missing piece itself and polls again.  A piece's winners
 // depend on the query alone, so it does not matter who publishes them or how
-// often, every workgroup gets the same tau, and after at most wgs pieces of
+// often, every workgroup gets the same tau, and after at most 32 pieces of
 // its own work all of them are there.  (The first workgroups of one launch
 // start first, but two launches in flight may hold each other's compute
 // units, each XCD starting another of them first.)
@@ -279,30 +293,22 @@ __device__ __forceinline__ void sample_publish(const QCols &q, uint64_t n, uint3
     }
     __syncthreads();
     if (wave == 0) {
-        constexpr int NB = STREAM_NW * SAMPLE_MAX_W / 64;
-        uint32_t hi[NB], lo[NB];
-#pragma unroll
-        for (int j = 0; j < NB; j++) {
-            const uint32_t i = j * 64 + lane;
-            const uint64_t v = i < STREAM_NW * W ? sc.keys[i] : 0ull;
-            hi[j] = (uint32_t)(v >> 32);
-            lo[j] = (uint32_t)v;
-        }
-        const uint64_t mine = wave_top<NB>(hi, lo, W);
+        const uint64_t mine = W <= 16 ? top_of_list<STREAM_NW * 16 / 64>(sc.keys, STREAM_NW * W, W)
+                                      : top_of_list<STREAM_NW * SAMPLE_MAX_W / 64>(sc.keys, STREAM_NW * W, W);
         if (lane < W) store_agent(reinterpret_cast<uint64_t *>(&st->win[piece * W + lane]), mine ? mine : 1ull);
     }
     __syncthreads();
 }
 
-// Consumer side, one wave: polls the winners (a winner is its own flag: a
+// Consumer side, one wave, W <= 16: polls the winners (a winner is its own flag: a
 // store and a load apart, where a counter would add two more trips to
 // memory).  With all of them there, tau is the ks-th largest and the result
 // NO_PIECE; after `polls` tries it is a missing piece, the first one from this
 // workgroup's own number on, so that many workgroups take different ones.
-__device__ __forceinline__ uint32_t sample_tau(FteState *__restrict__ st, uint32_t wgs, uint32_t W, uint32_t ks,
-                                               uint32_t polls, uint64_t &tau) {
-    constexpr int NPL = SAMPLE_WIN / 64;
-    const uint32_t nwin = wgs * W;
+__device__ __forceinline__ uint32_t sample_tau(FteState *__restrict__ st, uint32_t W, uint32_t ks, uint32_t polls,
+                                               uint64_t &tau) {
+    constexpr int NPL = SAMPLE_WGS * 16 / 64;
+    const uint32_t nwin = SAMPLE_WGS * W;
     for (uint32_t s = 1;; s++) {
         uint32_t hi[NPL], lo[NPL];
         bool all = true;
@@ -322,17 +328,45 @@ __device__ __forceinline__ uint32_t sample_tau(FteState *__restrict__ st, uint32
             return NO_PIECE;
         }
         if (s >= polls) {
-            const uint32_t from = blockIdx.x % wgs;
-            uint32_t near = 0;  // wgs less the steps from there to the nearest missing piece
+            const uint32_t from = blockIdx.x % SAMPLE_WGS;
+            uint32_t near = 0;  // SAMPLE_WGS less the steps from there to the nearest missing piece
 #pragma unroll
             for (int j = 0; j < NPL; j++) {
                 const uint32_t i = j * 64 + lane_id(), p = i / W;
-                const uint32_t left = p >= from ? wgs - (p - from) : from - p;
+                const uint32_t left = p >= from ? SAMPLE_WGS - (p - from) : from - p;
                 near = i < nwin && (hi[j] | lo[j]) == 0 && left > near ? left : near;
             }
-            const uint32_t p = from + wgs - wave_max_u32(near);
-            return p < wgs ? p : p - wgs;
+            return (from + SAMPLE_WGS - wave_max_u32(near)) % SAMPLE_WGS;
         }
+        __builtin_amdgcn_s_sleep(8);
+    }
+}
+
+// The same by the whole workgroup, a winner a thread, for any W: more than
+// eight winners a lane and the tile in flight don't fit the registers.
+__device__ __forceinline__ uint32_t sample_tau_deep(FteState *__restrict__ st, uint32_t W, uint32_t ks, uint32_t polls,
+                                                    uint64_t &tau, uint32_t &s_near, SelectScratchT<256> &ss) {
+    const uint32_t i = threadIdx.x;
+    const bool mine = i < SAMPLE_WGS * W;
+    for (uint32_t s = 1;; s++) {
+        uint64_t v = 0;
+        if (mine) v = __hip_atomic_load(&st->win[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (i == 0) s_near = 0;
+        __syncthreads();
+        if (mine && v == 0) {
+            const uint32_t p = i / W, from = blockIdx.x % SAMPLE_WGS;
+            atomicMax(&s_near, p >= from ? SAMPLE_WGS - (p - from) : from - p);
+        }
+        __syncthreads();
+        const uint32_t near = s_near;
+        __syncthreads();
+        if (near == 0) {
+            RegKeys<1> rk;
+            rk.k[0] = v;
+            tau = block_kth_largest<STREAM_BS, RegKeys<1>, 8>(rk, SAMPLE_WGS * W, ks, ss);
+            return NO_PIECE;
+        }
+        if (s >= polls) return (blockIdx.x % SAMPLE_WGS + SAMPLE_WGS - near) % SAMPLE_WGS;
         __builtin_amdgcn_s_sleep(8);
     }
 }
@@ -406,7 +440,7 @@ struct StreamArgs {
     CandSet cs;
     int tau;               // TAU_*: every object a candidate, st->tau, the shared sample, the own sample
     uint32_t ks;           // rank of tau in the sample
-    uint32_t chunks, wgs, W;  // shared sample: chunks, pieces, winners per piece
+    uint32_t chunks, W;    // shared sample: chunks, winners per piece
     uint64_t chunk_stride; // objects between the chunks' first objects
     uint32_t polls;        // tries before a workgroup takes a missing piece of the sample
     int select;            // the last workgroup selects and emits (else a later launch does)
@@ -478,30 +512,36 @@ __global__ __launch_bounds__(STREAM_BS, 4) void fte_stream_kernel(QCols q, Strea
     const uint32_t first_v = (uint32_t)((a.obj_begin + t * TILE) / 4) + threadIdx.x;  // the grid never exceeds the tiles
     uint64_t tau = 0;
     if (a.tau == TAU_SHARED) {
-        auto publish = [&](uint32_t piece) {
+        auto publish = [&](uint32_t piece) __attribute__((always_inline)) {
             sample_publish<M>(q, a.n, a.chunks, a.chunk_stride, a.W, piece, a.st, sh.sam);
         };
-        auto missing = [&]() -> uint32_t {
+        if (blockIdx.x < SAMPLE_WGS) publish(blockIdx.x);
+        uint32_t piece = NO_PIECE;
+        const bool deep = a.W > 16;
+        if (!deep) {
+            load(first_v);
             if (threadIdx.x < 64) {
                 uint64_t v = 0;
-                const uint32_t p = sample_tau(a.st, a.wgs, a.W, a.ks, a.polls, v);
+                const uint32_t p = sample_tau(a.st, a.W, a.ks, a.polls, v);
                 if (lane == 0) {
                     s_tau = v;
                     s_piece = p;
                 }
             }
             __syncthreads();
-            return __builtin_amdgcn_readfirstlane(s_piece);
-        };
-        if (blockIdx.x < a.wgs) publish(blockIdx.x);
-        load(first_v);
-        for (uint32_t piece = missing(); piece != NO_PIECE; piece = missing()) {
-            publish(piece);
+            tau = s_tau;
+            piece = __builtin_amdgcn_readfirstlane(s_piece);
+        }
+        if (deep || piece != NO_PIECE) {
+            for (;;) {
+                if (piece != NO_PIECE) publish(piece);
+                piece = sample_tau_deep(a.st, a.W, a.ks, a.polls, tau, s_piece, sh.sel.rs);
+                if (piece == NO_PIECE) break;
+            }
             uint32_t v0 = first_v;
             asm volatile("" : "+v"(v0));  // the addresses are made anew, not kept over the sample
             load(v0);
         }
-        tau = s_tau;
     } else {
         load(first_v);
         if (a.tau == TAU_OWN) {
@@ -781,8 +821,7 @@ static CandSet fte_launch(const FteRun &r, uint32_t k, const QCols &q, const Fin
     uint32_t cap = FUSE_CAP_MIN;
     while (cap < FUSE_CAP_MAX && (cap < 2 * a.kp2 || cap < 2 * sp.expect)) cap += FUSE_CAP_MIN;
     a.cap = cap;
-    a.wgs = g < SAMPLE_WGS ? g : SAMPLE_WGS;
-    a.polls = r.polls ? r.polls : SAMPLE_POLLS;
+    a.polls = r.polls ? r.polls : (g < SAMPLE_WGS ? 1u : SAMPLE_POLLS);
     CandSet &cs = a.cs;
     cs.keys = r.cand;
     cs.counts = r.counts;

@@ -25,9 +25,9 @@ constexpr uint32_t FUSE_CAP_MIN = 1024, FUSE_CAP_MAX = 4096;  // candidates the 
 constexpr uint32_t SEED_TILE = 4096;     // exact mode: objects per seed block (16 per thread)
 constexpr uint32_t SAMPLE_TILE = 1024;   // shared sample: objects per chunk
 constexpr uint32_t SAMPLE_CHUNKS = 128;  // shared sample: chunks at most, spread over the ids
-constexpr uint32_t SAMPLE_WGS = 32;      // workgroups that take the shared sample
-constexpr uint32_t SAMPLE_WIN = 512;     // shared sample: winners of all workgroups at most
-constexpr uint32_t SAMPLE_MAX_W = SAMPLE_WIN / SAMPLE_WGS;  // winners each of them publishes at most
+constexpr uint32_t SAMPLE_WGS = 32;      // shared sample: pieces, each a workgroup's
+constexpr uint32_t SAMPLE_WIN = 1024;    // shared sample: winners of all pieces at most
+constexpr uint32_t SAMPLE_MAX_W = SAMPLE_WIN / SAMPLE_WGS;  // winners of a piece at most
 constexpr uint32_t SAMPLE_POLLS = 32;    // tries before a workgroup takes a missing piece of the sample
 constexpr int SAMPLE_VEC = SAMPLE_CHUNKS * SAMPLE_TILE / (SAMPLE_WGS * STREAM_BS * 4);  // float4 per thread
 constexpr int OWN_VEC = 4096 / (STREAM_BS * 4);  // own sample: float4 vectors per thread
@@ -100,11 +100,23 @@ static inline uint32_t sample_rank(double q) {
 // exp(-q) (e q / ks)^ks (Chernoff, ten times the truth): here 1e-8, and 1e-5
 // below q = 1, where every rank adds candidates the most (32 queries of 16M x
 // 5, k = 32, q = 0.25: rank 4, 1e-4, 1797 us; rank 6 1820; rank 8 1872).
-static inline uint32_t queued_rank(double q) {
+//
+// These chances are for scores that do not depend on the id.  Stores in
+// score order, or with their best objects side by side, put whole runs of the
+// top k into one chunk: the rank leaves 8 k candidates at least, and k, a proven
+// bound, where that takes one (up to 2^20 objects).
+static inline uint32_t queued_rank(double q, uint32_t k) {
     const double rare = q < 1.0 ? 11.5 : 18.4;
-    uint32_t ks = 4;
+    uint32_t ks = std::max(4u, (uint32_t)std::min(std::ceil(8.0 * q), 4096.0));
     while (ks < 4096 && (ks <= q || ks * (std::log(ks / q) - 1.0) + q < rare)) ks++;
-    return ks;
+    return std::min(ks, std::max(k, 4u));
+}
+
+// Keys a piece of the shared sample publishes for a rank of ks: all of them
+// up to 16, then twice its share or more (the pieces' chunks alternate over
+// the id range; a piece that holds more of the ks best lowers tau).
+static inline uint32_t piece_winners(uint32_t ks) {
+    return ks < 16 ? ks : (ks <= 256 ? 16u : SAMPLE_MAX_W);
 }
 
 // Where a stream workgroup takes tau from: every object is a candidate,
@@ -141,15 +153,13 @@ static inline SeedPlan seed_plan(uint64_t n, uint32_t k, int mode) {
         // As many chunks as make tau the 8th largest of the sample (q =
         // 1.13).  A long list on a small store would leave few of them, large
         // jumps of the id range: below 32 chunks, all 128 and a deeper rank.
+        // Queued: all 128.
         const uint64_t c8 = (uint64_t)(1.13 * (double)n / ((double)k * SAMPLE_TILE));
-        p.blocks = c8 >= SAMPLE_CHUNKS / 4 && c8 < SAMPLE_CHUNKS ? (uint32_t)c8 : SAMPLE_CHUNKS;
+        p.blocks = mode == FTE_SAMPLE && c8 >= SAMPLE_CHUNKS / 4 && c8 < SAMPLE_CHUNKS ? (uint32_t)c8 : SAMPLE_CHUNKS;
         p.stride = ((n / p.blocks) / SAMPLE_TILE) * SAMPLE_TILE;
         const double s = (double)p.blocks * SAMPLE_TILE;
-        p.ks = mode == FTE_QUEUED ? queued_rank(k * s / (double)n) : sample_rank(k * s / (double)n);
-        // each piece's share of the ks best: all of them up to 16 (the
-        // pieces' chunks alternate over the id range, so more than 16 of
-        // a deep rank's best rarely meet in one; missing some lowers tau)
-        p.W = p.ks < SAMPLE_MAX_W ? p.ks : SAMPLE_MAX_W;
+        p.ks = mode == FTE_QUEUED ? queued_rank(k * s / (double)n, k) : sample_rank(k * s / (double)n);
+        p.W = piece_winners(p.ks);
         p.expect = (double)p.ks * n / s;
     } else {
         p.tau = TAU_STATE;

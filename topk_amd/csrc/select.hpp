@@ -145,6 +145,7 @@ __device__ void fused_select(FteState *__restrict__ st, const CandSet &cs, uint3
         if (fo.status) *fo.status = bad;
     }
     if (tid < ARRIVE_GROUPS) st->group[tid * ARRIVE_STRIDE] = 0;
+    static_assert(SAMPLE_WIN <= BS, "a winner a thread");
     if (tid < SAMPLE_WIN) st->win[tid] = 0;
     if (bad) return;
     const SlotView v{cs.pre, npre, cs.keys, cs.slot, off, cs.nblk, ntotal, cs.spill};
