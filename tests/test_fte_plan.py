@@ -87,6 +87,41 @@ int main() {
 }
 """
 
+ORDERED = HEADER + r"""
+// Candidates that reach tau in a store whose score falls with the id, from the plan alone: the sample's positions,
+// W winners of each piece or wave, the ks-th best of them.
+static uint64_t reach(const SeedPlan &p, uint64_t n) {
+    std::vector<uint64_t> best;
+    if (p.tau == TAU_SHARED) {
+        for (uint32_t piece = 0; piece < SAMPLE_WGS; piece++)
+            for (uint32_t w = 0, c = piece, i = 0; w < p.W && c < p.blocks; w++) {
+                best.push_back(c * p.stride + i);
+                if (++i == SAMPLE_TILE) c += SAMPLE_WGS, i = 0;
+            }
+    } else {
+        const uint64_t lines = (n + 15) / 16;
+        for (uint32_t wave = 0; wave < STREAM_BS / 64; wave++)
+            for (uint32_t w = 0; w < p.W; w++) {
+                const uint64_t spot = w / 16 * (STREAM_BS / 64) + wave, id = spot * lines / OWN_SPOTS * 16 + w % 16;
+                if (id < n) best.push_back(id);
+            }
+    }
+    std::sort(best.begin(), best.end());
+    return best.size() < p.ks ? n : best[p.ks - 1] + 1;
+}
+int main() {
+    for (uint64_t n : {4097ull, 16411ull, 65521ull, 131072ull, 300007ull, 1ull << 19, (1ull << 19) + 1, 700001ull, 1ull << 20})
+        for (uint32_t k = 1; k <= 1024; k++) {
+            const SeedPlan p = seed_plan(n, k, FTE_SAMPLE);
+            if (p.tau == TAU_ALL) continue;
+            const uint64_t c = reach(p, n);
+            CHECK(c >= k, "n %llu k %u: rank %u, %u winners a piece, %llu candidates", (unsigned long long)n, k, p.ks, p.W,
+                  (unsigned long long)c);
+        }
+    return fails ? 1 : 0;
+}
+"""
+
 
 def _run(program, tmp_path):
     if not shutil.which("g++"):
@@ -105,3 +140,7 @@ def test_reads_and_slots_stay_inside_their_buffers(tmp_path):
 
 def test_queued_ranks_are_as_deep_as_a_proven_bound(tmp_path):
     _run(RANKS, tmp_path)
+
+
+def test_stores_in_score_order_take_one_run(tmp_path):
+    _run(ORDERED, tmp_path)

@@ -56,7 +56,7 @@ def _ordered(n, kind):
     if kind == "best-last":
         return i.reshape(1, n)
     x = topk_amd.generate(n, 1, topk_amd.INDEPENDENT, 2) * np.float32(0.5)
-    at = (n // 128 // 1024) * 1024 * 40  # the first object of a sampled chunk
+    at = n // 128 // 16 * 16 * 40  # the first object of a sampled chunk
     x[0, at:at + 2000] += np.linspace(1, 0.5, 2000, dtype=np.float32)
     return x
 
@@ -96,3 +96,26 @@ def test_late_sample_with_queries_queued_on_both_lanes(gpu, polls):
     for i in range(2):
         for j, (rid, rsc, _) in enumerate(want):
             assert np.array_equal(got[i][0][j], rid) and np.array_equal(got[i][1][j], rsc), (i, j)
+
+
+@pytest.mark.parametrize("kind", ["best-first", "best-last", "one-value", "two-values", "few-below"])
+@pytest.mark.parametrize("n,k", [(4097, 1024), (6000, 1000), (8191, 1024), (65_521, 10), (1 << 19, 64), (1 << 20, 1),
+                                 (1 << 20, 10), (1 << 20, 256), (1 << 20, 1000)])
+def test_select_of_many_candidates(gpu, kind, n, k):
+    # candidates past the select's LDS: spread by score, all tied, and an interval too full for it
+    if kind in ("best-first", "best-last"):
+        x = _ordered(n, kind)
+    else:
+        x = np.full((1, n), 0.75, np.float32)
+        if kind == "two-values":
+            x[0, ::2] = 0.25
+        if kind == "few-below":
+            x[0, n // 2:n // 2 + 90] = 0.25
+    w = np.ones(1, np.float32)
+    rid, rsc, rthr = oracle.fte_topk(x, n, k, w, [0])
+    with topk_amd.Engine(x) as eng:
+        for _ in range(2):
+            ids, sc, thr = eng.fte(k, w, [0])
+            assert np.array_equal(ids, rid) and np.array_equal(sc, rsc) and thr == rthr
+        if kind.startswith("best"):
+            assert eng.stats()["fallback"] == 0  # one run

@@ -378,16 +378,14 @@ __device__ __forceinline__ uint32_t sample_tau_deep(FteState *__restrict__ st, u
 // half is widened to the end of the stratum the key lies in: among tied
 // scores a run's ids are consecutive, and the key of one of them alone would
 // admit only that run's ids.
-constexpr uint32_t OWN_MAX_W = 32;
 struct OwnScratch {
     uint64_t keys[STREAM_NW * OWN_MAX_W];
     uint64_t tau;
 };
 template <int M>
-__device__ __forceinline__ uint64_t own_sample_tau(const QCols &q, uint64_t n, uint32_t ks, OwnScratch &os) {
+__device__ __forceinline__ uint64_t own_sample_tau(const QCols &q, uint64_t n, uint32_t ks, uint32_t W, OwnScratch &os) {
     const uint32_t wave = threadIdx.x / 64, lane = lane_id();
     const uint32_t lines = (uint32_t)((n + 15) / 16);
-    const uint32_t W = ks < 8 + ks / 4 ? ks : (8 + ks / 4 < OWN_MAX_W ? 8 + ks / 4 : OWN_MAX_W);
     {
         uint32_t hi[4 * OWN_VEC], lo[4 * OWN_VEC];
 #pragma unroll
@@ -440,7 +438,8 @@ struct StreamArgs {
     CandSet cs;
     int tau;               // TAU_*: every object a candidate, st->tau, the shared sample, the own sample
     uint32_t ks;           // rank of tau in the sample
-    uint32_t chunks, W;    // shared sample: chunks, winners per piece
+    uint32_t chunks;       // of the shared sample
+    uint32_t W;            // winners per piece of the shared sample, or per wave of the own one
     uint64_t chunk_stride; // objects between the chunks' first objects
     uint32_t polls;        // tries before a workgroup takes a missing piece of the sample
     int select;            // the last workgroup selects and emits (else a later launch does)
@@ -545,7 +544,7 @@ __global__ __launch_bounds__(STREAM_BS, 4) void fte_stream_kernel(QCols q, Strea
     } else {
         load(first_v);
         if (a.tau == TAU_OWN) {
-            tau = own_sample_tau<M>(q, a.n, a.ks, sh.own);
+            tau = own_sample_tau<M>(q, a.n, a.ks, a.W, sh.own);
         } else {
             if (a.tau == TAU_STATE) tau = a.st->tau;
             __syncthreads();

@@ -33,6 +33,7 @@ constexpr int SAMPLE_VEC = SAMPLE_CHUNKS * SAMPLE_TILE / (SAMPLE_WGS * STREAM_BS
 constexpr int OWN_VEC = 4096 / (STREAM_BS * 4);  // own sample: float4 vectors per thread
 constexpr uint32_t OWN_OBJS = STREAM_BS * 4 * OWN_VEC;
 constexpr uint32_t OWN_SPOTS = OWN_OBJS / 16;   // own sample: 256 runs of 16 objects, one 64-byte line per column each
+constexpr uint32_t OWN_MAX_W = 32;              // own sample: keys of a wave at most
 constexpr uint64_t OWN_MAX_N = 1ull << 19;      // stores up to this size take their own sample
 
 // A column of n objects is readable to its n-th value rounded up to 16
@@ -112,12 +113,22 @@ static inline uint32_t queued_rank(double q, uint32_t k) {
     return std::min(ks, std::max(k, 4u));
 }
 
-// Keys a piece of the shared sample publishes for a rank of ks: all of them
-// up to 16, then twice its share or more (the pieces' chunks alternate over
-// the id range; a piece that holds more of the ks best lowers tau).
-static inline uint32_t piece_winners(uint32_t ks) {
-    return ks < 16 ? ks : (ks <= 256 ? 16u : SAMPLE_MAX_W);
+// Keys a piece of the shared sample publishes.  Up to 2^20 objects half of a
+// rank below k, so that tau lies below the best of at least two pieces: of a
+// store in score order one piece holds the whole top ks, and with all of them
+// published ks objects would reach tau instead of k (2^20 objects, k = 10: a
+// second, exact run, 100 us in all instead of 63).  Larger stores take that
+// run, as they always did.  From a rank of 16 on a piece's share, with room: a
+// piece that holds more lowers tau.
+static inline uint32_t piece_winners(uint32_t ks, uint32_t k, uint64_t n) {
+    const uint32_t w = ks < k && n <= 1ull << 20 ? (ks + 1) / 2 : ks;
+    return w < 16 ? w : (ks <= 256 ? 16u : SAMPLE_MAX_W);
 }
+
+// Keys a wave of the own sample contributes: half, for the same reason (2^19
+// objects, k = 64: 100 us in two runs, 40 in one; the exact run alone took
+// 80), which also halves its rounds (16k objects, k = 10: 35.4 -> 33.8 us).
+static inline uint32_t wave_winners(uint32_t ks) { return std::min({(ks + 1) / 2, 8 + ks / 4, OWN_MAX_W}); }
 
 // Where a stream workgroup takes tau from: every object is a candidate,
 // st->tau, the shared sample, the own sample.
@@ -127,7 +138,7 @@ enum { TAU_ALL = 0, TAU_STATE = 1, TAU_SHARED = 2, TAU_OWN = 3 };
 struct SeedPlan {
     int tau;               // TAU_*
     uint32_t blocks, ks;   // chunks of the sample or blocks of the exact seed; rank of tau (exact: winners per block)
-    uint32_t W;            // shared sample: winners per piece
+    uint32_t W;            // winners per piece of the shared sample, or per wave of the own one
     uint64_t stride;       // objects between the chunks' first objects
     uint64_t n_eff;        // exact: objects of the prefix
     uint32_t total_valid;  // exact: keys the blocks deposit
@@ -146,6 +157,7 @@ static inline SeedPlan seed_plan(uint64_t n, uint32_t k, int mode) {
     } else if (mode == FTE_SAMPLE && n <= OWN_MAX_N) {
         p.tau = TAU_OWN;
         p.ks = sample_rank((double)k * OWN_OBJS / (double)n);
+        p.W = wave_winners(p.ks);
         p.expect = (double)p.ks * n / OWN_OBJS;
         if (p.expect >= n) p.tau = TAU_ALL;
     } else if ((mode == FTE_SAMPLE || mode == FTE_QUEUED) && n > OWN_MAX_N) {
@@ -156,10 +168,10 @@ static inline SeedPlan seed_plan(uint64_t n, uint32_t k, int mode) {
         // Queued: all 128.
         const uint64_t c8 = (uint64_t)(1.13 * (double)n / ((double)k * SAMPLE_TILE));
         p.blocks = mode == FTE_SAMPLE && c8 >= SAMPLE_CHUNKS / 4 && c8 < SAMPLE_CHUNKS ? (uint32_t)c8 : SAMPLE_CHUNKS;
-        p.stride = ((n / p.blocks) / SAMPLE_TILE) * SAMPLE_TILE;
+        p.stride = (n / p.blocks) & ~15ull;  // a line; the chunks reach to the end of the store
         const double s = (double)p.blocks * SAMPLE_TILE;
         p.ks = mode == FTE_QUEUED ? queued_rank(k * s / (double)n, k) : sample_rank(k * s / (double)n);
-        p.W = piece_winners(p.ks);
+        p.W = piece_winners(p.ks, k, n);
         p.expect = (double)p.ks * n / s;
     } else {
         p.tau = TAU_STATE;

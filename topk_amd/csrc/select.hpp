@@ -60,6 +60,41 @@ struct FuseScratch {
     uint32_t cut, ncut;   // the interval holding the k-th key, and the keys up to its end
 };
 
+// f on every candidate, c of them.  Spread thin over the workgroups' slots they
+// are taken by flat index, four at a time; else a workgroup's slots by a wave,
+// eight loads in flight, without a search for each.
+template <int BS, class F>
+__device__ __forceinline__ void for_candidates(const SlotView &v, uint32_t c, F f) {
+    const uint32_t tid = threadIdx.x;
+    if (c < 64 * v.nblk) {
+        for (uint32_t i0 = tid; i0 < c; i0 += 4 * BS) {
+            uint64_t x[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = i0 + j * BS < c ? v.get(i0 + j * BS) : 0ull;
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (x[j]) f(x[j]);
+        }
+        return;
+    }
+    auto range = [&](const uint64_t *p, uint32_t n, uint32_t first, uint32_t step) __attribute__((always_inline)) {
+        for (uint32_t i0 = first; i0 < n; i0 += 8 * step) {
+            uint64_t x[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) x[j] = i0 + j * step < n ? p[i0 + j * step] : 0ull;
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                if (x[j]) f(x[j]);
+        }
+    };
+    range(v.pre, v.npre, tid, BS);
+    for (uint32_t b = tid / 64; b < v.nblk; b += BS / 64) {
+        const uint32_t at = v.off[b], end = b + 1 < v.nblk ? v.off[b + 1] : v.total;
+        range(v.keys + (uint64_t)b * v.slot, end - at, lane_id(), 64);
+    }
+    range(v.spill, c - v.npre - v.total, tid, BS);
+}
+
 // Writes the first want keys, best first, and sentinels up to k.
 template <int BS>
 __device__ __forceinline__ void emit_sorted(const uint64_t *sorted, uint32_t want, uint32_t k, const FinalOut &fo) {
@@ -76,10 +111,13 @@ __device__ __forceinline__ void emit_sorted(const uint64_t *sorted, uint32_t wan
 // gathered into LDS (lkeys, cap keys), counting-sorted by 1024 equal
 // intervals of their key range -- only as far as the interval that holds the
 // k-th -- and each key is ranked inside its interval; results go out best
-// first.  Ties crowding one interval, and more candidates than cap, take a
-// radix select.  lkeys and regb hold cap keys each (2 * kp2 at least).
+// first.  Of more candidates than cap, the intervals that hold the first want
+// of them are gathered (three passes; the radix select of 90000 candidates
+// took 500 us and 11 passes, a binary search a key).  Ties crowding one
+// interval, or past cap, take a radix select.  lkeys and regb hold cap keys
+// each (2 * kp2 at least).
 template <int BS>
-__device__ void fused_select(FteState *__restrict__ st, const CandSet &cs, uint32_t k, uint32_t kreq, uint32_t cap,
+__device__ __forceinline__ void fused_select(FteState *__restrict__ st, const CandSet &cs, uint32_t k, uint32_t kreq, uint32_t cap,
                              uint32_t kp2, const FinalOut &fo, uint64_t *lkeys, uint64_t *regb, FuseScratch &fs) {
     __shared__ uint32_t wsum[BS / 64];
     __shared__ uint32_t total, s_spill, s_pre;
@@ -171,14 +209,12 @@ __device__ void fused_select(FteState *__restrict__ st, const CandSet &cs, uint3
         emit_sorted<BS>(regb, want, k, fo);
         return;
     }
-    if (c <= cap) {
-        uint64_t lo = ~0ull, hi = 0;
-        for (uint32_t i = tid; i < c; i += BS) {
-            const uint64_t x = v.get(i);
-            lkeys[i] = x;
-            lo = x < lo ? x : lo;
-            hi = x > hi ? x : hi;
-        }
+    // the interval of a key, and the cut: the interval that holds the want-th
+    // (bins[] counts, then starts)
+    uint64_t lo = ~0ull, hi = 0;
+    int shift = 0;
+    auto interval = [&](uint64_t x) __attribute__((always_inline)) { return (uint32_t)((hi - x) >> shift); };
+    auto range = [&]() __attribute__((always_inline)) {
         lo = wave_min_u64(lo);
         hi = wave_max_u64(hi);
         if (lane_id() == 0) {
@@ -192,10 +228,10 @@ __device__ void fused_select(FteState *__restrict__ st, const CandSet &cs, uint3
             hi = fs.whi[w] > hi ? fs.whi[w] : hi;
         }
         const int width = 64 - (hi > lo ? __builtin_clzll(hi - lo) : 63);
-        const int shift = width > 10 ? width - 10 : 0;  // interval 0 holds the largest keys
-        for (uint32_t i = tid; i < c; i += BS) atomicAdd(&fs.bins[(uint32_t)((hi - lkeys[i]) >> shift)], 1u);
-        __syncthreads();
-        constexpr int BPT = FUSE_BINS / BS;
+        shift = width > 10 ? width - 10 : 0;  // interval 0 holds the largest keys
+    };
+    constexpr int BPT = FUSE_BINS / BS;
+    auto starts = [&](uint32_t most) __attribute__((always_inline)) {
         uint32_t n_[BPT], sum = 0;
 #pragma unroll
         for (int j = 0; j < BPT; j++) {
@@ -207,7 +243,7 @@ __device__ void fused_select(FteState *__restrict__ st, const CandSet &cs, uint3
         for (int j = 0; j < BPT; j++) {
             fs.bins[tid * BPT + j] = at;
             if (at < want) {
-                if (n_[j] > FUSE_BIN_MAX) fs.crowded = 1;
+                if (n_[j] > most) fs.crowded = 1;
                 if (at + n_[j] >= want) {  // holds the last result
                     fs.cut = tid * BPT + j;
                     fs.ncut = at + n_[j];
@@ -216,19 +252,57 @@ __device__ void fused_select(FteState *__restrict__ st, const CandSet &cs, uint3
             at += n_[j];
         }
         __syncthreads();
+    };
+    uint32_t held = c;  // keys in lkeys
+    bool few = c <= cap;
+    if (!few) {
+        for_candidates<BS>(v, c, [&](uint64_t x) __attribute__((always_inline)) {
+            lo = x < lo ? x : lo;
+            hi = x > hi ? x : hi;
+        });
+        range();
+        for_candidates<BS>(v, c, [&](uint64_t x) __attribute__((always_inline)) { atomicAdd(&fs.bins[interval(x)], 1u); });
+        __syncthreads();
+        starts(0xFFFFFFFFu);
+        if (fs.ncut <= cap) {
+            held = fs.ncut;
+            const uint32_t cut = fs.cut;
+            if (tid == 0) s_spill = 0;  // used up: the next free place in lkeys
+            __syncthreads();
+            for_candidates<BS>(v, c, [&](uint64_t x) __attribute__((always_inline)) {
+                if (interval(x) <= cut) lkeys[atomicAdd(&s_spill, 1u)] = x;
+            });
+            for (uint32_t b = tid; b < FUSE_BINS; b += BS) fs.bins[b] = 0;
+            few = true;
+            lo = ~0ull;
+            hi = 0;
+        }
+        __syncthreads();
+    }
+    if (few) {
+        for (uint32_t i = tid; i < held; i += BS) {
+            const uint64_t x = c <= cap ? v.get(i) : lkeys[i];
+            if (c <= cap) lkeys[i] = x;
+            lo = x < lo ? x : lo;
+            hi = x > hi ? x : hi;
+        }
+        range();
+        for (uint32_t i = tid; i < held; i += BS) atomicAdd(&fs.bins[interval(lkeys[i])], 1u);
+        __syncthreads();
+        starts(FUSE_BIN_MAX);
         if (!fs.crowded) {
             // the intervals up to the cut, in order; bins[] turns from an
             // interval's start into its end (the offsets in regb are used up)
-            for (uint32_t i = tid; i < c; i += BS) {
+            for (uint32_t i = tid; i < held; i += BS) {
                 const uint64_t x = lkeys[i];
-                const uint32_t b = (uint32_t)((hi - x) >> shift);
+                const uint32_t b = interval(x);
                 if (b <= fs.cut) regb[atomicAdd(&fs.bins[b], 1u)] = x;
             }
             __syncthreads();
             sorted = lkeys;
             for (uint32_t i = tid; i < fs.ncut; i += BS) {
                 const uint64_t x = regb[i];
-                const uint32_t b = (uint32_t)((hi - x) >> shift);
+                const uint32_t b = interval(x);
                 const uint32_t s0 = b ? fs.bins[b - 1] : 0u, s1 = fs.bins[b];
                 uint32_t r = s0;
                 for (uint32_t j = s0; j < s1; j++) r += regb[j] > x ? 1u : 0u;
@@ -237,12 +311,12 @@ __device__ void fused_select(FteState *__restrict__ st, const CandSet &cs, uint3
             __syncthreads();
         }
     }
-    if (c > cap || fs.crowded) {
+    if (!few || fs.crowded) {
         uint32_t got;
-        if (c <= cap) {
+        if (few) {
             const uint64_t thr =
-                c > k ? block_kth_largest<BS, MemKeys<BS>, 8>(MemKeys<BS>{lkeys, c}, c, k, fs.rs) : 1ull;
-            got = block_gather_ge<BS>(MemKeysUniform<BS>{lkeys, c}, thr, regb, fs.rs);
+                held > k ? block_kth_largest<BS, MemKeys<BS>, 8>(MemKeys<BS>{lkeys, held}, held, k, fs.rs) : 1ull;
+            got = block_gather_ge<BS>(MemKeysUniform<BS>{lkeys, held}, thr, regb, fs.rs);
             sorted = regb;
         } else {
             const uint64_t thr = block_kth_largest<BS, ViewKeys<BS, SlotView, false>, 8>(
