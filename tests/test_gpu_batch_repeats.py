@@ -1,0 +1,29 @@
+"""Batches over stores of repeated values, where every object of a value lies in
+one partition of many chunks: results against the oracle, and no more work
+items than a budget of 128 queries an item gives."""
+import numpy as np
+import pytest
+
+import topk_amd
+from test_gpu_batch import make_queries
+from test_gpu_batch_items import check
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nq", [1, 65, 300])
+@pytest.mark.parametrize("values", [1, 2])
+def test_partitions_of_many_chunks(gpu, values, nq):
+    n, d = 300_007, 4
+    rng = np.random.default_rng(values)
+    x = (rng.integers(0, values, size=(d, n)) + 0.5).astype(np.float32)
+    qs = make_queries(rng, nq, d, [1, 16, 100])
+    with topk_amd.Engine(x) as eng:
+        eng.set_tuning("batch_fused", 1)
+        eng.set_tuning("batch_item", 2048)
+        for qpi in (0, 16, 128):
+            eng.set_tuning("batch_qpi", qpi)
+            check(eng, x, qs)
+            s = eng.stats()
+            if qpi == 0 and values == 1:
+                assert s["items"] <= -(-nq // 128) * -(-n // 2048)

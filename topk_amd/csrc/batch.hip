@@ -716,7 +716,15 @@ __global__ __launch_bounds__(BMASK_BS) void batch_mask_kernel(const BatchQuery *
 // load of its objects.  Correlated, d = 8, 128 queries, N = 2^18: 128
 // queries an item 451 us, 16 206 us, 4 169 us; anticorrelated, d = 16, 1024
 // queries, N = 2^24: 128 and 64 27.4 ms, 32 29.4 ms, 16 33.3 ms.
-constexpr uint32_t QPI_MIN = 4, QPI_MAX = 64, QPI_ITEMS = 4096;
+//
+// Partitions of many chunks (repeated values: every object of a value shares
+// one) have few entries and many items each, and their objects are worth
+// loading for more queries: the budget grows with their chunks, to 128.  Their
+// items are written by the whole wave, a partition at a time: alone in its
+// lane, such a partition took a step an item.  512 queries, k <= 256, N = 2^23,
+// d = 8, all objects equal / binary attributes: 194 / 28 -> 129 / 3.9 ms.
+constexpr uint32_t QPI_MIN = 4, QPI_MAX = 64, QPI_MAX_LARGE = 128, QPI_ITEMS = 4096;
+constexpr uint32_t ITEM_STEPS = 256;  // items at most of a partition that takes its turn with the others
 __global__ __launch_bounds__(BAUX_BS) void batch_compact_kernel(const unsigned int *__restrict__ pcnt, uint32_t L,
                                                                 uint32_t qfix, uint32_t target, uint32_t ochunk, uint64_t cap,
                                                                 const uint32_t *__restrict__ psz,
@@ -727,14 +735,15 @@ __global__ __launch_bounds__(BAUX_BS) void batch_compact_kernel(const unsigned i
     __shared__ uint32_t tot_h, tot_l, base_h, base_l;
     const uint32_t lane = lane_id();
     const uint32_t p = (lane * (BAUX_BS / 64) + threadIdx.x / 64) * gridDim.x + blockIdx.x;
+    const uint32_t cnt = p < L ? pcnt[p] : 0u;
+    const uint32_t sz = cnt ? psz[p] : 0u;
+    const uint32_t nch = (sz + ochunk - 1) / ochunk;
     uint32_t qmax = qfix;
     if (!qfix) {
         const unsigned long long e = *reinterpret_cast<const unsigned long long *>(ctr + 2) / target;
         qmax = e < QPI_MIN ? QPI_MIN : (e > QPI_MAX ? QPI_MAX : (uint32_t)e);
+        if (nch > 3) qmax = nch > 2 * QPI_MAX_LARGE / qmax ? QPI_MAX_LARGE : qmax * nch / 2;
     }
-    const uint32_t cnt = p < L ? pcnt[p] : 0u;
-    const uint32_t sz = cnt ? psz[p] : 0u;
-    const uint32_t nch = (sz + ochunk - 1) / ochunk;
     const uint32_t heavy_min = (qmax + 1) / 2;
     const uint32_t nr = (cnt + qmax - 1) / qmax;
     const uint32_t last = cnt - (nr ? (nr - 1) * qmax : 0u);
@@ -762,11 +771,12 @@ __global__ __launch_bounds__(BAUX_BS) void batch_compact_kernel(const unsigned i
     __syncthreads();
     uint32_t kh = base_h + (uint32_t)__builtin_amdgcn_readfirstlane((int)offh);
     uint32_t kl = base_l + (uint32_t)__builtin_amdgcn_readfirstlane((int)offl);
-    const uint32_t maxc = wave_max_u32(nch), maxr = wave_max_u32(nr);
+    const bool large = (unsigned long long)nr * nch > ITEM_STEPS;
+    const uint32_t maxc = wave_max_u32(large ? 0u : nch), maxr = wave_max_u32(large ? 0u : nr);
     const uint64_t below = (1ull << lane) - 1ull;
     for (uint32_t r = 0; r < maxr; r++)
         for (uint32_t c = 0; c < maxc; c++) {
-            const bool on = r < nr && c < nch, heavy = on && r < nhr;
+            const bool on = !large && r < nr && c < nch, heavy = on && r < nhr;
             const uint64_t mh = __ballot(heavy), ml = __ballot(on && !heavy);
             const uint32_t q0 = r * qmax;
             const BatchItem it{p, q0, cnt - q0 < qmax ? cnt - q0 : qmax, c};
@@ -775,6 +785,20 @@ __global__ __launch_bounds__(BAUX_BS) void batch_compact_kernel(const unsigned i
             kh += (uint32_t)__popcll(mh);
             kl += (uint32_t)__popcll(ml);
         }
+    for (uint64_t m = __ballot(large); m; m &= m - 1) {
+        const int src = __builtin_ctzll(m);
+        auto of = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, src); };
+        const uint32_t sp = of(p), scnt = of(cnt), snch = of(nch), snr = of(nr), snhr = of(nhr), sq = of(qmax);
+        const uint32_t all = snr * snch, hv = snhr * snch;
+        for (uint32_t i = lane; i < all; i += 64) {
+            const uint32_t r = i / snch, c = i - r * snch, q0 = r * sq;
+            const BatchItem it{sp, q0, scnt - q0 < sq ? scnt - q0 : sq, c};
+            if (i < hv) items[kh + i] = it;
+            else items[cap - 1 - (kl + i - hv)] = it;
+        }
+        kh += hv;
+        kl += all - hv;
+    }
 }
 
 struct ScoreArgs {
