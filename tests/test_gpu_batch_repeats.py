@@ -27,3 +27,21 @@ def test_partitions_of_many_chunks(gpu, values, nq):
             s = eng.stats()
             if qpi == 0 and values == 1:
                 assert s["items"] <= -(-nq // 128) * -(-n // 2048)
+
+
+@pytest.mark.parametrize("fused", [1, 2])
+def test_large_partitions_keep_id_order(gpu, fused):
+    # one partition holds every object; its first positions are the lowest ids,
+    # so a seed threshold admits few ties and no query takes a second pass
+    n, d, nq = 1_000_003, 3, 40
+    x = np.full((d, n), 0.5, np.float32)
+    qs = make_queries(np.random.default_rng(3), nq, d, [1, 16, 256])
+    with topk_amd.Engine(x) as eng:
+        eng.init(topk_amd.TOPK_INIT_PTA)
+        eng.set_tuning("batch_fused", fused)
+        check(eng, x, qs)
+        s = eng.stats()
+        assert s["fallback"] == 0 and s["partitions_scored"] == nq
+        k, w, attr = qs[0]
+        ids, _, _ = eng.pta(256, w, attr)
+        assert np.array_equal(ids, np.arange(256, dtype=np.uint64)) and eng.stats()["fallback"] == 0

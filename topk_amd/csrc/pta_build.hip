@@ -575,6 +575,41 @@ __global__ __launch_bounds__(PA_BS) void pta_assign_kernel(AssignArgs a) {
     }
 }
 
+// Partitions past PTA_SORT_MAX objects stay as scattered.  They hold repeated
+// values, whose best objects are those of the lowest ids, and a query's seed
+// takes a partition's first objects: in the order in which the assign
+// workgroups happened to reserve their shares, 512 queries over N = 2^23 equal
+// objects (d = 8) all kept more ties than a list holds, 129 ms; in id order
+// 0.9 ms.  So the shares are given out again, workgroup by workgroup: recounted
+// here, and made prefixes over the workgroups, a thread per leaf, below.
+__global__ __launch_bounds__(PA_BS) void pta_recount_kernel(AssignArgs a) {
+    extern __shared__ float pa_lds[];
+    uint32_t *h = reinterpret_cast<uint32_t *>(pa_lds);
+    for (uint32_t l = threadIdx.x; l < a.L; l += PA_BS) h[l] = 0;
+    __syncthreads();
+    const uint64_t i0 = (uint64_t)blockIdx.x * a.per, i1 = i0 + a.per < a.n ? i0 + a.per : a.n;
+    for (uint64_t i = i0 + threadIdx.x; i < i1; i += PA_BS) atomicAdd(&h[a.place[i].x], 1u);
+    __syncthreads();
+    for (uint32_t l = threadIdx.x; l < a.L; l += PA_BS) a.base[(uint64_t)blockIdx.x * a.L + l] = h[l];
+}
+
+__global__ __launch_bounds__(256) void pta_base_kernel(uint32_t *__restrict__ base, uint32_t L, uint32_t groups) {
+    const uint32_t l = blockIdx.x * 256 + threadIdx.x;
+    if (l >= L) return;
+    uint32_t at = 0;
+    for (uint32_t g0 = 0; g0 < groups; g0 += 8) {
+        uint32_t c[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; j++) c[j] = g0 + j < groups ? base[(uint64_t)(g0 + j) * L + l] : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < 8; j++)
+            if (g0 + j < groups) {
+                base[(uint64_t)(g0 + j) * L + l] = at;
+                at += c[j];
+            }
+    }
+}
+
 // Padded offsets of the partitions (one workgroup); rep (pinned): padded
 // total (two words), nonempty partitions, largest partition.
 __global__ __launch_bounds__(1024) void pta_offsets_kernel(const uint32_t *__restrict__ cnt, uint32_t L,
@@ -629,21 +664,22 @@ __global__ __launch_bounds__(1024) void pta_offsets_kernel(const uint32_t *__res
 // ---------------------------------------------------------------------------
 // Ordering keys, and rows (if out != null), of assign workgroup blockIdx.y's
 // objects to their places in the partition order (unordered inside a
-// partition): in leaf order, so that a leaf's rows follow each other.
+// partition): in leaf order, so that a leaf's rows follow each other, or
+// (order null, bases by pta_base_kernel) in id order.
 __global__ __launch_bounds__(256) void pta_scatter_kernel(AssignArgs a, const uint32_t *__restrict__ poff,
                                                           uint64_t *__restrict__ keys, float *__restrict__ out) {
     const uint64_t i0 = (uint64_t)blockIdx.y * a.per, i1 = i0 + a.per < a.n ? i0 + a.per : a.n;
     const uint32_t *base = a.base ? a.base + (uint64_t)blockIdx.y * a.L : nullptr;
     for (uint64_t q = i0 + blockIdx.x * 256 + threadIdx.x; q < i1; q += gridDim.x * 256) {
         uint32_t i, pos;
-        if (base) {
+        if (a.order) {
             const uint2 o = a.order[q];
             i = o.x;
             pos = poff[o.y] + base[o.y] + (uint32_t)(q - i0);
         } else {
             const uint2 pl = a.place[q];
             i = (uint32_t)q;
-            pos = poff[pl.x] + pl.y;
+            pos = poff[pl.x] + (base ? base[pl.x] : 0u) + pl.y;
         }
         float s = 0.0f;  // attribute sum, in attribute order
         for (uint32_t m = 0; m < a.dp; m += 4) {
@@ -1451,6 +1487,11 @@ int pta_build(topk_ctx *ctx) {
         // 4, 5: objects to their partitions, the partitions in order
         const bool fused = with_rows && P.maxsz <= PTA_SORT_MAX;
         if (!fused) TK_TRY(hipMemsetAsync(keys, 0, sizeof(uint64_t) * P.ld, s));
+        if (P.maxsz > PTA_SORT_MAX && counted) {
+            hipLaunchKernelGGL(pta_recount_kernel, dim3(groups), dim3(PA_BS), sizeof(uint32_t) * L, s, as);
+            hipLaunchKernelGGL(pta_base_kernel, dim3((L + 255) / 256), dim3(256), 0, s, as.base, L, groups);
+            as.order = nullptr;
+        }
         hipLaunchKernelGGL(pta_scatter_kernel, dim3((uint32_t)std::min<uint64_t>(16, (as.per + 255) / 256), groups),
                            dim3(256), 0, s, as, P.poff, keys, fused ? srows : (float *)nullptr);
         if (fused) {
