@@ -154,7 +154,13 @@ int topk_ctx_read_columns(topk_ctx *ctx, float *out);
 #define TOPK_INIT_NORMALIZE 0x1u   /* per-column min-max normalisation, common/common.h:29-60 */
 #define TOPK_INIT_PTA       0x2u   /* build the PTA partition layout + per-partition bounds */
 
-/* Runs the requested preprocessing; its wall time is reported as tt_init. */
+/* Runs the requested preprocessing; its wall time is reported as tt_init.
+ * A layout build takes scratch of up to 24 + 8 d bytes an object while it
+ * runs; without room for that it takes 24, and without room for those nothing
+ * per object (slower; "init_lean" asks for it).  Up to 4 GiB of the scratch
+ * stays with the context for the next build, until topk_ctx_destroy,
+ * topk_reorder_attr, a topk_init without a build, or an allocation of the
+ * context that finds no room without it. */
 int topk_init(topk_ctx *ctx, uint32_t flags);
 
 /* Partition size used by TOPK_INIT_PTA (default 4096 objects). Must be a
@@ -363,6 +369,8 @@ void *topk_stream(topk_ctx *ctx);
  *   "stream_grid"     blocks of the FTE stream pass (0 = default)
  *   "stream_vpt"      float4 vectors per lane per column of a stream tile:
  *                     1, 2, 4 or 8 (0 = chosen from the query width)
+ *   "init_lean"       1 = layout builds take the least device memory: no
+ *                     scratch per object, none kept afterwards
  *   "sample_polls"    tries (about 1.5 us each) of an FTE stream workgroup to
  *                     get the shared threshold sample before it scores the
  *                     missing part of it itself (0 = default)

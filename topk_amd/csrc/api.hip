@@ -335,9 +335,9 @@ static int ensure_big(topk_ctx *ctx, uint64_t n) {
     hipFree(ctx->flat);
     ctx->cand_big = nullptr;
     ctx->flat = nullptr;
-    TK_HIP(hipMalloc(&ctx->cand_big, sizeof(uint64_t) * need));
+    TK_HIP(ctx_malloc(ctx, &ctx->cand_big, sizeof(uint64_t) * need));
     ctx->cand_big_cap = need;
-    TK_HIP(hipMalloc(&ctx->flat, sizeof(uint64_t) * (n + TOPK_MAX_K)));
+    TK_HIP(ctx_malloc(ctx, &ctx->flat, sizeof(uint64_t) * (n + TOPK_MAX_K)));
     ctx->flat_cap = n + TOPK_MAX_K;
     return TOPK_OK;
 }
@@ -483,6 +483,8 @@ int topk_set_tuning(topk_ctx *ctx, const char *name, int64_t value) {
     if (key == "stream_grid") {
         if (value < 0 || value > (int64_t)MAX_STREAM_GRID) return TOPK_ERR_INVALID;
         ctx->tune.stream_grid = (uint32_t)value;
+    } else if (key == "init_lean") {
+        ctx->tune.init_lean = value ? 1 : 0;
     } else if (key == "sample_polls") {
         if (value < 0 || value > 1 << 20) return TOPK_ERR_INVALID;
         ctx->tune.sample_polls = (uint32_t)value;

@@ -1972,13 +1972,13 @@ void batch_free(topk_ctx *ctx) {
 }
 
 template <class T>
-static int grow_dev(T *&p, uint64_t &cap, uint64_t need, bool &changed) {
+static int grow_dev(topk_ctx *ctx, T *&p, uint64_t &cap, uint64_t need, bool &changed) {
     if (need <= cap) return TOPK_OK;
     hipFree(p);
     p = nullptr;
     cap = 0;
     changed = true;
-    if (hipMalloc(&p, sizeof(T) * need) != hipSuccess) return TOPK_ERR_NOMEM;
+    if (ctx_malloc(ctx, &p, sizeof(T) * need) != hipSuccess) return TOPK_ERR_NOMEM;
     cap = need;
     return TOPK_OK;
 }
@@ -2028,9 +2028,9 @@ static int ensure(topk_ctx *ctx, BatchState &B, uint32_t nq, uint32_t ks, int si
         H.d_flist = nullptr;
         H.nq_cap = 0;
         changed = true;
-        TK_HIP(hipMalloc(&H.d_flist, sizeof(unsigned int) * (cap + 1)));
-        TK_HIP(hipMalloc(&H.d_ccount, sizeof(unsigned int) * cap));
-        TK_HIP(hipMalloc(&H.d_cand, sizeof(uint64_t) * BATCH_CAP * cap));
+        TK_HIP(ctx_malloc(ctx, &H.d_flist, sizeof(unsigned int) * (cap + 1)));
+        TK_HIP(ctx_malloc(ctx, &H.d_ccount, sizeof(unsigned int) * cap));
+        TK_HIP(ctx_malloc(ctx, &H.d_cand, sizeof(uint64_t) * BATCH_CAP * cap));
         H.nq_cap = cap;
     }
     if (in_need > H.din_cap) {
@@ -2038,7 +2038,7 @@ static int ensure(topk_ctx *ctx, BatchState &B, uint32_t nq, uint32_t ks, int si
         H.d_in = nullptr;
         H.din_cap = 0;
         changed = true;
-        TK_HIP(hipMalloc(&H.d_in, in_need));
+        TK_HIP(ctx_malloc(ctx, &H.d_in, in_need));
         H.din_cap = in_need;
     }
     if (out_need > H.dout_cap) {
@@ -2046,7 +2046,7 @@ static int ensure(topk_ctx *ctx, BatchState &B, uint32_t nq, uint32_t ks, int si
         H.d_out = nullptr;
         H.dout_cap = 0;
         changed = true;
-        TK_HIP(hipMalloc(&H.d_out, out_need));
+        TK_HIP(ctx_malloc(ctx, &H.d_out, out_need));
         H.dout_cap = out_need;
     }
     if (in_need > H.in_cap) {
@@ -2069,10 +2069,10 @@ static int ensure(topk_ctx *ctx, BatchState &B, uint32_t nq, uint32_t ks, int si
     // slot i runs on pipeline lane i's stream: no streams beyond the
     // context's, so the two slots keep hardware queues of their own
     H.stream = ctx->lane[si].stream;
-    rc = grow_dev(H.d_plist, H.plist_cap, (uint64_t)L * nq, changed);
-    if (!rc) rc = grow_dev(H.d_pcnt, H.pcnt_cap, (uint64_t)L, changed);
+    rc = grow_dev(ctx, H.d_plist, H.plist_cap, (uint64_t)L * nq, changed);
+    if (!rc) rc = grow_dev(ctx, H.d_pcnt, H.pcnt_cap, (uint64_t)L, changed);
     // chunks >= ITEM_MIN_OBJECTS objects
-    if (!rc) rc = grow_dev(H.d_items, H.item_cap, items_need, changed);
+    if (!rc) rc = grow_dev(ctx, H.d_items, H.item_cap, items_need, changed);
     if (rc) return rc;
     {
         const uint32_t units = nq * BQ_MAX_S;
@@ -2083,7 +2083,7 @@ static int ensure(topk_ctx *ctx, BatchState &B, uint32_t nq, uint32_t ks, int si
             changed = true;
         }
         if (te) {
-            rc = grow_dev(H.d_tasks, H.tasks_cap, te, changed);
+            rc = grow_dev(ctx, H.d_tasks, H.tasks_cap, te, changed);
             if (!rc && units > H.unit_cap) {
                 hipFree(H.d_ucnt);
                 hipFree(H.d_uoff);
@@ -2091,8 +2091,8 @@ static int ensure(topk_ctx *ctx, BatchState &B, uint32_t nq, uint32_t ks, int si
                 H.d_uoff = nullptr;
                 H.unit_cap = 0;
                 changed = true;
-                TK_HIP(hipMalloc(&H.d_ucnt, sizeof(uint2) * units));
-                TK_HIP(hipMalloc(&H.d_uoff, sizeof(uint32_t) * (units + 1)));
+                TK_HIP(ctx_malloc(ctx, &H.d_ucnt, sizeof(uint2) * units));
+                TK_HIP(ctx_malloc(ctx, &H.d_uoff, sizeof(uint32_t) * (units + 1)));
                 H.unit_cap = units;
             }
             if (rc) return rc;
@@ -2100,8 +2100,8 @@ static int ensure(topk_ctx *ctx, BatchState &B, uint32_t nq, uint32_t ks, int si
     }
     if (!H.d_ctr) {
         changed = true;
-        TK_HIP(hipMalloc(&H.d_ctr, sizeof(unsigned int) * BCTR_WORDS));
-        TK_HIP(hipMalloc(&H.d_scored, sizeof(unsigned long long) * 2 * BATCH_MAX_GRID));
+        TK_HIP(ctx_malloc(ctx, &H.d_ctr, sizeof(unsigned int) * BCTR_WORDS));
+        TK_HIP(ctx_malloc(ctx, &H.d_scored, sizeof(unsigned long long) * 2 * BATCH_MAX_GRID));
     }
     if (!B.cus) {
         TK_HIP(hipDeviceGetAttribute(&B.cus, hipDeviceAttributeMultiprocessorCount, ctx->device));

@@ -699,8 +699,8 @@ int topk_bta(topk_ctx *ctx, uint32_t k, uint8_t qq, const float *weights, const 
         hipFree(A.bta[1]);
         A.bta[0] = A.bta[1] = nullptr;
         A.bta_cap = 0;
-        TK_HIP(hipMalloc(&A.bta[0], sizeof(uint64_t) * need));
-        TK_HIP(hipMalloc(&A.bta[1], sizeof(uint64_t) * need));
+        TK_HIP(ctx_malloc(ctx, &A.bta[0], sizeof(uint64_t) * need));
+        TK_HIP(ctx_malloc(ctx, &A.bta[1], sizeof(uint64_t) * need));
         A.bta_cap = need;
     }
     hipStream_t s = ctx->stream;
@@ -765,8 +765,8 @@ int topk_gpa(topk_ctx *ctx, uint32_t k, uint8_t qq, const float *weights, const 
         }
         A.gcap = 0;
         for (int b = 0; b < 2; b++) {
-            TK_HIP(hipMalloc(&A.gids[b], sizeof(uint32_t) * n));
-            TK_HIP(hipMalloc(&A.gs[b], sizeof(float) * n));
+            TK_HIP(ctx_malloc(ctx, &A.gids[b], sizeof(uint32_t) * n));
+            TK_HIP(ctx_malloc(ctx, &A.gs[b], sizeof(float) * n));
         }
         A.gcap = n;
     }

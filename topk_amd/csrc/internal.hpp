@@ -76,6 +76,7 @@ inline uint32_t id_shards(uint64_t n) { return n >= ID_LIMIT ? (uint32_t)((n + I
 // Launch-shape knobs (set by topk_set_tuning / the autotuner).
 struct Tuning {
     uint32_t stream_grid = 0;   // 0: default grid cap
+    int init_lean = 0;          // 1: layout builds take the least memory
     uint32_t sample_polls = 0;  // 0: default tries for the shared sample
     int stream_vpt = 0;         // float4 vectors per lane per column in a stream tile (0: by width)
     int fte_force_exact = 0;    // 1: skip the sample seed (testing / comparison)
@@ -364,6 +365,19 @@ void batch_free(topk_ctx *ctx);
 void aux_free(topk_ctx *ctx);
 int pta_build(topk_ctx *ctx);
 void pta_release(topk_ctx *ctx);
+void pta_trim(topk_ctx *ctx);
+// hipMalloc for a context: out of memory, the scratch that a layout build kept
+// for the next one is given back first.
+template <class T>
+inline hipError_t ctx_malloc(topk_ctx *ctx, T **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && ctx->pta.scratch) {
+        (void)hipGetLastError();
+        pta_trim(ctx);
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
 int pta_extreme_bits(topk_ctx *ctx);
 
 // Event bracketing for topk_timing_*.

@@ -495,7 +495,7 @@ struct AssignArgs {
     uint32_t d, dp, L;
     const KdNode *nodes;
     int tree_lds;         // the tree fits in LDS
-    uint2 *place;         // leaf and rank of each object
+    uint2 *place;         // leaf and rank of each object (null: not kept)
     uint32_t *cnt;        // objects per leaf
     // counted in LDS (else null): per workgroup and leaf, what added to the
     // leaf's offset and an index in leaf order gives the position; the range
@@ -503,6 +503,9 @@ struct AssignArgs {
     uint32_t *base;
     uint2 *order;
     float *rows;
+    // without place: ids to their partitions (cnt then counts them again)
+    const uint32_t *poff;
+    uint32_t *pid;
 };
 
 // Dynamic LDS: d x PA_BS attribute values (a lane reads its own column of
@@ -553,7 +556,9 @@ __global__ __launch_bounds__(PA_BS) void pta_assign_kernel(AssignArgs a) {
             lo += left ? 0u : nleft;
             nl = left ? nleft : nl - nleft;
         }
-        a.place[i] = make_uint2(lo, a.base ? atomicAdd(&h[lo], 1u) : atomicAdd(&a.cnt[lo], 1u));
+        const uint32_t r = a.base ? atomicAdd(&h[lo], 1u) : atomicAdd(&a.cnt[lo], 1u);
+        if (a.place) a.place[i] = make_uint2(lo, r);
+        else if (a.pid) a.pid[a.poff[lo] + r] = (uint32_t)i;
     }
     if (!a.base) return;
     __syncthreads();
@@ -934,7 +939,8 @@ __global__ __launch_bounds__(256) void pta_tail_kernel(uint64_t npos, uint64_t l
 }
 
 // ---- stores with a partition past PTA_SORT_MAX objects, or no room for the
-//      scattered rows: the same layout by separate passes ----
+//      scattered rows or for anything per object: the same layout by separate
+//      passes ----
 
 // Sorts each partition's keys, largest first (over PTA_SORT_MAX: as scattered).
 __global__ __launch_bounds__(1024) void pta_sort_kernel(const uint32_t *__restrict__ poff,
@@ -952,13 +958,40 @@ __global__ __launch_bounds__(1024) void pta_sort_kernel(const uint32_t *__restri
     for (uint32_t i = threadIdx.x; i < s; i += 1024) seg[i] = a[i];
 }
 
+// The same for ids without their keys: the attribute sums are gathered.
+__global__ __launch_bounds__(1024) void pta_sort_ids_kernel(const float *__restrict__ cols, uint64_t ld, uint32_t d,
+                                                            const uint32_t *__restrict__ poff,
+                                                            const uint32_t *__restrict__ psz,
+                                                            uint32_t *__restrict__ pid) {
+    __shared__ uint64_t a[PTA_SORT_MAX];
+    const uint32_t p = blockIdx.x, s = psz[p];
+    if (s < 2 || s > PTA_SORT_MAX) return;
+    uint32_t *seg = pid + poff[p];
+    uint32_t n2 = 1;
+    while (n2 < s) n2 <<= 1;
+    for (uint32_t i = threadIdx.x; i < n2; i += 1024) {
+        uint64_t key = 0;
+        if (i < s) {
+            const uint32_t id = seg[i];
+            float sum = 0.0f;  // attribute sum, in attribute order
+            for (uint32_t m = 0; m < d; m++) sum += cols[(uint64_t)m * ld + id];
+            key = rkey(sum, id);
+        }
+        a[i] = key;
+    }
+    __syncthreads();
+    bitonic_sort_desc<1024>(a, n2);
+    for (uint32_t i = threadIdx.x; i < s; i += 1024) seg[i] = rkey_id(a[i]);
+}
+
+// keys null: the ids are in pid[].
 __global__ void pta_gather_kernel(const float *__restrict__ cols, uint64_t ld, uint32_t d, uint64_t npos,
                                   const uint64_t *__restrict__ keys, float *__restrict__ pcols, uint64_t ldp,
                                   uint32_t *__restrict__ pid) {
     const uint64_t pos = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (pos >= npos) return;
-    const uint32_t id = rkey_id(keys[pos]);  // key 0: no object, id 0xFFFFFFFF
-    pid[pos] = id;
+    const uint32_t id = keys ? rkey_id(keys[pos]) : pid[pos];  // key 0: no object, id 0xFFFFFFFF
+    if (keys) pid[pos] = id;
     for (uint32_t m = 0; m < d; m++) pcols[(uint64_t)m * ldp + pos] = id != 0xFFFFFFFFu ? cols[(uint64_t)m * ld + id] : 0.0f;
 }
 
@@ -1221,6 +1254,13 @@ void pta_stale(topk_ctx *ctx) {
     pta_forget(ctx->pta, true);
 }
 
+// Gives back the scratch a build left for the next one.
+void pta_trim(topk_ctx *ctx) {
+    hipFree(ctx->pta.scratch);
+    ctx->pta.scratch = nullptr;
+    ctx->pta.scratch_cap = 0;
+}
+
 // Room for `need` bytes at p (cap bytes so far), whose contents may go.
 static int pta_room(unsigned char *&p, size_t &cap, size_t need) {
     if (need <= cap) return TOPK_OK;
@@ -1323,7 +1363,9 @@ static int kd_enqueue(const KdPlan &plan, hipStream_t s, const KdSeg *d_segs, co
 // A rebuild reuses the memory of the layout it replaces, and the scratch of
 // the build before if that is at most PTA_KEEP_SCRATCH: device memory freed
 // and allocated again at the pace of the build (1.5 GB in 3 ms) ends in the
-// driver's clearing of freed pages, which stalled builds for up to seconds.
+// driver's clearing of freed pages, which stalled builds for up to seconds.  An
+// allocation of the context that finds no room takes the scratch back
+// (ctx_malloc).
 constexpr size_t PTA_KEEP_SCRATCH = 4ull << 30;
 
 int pta_build(topk_ctx *ctx) {
@@ -1365,18 +1407,20 @@ int pta_build(topk_ctx *ctx) {
     as.dp = dp;
     as.L = L;
 
-    // the layout's own arrays, sized for the most padding
-    const uint64_t npos_max = (n + (uint64_t)(PART_ALIGN - 1) * L + 8191) / 8192 * 8192;
+    // the layout's own arrays, for npos positions (before they are counted: the
+    // most padding)
+    uint64_t npos_room = (n + (uint64_t)(PART_ALIGN - 1) * L + 8191) / 8192 * 8192;
     uint32_t p2 = 1;
     while (p2 < L) p2 <<= 1;
-    const size_t nn = 2 * (size_t)p2, nchunks_max = npos_max / PTA_CHUNK;
+    const size_t nn = 2 * (size_t)p2;
     P.crow = 2 * d + 2;
     auto own = [&](unsigned char *p) {
+        const size_t nchunks = npos_room / PTA_CHUNK;
         Carve c;
         c.base = p;
-        c.take(P.pid, npos_max);
-        c.take(P.cstat, nchunks_max * P.crow);
-        c.take(P.cminid, nchunks_max);
+        c.take(P.pid, npos_room);
+        c.take(P.cstat, nchunks * P.crow);
+        c.take(P.cminid, nchunks);
         c.take(P.poff, L + 1);
         c.take(P.psz, L);
         c.take(P.pmax, (size_t)L * d);
@@ -1395,20 +1439,31 @@ int pta_build(topk_ctx *ctx) {
         c.take(P.tminid, nn);
         return c.at;
     };
+    auto room = [&]() {
+        int rc = pta_room(P.arena, P.arena_cap, own(nullptr));
+        unsigned char *pc = reinterpret_cast<unsigned char *>(P.pcols);
+        if (!rc) rc = pta_room(pc, P.pcols_cap, sizeof(float) * (npos_room * d + 8192));
+        P.pcols = reinterpret_cast<float *>(pc);
+        if (!rc) own(P.arena);
+        return rc;
+    };
     // scratch of the build in one piece.  The rows in object order may lie in
     // the columns' memory, which is written after their last use; without
-    // room for the scattered rows the columns are gathered by id instead.
-    const size_t pcols_floats = npos_max * d + 8192;
-    const bool rows_in_pcols = n * dp <= pcols_floats;
+    // room for the scattered rows the columns are gathered by id instead, and
+    // without room for anything per object (24 bytes of it) the tree is walked
+    // twice, the arrays are sized after the first walk has counted, and the
+    // columns are read once more for the sums: no more memory at any time than
+    // the store, the layout and the sample.
+    const bool rows_in_pcols = n * dp <= npos_room * d + 8192;
     float *rows = nullptr, *own_rows = nullptr, *srows = nullptr;
-    uint32_t *idx = nullptr, *idx2 = nullptr, *val = nullptr;
+    uint32_t *idx = nullptr, *idx2 = nullptr, *val = nullptr, *off = nullptr, *sz = nullptr;
     KdState *states = nullptr;
     uint2 *share_cnt = nullptr;
     KdNode *nodes = nullptr;
     KdSeg *segs = nullptr, *subs = nullptr;
     KdShare *shares = nullptr;
     uint64_t *keys = nullptr;
-    bool with_rows = true;
+    bool with_rows = true, lean = ctx->tune.init_lean != 0;
     auto carve = [&](unsigned char *p) {
         Carve c;
         c.base = p;
@@ -1418,37 +1473,43 @@ int pta_build(topk_ctx *ctx) {
         c.take(val, ns);
         c.take(states, plan.max_seg);
         c.take(share_cnt, plan.max_share);
-        c.take(nodes, L);
         c.take(segs, plan.segs.size());
         c.take(shares, plan.shares.size());
         c.take(subs, plan.subs.size());
+        c.take(nodes, L);
         c.take(as.cnt, L);
-        c.take(as.place, n);
-        c.take(as.base, counted ? (size_t)groups * L : 0);
-        c.take(as.order, counted ? n : 0);
-        c.take(keys, npos_max);
-        c.take(own_rows, with_rows && counted && !rows_in_pcols ? n * dp : 0);
-        c.take(srows, with_rows ? npos_max * dp : 0);
+        c.take(off, lean ? L + 1 : 0);
+        c.take(sz, lean ? L : 0);
+        c.take(as.place, lean ? 0 : n);
+        c.take(as.base, counted && !lean ? (size_t)groups * L : 0);
+        c.take(as.order, counted && !lean ? n : 0);
+        c.take(keys, lean ? 0 : npos_room);
+        c.take(own_rows, with_rows && counted && !lean && !rows_in_pcols ? n * dp : 0);
+        c.take(srows, with_rows && !lean ? npos_room * dp : 0);
         return c.at;
     };
-    int rc = pta_room(P.arena, P.arena_cap, own(nullptr));
-    if (!rc) {
-        unsigned char *pc = reinterpret_cast<unsigned char *>(P.pcols);
-        rc = pta_room(pc, P.pcols_cap, sizeof(float) * pcols_floats);
-        P.pcols = reinterpret_cast<float *>(pc);
+    int rc = lean ? TOPK_ERR_NOMEM : room();
+    if (!rc && pta_room(P.scratch, P.scratch_cap, carve(nullptr))) {
+        with_rows = false;
+        rc = pta_room(P.scratch, P.scratch_cap, carve(nullptr));
     }
-    if (!rc && with_rows && pta_room(P.scratch, P.scratch_cap, carve(nullptr))) with_rows = false;
-    if (!rc && !with_rows) rc = pta_room(P.scratch, P.scratch_cap, carve(nullptr));
+    if (rc) {
+        pta_forget(P, false);
+        P.crow = 2 * d + 2;
+        lean = true;
+        with_rows = false;
+        rc = pta_room(P.scratch, P.scratch_cap, carve(nullptr));
+    }
     if (rc) {
         pta_forget(P, false);
         return rc;
     }
-    own(P.arena);
     carve(P.scratch);
-    if (!counted) {
+    if (!counted || lean) {
         as.base = nullptr;
         as.order = nullptr;
     }
+    if (lean) as.place = nullptr;
     as.nodes = nodes;
     as.rows = !with_rows || !counted ? nullptr : (rows_in_pcols ? P.pcols : own_rows);
 #define TK_TRY(call)                                              \
@@ -1472,7 +1533,8 @@ int pta_build(topk_ctx *ctx) {
         // 3: leaves
         TK_TRY(hipMemsetAsync(as.cnt, 0, sizeof(uint32_t) * L, s));
         hipLaunchKernelGGL(pta_assign_kernel, dim3(groups), dim3(PA_BS), lds, s, as);
-        hipLaunchKernelGGL(pta_offsets_kernel, dim3(1), dim3(1024), 0, s, as.cnt, L, P.poff, P.psz, P.h_report);
+        hipLaunchKernelGGL(pta_offsets_kernel, dim3(1), dim3(1024), 0, s, as.cnt, L, lean ? off : P.poff,
+                           lean ? sz : P.psz, P.h_report);
         TK_TRY(hipGetLastError());
         TK_TRY(hipStreamSynchronize(s));
         const uint64_t npos = *reinterpret_cast<volatile uint64_t *>(P.h_report);
@@ -1484,16 +1546,31 @@ int pta_build(topk_ctx *ctx) {
         P.ld = (npos + 8191) / 8192 * 8192;
         P.nchunks = npos / PTA_CHUNK;
         P.p2 = p2;
+        if (lean) {
+            npos_room = P.ld;
+            rc = room();
+            if (rc) goto fail;
+            TK_TRY(hipMemcpyAsync(P.poff, off, sizeof(uint32_t) * (L + 1), hipMemcpyDeviceToDevice, s));
+            TK_TRY(hipMemcpyAsync(P.psz, sz, sizeof(uint32_t) * L, hipMemcpyDeviceToDevice, s));
+        }
         // 4, 5: objects to their partitions, the partitions in order
         const bool fused = with_rows && P.maxsz <= PTA_SORT_MAX;
-        if (!fused) TK_TRY(hipMemsetAsync(keys, 0, sizeof(uint64_t) * P.ld, s));
-        if (P.maxsz > PTA_SORT_MAX && counted) {
+        if (!fused && !lean) TK_TRY(hipMemsetAsync(keys, 0, sizeof(uint64_t) * P.ld, s));
+        if (P.maxsz > PTA_SORT_MAX && as.base) {
             hipLaunchKernelGGL(pta_recount_kernel, dim3(groups), dim3(PA_BS), sizeof(uint32_t) * L, s, as);
             hipLaunchKernelGGL(pta_base_kernel, dim3((L + 255) / 256), dim3(256), 0, s, as.base, L, groups);
             as.order = nullptr;
         }
-        hipLaunchKernelGGL(pta_scatter_kernel, dim3((uint32_t)std::min<uint64_t>(16, (as.per + 255) / 256), groups),
-                           dim3(256), 0, s, as, P.poff, keys, fused ? srows : (float *)nullptr);
+        if (lean) {
+            TK_TRY(hipMemsetAsync(as.cnt, 0, sizeof(uint32_t) * L, s));
+            TK_TRY(hipMemsetAsync(P.pid, 0xFF, sizeof(uint32_t) * P.ld, s));
+            as.poff = P.poff;
+            as.pid = P.pid;
+            hipLaunchKernelGGL(pta_assign_kernel, dim3(groups), dim3(PA_BS), lds, s, as);
+        } else {
+            hipLaunchKernelGGL(pta_scatter_kernel, dim3((uint32_t)std::min<uint64_t>(16, (as.per + 255) / 256), groups),
+                               dim3(256), 0, s, as, P.poff, keys, fused ? srows : (float *)nullptr);
+        }
         if (fused) {
             const uint32_t cap = (std::max(P.maxsz, 1u) + 255) / 256 * 256;
             const PartOut po{P.pcols, P.ld, P.pid, P.nchunks, P.cstat, P.cminid, P.pmax, P.pmin, P.psum, P.pminsum};
@@ -1501,10 +1578,13 @@ int pta_build(topk_ctx *ctx) {
                                keys, srows, d, dp, P.poff, P.psz, cap, po);
             hipLaunchKernelGGL(pta_tail_kernel, dim3(32), dim3(256), 0, s, P.npos, P.ld, d, P.pcols, P.pid);
         } else {
-            hipLaunchKernelGGL(pta_sort_kernel, dim3(L), dim3(1024), 0, s, P.poff, P.psz, keys);
+            if (lean)
+                hipLaunchKernelGGL(pta_sort_ids_kernel, dim3(L), dim3(1024), 0, s, ctx->cols, ctx->ld, d, P.poff, P.psz,
+                                   P.pid);
+            else hipLaunchKernelGGL(pta_sort_kernel, dim3(L), dim3(1024), 0, s, P.poff, P.psz, keys);
             TK_TRY(hipMemsetAsync(P.pcols + P.ld * d, 0, sizeof(float) * 8192, s));
             hipLaunchKernelGGL(pta_gather_kernel, dim3((uint32_t)((P.ld + 255) / 256)), dim3(256), 0, s, ctx->cols,
-                               ctx->ld, d, P.ld, keys, P.pcols, P.ld, P.pid);
+                               ctx->ld, d, P.ld, lean ? (const uint64_t *)nullptr : keys, P.pcols, P.ld, P.pid);
             hipLaunchKernelGGL(pta_bounds_kernel, dim3(L), dim3(PB_BS), 0, s, P.pcols, P.ld, d, P.poff, P.psz, P.pmax,
                                P.pmin, P.psum, P.pminsum);
             if (P.nchunks) {
@@ -1526,11 +1606,7 @@ int pta_build(topk_ctx *ctx) {
         TK_TRY(hipStreamSynchronize(s));
     }
 #undef TK_TRY
-    if (P.scratch_cap > PTA_KEEP_SCRATCH) {
-        hipFree(P.scratch);
-        P.scratch = nullptr;
-        P.scratch_cap = 0;
-    }
+    if (lean || P.scratch_cap > PTA_KEEP_SCRATCH) pta_trim(ctx);
     P.built = true;
     P.tt_build_ms = now_ms() - t0;
     return TOPK_OK;
@@ -1569,7 +1645,7 @@ int pta_extreme_bits(topk_ctx *ctx) {
     if (!P.built) return TOPK_ERR_STATE;
     if (P.xbits) return TOPK_OK;
     const uint64_t nw = ((ctx->n + 63) / 64 + 15) & ~15ull;  // padding words hold ids >= n: zero
-    TK_HIP(hipMalloc(&P.xbits, sizeof(uint64_t) * 2 * ctx->d * nw));
+    TK_HIP(ctx_malloc(ctx, &P.xbits, sizeof(uint64_t) * 2 * ctx->d * nw));
     P.nw = nw;
     const uint64_t waves = (uint64_t)ctx->d * nw;
     const uint32_t grid = (uint32_t)std::min<uint64_t>((waves + 3) / 4, 65536);
