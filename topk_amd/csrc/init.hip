@@ -214,6 +214,14 @@ static double now_ms() {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 
+// Queries queued on the lanes read the store that is about to change.  (A
+// layout's hipFree used to wait for them; a rebuild frees nothing.)
+static int lanes_wait(topk_ctx *ctx) {
+    for (int i = 0; i < NUM_LANES; i++)
+        if (ctx->lane[i].stream) TK_HIP(hipStreamSynchronize(ctx->lane[i].stream));
+    return TOPK_OK;
+}
+
 extern "C" {
 
 int topk_init(topk_ctx *ctx, uint32_t flags) {
@@ -226,6 +234,8 @@ int topk_init(topk_ctx *ctx, uint32_t flags) {
         // reuses its memory
         if (flags & TOPK_INIT_PTA) pta_stale(ctx);
         else pta_release(ctx);
+        rc = lanes_wait(ctx);
+        if (rc) return rc;
         ctx->store_gen++;
         rc = normalize_store(ctx);
         if (rc) {
@@ -250,6 +260,8 @@ int topk_set_partition_size(topk_ctx *ctx, uint32_t objects) {
 int topk_reorder_attr(topk_ctx *ctx) {
     if (!ctx) return TOPK_ERR_INVALID;
     pta_release(ctx);
+    const int rc = lanes_wait(ctx);
+    if (rc) return rc;
     ctx->store_gen++;
     hipEvent_t ev0 = nullptr;
     timing_begin(ctx, ctx->stream, ev0);
