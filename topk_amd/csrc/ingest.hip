@@ -575,7 +575,8 @@ struct CsvText {
         hipFree(mem[1]);
     }
 
-    int load(const char *path, hipStream_t s) {
+    // want: rows that parse will be asked for at most (0: all of the text's).
+    int load(const char *path, hipStream_t s, uint64_t want) {
         st = s;
         int rc = f.open(path);
         if (rc) return rc;
@@ -594,22 +595,24 @@ struct CsvText {
         rc = io.init(st, f.size);
         if (!rc) rc = io.upload(f.fd, 0, f.size, text);
         if (rc) return rc;
+        IK_HIP(hipStreamSynchronize(st));
+        ms_read = ms_since(t0);
+        t0 = std::chrono::steady_clock::now();
         hipLaunchKernelGGL(csv_count_kernel, dim3((uint32_t)ntiles), dim3(CSV_BS), 0, st, (const uint4 *)text,
                            tile_nl);
         hipLaunchKernelGGL(csv_scan_kernel, dim3(1), dim3(CSV_SCAN_BS), 0, st, tile_nl, ntiles, tile_base);
         IK_HIP(hipGetLastError());
-        IK_HIP(hipStreamSynchronize(st));
-        ms_read = ms_since(t0);
-        t0 = std::chrono::steady_clock::now();
         rc = io.word(tile_base + ntiles, nl);
         if (rc) return rc;
         // lines: nl terminated ones plus the text after the last newline
         groups = (nl + 1 + CSV_BS - 1) / CSV_BS;
-        // slow (nl + 1) | ends (nl + 1) | row_base (groups + 1) | nslow | grp (groups)
-        if (hipMalloc(&mem[1], 24 * (nl + 1) + 8 * (groups + 2) + 4 * groups) != hipSuccess) return TOPK_ERR_NOMEM;
+        // slow (a row each) | ends (nl + 1) | row_base (groups + 1) | nslow | grp (groups)
+        const uint64_t most = want ? std::min(want, nl + 1) : nl + 1;
+        if (hipMalloc(&mem[1], sizeof(CsvSlow) * most + 8 * (nl + 1) + 8 * (groups + 2) + 4 * groups) != hipSuccess)
+            return TOPK_ERR_NOMEM;
         static_assert(sizeof(CsvSlow) == 16, "slow lines lead the block");
         slow = reinterpret_cast<CsvSlow *>(mem[1]);
-        ends = reinterpret_cast<uint64_t *>(slow + nl + 1);
+        ends = reinterpret_cast<uint64_t *>(slow + most);
         row_base = ends + nl + 1;
         nslow = reinterpret_cast<unsigned long long *>(row_base + groups + 1);
         uint32_t *grp = reinterpret_cast<uint32_t *>(nslow + 1);
@@ -789,7 +792,7 @@ static int load_text(topk_ctx *ctx, const char *path, uint64_t n, uint32_t d, to
     if (rc) return rc;
     {
         CsvText t;  // released (its stream drained) before the stream is destroyed
-        rc = t.load(path, ls);
+        rc = t.load(path, ls, n);
         if (!rc) rc = csv_shape(t, n, d);
         if (!rc) {
             ctx->n = n;
@@ -880,7 +883,7 @@ int topk_csv_read(const char *path, uint64_t n, uint32_t d, uint32_t flags, floa
     uint64_t slow = 0;
     double ms_parse = 0;
     CsvText *t = new CsvText();
-    rc = t->load(path, st);
+    rc = t->load(path, st, n);
     if (!rc) rc = csv_shape(*t, n, d);
     if (!rc && hipMalloc(&dout, sizeof(float) * n * d) != hipSuccess) rc = TOPK_ERR_NOMEM;
     if (!rc) {
