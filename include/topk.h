@@ -255,7 +255,9 @@ int topk_batch_wait(topk_ctx *ctx, uint64_t ticket);
  * per CU), query budget per work item and select digit width, and installs
  * the fastest in the context (as topk_set_tuning would). */
 typedef struct topk_batch_tuning {
-    uint32_t vpt, bs, qpi, digit, grid, item;
+    uint32_t vpt, bs;
+    uint32_t qpi;                /* 64 also where the budget goes by the entries of each batch (batch_qpi 0) */
+    uint32_t digit, grid, item;
     uint32_t variants;           /* shapes timed */
     double ms_best, ms_default;  /* device time of one batch: chosen / defaults */
     uint32_t fused;              /* 1: the query-major fused pass was chosen (batch_fused 2) */

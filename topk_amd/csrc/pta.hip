@@ -17,7 +17,7 @@
 //    rounded up to binary32.  It is never below an object's score.
 //  * query: bound keys for all partitions; the exact k-th key among the best
 //    partitions' objects (seed) is a proven lower bound tau of the global
-//    k-th key; the task pass lists the partitions whose bound reaches tau's
+//    k-th key; the cut pass finds the partitions whose bound reaches tau's
 //    score (skip iff bound < tau strictly), each up to its first suffix row
 //    whose bound falls below tau, as chunk ranges; the scoring pass spreads
 //    those chunks evenly over every wave of the GPU and keeps keys >= tau;
@@ -529,8 +529,8 @@ __global__ __launch_bounds__(STREAM_BS) void pta_score_kernel(QCols q, uint32_t 
 // ---------------------------------------------------------------------------
 // host: query
 // ---------------------------------------------------------------------------
-// bound -> seed -> chunk tasks -> chunk scoring -> final select, all on the
-// context's stream; fo points at pinned host memory, so the caller only
+// Four launches on the context's stream: bound, seed, cut, and scoring, whose
+// last workgroup selects; fo points at pinned host memory, so the caller only
 // synchronises.
 int pta_query(topk_ctx *ctx, uint32_t k, uint8_t qq, const float *weights, const uint8_t *attr, const FinalOut &fo) {
     PtaLayout &P = ctx->pta;
