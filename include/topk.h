@@ -342,8 +342,8 @@ int topk_fte_async(topk_ctx *ctx, uint32_t k, uint8_t qq, const float *weights, 
  * device memory in the call (code under HIP graph capture, serving loops,
  * harnesses that forbid hipMalloc).  No context: column m of the store is at
  * d_cols + m*ld (ld >= n, a multiple of 4; d_cols 16-byte aligned), and the
- * buffer must hold d*ld + 8192 floats, since stream tiles read up to 8191
- * values past a column's n-th (ignored).  The same results as topk_fte
+ * buffer must hold d*ld + 8192 floats: up to 8191 values past a column's n-th
+ * may be read (ignored).  The same results as topk_fte
  * (best first into d_ids / d_scores, k entries; d_threshold may be NULL),
  * written to device memory; *d_status (device) becomes TOPK_OK, or
  * TOPK_ERR_OVERFLOW when more than 2^20 candidates beat even the exact

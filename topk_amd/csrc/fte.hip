@@ -456,7 +456,7 @@ struct StreamArgs {
 //
 // One workgroup of 16 waves per CU holds 8 or more loads of 16 bytes per lane
 // in flight, which is all HBM needs (512 to 3072 workgroups of 256 threads
-// stream at the same 6.7 TB/s), leaves few arrivals at the end and 1024
+// stream at the same 6.8 TB/s), leaves few arrivals at the end and 1024
 // threads to the select.  Of two workgroups on a CU the older one goes
 // first: two of 512 threads per CU ended between 203 and 334 us at N = 2^26.
 //
@@ -465,13 +465,15 @@ struct StreamArgs {
 // tile before is processed (device atomics on one address serialise at
 // about 20 ns, so only the last ones).
 //
-// Bound by HBM above a few million objects (6.9 TB/s at N = 2^26, m = 8),
-// by the chain of launch, sample, arrival and select below.  A synchronous
-// call, before (seed, stream and select launches, two result copies) and
-// now: 16k objects 50 -> 35 us, 2^20 65 -> 39, 8M x 7 divided 114 -> 78, 4.2M
-// x 20 with k = 1000 245 -> 106, 2^26 x 8 373 -> 349; 32 queued queries of
-// 16M x 5 1945 -> 1807.  At 2^20 tau is known after 10 us, the last
-// workgroup arrives at 13 and has selected at 19.
+// Bound by HBM above a few million objects: at N = 2^26, m = 8 the launch takes
+// 332.7 us on average under a kernel trace (6.45 TB/s with its sample and
+// select; as launches of their own sample, stream and select took 13.8 + 317.2
+// + 17.5), and two queries in flight hide those, 6.9 TB/s.  Below, by the chain
+// of launch, sample, arrival and select.  A synchronous call, before (three
+// launches, two result copies) and now: 16k objects 50.7 -> 34.0 us, 2^20 x 4
+// 64.0 -> 36.2, 8M x 7 divided 115 -> 78, 4.2M x 20 with k = 1000 223 -> 107,
+// 2^26 x 8 374 -> 344; 32 queued queries of 16M x 5 1945 -> 1844.  At 2^20 tau is
+// known after 10 us, the last workgroup arrives at 13 and has selected at 19.
 //
 // The select runs in the last workgroup to finish.  Its inputs cross XCDs
 // without an L2 write-back per workgroup: candidates, counts and spilled

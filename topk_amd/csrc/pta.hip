@@ -248,9 +248,9 @@ __global__ __launch_bounds__(PTA_BS) void pta_seed_kernel(QCols q, const uint64_
 // each for the bounds.  The survivors are then cut four at a time, 16 lanes
 // each, one chunk row per lane (a 4096-object partition in one round).  The
 // group's cuts, chunk total and report go out without atomics; the scoring
-// pass scans the totals.  Bound by the chain of one wave's loads; one
-// workgroup per 16 partitions, most of which did not survive, took 11.5 us at
-// 65536 partitions, this 7.4.
+// pass scans the totals.  Bound by the chain of one wave's loads.  One
+// workgroup per 16 partitions, most of which did not survive, took 12.2 us on
+// average at 65536 partitions (9.2 at the least), this 11.0 (7.1).
 template <int NB>
 __global__ __launch_bounds__(PTA_BS) void pta_cut_kernel(BoundArgs b, uint32_t L, uint32_t R, uint32_t G,
                                                          const uint64_t *__restrict__ pbound,
@@ -330,8 +330,9 @@ __global__ __launch_bounds__(PTA_BS) void pta_cut_kernel(BoundArgs b, uint32_t L
 // candidate buffer (an LDS counter; past the slot, the shared spill region),
 // its count to cs.counts[workgroup]; the last workgroup selects, as the
 // plain stream's does.  One workgroup of 16 waves per CU keeps the arrivals
-// few and gives the select its threads; with four of 4 waves and a select
-// launch, scoring and select took 12 + 7 us at N = 2^28, now 14.2 together.
+// few and gives the select its threads: 22.6 us on average at N = 2^28 (17.5 at
+// the least), select included; with four of 4 waves scoring alone took 15.1
+// (12.7), and a select launch followed.
 // Workgroup 0 also reports the partitions and objects scored.
 struct ScoreSelect {
     uint32_t cap, kp2, k, kreq;
