@@ -35,10 +35,11 @@ int main() {
                     for (int vpt : {0, 1, 2, 4, 8})
                         for (uint32_t grid : {0u, 1u, 257u, MAX_STREAM_GRID}) {
                             const SeedPlan s = seed_plan(n, k, mode);
-                            const uint64_t first = s.tau == TAU_STATE ? s.n_eff : 0, pad = (n + 3) / 4 * 4;
+                            const uint64_t first = s.first, pad = (n + 3) / 4 * 4;
                             const bool big = mode == FTE_EXACT_BIG;
                             const StreamPlan p = stream_plan(n, first, m, big, vpt, grid, 1ull << 21);
                             // the stream: every object of [first, n), nothing past the column's last vector
+                            CHECK(first == 0 || (s.tau == TAU_STATE && first == s.n_eff), "n %llu", (unsigned long long)n);
                             CHECK(first + p.ntiles * p.tile >= n && (!p.ntiles || first % 4 == 0), "n %llu", (unsigned long long)n);
                             const uint32_t last = (uint32_t)((n - 1) / 4);
                             uint64_t most = 0;

@@ -119,3 +119,18 @@ def test_select_of_many_candidates(gpu, kind, n, k):
             assert np.array_equal(ids, rid) and np.array_equal(sc, rsc) and thr == rthr
         if kind.startswith("best"):
             assert eng.stats()["fallback"] == 0  # one run
+
+
+@pytest.mark.parametrize("n", [1, 4095, 100_003, 1 << 19])
+@pytest.mark.parametrize("k", [1, 31, 33, 163, 164, 256, 257, 1024])
+def test_queued_queries_on_small_stores(gpu, n, k):
+    # the prefix's top k listed by the seed, or the prefix streamed again
+    x = _store(n, 3)
+    w = np.array([0.5, -0.2, 1.0], np.float32)
+    rid, rsc, _ = oracle.fte_topk(x, n, k, w, [2, 0, 1])
+    with topk_amd.Engine(x) as eng:
+        ids, sc = _queue(eng, [(w, [2, 0, 1])] * 3, k)
+    c = rid.size  # min(k, n), then padding
+    for j in range(3):
+        assert np.array_equal(ids[j][:c], rid) and np.array_equal(sc[j][:c], rsc)
+        assert np.all(ids[j][c:] == np.uint64(0xFFFFFFFFFFFFFFFF)) and np.all(sc[j][c:] == -np.inf)

@@ -786,24 +786,21 @@ static CandSet fte_launch(const FteRun &r, uint32_t k, const QCols &q, const Fin
     const uint64_t n = r.n;
     hipStream_t s = r.s;
     const SeedPlan sp = seed_plan(n, k, mode);
-    const bool exact = sp.tau == TAU_STATE;
-    uint64_t *pre = exact ? r.pre : nullptr;
+    uint64_t *pre = sp.first ? r.pre : nullptr;
     // kernels unrolled for the query width, or the runtime-width ones (the
     // only ones that divide real-data scores)
     const uint32_t msw = q.div != 0.0f ? 0u : q.m;
 #define TK_SEED(MM)                                                                                              \
     hipLaunchKernelGGL((fte_seed_kernel<MM, SEED_TILE / SEED_BS>), dim3(sp.blocks), dim3(SEED_BS), 0, s, q, sp.n_eff, \
                        sp.stride, sp.ks, sp.total_valid, r.blk, pre, r.st, r.gate)
-    if (exact) TK_SWITCH_M(msw, TK_SEED);
+    if (sp.tau == TAU_STATE) TK_SWITCH_M(msw, TK_SEED);
 #undef TK_SEED
 
-    // exact mode streams only the objects after the prefix
-    const uint64_t first = exact ? sp.n_eff : 0;
-    const StreamPlan pl = stream_plan(n, first, q.m, r.big, r.vpt, r.grid_cap, r.cand_cap);
+    const StreamPlan pl = stream_plan(n, sp.first, q.m, r.big, r.vpt, r.grid_cap, r.cand_cap);
     const uint32_t g = pl.grid;
     StreamArgs a{};
     a.n = n;
-    a.obj_begin = first;
+    a.obj_begin = sp.first;
     a.ntiles = pl.ntiles;
     a.nstatic = pl.nstatic;
     a.st = r.st;

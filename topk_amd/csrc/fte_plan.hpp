@@ -141,6 +141,7 @@ struct SeedPlan {
     uint32_t W;            // winners per piece of the shared sample, or per wave of the own one
     uint64_t stride;       // objects between the chunks' first objects
     uint64_t n_eff;        // exact: objects of the prefix
+    uint64_t first;        // first object to stream: n_eff where the seed hands on the prefix's top k
     uint32_t total_valid;  // exact: keys the blocks deposit
     double expect;         // candidates expected
 };
@@ -148,7 +149,7 @@ struct SeedPlan {
 // FTE_SAMPLE may guess on any store (the caller re-runs a bad guess): every
 // object of a store that fits the select, the own sample up to 2^19 objects,
 // the shared sample above.  FTE_QUEUED guesses only above 2^19 objects:
-// nothing re-runs it.
+// nothing re-runs it; below, tau is the k-th key of the exact prefix.
 static inline SeedPlan seed_plan(uint64_t n, uint32_t k, int mode) {
     SeedPlan p{};
     if (mode == FTE_SAMPLE && n <= FUSE_CAP_MAX) {
@@ -179,6 +180,14 @@ static inline SeedPlan seed_plan(uint64_t n, uint32_t k, int mode) {
         p.stride = SEED_TILE;
         const uint64_t pre = (uint64_t)p.blocks * SEED_TILE;
         p.n_eff = n < pre ? n : pre;
+        // Queued: past 4096 seed winners or k = 256 the prefix is streamed
+        // again, with the select in the last stream workgroup, instead of
+        // listed by the seed's last workgroup (a search of all winners) and
+        // selected by a launch of its own.  Listed / streamed, us a query:
+        // 100,000 objects (25 blocks), k = 16 17.6 / 20.6, 100 21.6 / 23.2, 400
+        // 37.7 / 32.5, 1000 70.6 / 45.3; 2^19 (128 blocks), k = 16 29.6 / 34.7,
+        // 100 42.6 / 39.8; 5000, k = 1000 36.8 / 24.6.
+        p.first = mode != FTE_QUEUED || (k <= 256 && p.blocks * k <= 4096) ? p.n_eff : 0;
         p.ks = k;
         const uint64_t full = p.n_eff / SEED_TILE, rem = p.n_eff % SEED_TILE;
         p.total_valid = (uint32_t)(full * (k < SEED_TILE ? k : SEED_TILE) + (rem < k ? rem : k));
