@@ -134,3 +134,18 @@ def test_queued_queries_on_small_stores(gpu, n, k):
     for j in range(3):
         assert np.array_equal(ids[j][:c], rid) and np.array_equal(sc[j][:c], rsc)
         assert np.all(ids[j][c:] == np.uint64(0xFFFFFFFFFFFFFFFF)) and np.all(sc[j][c:] == -np.inf)
+
+
+@pytest.mark.parametrize("n,values", [((1 << 21) + 5, 1), (3_000_001, 2), (5_000_003, 7)])
+def test_tied_scores_take_one_run(gpu, n, values):
+    # every chunk of the sample holds more ties than the threshold's rank
+    rng = np.random.default_rng(values)
+    x = rng.integers(0, values, size=(2, n)).astype(np.float32)
+    w, k = np.array([0.5, 1.0], np.float32), 100
+    rid, rsc, _ = oracle.fte_topk(x, n, k, w, [0, 1])
+    with topk_amd.Engine(x) as eng:
+        ids, sc, _ = eng.fte(k, w, [0, 1])
+        assert np.array_equal(ids, rid) and np.array_equal(sc, rsc) and eng.stats()["fallback"] == 0
+        qi, qs = _queue(eng, [(w, [0, 1])] * 2, k)
+    for j in range(2):
+        assert np.array_equal(qi[j], rid) and np.array_equal(qs[j], rsc)
