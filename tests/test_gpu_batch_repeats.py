@@ -45,3 +45,15 @@ def test_large_partitions_keep_id_order(gpu, fused):
         k, w, attr = qs[0]
         ids, _, _ = eng.pta(256, w, attr)
         assert np.array_equal(ids, np.arange(256, dtype=np.uint64)) and eng.stats()["fallback"] == 0
+
+
+@pytest.mark.parametrize("nq", [1, 7, 8])
+def test_few_queries_over_a_larger_store(gpu, nq):
+    # the two passes' limit above 2^20 objects, over values that bounds rule out little of
+    n, d = (1 << 20) + 4097, 5
+    rng = np.random.default_rng(nq)
+    x = (rng.random((d, n)) * (rng.random((d, n)) < 0.02)).astype(np.float32)
+    qs = make_queries(rng, nq, d, [1, 64, 300])
+    with topk_amd.Engine(x) as eng:
+        check(eng, x, qs)
+        assert (eng.stats()["items"] == 0) == (nq >= 8)  # the query-major pass has no work items

@@ -2138,23 +2138,27 @@ static BatchVariant pick_variant(const topk_ctx *ctx, const BatchState &B, uint3
     v.grid = ctx->tune.batch_grid ? ctx->tune.batch_grid : B.cus * (v.bs == 256 ? 4 : 2);
     v.item = ctx->tune.batch_item ? ctx->tune.batch_item : 4096;
     // The query-major pass when neither it nor a work-item shape was asked
-    // for: no work list to build and no
-    // reuse of loaded objects, so it is ahead while queries x objects are
-    // few.  Measured limits, worst distribution (anticorrelated or
+    // for: no work list to build and no reuse of loaded objects, so it is
+    // ahead while queries x objects are few.  Measured limits, worst distribution (anticorrelated or
     // independent) and best (correlated), work items against query-major in
     // us, k <= 256:
     //   d <= 8:  2^28 pairs in at most 2^22 objects; 2^20 x 128: 518 / 479
     //            and 181 / 148, 2^18 x 1024: 643 / 702 and 369 / 351;
     //            2^22 x 512: 1250 / 1520 and 337 / 296;
     //            8 queries over 2^24 (one workgroup bounds a whole tree):
-    //            209 / 247
+    //            209 / 247; above 2^20 objects at least 8 queries: sparse values
+    //            (2% nonzero), whose bounds rule out little, 2^22, 1 query 271 /
+    //            447, 2 314 / 550, 4 429 / 716, 16 959 / 909 (independent, 1
+    //            query 116 / 104)
     //   d <= 16: 2^24 pairs in at most 2^18 objects; 2^18 x 32: 321 / 315
     //            and 160 / 126; 2^20 x 8: 297 / 337; 2^20 x 32: 491 / 586
     //            and 187 / 154
     const bool shaped = ctx->tune.batch_vpt || ctx->tune.batch_bs || ctx->tune.batch_qpi || ctx->tune.batch_grid ||
                         ctx->tune.batch_item || ctx->tune.batch_mask;
     const uint64_t most = D == 8 ? 1ull << 28 : (D == 16 ? 1ull << 24 : 0), most_n = D == 8 ? 1ull << 22 : 1ull << 18;
-    v.fused = ctx->tune.batch_fused ? ctx->tune.batch_fused == 2 : !shaped && ctx->n <= most_n && ctx->n * nq <= most;
+    v.fused = ctx->tune.batch_fused ? ctx->tune.batch_fused == 2
+                                    : !shaped && ctx->n <= most_n && ctx->n * nq <= most &&
+                                          (nq >= 8 || ctx->n <= 1ull << 20);
     return v;
 }
 
